@@ -260,14 +260,34 @@ __global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(2))) 
     }
 }
 
-#ifndef VX_FRIC_ROWS
-#define VX_FRIC_ROWS 24  // rows per block of the walk kernel
-#endif
+// Rows per block of the walk kernel. A block walks `rows` rows of two face
+// solves each and one extra row of u faces, and two blocks fit a CU (one from
+// 14 levels per lane on, by their LDS), so a launch of n blocks takes about ceil(n / slots) passes of 2 * rows + 1 solves;
+// the row count with the cheapest product is taken (at most 24: longer chunks
+// leave the last pass emptier than the row they save). With 24 rows whatever
+// the grid, 360x160x60 (levels innermost) launched 96 blocks for 256 CUs: 459 us,
+// 163 us with the 5 rows (438 blocks) chosen here; 1440x720x80: 2.01 -> 1.94 ms
+// with 23.
+int fric_rows(int64_t nrows, int64_t nstrips, int blocks_per_cu) {
+    const int64_t slots = (int64_t)blocks_per_cu * cu_count();
+    int best = 1;
+    int64_t best_cost = INT64_MAX;
+    for (int rows = 1; rows <= 24; ++rows) {
+        const int64_t nblocks = nstrips * ((nrows + rows - 1) / rows);
+        const int64_t cost = (nblocks + slots - 1) / slots * (2 * rows + 1);
+        if (cost <= best_cost) {
+            best_cost = cost;
+            best = rows;
+        }
+    }
+    return best;
+}
 
 template <int S>
 void launch_fric_walk(const FricArgs& p, bool vec, bool pv, hipStream_t s) {
-    const int rows = VX_FRIC_ROWS;
-    const int64_t nstrips = (p.Y - 3 + 30) / 31, nchunks = (p.X - 3 + rows - 1) / rows;
+    const int64_t nstrips = (p.Y - 3 + 30) / 31;
+    const int rows = fric_rows(p.X - 3, nstrips, S >= 14 ? 1 : 2);
+    const int64_t nchunks = (p.X - 3 + rows - 1) / rows;
     const int64_t nblocks = nstrips * nchunks;
     const dim3 grid((unsigned)((nblocks + 7) / 8 * 8));
     if (vec)

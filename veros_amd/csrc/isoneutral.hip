@@ -1620,21 +1620,6 @@ int join_aux(hipStream_t s, hipStream_t sd, const char* who) {
     return VX_OK;
 }
 
-// Compute units of the current device (0 if it cannot be queried), cached
-// per device.
-int device_cu_count() {
-    static std::mutex m;
-    static std::map<int, int> per_device;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    std::lock_guard<std::mutex> lk(m);
-    auto it = per_device.find(dev);
-    if (it != per_device.end()) return it->second;
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-    return per_device[dev] = n;
-}
-
 #ifndef VX_PRE_CELLS
 #define VX_PRE_CELLS 3840
 #endif
@@ -1718,8 +1703,7 @@ int launch_wet_plan(const Grid& g, const WetPlan& wp, hipStream_t s, const char*
 template <int NTR, bool IMPLICIT, bool WETFLUX>
 int launch_wet_step(const Grid& g, const Prm& p, const StepArgs& a, const WetPlan& wp, hipStream_t s,
                     const char* who) {
-    const int ncu = device_cu_count();
-    const unsigned nblk = (unsigned)(((ncu > 0 ? ncu : 256) * VX_WET_BPC + 7) / 8 * 8);
+    const unsigned nblk = (unsigned)((cu_count() * VX_WET_BPC + 7) / 8 * 8);
     const size_t lds = (size_t)(3 + kStepArrays * NTR) * kWetThreads * sizeof(double) +
                        (2 * kWetThreads + 1) * sizeof(int);
     hipLaunchKernelGGL((iso_step_wet_kernel<NTR, IMPLICIT, WETFLUX>), dim3(nblk), dim3(kWetThreads), lds, s, g, p, a,
@@ -1795,7 +1779,7 @@ int launch_pre(const Grid& g, const Prm& p, const Fields& f, const double* K_iso
     // (on the caller's stream, without the helper, the fill runs before pre:
     // the whole grid of it)
     const unsigned eighths = (dry_stream && use_aux) ? VX_DRY_EIGHTHS_FUSED : VX_DRY_EIGHTHS_PRE;
-    const unsigned dry_full = blocks_for(ncol, 4), ndry = eighths * (unsigned)device_cu_count() / 8;
+    const unsigned dry_full = blocks_for(ncol, 4), ndry = eighths * (unsigned)cu_count() / 8;
     const unsigned dry_grid = ndry > 0 && ndry < dry_full ? ndry : dry_full;
     hipLaunchKernelGGL(iso_pre_dry_kernel, dim3(dry_grid), dim3(256), 0, sd, g, Ai_ez, Ai_nz, Ai_bx, Ai_by,
                        K_11, K_22, K_33);

@@ -38,6 +38,10 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 constexpr int kMaxNz = 128;
 
+// Compute units of the current device (256 if it cannot be queried), cached
+// per device.
+int cu_count();
+
 // Blocks are dispatched round-robin over the 8 XCDs, each with its own L2.
 // With gridDim.x a multiple of 8 this gives block b the index of the
 // (b / 8)-th block of the x-th eighth of the grid (x = b % 8), so that each
