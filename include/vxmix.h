@@ -360,6 +360,14 @@ int vx_enforce_boundaries_f64(void* stream, double* arr, int64_t X, int64_t row_
                               int64_t elem_stride, int32_t enable_cyclic_x);
 
 /*
+ * kbot of ncol columns from the edge mask that create_water_masks builds
+ * (veros/core/utilities.py:38-48): edge_mask holds ncol * nz bytes (bool), a
+ * column's nz levels contiguous; kbot[c] = 1 + the first level with a nonzero
+ * byte, 0 where a column has none.
+ */
+int vx_kbot_from_edge_mask(void* stream, const void* edge_mask, int64_t ncol, int32_t nz, int32_t* kbot);
+
+/*
  * isoneutral_diag_streamfunction_kernel (veros/core/isoneutral/isoneutral.py:232-255):
  * B2_gm[1:-2, 2:-2] = 0.25 * diffloc_e * sum(Ai_ez) and
  * B1_gm[2:-2, 1:-2] = -0.25 * diffloc_n * sum(Ai_nz), diffloc the 4-point

@@ -34,6 +34,14 @@ def create_water_masks(ks, nz):
 def kbot_from_masks(water_mask, edge_mask):
     """kbot = (index of the edge cell) + 1, 0 where a column has no edge."""
     edge, _ = to_device(edge_mask)
+    if (edge.dtype == torch.bool and edge.dim() == 3 and edge.numel() > 0
+            and edge.device.index == torch.cuda.current_device()):
+        edge = edge.contiguous()
+        nx, ny, nz = edge.shape
+        kbot = torch.empty((nx, ny), dtype=torch.int32, device=edge.device)
+        _native.check(_native.lib().vx_kbot_from_edge_mask(stream_handle(), ptr(edge), nx * ny, nz, ptr(kbot)),
+                      "kbot_from_masks")
+        return kbot
     e = edge.to(torch.uint8)
     has = e.amax(dim=-1) > 0
     first = torch.argmax(e, dim=-1)
