@@ -1,0 +1,96 @@
+"""The column-tile kernels at the edges of their tiles: depths around the
+multiples of 16 levels that change the levels per lane, column counts that
+leave the last tile short (9 x 6 interior columns: 130 = 32 * 4 + 2), and
+arrays that start 8 bytes off a 16-byte boundary.
+
+TKE and EKE against the oracle at 1e-12. IDEMIX's rows carry entries of 1e7
+around a row sum of about 1, so two correct eliminations differ by an amount
+that only the system's conditioning sets; its solve is held to its backward
+error instead: |d - A x| <= 1e-13 (|A| |x| + |d|) row by row (about 450 eps; an
+elimination without pivoting of a diagonally dominant row and the rows'
+own roundings stay well below), and its lateral term and diagnostic, which are
+well conditioned, to 1e-12 on their own."""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_turbulence as TT
+from conftest import rel_err
+from oracle import turbulence as OT
+
+pytestmark = pytest.mark.gpu
+DEPTHS = [3, 16, 17, 32, 33, 49, 65, 96, 97, 113, 127]
+
+
+def shift_arrays(ds):
+    """The state's float arrays re-stored 8 bytes off their allocation's start (strides kept)."""
+    vs = ds.variables
+    for k, v in vars(vs).items():
+        if isinstance(v, torch.Tensor) and v.dtype == torch.float64 and v.dim() >= 3:
+            buf = torch.empty(v.numel() + 1, dtype=v.dtype, device=v.device)
+            w = buf[1:].as_strided(v.shape, v.stride(), 1)
+            w.copy_(v)
+            setattr(vs, k, w)
+    return ds
+
+
+def _state(nz, **kw):
+    from veros_amd.workloads import masks_from_kbot
+    st = TT._state(nz, 9, 6, nz, enable_eke=True, enable_tke_hor_diffusion=True, **kw)
+    st.variables.kbot[5, 3] = nz  # a column of one wet level (rows 4 to X-5 have no halo copy)
+    st.variables.kbot[6, 4] = 1
+    for k, m in masks_from_kbot(st.variables.kbot, nz).items():
+        setattr(st.variables, k, m)
+    return st
+
+
+def _run(model, st, levels, shift, monkeypatch):
+    import veros_amd.state as S
+    with monkeypatch.context() as m:
+        if shift:
+            inner = S.to_device_state
+            m.setattr(S, "to_device_state", lambda *a, **k: shift_arrays(inner(*a, **k)))
+        return TT._gpu(model, st, levels)
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+@pytest.mark.parametrize("model,levels,shift", [("tke", "inner", False), ("eke", "outer", True)])
+def test_turbulence_depths(model, nz, levels, shift, monkeypatch):
+    st = _state(nz)
+    ref = TT.ORACLE[model](st)
+    out = _run(model, st, levels, shift, monkeypatch)
+    for k, r in ref._asdict().items():
+        assert rel_err(out[k], r) <= 1e-12, k
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+@pytest.mark.parametrize("levels,shift", [("outer", False), ("inner", True)])
+def test_idemix_depths(nz, levels, shift, monkeypatch):
+    kw = dict(enable_eke_diss_surfbot=nz % 2 == 0, eke_diss_surfbot_frac=0.3)
+    st = _state(nz, **kw)
+    rows = {}
+
+    def capture(a, b, c, d, water, edge, b_edge=None, d_edge=None, solver=None):
+        rows.update(a=np.where(edge, 0.0, a), b=np.where(edge, b_edge, b), c=c, d=np.where(edge, d_edge, d), water=water)
+        return np.zeros_like(a)
+
+    with monkeypatch.context() as m:
+        m.setattr(OT, "solve_implicit", capture)
+        OT.integrate_idemix_kernel(st)
+    t1 = st.variables.taup1
+    plain = _run("idemix", st, levels, shift, monkeypatch)
+    x = plain["E_iw"][2:-2, 2:-2, :, t1]
+    up, dn = np.zeros_like(x), np.zeros_like(x)
+    up[..., :-1], dn[..., 1:] = x[..., 1:], x[..., :-1]
+    up[..., -1] = 0.0
+    dn = np.where(rows["a"] == 0.0, 0.0, dn)
+    terms = [rows["d"], -rows["a"] * dn, -rows["b"] * x, -np.where(rows["water"], rows["c"], 0.0) * up]
+    res, scale = sum(terms), sum(np.abs(t) for t in terms)
+    assert np.all(np.abs(res)[rows["water"]] <= 1e-13 * scale[rows["water"]])
+    E0 = st.variables.E_iw[..., st.variables.tau]
+    assert rel_err(plain["iw_diss"], st.variables.alpha_c * np.maximum(0.0, E0) * plain["E_iw"][..., t1]) <= 1e-14
+    off = TT.ORACLE["idemix"](st).E_iw
+    st.settings.enable_idemix_hor_diffusion = True
+    lat = TT.ORACLE["idemix"](st).E_iw - off
+    got = _run("idemix", st, levels, shift, monkeypatch)["E_iw"] - plain["E_iw"]
+    assert np.max(np.abs(got - lat)) <= 1e-12 * np.max(np.abs(off))

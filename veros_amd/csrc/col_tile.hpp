@@ -1,0 +1,259 @@
+// Column tiles: a wave owns kTileC consecutive (i, j) columns of an (X, Y, nz)
+// grid, which are one contiguous run of kTileC * nz cells, and sees them in
+// two layouts.
+//
+//   flat:     element t of lane l is cell 64 t + l of the run. Every global
+//             access is made here: consecutive lanes touch consecutive cells
+//             whatever nz's parity, the arrays' alignment or the storage of the
+//             time levels (levels innermost: every third double). Loads and
+//             stores are raw buffer accesses whose descriptor spans the run; a
+//             lane that must not take part gets an offset past its end, which
+//             the hardware turns into 0 (a dropped store) without traffic and
+//             without a branch, so all loads of a phase are in flight together.
+//   segments: lane s of a column's kTileP lanes holds levels [s S, s S + S),
+//             the layout of the segmented tridiagonal solve.
+//
+// Values pass between the layouts through an LDS image of the run (odd
+// segment stride, so that the segments' starts spread over the banks).
+// Everything elementwise (forcing sums, right-hand sides, diagnostics, lateral
+// fluxes) is done flat, only the rows' neighbours and the solve need
+// segments. With 16 lanes per column a lane holds nz/16 values per array, half
+// of what 8 lanes need, which leaves registers for twice the waves.
+#pragma once
+#include "tdma_seg.hpp"
+
+namespace vx {
+
+constexpr int kTileP = 16;           // lanes per column: one DPP row
+constexpr int kTileC = 64 / kTileP;  // columns per wave
+
+// levels per lane for a depth nz (>= 2)
+__host__ __device__ constexpr int tile_levels(int nz) {
+    const int s = (nz + kTileP - 1) / kTileP;
+    return s < 2 ? 2 : s;
+}
+
+// An offset past the end of every buffer, also when scaled by 3.
+constexpr uint32_t kNoAccess = 0x20000000u;
+
+typedef __amdgpu_buffer_rsrc_t BufRsrc;
+// A buffer of `bytes` bytes at the wave-uniform address p; accesses past its
+// end read 0 or are dropped.
+__device__ __forceinline__ BufRsrc make_buf(const double* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, bytes, 0x00027000);
+}
+typedef unsigned int vx_u2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ double buf_load(BufRsrc b, uint32_t off) {
+    const vx_u2 v = __builtin_amdgcn_raw_buffer_load_b64(b, off, 0, 0);
+    return __builtin_bit_cast(double, v);
+}
+__device__ __forceinline__ void buf_store(BufRsrc b, uint32_t off, double v) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(vx_u2, v), b, off, 0, 0);
+}
+
+template <int S>
+struct Tile {
+    static constexpr int SP = S | 1;              // segment stride in an image
+    static constexpr int CS = kTileP * SP;        // column stride
+    static constexpr int DUMMY = kTileC * CS;     // slot of the lanes past the run
+    static constexpr int IMG = kTileC * CS + 2;   // doubles of an image
+    int lane, s, q;       // lane of the wave; segment and column (segments)
+    int lo;               // first level of the segment
+    int seg;              // the segment's position in an image
+    int k[S], c[S];       // level and column of the flat elements
+    int pos[S];           // their positions in an image
+    uint32_t off[S];      // their byte offsets in an (X, Y, nz) array's run
+    uint32_t bytes;       // bytes of that run
+    int64_t col0, cell0;  // first column and cell of the run
+    int ncol;             // columns of the run (< kTileC in the last tile)
+};
+
+// Tile `w` (wave-uniform) of a grid of `cols` columns.
+template <int S>
+__device__ __forceinline__ Tile<S> make_tile(int64_t w, int64_t cols, int nz) {
+    Tile<S> t;
+    t.lane = (int)(threadIdx.x & 63);
+    t.s = t.lane % kTileP;
+    t.q = t.lane / kTileP;
+    t.lo = t.s * S;
+    t.seg = t.q * Tile<S>::CS + t.s * Tile<S>::SP;
+    const int64_t left = cols - w * kTileC;
+    t.ncol = left < kTileC ? (left < 0 ? 0 : (int)left) : kTileC;
+    t.col0 = t.ncol > 0 ? w * kTileC : 0;  // a tile past the grid: no columns, addresses of the first
+    t.cell0 = t.col0 * nz;
+    t.bytes = (uint32_t)(t.ncol * nz) * 8u;
+    // e / nz for e < 512 + 64, nz <= 128, by a 20-bit reciprocal (exact)
+    const uint32_t m = ((1u << 20) + (uint32_t)nz - 1u) / (uint32_t)nz;
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        const uint32_t e = 64u * r + (uint32_t)t.lane;
+        const uint32_t c = (e * m) >> 20;
+        const bool in = (int)e < t.ncol * nz;
+        t.k[r] = (int)(e - c * (uint32_t)nz);
+        t.c[r] = in ? (int)c : 0;
+        t.pos[r] = (int)c < kTileC ? (int)c * Tile<S>::CS + t.k[r] + t.k[r] / S * (Tile<S>::SP - S) : Tile<S>::DUMMY;
+        t.off[r] = in ? e * 8u : kNoAccess;
+    }
+    return t;
+}
+
+// The run of a (X, Y, nz) array, `d` cells further on, cs doubles per cell.
+template <int S>
+__device__ __forceinline__ BufRsrc tile_buf(const Tile<S>& t, const double* a, int64_t d = 0, int cs = 1) {
+    return make_buf(a + (t.cell0 + d) * cs, t.bytes * (uint32_t)cs);
+}
+
+// flat elements where on[r] (0 elsewhere)
+template <int S>
+__device__ __forceinline__ void tile_load(BufRsrc b, const uint32_t (&off)[S], uint32_t cs, double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) v[r] = buf_load(b, off[r] * cs);
+}
+template <int S>
+__device__ __forceinline__ void tile_store(BufRsrc b, const uint32_t (&off)[S], uint32_t cs, const double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) buf_store(b, off[r] * cs, v[r]);
+}
+// flat <-> image
+template <int S>
+__device__ __forceinline__ void tile_put(const Tile<S>& t, double* img, const double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) img[t.pos[r]] = v[r];
+}
+template <int S>
+__device__ __forceinline__ void tile_get(const Tile<S>& t, const double* img, double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) v[r] = img[t.pos[r]];
+}
+// segments <-> image
+template <int S>
+__device__ __forceinline__ void seg_get(const Tile<S>& t, const double* img, double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) v[r] = img[t.seg + r];
+}
+template <int S>
+__device__ __forceinline__ void seg_put(const Tile<S>& t, double* img, const double (&v)[S]) {
+#pragma unroll
+    for (int r = 0; r < S; ++r) img[t.seg + r] = v[r];
+}
+// the value of the level below lo (lane s = 0: unspecified) and above lo + S - 1
+// (lane s = kTileP - 1: unspecified) in an image
+template <int S>
+__device__ __forceinline__ double seg_below(const Tile<S>& t, const double* img) {
+    return img[t.s > 0 ? t.seg - 1 - (Tile<S>::SP - S) : t.seg];
+}
+template <int S>
+__device__ __forceinline__ double seg_above(const Tile<S>& t, const double* img) {
+    return img[t.s < kTileP - 1 ? t.seg + Tile<S>::SP : t.seg];
+}
+
+// ---------------------------------------------------------------------------
+// The segmented solve of tdma_seg.hpp with kTileP lanes per column: the
+// interface system has kTileP rows and its cyclic reduction one more stride.
+// A DPP row holds exactly one column, so a move past the column's end reads 0.
+// ---------------------------------------------------------------------------
+template <int D, int NR>
+__device__ __forceinline__ void tile_pcr_step(int s, double& A, double& B, double& C, double (&R)[NR], double& al,
+                                              double& ga) {
+    double Bm = dpp_move<kDppShr + D>(B), Bp = dpp_move<kDppShl + D>(B);  // every lane moves
+    Bm = s < D ? 1.0 : Bm;
+    Bp = s + D >= kTileP ? 1.0 : Bp;
+    const double Am = dpp_move<kDppShr + D>(A), Cm = dpp_move<kDppShr + D>(C);
+    const double Ap = dpp_move<kDppShl + D>(A), Cp = dpp_move<kDppShl + D>(C);
+    al = -A * seg_rcp(Bm);
+    ga = -C * seg_rcp(Bp);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        const double Rm = dpp_move<kDppShr + D>(R[q]), Rp = dpp_move<kDppShl + D>(R[q]);
+        R[q] = R[q] + al * Rm + ga * Rp;
+    }
+    A = al * Am;
+    C = ga * Cp;
+    B = B + al * Cm + ga * Ap;
+}
+template <int D>
+__device__ __forceinline__ double tile_rhs_step(double R, double al, double ga) {
+    return R + al * dpp_move<kDppShr + D>(R) + ga * dpp_move<kDppShl + D>(R);
+}
+
+// The interface system with NR right-hand sides; in columns with a row that is
+// not strongly diagonally dominant one step of iterative refinement follows,
+// as in iface_solve.
+template <int NR>
+__device__ __forceinline__ void tile_iface(int s, double A, double B, double C, const double (&R)[NR],
+                                           double (&Ls)[NR], double (&Lm)[NR]) {
+    double a = A, b = B, c = C, al[4], ga[4];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) Ls[q] = R[q];
+    tile_pcr_step<1, NR>(s, a, b, c, Ls, al[0], ga[0]);
+    tile_pcr_step<2, NR>(s, a, b, c, Ls, al[1], ga[1]);
+    tile_pcr_step<4, NR>(s, a, b, c, Ls, al[2], ga[2]);
+    tile_pcr_step<8, NR>(s, a, b, c, Ls, al[3], ga[3]);
+    const double rb = seg_rcp(b);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) Ls[q] *= rb;
+    const unsigned long long weak = __ballot(fabs(A) + fabs(C) > 0.25 * fabs(B));
+    if (weak != 0) {
+        const bool gw = ((weak >> (threadIdx.x & 48)) & 0xffffull) != 0;  // this column has such a row
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            double r = R[q] - (A * dpp_move<kDppShr + 1>(Ls[q]) + B * Ls[q] + C * dpp_move<kDppShl + 1>(Ls[q]));
+            r = tile_rhs_step<1>(r, al[0], ga[0]);
+            r = tile_rhs_step<2>(r, al[1], ga[1]);
+            r = tile_rhs_step<4>(r, al[2], ga[2]);
+            r = tile_rhs_step<8>(r, al[3], ga[3]);
+            Ls[q] = gw ? Ls[q] + r * rb : Ls[q];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) Lm[q] = dpp_move<kDppShr + 1>(Ls[q]);
+}
+
+// NR right-hand sides of one matrix; z in, their solutions out. va and vc are
+// overwritten by the sweep's factors (see seg_solve_f64).
+template <int S, int NR>
+__device__ __forceinline__ void tile_solve(const Tile<S>& t, double (&va)[S], const double (&vb)[S], double (&vc)[S],
+                                           double (&z)[NR][S]) {
+    const double aL = va[S - 1], bL = vb[S - 1], cL = vc[S - 1];
+    {
+        const double r = seg_rcp(vb[0]);
+        vc[0] *= r;
+        va[0] *= r;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) z[q][0] *= r;
+    }
+#pragma unroll
+    for (int i = 1; i < S - 1; ++i) {
+        const double at = va[i];
+        const double r = seg_rcp(vb[i] - at * vc[i - 1]);
+        vc[i] *= r;
+        va[i] = -at * va[i - 1] * r;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) z[q][i] = (z[q][i] - at * z[q][i - 1]) * r;
+    }
+    va[S - 2] = -va[S - 2];
+    vc[S - 2] = -vc[S - 2];
+#pragma unroll
+    for (int i = S - 3; i >= 0; --i) {
+        const double cp = vc[i];
+#pragma unroll
+        for (int q = 0; q < NR; ++q) z[q][i] = z[q][i] - cp * z[q][i + 1];
+        va[i] = -va[i] - cp * va[i + 1];
+        vc[i] = -cp * vc[i + 1];
+    }
+    const double RA = aL * va[S - 2];
+    const double RB = bL + aL * vc[S - 2] + cL * dpp_move<kDppShl + 1>(va[0]);
+    const double RC = cL * dpp_move<kDppShl + 1>(vc[0]);
+    double RD[NR], Ls[NR], Lm[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) RD[q] = z[q][S - 1] - aL * z[q][S - 2] - cL * dpp_move<kDppShl + 1>(z[q][0]);
+    tile_iface<NR>(t.s, RA, RB, RC, RD, Ls, Lm);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+#pragma unroll
+        for (int i = 0; i < S - 1; ++i) z[q][i] = z[q][i] + va[i] * Lm[q] + vc[i] * Ls[q];
+        z[q][S - 1] = Ls[q];
+    }
+}
+
+}  // namespace vx

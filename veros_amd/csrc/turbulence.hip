@@ -3,19 +3,27 @@
 // integrate_eke_kernel (veros/core/eke.py:93-255) and integrate_idemix_kernel
 // (veros/core/idemix.py:47-265), without their advection branches.
 //
-// One kernel per model. A group of kSegP lanes owns one (i, j) column of the
-// whole (X, Y) grid and lane s holds levels [s*S, s*S + S) (tdma_seg.hpp):
-// each lane sums the forcing terms, forms its rows of the implicit system
-// (delta from the diffusivity at k and k+1, the dissipation on the diagonal,
-// the edge row at kbot-1, the surface flux in the top rhs) in registers,
-// the group solves the column by the segmented elimination, and each lane
-// then writes its levels: the new energy at taup1 on the wet levels of the
-// interior columns, the dissipation diagnostic over the whole array, the
-// lateral diffusion of the tau level added on top (its fluxes read the four
-// neighbouring columns), and for TKE the surface correction. Halo columns
-// only produce the diagnostics. Masks come from kbot (maskT = maskW = wet
-// suffix, maskU / maskV the products of the two adjacent maskT).
-#include "tdma_seg.hpp"
+// One kernel per model. A wave owns a tile of four columns of the whole (X, Y)
+// grid (col_tile.hpp): it loads its cells flat and coalesced, sums the forcing
+// terms and forms the right-hand side and the dissipation coefficient cell by
+// cell, passes those and the diffusivity through LDS to the segment layout,
+// where the rows of the implicit system are formed (delta from the diffusivity
+// at k and k+1, the edge row at kbot-1) and the columns solved, and takes the
+// solution back through LDS to store, cell by cell, the new energy at taup1 on
+// the wet levels of the interior columns, the dissipation diagnostic over the
+// whole array and the lateral diffusion of the tau level on top (its fluxes
+// read the four neighbouring columns, cells whose face is wet only). Halo
+// columns only produce the diagnostics. Masks come from kbot (maskT = maskW =
+// wet suffix, maskU / maskV the products of the two adjacent maskT).
+//
+// What bounds the three: the chain of memory round trips of a wave (kbot, the
+// arrays, the lateral neighbours), behind it HBM. The earlier kernels (8 lanes
+// per column, each lane loading its own levels, two waves per SIMD, a scalar
+// variant for odd nz or levels innermost) took, TKE + EKE + IDEMIX together,
+// 4.91 ms on 1440x720x80 (levels outermost), these 4.13; on 360x160x45 (odd,
+// levels innermost) 336 -> 189 us; 700x400x75, innermost, 2.55 -> 1.28 ms. Of
+// the 4.1 ms the lateral terms cost 1.1, the forcing terms 0.8, the solve 0.2.
+#include "col_tile.hpp"
 
 namespace vx {
 
@@ -38,191 +46,128 @@ struct Terms {
     int n;
 };
 
-__device__ __forceinline__ double sum_terms(const Terms& T, int64_t c) {
-    double f = 0.0;
-    for (int q = 0; q < T.n; ++q) f = q == 0 ? T.sgn[0] * T.p[0][c] : f + T.sgn[q] * T.p[q][c];
-    return f;
-}
-
-__device__ __forceinline__ bool wet_at(int kb, int k) { return kb > 0 && k >= kb - 1; }
-
-// The column of a lane group, over the whole (X, Y) grid.
-struct TurbCol {
-    int i, j, s, lo;
-    int64_t col;    // i * Y + j
-    bool valid;     // inside the grid
-    bool interior;  // 2 <= i < X-2, 2 <= j < Y-2
-    int kb;         // kbot
-    int k0;         // first solved level (nz: none)
+// The lateral faces of a tile's columns: east, west, north, south.
+struct TurbCols {
+    double w[kTileC][4];  // weights
+    int face[kTileC][4];  // first level at which the face is wet (nz: none)
 };
 
-__device__ __forceinline__ TurbCol turb_col(const TurbGrid& g, int S) {
-    TurbCol t;
-    const int64_t gt = xcd_contiguous_block() * kTurbBlock + threadIdx.x;
-    const int64_t col = gt / kSegP;
-    t.s = (int)(gt % kSegP);
-    t.lo = t.s * S;
-    t.valid = col < (int64_t)g.X * g.Y;
-    t.col = t.valid ? col : 0;
-    t.i = (int)(t.col / g.Y);
-    t.j = (int)(t.col - (int64_t)t.i * g.Y);
-    t.interior = t.valid && t.i >= 2 && t.i < g.X - 2 && t.j >= 2 && t.j < g.Y - 2;
-    t.kb = t.valid ? g.kbot[t.col] : 0;
-    t.k0 = (t.interior && t.kb >= 1 && t.kb <= g.nz) ? t.kb - 1 : g.nz;
-    return t;
+// Level tables of a block: dd[k] = the diffusivity's factor in delta at level k
+// (0 on the top level), rz[k] = 1 / dzw (1 / (0.5 dzw) on the top level).
+struct TurbLevels {
+    double dd[kMaxNz], rz[kMaxNz], zw[kMaxNz];
+};
+
+__device__ __forceinline__ int first_wet_of(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
+
+// The lane's group column (segments): what the masks need, known before the
+// first load is issued.
+struct TurbLane {
+    int i, j;
+    bool interior;
+    int kw, k0;  // first wet and first solved level (nz: none)
+};
+template <int S>
+__device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S>& t) {
+    TurbLane l;
+    const bool valid = t.q < t.ncol;
+    const int64_t col = t.col0 + (valid ? t.q : 0);
+    const int kb = t.ncol > 0 ? g.kbot[col] : 0;
+    l.i = (int)(col / g.Y);
+    l.j = (int)(col - (int64_t)l.i * g.Y);
+    l.interior = valid && l.i >= 2 && l.i < g.X - 2 && l.j >= 2 && l.j < g.Y - 2;
+    l.kw = valid ? first_wet_of(kb, g.nz) : g.nz;
+    l.k0 = l.interior ? l.kw : g.nz;
+    return l;
 }
 
-// Lateral diffusion of the tau level at (i, j, k) of an interior column
-// (veros/core/tke.py:250-276; eke.py:168-200; idemix.py:186-218):
-//   fe(i) = ce(i) * (F(i+1) - F(i)) / (cost dxu(i)) * maskU(i)
-//   fn(j) = cn(j) * (F(j+1) - F(j)) / dyu(j) * maskV(j) * cosu(j)
-//   div   = (fe(i) - fe(i-1)) / (cost dxt) + (fn(j) - fn(j-1)) / (cost dyt)
-// F(ii, jj) and the coefficients come from functors of the cell offset.
-template <class FV, class CE, class CN>
-__device__ __forceinline__ double lateral_div(const TurbGrid& g, int i, int j, int k, FV F, CE ce, CN cn) {
-    const int64_t Y = g.Y, nz = g.nz;
-    const int64_t c = ((int64_t)i * Y + j) * nz + k;
-    const int64_t cE = c + Y * nz, cW = c - Y * nz, cN = c + nz, cS = c - nz;
-    const bool mC = wet_at(g.kbot[(int64_t)i * Y + j], k);
-    const bool mE = wet_at(g.kbot[(int64_t)(i + 1) * Y + j], k), mW = wet_at(g.kbot[(int64_t)(i - 1) * Y + j], k);
-    const bool mN = wet_at(g.kbot[(int64_t)i * Y + j + 1], k), mS = wet_at(g.kbot[(int64_t)i * Y + j - 1], k);
-    const double cost = g.cost[j];
-    const double Fc = F(c), Fe = F(cE), Fw = F(cW), Fn = F(cN), Fs = F(cS);
-    const double fe = ce(c, cE) * (Fe - Fc) / (cost * g.dxu[i]) * ((mC && mE) ? 1.0 : 0.0);
-    const double fw = ce(cW, c) * (Fc - Fw) / (cost * g.dxu[i - 1]) * ((mW && mC) ? 1.0 : 0.0);
-    const double fn = cn(c, cN) * (Fn - Fc) / g.dyu[j] * ((mC && mN) ? 1.0 : 0.0) * g.cosu[j];
-    const double fs = cn(cS, c) * (Fc - Fs) / g.dyu[j - 1] * ((mS && mC) ? 1.0 : 0.0) * g.cosu[j - 1];
-    return (fe - fw) / (cost * g.dxt[i]) + (fn - fs) / (cost * g.dyt[j]);
-}
-
-__device__ __forceinline__ double2 ld2(const double* __restrict__ p) { return *reinterpret_cast<const double2*>(p); }
-
-// lateral_div at the levels k and k+1 together: F2 and the coefficient
-// functors return the two levels' values from 16-byte loads (levels
-// outermost, k even), the arithmetic of each level that of lateral_div.
-template <class FV2, class CE2, class CN2>
-__device__ __forceinline__ double2 lateral_div_pair(const TurbGrid& g, int i, int j, int k, FV2 F, CE2 ce, CN2 cn) {
-    const int64_t Y = g.Y, nz = g.nz;
-    const int64_t c = ((int64_t)i * Y + j) * nz + k;
-    const int64_t cE = c + Y * nz, cW = c - Y * nz, cN = c + nz, cS = c - nz;
-    const int kC = g.kbot[(int64_t)i * Y + j], kE = g.kbot[(int64_t)(i + 1) * Y + j];
-    const int kW = g.kbot[(int64_t)(i - 1) * Y + j], kN = g.kbot[(int64_t)i * Y + j + 1];
-    const int kS = g.kbot[(int64_t)i * Y + j - 1];
-    const double cost = g.cost[j], dxu = g.dxu[i], dxuw = g.dxu[i - 1], dyu = g.dyu[j], dyus = g.dyu[j - 1];
-    const double cosu = g.cosu[j], cosus = g.cosu[j - 1], dxt = g.dxt[i], dyt = g.dyt[j];
-    const double2 Fc = F(c), Fe = F(cE), Fw = F(cW), Fn = F(cN), Fs = F(cS);
-    const double2 ceE = ce(c, cE), ceW = ce(cW, c), cnN = cn(c, cN), cnS = cn(cS, c);
-    double r[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int kk = k + h;
-        const bool mC = wet_at(kC, kk), mE = wet_at(kE, kk), mW = wet_at(kW, kk);
-        const bool mN = wet_at(kN, kk), mS = wet_at(kS, kk);
-        const double fc = h ? Fc.y : Fc.x, fe_ = h ? Fe.y : Fe.x, fw_ = h ? Fw.y : Fw.x;
-        const double fn_ = h ? Fn.y : Fn.x, fs_ = h ? Fs.y : Fs.x;
-        const double fe = (h ? ceE.y : ceE.x) * (fe_ - fc) / (cost * dxu) * ((mC && mE) ? 1.0 : 0.0);
-        const double fw = (h ? ceW.y : ceW.x) * (fc - fw_) / (cost * dxuw) * ((mW && mC) ? 1.0 : 0.0);
-        const double fn = (h ? cnN.y : cnN.x) * (fn_ - fc) / dyu * ((mC && mN) ? 1.0 : 0.0) * cosu;
-        const double fs = (h ? cnS.y : cnS.x) * (fc - fs_) / dyus * ((mS && mC) ? 1.0 : 0.0) * cosus;
-        r[h] = (fe - fw) / (cost * dxt) + (fn - fs) / (cost * dyt);
+// Fills the block's level tables (scale = dt * coefficient) and the wave's
+// columns; every thread of the block calls it, after it has issued its first
+// loads (whose latency the divisions here hide). `lateral`: the weights times
+// `lw` and the faces are wanted.
+template <int S>
+__device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S>& t, const TurbLane& l, double scale,
+                                           double lw, bool lateral, TurbLevels& lv, TurbCols& tc) {
+    const int nz = g.nz;
+    for (int k = threadIdx.x; k < nz; k += kTurbBlock) {
+        const double dzw = g.dzw[k];
+        lv.zw[k] = dzw;
+        lv.rz[k] = 1.0 / (k == nz - 1 ? 0.5 * dzw : dzw);
+        lv.dd[k] = k < nz - 1 ? scale / g.dzt[k + 1] * 0.5 : 0.0;
     }
-    return make_double2(r[0], r[1]);
-}
-
-// The lateral term of the lane's levels where need(k) (0 elsewhere): per
-// level with lateral_div, or with VEC per level pair with lateral_div_pair.
-template <int S, bool VEC, class NEED, class L1, class L2>
-__device__ __forceinline__ void lateral_levels(int lo, NEED need, L1 one, L2 pair, double (&lat)[S]) {
-#pragma unroll
-    for (int t = 0; t < S; ++t) lat[t] = 0.0;
-    if constexpr (VEC) {
-#pragma unroll
-        for (int t = 0; t < S; t += 2) {
-            const int k = lo + t;
-            if (need(k) || need(k + 1)) {
-                const double2 v = pair(k);
-                lat[t] = v.x;
-                lat[t + 1] = v.y;
-            }
+    if (lateral) {
+        // div = (fe - fw) / (cost dxt) + (fn - fs) / (cost dyt) with fe = ce (F(i+1) - F(i)) / (cost dxu),
+        // fn = cn (F(j+1) - F(j)) / dyu cosu: one factor per face; lane s < 4 of a column forms face s
+        // (east, west, north, south)
+        const bool on = l.interior && l.kw < nz;
+        const int ii = on ? l.i : 1, jj = on ? l.j : 1, f = t.s & 3;
+        const double cost = g.cost[jj];
+        const int io = f == 1 ? ii - 1 : ii, jo = f == 3 ? jj - 1 : jj;
+        const double den = f < 2 ? cost * g.dxt[ii] * (cost * g.dxu[io]) : cost * g.dyt[jj] * g.dyu[jo];
+        const double num = f < 2 ? lw : lw * g.cosu[jo];
+        const int64_t cc = (int64_t)ii * g.Y + jj;
+        const int kn = first_wet_of(g.kbot[cc + (f == 0 ? g.Y : (f == 1 ? -g.Y : (f == 2 ? 1 : -1)))], nz);
+        if (t.s < 4) {
+            tc.w[t.q][f] = num / den;
+            tc.face[t.q][f] = on ? (kn > l.kw ? kn : l.kw) : nz;
         }
-    } else {
-#pragma unroll
-        for (int t = 0; t < S; ++t) {
-            if (need(lo + t)) lat[t] = one(lo + t);
-        }
-    }
-}
-
-// dzt (s[0, nz)) and dzw (s[kMaxNz, kMaxNz + nz)) of the grid in LDS; every
-// thread of the block calls it. The row loops read the spacings of their
-// levels inside per-lane branches, where a global load is waited for at once:
-// from LDS that wait is short.
-__device__ __forceinline__ void stage_dz(const TurbGrid& g, double* s) {
-    for (int k = threadIdx.x; k < g.nz; k += kTurbBlock) {
-        s[k] = g.dzt[k];
-        s[kMaxNz + k] = g.dzw[k];
     }
     __syncthreads();
 }
 
-// levels lo-1 .. lo+S of a (X, Y, nz) array at column `base` (0 outside
-// [0, nz)), in two steps so that other loads can be issued between them:
-// load_halo_issue loads the lane's levels (VEC: its own, in pairs; otherwise
-// all S+2), and load_halo_finish takes lo-1 and lo+S from the lanes below
-// and above (VEC; every lane must call it).
-template <int S, bool VEC>
-__device__ __forceinline__ void load_halo_issue(const double* __restrict__ p, int64_t base, int lo, int nz,
-                                                double (&v)[S + 2]) {
-    if constexpr (VEC) {
-        double w[S];
+// Adds the lateral diffusion of the tau level (veros/core/tke.py:250-276;
+// eke.py:168-200; idemix.py:186-218) to v on the cells with a wet face:
+// sum over the faces of weight * coefficient * (F(neighbour) - F(cell)).
+// F and the coefficient come from the arrays A and B (one or two of them):
+// COMB(face values of the neighbour's A and B, the cell's a and b) returns
+// coefficient * difference. Two directions at a time, so that the loads of a
+// pair are in flight together and hold few registers.
+template <int S, bool TWO, class COMB>
+__device__ __forceinline__ void add_lateral(const TurbGrid& g, const Tile<S>& t, const TurbCols& tc, const double* A,
+                                            uint32_t csA, const double* B, const double (&a)[S],
+                                            const double (&b)[TWO ? S : 1], COMB comb, double (&v)[S]) {
+    const int64_t nz = g.nz, row = (int64_t)g.Y * nz;
+    const int64_t d[4] = {row, -row, nz, -nz};
 #pragma unroll
-        for (int t = 0; t < S; ++t) w[t] = 0.0;
-        col_load<S, true>(p + base, 1, lo, nz, [](int) { return true; }, w);
-        v[0] = v[S + 1] = 0.0;
+    for (int h = 0; h < 4; h += 2) {
+        double nA[2][S], nB[2][TWO ? S : 1];
 #pragma unroll
-        for (int t = 0; t < S; ++t) v[t + 1] = w[t];
-    } else {
+        for (int f = 0; f < 2; ++f) {
+            const BufRsrc ra = tile_buf(t, A, d[h + f], (int)csA);
+            const BufRsrc rb = tile_buf(t, TWO ? B : A, d[h + f]);
 #pragma unroll
-        for (int t = 0; t < S + 2; ++t) {
-            const int k = lo - 1 + t;
-            v[t] = (k >= 0 && k < nz) ? p[base + k] : 0.0;
+            for (int r = 0; r < S; ++r) {
+                const uint32_t o = t.k[r] >= tc.face[t.c[r]][h + f] ? t.off[r] : kNoAccess;
+                nA[f][r] = buf_load(ra, o * csA);
+                if constexpr (TWO) nB[f][r] = buf_load(rb, o);
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+#pragma unroll
+            for (int r = 0; r < S; ++r) {
+                const double x = tc.w[t.c[r]][h + f] * comb(nA[f][r], TWO ? nB[f][TWO ? r : 0] : 0.0, a[r], TWO ? b[TWO ? r : 0] : 0.0);
+                v[r] += t.k[r] >= tc.face[t.c[r]][h + f] ? x : 0.0;
+            }
         }
     }
-}
-template <int S, bool VEC>
-__device__ __forceinline__ void load_halo_finish(int s, double (&v)[S + 2]) {
-    if constexpr (VEC) {
-        v[0] = grp_prev(s, v[S]);
-        v[S + 1] = grp_next(s, v[1]);
-    }
-}
-
-// levels lo .. lo+S-1 (0 from nz on)
-template <int S, bool VEC>
-__device__ __forceinline__ void load_lv(const double* __restrict__ p, int64_t base, int lo, int nz, double (&v)[S]) {
-#pragma unroll
-    for (int t = 0; t < S; ++t) v[t] = 0.0;
-    col_load<S, VEC>(p + base, 1, lo, nz, [](int) { return true; }, v);
 }
 
 #ifndef VX_TERMS_GROUP
 #define VX_TERMS_GROUP 3
 #endif
-// f (levels lo .. lo+S-1) plus the sum of the forcing terms where want(k),
-// summed left to right as sum_terms; with `first` the sum replaces f. The
-// terms are loaded VX_TERMS_GROUP at a time, all loads of a group before its
-// first use, so a group costs one memory round trip instead of one per term.
-template <int S, bool VEC, class W>
-__device__ __forceinline__ void add_terms(const Terms& T, int64_t base, int lo, int nz, W want, bool first,
+// f plus the signed forcing terms on the cells of `off`, summed left to right;
+// with `first` the sum replaces f. VX_TERMS_GROUP terms are loaded at a time,
+// before the group's first use.
+template <int S>
+__device__ __forceinline__ void add_terms(const Terms& T, const Tile<S>& t, const uint32_t (&off)[S], bool first,
                                           double (&f)[S]) {
     constexpr int G = VX_TERMS_GROUP;
     for (int q0 = 0; q0 < T.n; q0 += G) {
         double v[G][S];
 #pragma unroll
         for (int r = 0; r < G; ++r) {
-#pragma unroll
-            for (int t = 0; t < S; ++t) v[r][t] = 0.0;
-            if (q0 + r < T.n) col_load<S, VEC>(T.p[q0 + r] + base, 1, lo, nz, want, v[r]);
+            if (q0 + r < T.n) tile_load(tile_buf(t, T.p[q0 + r]), off, 1, v[r]);
         }
 #pragma unroll
         for (int r = 0; r < G; ++r) {
@@ -230,20 +175,78 @@ __device__ __forceinline__ void add_terms(const Terms& T, int64_t base, int lo, 
                 const double sg = T.sgn[q0 + r];
                 const bool set = first && q0 + r == 0;
 #pragma unroll
-                for (int t = 0; t < S; ++t) f[t] = set ? sg * v[r][t] : f[t] + sg * v[r][t];
+                for (int x = 0; x < S; ++x) f[x] = set ? sg * v[r][x] : f[x] + sg * v[r][x];
             }
         }
     }
 }
 
-// sum of the forcing terms at levels lo .. lo+S-1 where want(k), summed
-// left to right as sum_terms (0 elsewhere)
-template <int S, bool VEC, class W>
-__device__ __forceinline__ void load_terms(const Terms& T, int64_t base, int lo, int nz, W want, double (&f)[S]) {
+// Forms and solves the group columns' systems: kap, diss (the diagonal's
+// dissipation) and rhs images in, the solution into the rhs image. MUL (IDEMIX):
+// the rows are scaled by kap at their own column's level,
+// a = -delta[k-1] kap[k-1], b = 1 + (delta[k] + delta[k-1]) kap[k], c = -delta[k] kap[k+1].
+template <int S, bool MUL>
+__device__ __forceinline__ void turb_solve(const Tile<S>& t, const TurbLevels& lv, int nz, int k0, const double* kap,
+                                           const double* diss, double* rhs) {
+    double km[S], va[S], vb[S], vc[S], z[1][S];
+    seg_get(t, kap, km);
+    seg_get(t, diss, vb);
+    seg_get(t, rhs, z[0]);
+    const double below = seg_below(t, kap), above = seg_above(t, kap);
+    const int kp = t.lo - 1;
+    double dm = kp >= k0 && kp < nz - 1 ? lv.dd[kp] * (below + km[0]) : 0.0;
 #pragma unroll
-    for (int t = 0; t < S; ++t) f[t] = 0.0;
-    add_terms<S, VEC>(T, base, lo, nz, want, true, f);
+    for (int r = 0; r < S; ++r) {
+        const int k = t.lo + r;
+        const bool wet = k >= k0 && k < nz;
+        const int kc = k < nz ? k : nz - 1;
+        const double kn = r < S - 1 ? km[r < S - 1 ? r + 1 : r] : above;
+        const double kb = r > 0 ? km[r > 0 ? r - 1 : 0] : below;
+        const double dk = wet && k < nz - 1 ? lv.dd[kc] * (km[r] + kn) : 0.0;
+        const bool edge = k == k0;
+        double A, B, C;
+        if constexpr (MUL) {
+            // entries of 1e7 around a row sum of about 1: formed in the
+            // reference's order (veros/core/idemix.py:134-153), since every
+            // other rounding of them moves the solution as much as another
+            // elimination order would
+            const double zw = lv.zw[kc];
+            if (k < nz - 1) {
+                A = -dm * kb / zw;
+                B = edge ? 1 + dk / zw * km[r] + vb[r] : 1 + dk * km[r] / zw + dm * km[r] / zw + vb[r];
+            } else {
+                A = -dm / (0.5 * zw) * kb;
+                B = edge ? 1 + vb[r] : 1 + dm / (0.5 * zw) * km[r] + vb[r];
+            }
+            C = -dk / zw * kn;
+        } else {
+            const double rz = lv.rz[kc];
+            A = -dm * rz;
+            B = 1 + (dk + (edge ? 0.0 : dm)) * rz + vb[r];
+            C = -dk * rz;
+        }
+        va[r] = wet && !edge ? A : 0.0;
+        vb[r] = wet ? B : 1.0;
+        vc[r] = wet && k < nz - 1 ? C : 0.0;
+        z[0][r] = wet ? z[0][r] : 0.0;
+        dm = dk;
+    }
+    tile_solve<S, 1>(t, va, vb, vc, z);
+    seg_put(t, rhs, z[0]);
 }
+
+// LDS of a block: three images per wave, the columns, the level tables.
+template <int S>
+struct TurbShared {
+    double img[kTurbBlock / 64][3][Tile<S>::IMG];
+    TurbCols cols[kTurbBlock / 64];
+    TurbLevels lv;
+};
+
+// Waves per SIMD: as many as the registers allow without spilling (5 levels
+// per lane at four waves: 24 to 44 bytes of scratch per lane, 4.61 ms for the
+// three on 1440x720x80 against 4.08 at three and 4.29 at two).
+#define VX_TURB_WAVES(S) ((S) < 5 ? 4 : ((S) <= 6 ? 3 : 2))
 
 // ---------------------------------------------------------------------------
 // TKE (veros/core/tke.py:123-321)
@@ -259,205 +262,86 @@ struct TkeArgs {
     int hor;
 };
 
-// VEC (all three kernels): levels outermost, nz even and every array
-// 16-byte aligned; the lanes then move their levels in 16-byte pairs. PV
-// (implied by VEC): nz even and the arrays without time levels aligned, which
-// then move in pairs whatever the layout of the energy's time levels.
-template <int S, bool VEC, bool PV>
-__global__ __launch_bounds__(kTurbBlock) void tke_kernel(TkeArgs a) {
+template <int S>
+__global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void tke_kernel(TkeArgs a) {
     const TurbGrid& g = a.g;
-    const TurbCol tc = turb_col(g, S);
-    __shared__ double sdz[2 * kMaxNz];
-    stage_dz(g, sdz);
-    const double* __restrict__ zt = sdz;           // dzt
-    const double* __restrict__ zw = sdz + kMaxNz;  // dzw
-    const int nz = g.nz, lo = tc.lo, k0 = tc.k0;
-    const int64_t base = tc.col * nz;
-    const double* __restrict__ E0 = a.tke + a.tau * g.ls;
-    double* __restrict__ E1 = a.tke + a.taup1 * g.ls;
-    // VEC: the lateral diffusion's east and west neighbour columns (and, for
-    // the wave's first and last groups, the south and north ones outside the
-    // wave) are copied into the wave's LDS now, asynchronously and without
-    // registers; the other north and south neighbours are the adjacent groups'
-    // own columns, taken from their registers after the solve. Lane l's pair
-    // of region r lands at lat_stage[wave][r][l], read back by lane l only.
-    constexpr int NP = S / 2;
-    __shared__ double lat_stage[VEC ? (kTurbBlock / 64) * 3 * NP * 128 : 1];
-    double* const stg = lat_stage + (VEC ? (threadIdx.x / 64) * 3 * NP * 128 : 0);
-    const int g8 = (int)((threadIdx.x & 63) / kSegP);  // group in the wave
-    const bool lat_on = a.hor && tc.interior;
-    int kE = 0, kW = 0, kX = 0;
-    double m_cost = 1.0, m_dxu = 1.0, m_dxuw = 1.0, m_dyu = 1.0, m_dyus = 1.0, m_cosu = 0.0, m_cosus = 0.0,
-           m_dxt = 1.0, m_dyt = 1.0;
-    if constexpr (VEC) {
-        if (a.hor) {
-            const int64_t Y = g.Y;
-            const int64_t dE = lat_on ? Y * nz : 0;
-            const int64_t dX = lat_on ? (g8 == 0 ? -(int64_t)nz : (g8 == kSegCols - 1 ? (int64_t)nz : 0)) : 0;
-            const double* pc = E0 + base;
-            // only the pairs that touch the column's wet suffix (the term is
-            // taken on wet levels only); the other lanes' slots are not read
-            const int kw = tc.kb >= 1 && tc.kb <= nz ? tc.kb - 1 : nz;
-#pragma unroll
-            for (int t = 0; t < S; t += 2) {
-                const int k = lo + t;
-                if (lat_on && k < nz && k + 1 >= kw) {
-                    __builtin_amdgcn_global_load_lds((const void*)(pc + dE + k),
-                                                     (lds_void_ptr)(stg + (0 * NP + t / 2) * 128), 16, 0, 0);
-                    __builtin_amdgcn_global_load_lds((const void*)(pc - dE + k),
-                                                     (lds_void_ptr)(stg + (1 * NP + t / 2) * 128), 16, 0, 0);
-                    __builtin_amdgcn_global_load_lds((const void*)(pc + dX + k),
-                                                     (lds_void_ptr)(stg + (2 * NP + t / 2) * 128), 16, 0, 0);
-                }
-            }
-            const int64_t cj = lat_on ? tc.col : (int64_t)Y + 1;  // column (1, 1) when unused
-            const int i = (int)(cj / Y), j = (int)(cj - (cj / Y) * Y);
-            kE = g.kbot[cj + Y], kW = g.kbot[cj - Y];
-            kX = g.kbot[cj + (g8 == 0 ? -1 : 1)];
-            m_cost = g.cost[j], m_dxu = g.dxu[i], m_dxuw = g.dxu[i - 1], m_dyu = g.dyu[j], m_dyus = g.dyu[j - 1];
-            m_cosu = g.cosu[j], m_cosus = g.cosu[j - 1], m_dxt = g.dxt[i], m_dyt = g.dyt[j];
-        }
-    }
-    double km[S + 2];
-    load_halo_issue<S, PV>(a.kappaM, base, lo, nz, km);
-    double sq[S], ml[S];
-    load_lv<S, PV>(a.sqrttke, base, lo, nz, sq);
-    load_lv<S, PV>(a.mxl, base, lo, nz, ml);
-    // tau on the wet levels, taup1 on the others (kept there and read by the
-    // diagnostic); VEC with lateral diffusion: tau on every column's wet
-    // levels, halo columns included, for the neighbours' exchange
-    double e0[S], e1[S], fo[S];
-#pragma unroll
-    for (int t = 0; t < S; ++t) e0[t] = e1[t] = 0.0;
-    if (VEC && a.hor)
-        col_load<S, VEC>(E0 + base * g.cs, g.cs, lo, nz, [&](int k) { return tc.valid && wet_at(tc.kb, k); }, e0);
-    else
-        col_load<S, VEC>(E0 + base * g.cs, g.cs, lo, nz, [&](int k) { return k >= k0; }, e0);
-    col_load<S, VEC>(E1 + base * g.cs, g.cs, lo, nz, [&](int k) { return tc.valid && k < k0; }, e1);
-    load_terms<S, PV>(a.forc, base, lo, nz, [&](int k) { return k >= k0; }, fo);
-    const double fsurf = a.forc_surf[tc.col];  // loaded with the rest, used by the top row
+    __shared__ TurbShared<S> sh;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
     const double dt = a.dt;
-    load_halo_finish<S, PV>(tc.s, km);  // after the other loads are issued
-    double va[S], vb[S], vc[S], vd[S];
-    auto delta = [&](int t) {  // delta at level lo - 1 + t
-        const int k = lo - 1 + t;
-        return (k >= 0 && k < nz - 1) ? dt / zt[k + 1] * a.alpha * 0.5 * (km[t] + km[t + 1]) : 0.0;
-    };
+    TurbCols& tc = sh.cols[wave];
+    const TurbLane l = turb_lane(g, t);
+    const int nz = g.nz;
+    const uint32_t cs = (uint32_t)g.cs;
+    const double* E0 = a.tke + a.tau * g.ls;
+    double* E1 = a.tke + a.taup1 * g.ls;
+    uint32_t wet[S], dry[S];  // solved cells; the others of the run
 #pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = lo + t;
-        const bool w = tc.valid && k < nz && k >= k0;
-        double A = 0.0, B = 1.0, C = 0.0, D = 0.0;
-        if (w) {
-            const double dk = delta(t + 1), dm = delta(t);
-            const double dzw = zw[k];
-            D = e0[t] + dt * fo[t];
-            if (k == k0) {
-                A = 0.0;
-                B = 1 + dk / dzw + dt * a.c_eps / ml[t] * sq[t];
-            } else if (k == nz - 1) {
-                A = -dm / (0.5 * dzw);
-                B = 1 + dm / (0.5 * dzw) + dt * a.c_eps / ml[t] * sq[t];
-            } else {
-                A = -dm / dzw;
-                B = 1 + (dk + dm) / dzw + dt * a.c_eps * sq[t] / ml[t];
-            }
-            C = k < nz - 1 ? -dk / dzw : 0.0;
-            if (k == nz - 1) D += dt * fsurf / (0.5 * dzw);
-        }
-        va[t] = A;
-        vb[t] = B;
-        vc[t] = C;
-        vd[t] = D;
+    for (int r = 0; r < S; ++r) {
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP);
+        wet[r] = w ? t.off[r] : kNoAccess;
+        dry[r] = w ? kNoAccess : t.off[r];
     }
-    SegLane L;
-    L.s = tc.s;
-    L.lo = lo;
-    L.k0 = k0;
-    L.valid = tc.valid;
-    L.base = base;
-    seg_solve_f64<S>(L, va, vb, vc, vd);
-    // the lateral diffusion of the tau level (:250-276)
-    double lat[S];
-    const double Kh = a.K_h;
-    if constexpr (VEC) {
+    const double fsurf = a.forc_surf[t.col0 + (t.q < t.ncol ? t.q : 0)];
+    double e0[S], e1[S], rate[S], f[S];
+    {
+        double km[S], sq[S], ml[S];
+        tile_load(tile_buf(t, a.kappaM), wet, 1, km);
+        tile_load(tile_buf(t, a.sqrttke), t.off, 1, sq);
+        tile_load(tile_buf(t, a.mxl), t.off, 1, ml);
+        tile_load(tile_buf(t, E0, 0, (int)cs), wet, cs, e0);
+        // taup1 off the solved cells (kept there and read by the diagnostic)
+        tile_load(tile_buf(t, E1, 0, (int)cs), dry, cs, e1);
+        turb_setup(g, t, l, dt * a.alpha, dt * a.K_h, a.hor != 0, sh.lv, tc);
+        add_terms(a.forc, t, wet, true, f);
+        tile_put(t, sh.img[wave][0], km);
 #pragma unroll
-        for (int t = 0; t < S; ++t) lat[t] = 0.0;
-        if (a.hor) {
-            // the adjacent groups' columns (j-1 and j+1 inside the wave): every
-            // lane takes part in the exchange
-            const int lane = (int)(threadIdx.x & 63);
-            const int kN_in = __shfl(tc.kb, (lane + kSegP) & 63), kS_in = __shfl(tc.kb, (lane - kSegP) & 63);
-            double eN[S], eS[S];
+        for (int r = 0; r < S; ++r) rate[r] = a.c_eps / ml[r] * sq[r];
+    }
+    {
+        double x[S];
 #pragma unroll
-            for (int t = 0; t < S; ++t) {
-                eN[t] = __shfl(e0[t], (lane + kSegP) & 63);
-                eS[t] = __shfl(e0[t], (lane - kSegP) & 63);
-            }
-            seg_wait_vmem();  // the staged neighbours have landed
-            if (lat_on) {
-                const int kC = tc.kb;
-                const int kN = g8 == kSegCols - 1 ? kX : kN_in, kS = g8 == 0 ? kX : kS_in;
+        for (int r = 0; r < S; ++r) x[r] = dt * rate[r];
+        tile_put(t, sh.img[wave][1], x);
+        const double rtop = dt * sh.lv.rz[nz - 1];
 #pragma unroll
-                for (int t = 0; t < S; ++t) {
-                    const int kk = lo + t, h = t & 1;
-                    const double* sp = stg + 2 * lane + h;
-                    const double fe_ = sp[(0 * NP + t / 2) * 128], fw_ = sp[(1 * NP + t / 2) * 128];
-                    const double fx_ = sp[(2 * NP + t / 2) * 128];
-                    const double fn_ = g8 == kSegCols - 1 ? fx_ : eN[t], fs_ = g8 == 0 ? fx_ : eS[t];
-                    const double fc = e0[t];
-                    const bool mC = wet_at(kC, kk), mE = wet_at(kE, kk), mW = wet_at(kW, kk);
-                    const bool mN = wet_at(kN, kk), mS = wet_at(kS, kk);
-                    const double fe = Kh * (fe_ - fc) / (m_cost * m_dxu) * ((mC && mE) ? 1.0 : 0.0);
-                    const double fw = Kh * (fc - fw_) / (m_cost * m_dxuw) * ((mW && mC) ? 1.0 : 0.0);
-                    const double fn = Kh * (fn_ - fc) / m_dyu * ((mC && mN) ? 1.0 : 0.0) * m_cosu;
-                    const double fs = Kh * (fc - fs_) / m_dyus * ((mS && mC) ? 1.0 : 0.0) * m_cosus;
-                    const double r = (fe - fw) / (m_cost * m_dxt) + (fn - fs) / (m_cost * m_dyt);
-                    lat[t] = (kk < nz && mC) ? r : 0.0;
-                }
+        for (int r = 0; r < S; ++r) {
+            x[r] = e0[r] + dt * f[r];
+            const double fs = __shfl(fsurf, t.c[r] * kTileP);
+            if (t.k[r] == nz - 1) x[r] += rtop * fs;
+        }
+        tile_put(t, sh.img[wave][2], x);
+    }
+    turb_solve<S, false>(t, sh.lv, nz, l.k0, sh.img[wave][0], sh.img[wave][1], sh.img[wave][2]);
+    double v[S], dg[S];
+    uint32_t st[S];
+    tile_get(t, sh.img[wave][2], v);
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        v[r] = wet[r] != kNoAccess ? v[r] : e1[r];
+        dg[r] = rate[r] * v[r];  // tke_diss over the whole array (:230)
+        st[r] = wet[r];
+    }
+    tile_store(tile_buf(t, a.diss), t.off, 1, dg);
+    // surface correction and clamp of every interior column (:235-244)
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        if (t.k[r] == nz - 1 && t.off[r] != kNoAccess) {
+            const int64_t col = t.col0 + t.c[r];
+            const int i = (int)(col / g.Y), j = (int)(col - (int64_t)i * g.Y);
+            if (i >= 2 && i < g.X - 2 && j >= 2 && j < g.Y - 2) {
+                a.surf_corr[col] = v[r] < 0.0 ? -v[r] * 0.5 * sh.lv.zw[nz - 1] / dt : 0.0;
+                v[r] = fmax(0.0, v[r]);
+                st[r] = t.off[r];
             }
         }
     }
-    if (!tc.valid) return;
-    if constexpr (!VEC) {
-        lateral_levels<S, VEC>(
-            lo, [&](int k) { return tc.interior && a.hor && k < nz && wet_at(tc.kb, k); },
-            [&](int k) {
-                return lateral_div(
-                    g, tc.i, tc.j, k, [&](int64_t cc) { return E0[cc * g.cs]; },
-                    [&](int64_t, int64_t) { return Kh; }, [&](int64_t, int64_t) { return Kh; });
-            },
-            [&](int k) {
-                return lateral_div_pair(
-                    g, tc.i, tc.j, k, [&](int64_t cc) { return ld2(E0 + cc); },
-                    [&](int64_t, int64_t) { return make_double2(Kh, Kh); },
-                    [&](int64_t, int64_t) { return make_double2(Kh, Kh); });
-            },
-            lat);
+    if (a.hor) {
+        const double none[1] = {0.0};
+        add_lateral<S, false>(g, t, tc, E0, cs, nullptr, e0, none,
+                              [](double nA, double, double ea, double) { return nA - ea; }, v);
     }
-    double dg[S];
-    bool st[S];
-#pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = lo + t;
-        const bool w = k >= k0;
-        double v = w ? vd[t] : e1[t];
-        dg[t] = a.c_eps / ml[t] * sq[t] * v;  // tke_diss over the whole array (:230)
-        bool store = tc.interior && w;
-        if (tc.interior && k == nz - 1) {  // surface correction and clamp of every interior column (:235-244)
-            a.surf_corr[tc.col] = v < 0.0 ? -v * 0.5 * zw[k] / dt : 0.0;
-            v = fmax(0.0, v);
-            store = true;
-        }
-        if (tc.interior && k < nz && a.hor && wet_at(tc.kb, k)) {
-            v += dt * 1.0 * lat[t];
-            store = true;
-        }
-        e1[t] = v;
-        st[t] = store;
-    }
-    col_store<S, PV>(a.diss + base, 1, lo, nz, dg);
-    col_store_if<S, VEC>(E1 + base * g.cs, g.cs, lo, nz, e1, st);
+    tile_store(tile_buf(t, E1, 0, (int)cs), st, cs, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -473,111 +357,68 @@ struct EkeArgs {
     double dt, alpha, c_eps;
 };
 
-template <int S, bool VEC, bool PV>
-__global__ __launch_bounds__(kTurbBlock) void eke_kernel(EkeArgs a) {
+template <int S>
+__global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void eke_kernel(EkeArgs a) {
     const TurbGrid& g = a.g;
-    const TurbCol tc = turb_col(g, S);
-    __shared__ double sdz[2 * kMaxNz];
-    stage_dz(g, sdz);
-    const double* __restrict__ zt = sdz;           // dzt
-    const double* __restrict__ zw = sdz + kMaxNz;  // dzw
-    const int nz = g.nz, lo = tc.lo, k0 = tc.k0;
-    const int64_t base = tc.col * nz;
-    double km[S + 2];
-    load_halo_issue<S, PV>(a.kappaM, base, lo, nz, km);
-    double sq[S], el[S];
-    load_lv<S, PV>(a.sqrteke, base, lo, nz, sq);
-    load_lv<S, PV>(a.eke_len, base, lo, nz, el);
-    double cint[S];  // eke_c_eps * sqrteke / eke_len * maskW (:121)
-#pragma unroll
-    for (int t = 0; t < S; ++t) cint[t] = a.c_eps * sq[t] / el[t] * (wet_at(tc.kb, lo + t) ? 1.0 : 0.0);
-    const double* __restrict__ E0 = a.eke + a.tau * g.ls;
-    double* __restrict__ E1 = a.eke + a.taup1 * g.ls;
-    double e0[S], e1[S], fo[S];
-#pragma unroll
-    for (int t = 0; t < S; ++t) e0[t] = e1[t] = 0.0;
-    col_load<S, VEC>(E0 + base * g.cs, g.cs, lo, nz, [&](int k) { return k >= k0; }, e0);
-    col_load<S, VEC>(E1 + base * g.cs, g.cs, lo, nz, [&](int k) { return tc.valid && k < k0; }, e1);
-    load_terms<S, PV>(a.forc, base, lo, nz, [&](int k) { return k >= k0; }, fo);
+    __shared__ TurbShared<S> sh;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
     const double dt = a.dt;
-    load_halo_finish<S, PV>(tc.s, km);  // after the other loads are issued
-    double va[S], vb[S], vc[S], vd[S];
-    auto delta = [&](int t) {
-        const int k = lo - 1 + t;
-        return (k >= 0 && k < nz - 1) ? dt / zt[k + 1] * 0.5 * (km[t] + km[t + 1]) * a.alpha : 0.0;
-    };
+    TurbCols& tc = sh.cols[wave];
+    const TurbLane l = turb_lane(g, t);
+    const int nz = g.nz;
+    const uint32_t cs = (uint32_t)g.cs;
+    const double* E0 = a.eke + a.tau * g.ls;
+    double* E1 = a.eke + a.taup1 * g.ls;
+    // solved cells; wet cells (c_int is 0 elsewhere, :121); wet cells that are not solved (halo columns)
+    uint32_t wet[S], sea[S], halo[S];
 #pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = lo + t;
-        const bool w = tc.valid && k < nz && k >= k0;
-        double A = 0.0, B = 1.0, C = 0.0, D = 0.0;
-        if (w) {
-            const double dk = delta(t + 1), dm = delta(t);
-            const double dzw = zw[k];
-            D = e0[t] + dt * fo[t];
-            if (k == k0) {
-                B = 1 + dk / dzw + dt * cint[t];
-            } else if (k == nz - 1) {
-                A = -dm / (0.5 * dzw);
-                B = 1 + dm / (0.5 * dzw) + dt * cint[t];
-            } else {
-                A = -dm / dzw;
-                B = 1 + (dk + dm) / dzw + dt * cint[t];
-            }
-            C = k < nz - 1 ? -dk / dzw : 0.0;
-        }
-        va[t] = A;
-        vb[t] = B;
-        vc[t] = C;
-        vd[t] = D;
+    for (int r = 0; r < S; ++r) {
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP), m = t.k[r] >= __shfl(l.kw, t.c[r] * kTileP);
+        wet[r] = w ? t.off[r] : kNoAccess;
+        sea[r] = m ? t.off[r] : kNoAccess;
+        halo[r] = m && !w ? t.off[r] : kNoAccess;
     }
-    SegLane L;
-    L.s = tc.s;
-    L.lo = lo;
-    L.k0 = k0;
-    L.valid = tc.valid;
-    L.base = base;
-    seg_solve_f64<S>(L, va, vb, vc, vd);
-    if (!tc.valid) return;
-    // the lateral diffusion of the tau level (:168-200)
-    double lat[S];
+    double e0[S], e1[S], cint[S], f[S], kg[S];
     {
-        const double* __restrict__ K = a.K_gm;
-        auto ce2 = [&](int64_t c0, int64_t c1) {
-            const double2 p0 = ld2(K + c0), p1 = ld2(K + c1);
-            return make_double2(0.5 * fmax(500.0, p0.x + p1.x), 0.5 * fmax(500.0, p0.y + p1.y));
-        };
-        lateral_levels<S, VEC>(
-            lo, [&](int k) { return tc.interior && k < nz && wet_at(tc.kb, k); },
-            [&](int k) {
-                return lateral_div(
-                    g, tc.i, tc.j, k, [&](int64_t cc) { return E0[cc * g.cs]; },
-                    [&](int64_t c0, int64_t c1) { return 0.5 * fmax(500.0, K[c0] + K[c1]); },
-                    [&](int64_t c0, int64_t c1) { return 0.5 * fmax(500.0, K[c0] + K[c1]); });
-            },
-            [&](int k) {
-                return lateral_div_pair(g, tc.i, tc.j, k, [&](int64_t cc) { return ld2(E0 + cc); }, ce2, ce2);
-            },
-            lat);
-    }
-    double di[S], zero[S];
-    bool st[S];
+        double km[S], sq[S], el[S];
+        tile_load(tile_buf(t, a.kappaM), wet, 1, km);
+        tile_load(tile_buf(t, a.sqrteke), sea, 1, sq);
+        tile_load(tile_buf(t, a.eke_len), sea, 1, el);
+        tile_load(tile_buf(t, E0, 0, (int)cs), wet, cs, e0);
+        tile_load(tile_buf(t, E1, 0, (int)cs), halo, cs, e1);
+        turb_setup(g, t, l, dt * a.alpha, dt, true, sh.lv, tc);
+        add_terms(a.forc, t, wet, true, f);
+        tile_load(tile_buf(t, a.K_gm), wet, 1, kg);
+        tile_put(t, sh.img[wave][0], km);
 #pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = lo + t;
-        double v = k >= k0 ? vd[t] : e1[t];
-        di[t] = cint[t] * v;  // (:151)
-        zero[t] = 0.0;        // (:152)
-        st[t] = false;
-        if (tc.interior && k < nz && wet_at(tc.kb, k)) {
-            v += dt * 1.0 * lat[t];
-            st[t] = true;
-        }
-        e1[t] = v;
+        for (int r = 0; r < S; ++r) cint[r] = sea[r] != kNoAccess ? a.c_eps * sq[r] / el[r] : 0.0;
     }
-    col_store<S, PV>(a.diss_iw + base, 1, lo, nz, di);
-    col_store<S, PV>(a.diss_tke + base, 1, lo, nz, zero);
-    col_store_if<S, VEC>(E1 + base * g.cs, g.cs, lo, nz, e1, st);
+    {
+        double x[S];
+#pragma unroll
+        for (int r = 0; r < S; ++r) x[r] = dt * cint[r];
+        tile_put(t, sh.img[wave][1], x);
+#pragma unroll
+        for (int r = 0; r < S; ++r) x[r] = e0[r] + dt * f[r];
+        tile_put(t, sh.img[wave][2], x);
+    }
+    turb_solve<S, false>(t, sh.lv, nz, l.k0, sh.img[wave][0], sh.img[wave][1], sh.img[wave][2]);
+    double v[S], dg[S];
+    tile_get(t, sh.img[wave][2], v);
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        v[r] = wet[r] != kNoAccess ? v[r] : e1[r];
+        dg[r] = cint[r] * v[r];  // (:151)
+    }
+    tile_store(tile_buf(t, a.diss_iw), t.off, 1, dg);
+#pragma unroll
+    for (int r = 0; r < S; ++r) dg[r] = 0.0;  // (:152)
+    tile_store(tile_buf(t, a.diss_tke), t.off, 1, dg);
+    add_lateral<S, true>(g, t, tc, E0, cs, a.K_gm, e0, kg, [](double nE, double nK, double ea, double ka) {
+        return 0.5 * fmax(500.0, nK + ka) * (nE - ea);
+    }, v);
+    tile_store(tile_buf(t, E1, 0, (int)cs), wet, cs, v);
 }
 
 // ---------------------------------------------------------------------------
@@ -596,152 +437,101 @@ struct IdemixArgs {
     int diss_mode;  // 0: as is; 1: column integral at the bottom cell; 2: split bottom / surface
 };
 
-template <int S, bool VEC, bool PV>
-__global__ __launch_bounds__(kTurbBlock) void idemix_kernel(IdemixArgs a) {
+template <int S>
+__global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void idemix_kernel(IdemixArgs a) {
     const TurbGrid& g = a.g;
-    const TurbCol tc = turb_col(g, S);
-    __shared__ double sdz[2 * kMaxNz];
-    stage_dz(g, sdz);
-    const double* __restrict__ zt = sdz;           // dzt
-    const double* __restrict__ zw = sdz + kMaxNz;  // dzw
-    const int nz = g.nz;
-    const int64_t base = tc.col * nz;
-    double c0[S + 2];
-    load_halo_issue<S, PV>(a.c0, base, tc.lo, nz, c0);
-    double al[S];
-    load_lv<S, PV>(a.alpha_c, base, tc.lo, nz, al);
-    const double* __restrict__ E0 = a.E + a.tau * g.ls;
-    double* __restrict__ E1 = a.E + a.taup1 * g.ls;
+    __shared__ TurbShared<S> sh;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
     const double dt = a.dt;
-    // the bottom and surface forcing of the column, used by the edge rows
-    const double fbot = a.forc_bot[tc.col], fsurf = a.forc_surf[tc.col];
-    // E_iw at tau on every level, at taup1 off the solve (kept there and read by the diagnostic)
-    double e0[S], e1[S], mx[S];
+    TurbCols& tc = sh.cols[wave];
+    const TurbLane l = turb_lane(g, t);
+    const int nz = g.nz;
+    const uint32_t cs = (uint32_t)g.cs;
+    const double* E0 = a.E + a.tau * g.ls;
+    double* E1 = a.E + a.taup1 * g.ls;
+    uint32_t wet[S], dry[S];
 #pragma unroll
-    for (int t = 0; t < S; ++t) e0[t] = e1[t] = 0.0;
-    col_load<S, VEC>(E0 + base * g.cs, g.cs, tc.lo, nz, [&](int) { return tc.valid; }, e0);
-    col_load<S, VEC>(E1 + base * g.cs, g.cs, tc.lo, nz, [&](int k) { return tc.valid && k < tc.k0; }, e1);
+    for (int r = 0; r < S; ++r) {
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP);
+        wet[r] = w ? t.off[r] : kNoAccess;
+        dry[r] = w ? kNoAccess : t.off[r];
+    }
+    const int64_t gcol = t.col0 + (t.q < t.ncol ? t.q : 0);
+    const double fbot = a.forc_bot[gcol], fsurf = a.forc_surf[gcol];
+    double e0[S], e1[S], rate[S], f[S];
+    {
+        double c0[S], al[S];
+        tile_load(tile_buf(t, a.c0), wet, 1, c0);
+        tile_load(tile_buf(t, a.alpha_c), t.off, 1, al);
+        // E_iw at tau on every cell, at taup1 off the solved ones (kept there and read by the diagnostic)
+        tile_load(tile_buf(t, E0, 0, (int)cs), t.off, cs, e0);
+        tile_load(tile_buf(t, E1, 0, (int)cs), dry, cs, e1);
+        turb_setup(g, t, l, dt * a.tau_v, dt * a.tau_h * 0.5, a.hor != 0, sh.lv, tc);
+        add_terms(a.forc, t, wet, true, f);
+        tile_put(t, sh.img[wave][0], c0);
 #pragma unroll
-    for (int t = 0; t < S; ++t) mx[t] = fmax(0.0, e0[t]);  // max(0, E_iw[tau]) (:118)
-    // the forcing of the lane's levels (interior columns; wet levels feed the
-    // solve, the column integral sums maskW-weighted levels)
-    double fo[S];
-    load_terms<S, PV>(a.forc, base, tc.lo, nz, [&](int k) { return tc.interior && wet_at(tc.kb, k); }, fo);
-#pragma unroll
-    for (int t = 0; t < S; ++t) fo[t] = (tc.interior && wet_at(tc.kb, tc.lo + t)) ? fo[t] : 0.0;
-    if (a.diss_mode != 0) {  // (:70-103)
+        for (int r = 0; r < S; ++r) rate[r] = al[r] * fmax(0.0, e0[r]);  // alpha_c max(0, E_iw[tau]) (:118)
+    }
+    if (a.diss_mode != 0) {  // (:70-103): the forcing's column integral moved to the bottom (and surface) cell
+        double* const img = sh.img[wave][1];
+        tile_put(t, img, f);
+        const int k0 = l.k0;
         double part = 0.0;
 #pragma unroll
-        for (int t = 0; t < S; ++t) {
-            const int k = tc.lo + t;
-            if (k < nz - 1) part += zw[k] * fo[t];
-            else if (k == nz - 1) part += 0.5 * fo[t] * zw[k];
+        for (int r = 0; r < S; ++r) {
+            const int k = t.lo + r;
+            const double fk = img[t.seg + r];
+            if (k >= k0 && k < nz) part += (k < nz - 1 ? sh.lv.zw[k] : 0.5 * sh.lv.zw[k]) * fk;
         }
-        part += __shfl_xor(part, 1, kSegP);
-        part += __shfl_xor(part, 2, kSegP);
-        part += __shfl_xor(part, 4, kSegP);
-        const double a_loc = part;
-        const int ks = tc.kb - 1 > 0 ? tc.kb - 1 : 0;
+        part += __shfl_xor(part, 1, kTileP);
+        part += __shfl_xor(part, 2, kTileP);
+        part += __shfl_xor(part, 4, kTileP);
+        part += __shfl_xor(part, 8, kTileP);
 #pragma unroll
-        for (int t = 0; t < S; ++t) {
-            const int k = tc.lo + t;
-            double f = 0.0;
-            if (k == ks) f = (a.diss_mode == 1 ? 1.0 : a.frac) * a_loc / zw[k];
-            if (a.diss_mode == 2 && k == nz - 1) f = (1.0 - a.frac) * a_loc / (0.5 * zw[k]);
-            fo[t] = f;
+        for (int r = 0; r < S; ++r) {
+            const double a_loc = __shfl(part, t.c[r] * kTileP);
+            const int k = t.k[r];
+            double x = 0.0;
+            if (k == __shfl(l.k0, t.c[r] * kTileP)) x = (a.diss_mode == 1 ? 1.0 : a.frac) * a_loc / sh.lv.zw[k];
+            if (a.diss_mode == 2 && k == nz - 1) x = (1.0 - a.frac) * a_loc / (0.5 * sh.lv.zw[k]);
+            f[r] = x;
         }
-        // the moved term applies to every interior column; rows of other
-        // columns are never solved
     }
-    // terms added afterwards, on the levels whose rows are solved
-    add_terms<S, PV>(a.forc_post, base, tc.lo, nz, [&](int k) { return k >= tc.k0; }, false, fo);
-    load_halo_finish<S, PV>(tc.s, c0);  // after the other loads are issued
-    double va[S], vb[S], vc[S], vd[S];
-    auto delta = [&](int t) {
-        const int k = tc.lo - 1 + t;
-        return (k >= 0 && k < nz - 1) ? dt * a.tau_v / zt[k + 1] * 0.5 * (c0[t] + c0[t + 1]) : 0.0;
-    };
-#pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = tc.lo + t;
-        const bool w = tc.valid && k < nz && k >= tc.k0;
-        double A = 0.0, B = 1.0, C = 0.0, D = 0.0;
-        if (w) {
-            const double dk = delta(t + 1), dm = delta(t);
-            const double dzw = zw[k];
-            const double diss = dt * al[t] * mx[t];
-            const double cc = c0[t + 1];
-            D = e0[t] + dt * fo[t];
-            if (k == tc.k0) {
-                B = 1 + dk / dzw * cc + diss;
-                D = D + dt * fbot / dzw;  // d_edge (:157-159)
-            } else if (k == nz - 1) {
-                A = -dm / (0.5 * dzw) * c0[t];
-                B = 1 + dm / (0.5 * dzw) * cc + diss;
-                D += dt * fsurf / (0.5 * dzw);
-            } else {
-                A = -dm * c0[t] / dzw;
-                B = 1 + dk * cc / dzw + dm * cc / dzw + diss;
-            }
-            C = k < nz - 1 ? -dk / dzw * c0[t + 2] : 0.0;
-        }
-        va[t] = A;
-        vb[t] = B;
-        vc[t] = C;
-        vd[t] = D;
-    }
-    SegLane L;
-    L.s = tc.s;
-    L.lo = tc.lo;
-    L.k0 = tc.k0;
-    L.valid = tc.valid;
-    L.base = base;
-    seg_solve_f64<S>(L, va, vb, vc, vd);
-    if (!tc.valid) return;
-    // the lateral diffusion of the tau level (:186-218)
-    double lat[S];
+    add_terms(a.forc_post, t, wet, false, f);
     {
-        const double* __restrict__ V = a.v0;
-        const double th = a.tau_h;
-        auto ce2 = [&](int64_t c0_, int64_t c1) {
-            const double2 p1 = ld2(V + c1), p0 = ld2(V + c0_);
-            return make_double2(th * 0.5 * (p1.x + p0.x), th * 0.5 * (p1.y + p0.y));
-        };
-        lateral_levels<S, VEC>(
-            tc.lo, [&](int k) { return tc.interior && k < nz && a.hor && wet_at(tc.kb, k); },
-            [&](int k) {
-                return lateral_div(
-                    g, tc.i, tc.j, k, [&](int64_t cc) { return V[cc] * E0[cc * g.cs]; },
-                    [&](int64_t c0_, int64_t c1) { return th * 0.5 * (V[c1] + V[c0_]); },
-                    [&](int64_t c0_, int64_t c1) { return th * 0.5 * (V[c1] + V[c0_]); });
-            },
-            [&](int k) {
-                return lateral_div_pair(
-                    g, tc.i, tc.j, k,
-                    [&](int64_t cc) {
-                        const double2 v = ld2(V + cc), e = ld2(E0 + cc);
-                        return make_double2(v.x * e.x, v.y * e.y);
-                    },
-                    ce2, ce2);
-            },
-            lat);
-    }
-    double di[S];
-    bool st[S];
+        double x[S];
 #pragma unroll
-    for (int t = 0; t < S; ++t) {
-        const int k = tc.lo + t;
-        double v = k >= tc.k0 ? vd[t] : e1[t];
-        di[t] = al[t] * mx[t] * v;  // (:174)
-        st[t] = tc.interior && k >= tc.k0;
-        if (tc.interior && k < nz && a.hor && wet_at(tc.kb, k)) {
-            v += dt * 1.0 * lat[t];
-            st[t] = true;
+        for (int r = 0; r < S; ++r) x[r] = dt * rate[r];
+        tile_put(t, sh.img[wave][1], x);
+        const double rtop = dt * sh.lv.rz[nz - 1];
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            x[r] = e0[r] + dt * f[r];
+            const bool edge = t.k[r] == __shfl(l.k0, t.c[r] * kTileP);
+            const double fb = __shfl(fbot, t.c[r] * kTileP), fs = __shfl(fsurf, t.c[r] * kTileP);
+            if (edge) x[r] += dt * fb / sh.lv.zw[t.k[r]];  // d_edge (:157-159)
+            else if (t.k[r] == nz - 1) x[r] += rtop * fs;
         }
-        e1[t] = v;
+        tile_put(t, sh.img[wave][2], x);
     }
-    col_store<S, PV>(a.iw_diss + base, 1, tc.lo, nz, di);
-    col_store_if<S, VEC>(E1 + base * g.cs, g.cs, tc.lo, nz, e1, st);
+    turb_solve<S, true>(t, sh.lv, nz, l.k0, sh.img[wave][0], sh.img[wave][1], sh.img[wave][2]);
+    double v[S], dg[S];
+    tile_get(t, sh.img[wave][2], v);
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        v[r] = wet[r] != kNoAccess ? v[r] : e1[r];
+        dg[r] = rate[r] * v[r];  // (:174)
+    }
+    tile_store(tile_buf(t, a.iw_diss), t.off, 1, dg);
+    if (a.hor) {  // (:186-218): the fluxes of v0 E with the coefficient 0.5 tau_h (v0 + v0')
+        double v0[S];
+        tile_load(tile_buf(t, a.v0), wet, 1, v0);
+        add_lateral<S, true>(g, t, tc, E0, cs, a.v0, e0, v0, [](double nE, double nV, double ea, double va) {
+            return (nV + va) * (nV * nE - va * ea);
+        }, v);
+    }
+    tile_store(tile_buf(t, E1, 0, (int)cs), wet, cs, v);
 }
 
 namespace {
@@ -784,67 +574,35 @@ int make_terms(const vx_terms* in, Terms& t, bool allow_empty, const char* who) 
     return VX_OK;
 }
 
-template <class Args, template <int, bool, bool> class K>
-int launch_turb(const Args& a, const TurbGrid& g, bool vec, bool pv, hipStream_t s, const char* who) {
-    const int S = seg_levels(g.nz);
-    const int64_t threads = (int64_t)g.X * g.Y * kSegP;
+template <class Args, template <int> class K>
+int launch_turb(const Args& a, const TurbGrid& g, hipStream_t s, const char* who) {
+    const int64_t threads = ((int64_t)g.X * g.Y + kTileC - 1) / kTileC * 64;
     const dim3 grid(blocks_mult8(threads, kTurbBlock)), block(kTurbBlock);
-#define VX_TURB_CASE(N)                                                     \
-    case N:                                                                 \
-        if (vec)                                                            \
-            hipLaunchKernelGGL((K<N, true, true>::fn), grid, block, 0, s, a); \
-        else if (pv)                                                        \
-            hipLaunchKernelGGL((K<N, false, true>::fn), grid, block, 0, s, a); \
-        else                                                                \
-            hipLaunchKernelGGL((K<N, false, false>::fn), grid, block, 0, s, a); \
-        break;
-    switch (S) {
-        VX_TURB_CASE(2)
-        VX_TURB_CASE(4)
-        VX_TURB_CASE(6)
-        VX_TURB_CASE(8)
-        VX_TURB_CASE(10)
-        VX_TURB_CASE(12)
-        VX_TURB_CASE(14)
-        VX_TURB_CASE(16)
+    switch (tile_levels(g.nz)) {
+        case 2: hipLaunchKernelGGL(K<2>::fn, grid, block, 0, s, a); break;
+        case 3: hipLaunchKernelGGL(K<3>::fn, grid, block, 0, s, a); break;
+        case 4: hipLaunchKernelGGL(K<4>::fn, grid, block, 0, s, a); break;
+        case 5: hipLaunchKernelGGL(K<5>::fn, grid, block, 0, s, a); break;
+        case 6: hipLaunchKernelGGL(K<6>::fn, grid, block, 0, s, a); break;
+        case 7: hipLaunchKernelGGL(K<7>::fn, grid, block, 0, s, a); break;
+        case 8: hipLaunchKernelGGL(K<8>::fn, grid, block, 0, s, a); break;
         default: return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, g.nz);
     }
-#undef VX_TURB_CASE
     return check_launch(who);
 }
 
-template <int N, bool V, bool P>
+template <int N>
 struct TkeK {
-    static constexpr auto fn = tke_kernel<N, V, P>;
+    static constexpr auto fn = tke_kernel<N>;
 };
-template <int N, bool V, bool P>
+template <int N>
 struct EkeK {
-    static constexpr auto fn = eke_kernel<N, V, P>;
+    static constexpr auto fn = eke_kernel<N>;
 };
-template <int N, bool V, bool P>
+template <int N>
 struct IdemixK {
-    static constexpr auto fn = idemix_kernel<N, V, P>;
+    static constexpr auto fn = idemix_kernel<N>;
 };
-
-// the 16-byte pair variant: levels outermost, nz even, every array aligned
-// level pairs for the arrays listed (nz even, every one 16-byte aligned)
-bool turb_pairs(const TurbGrid& g, std::initializer_list<const void*> arrays, const Terms& t1, const Terms* t2) {
-    if (g.nz & 1) return false;
-    for (const void* p : arrays)
-        if (!aligned16(p)) return false;
-    for (int q = 0; q < t1.n; ++q)
-        if (!aligned16(t1.p[q])) return false;
-    if (t2)
-        for (int q = 0; q < t2->n; ++q)
-            if (!aligned16(t2->p[q])) return false;
-    return true;
-}
-
-// the 16-byte pair variant for every array, the energy's time levels too
-// (they must be stored outermost)
-bool turb_vec(const TurbGrid& g, std::initializer_list<const void*> arrays, const Terms& t1, const Terms* t2) {
-    return g.cs == 1 && turb_pairs(g, arrays, t1, t2);
-}
 
 bool levels_ok(int tau, int taup1) { return tau >= 0 && tau <= 2 && taup1 >= 0 && taup1 <= 2 && tau != taup1; }
 
@@ -871,11 +629,7 @@ extern "C" int vx_integrate_tke_f64(void* stream, const vx_grid* grid, const vx_
     a.surf_corr = tke_surf_corr, a.diss = tke_diss;
     a.dt = prm->dt_mom, a.alpha = prm->alpha_tke, a.c_eps = prm->c_eps, a.K_h = prm->K_h_tke;
     a.hor = prm->hor_diffusion != 0;
-    const bool vec = turb_vec(a.g, {tke, tke + tau * a.g.ls, tke + taup1 * a.g.ls, kappaM, sqrttke, mxl, tke_diss},
-                              a.forc, nullptr);
-    // the arrays without time levels in pairs whatever the layout
-    const bool pv = vec || turb_pairs(a.g, {kappaM, sqrttke, mxl, tke_diss}, a.forc, nullptr);
-    return launch_turb<TkeArgs, TkeK>(a, a.g, vec, pv, (hipStream_t)stream, who);
+    return launch_turb<TkeArgs, TkeK>(a, a.g, (hipStream_t)stream, who);
 }
 
 extern "C" int vx_integrate_eke_f64(void* stream, const vx_grid* grid, const vx_eke_params* prm, double* eke,
@@ -897,10 +651,7 @@ extern "C" int vx_integrate_eke_f64(void* stream, const vx_grid* grid, const vx_
     a.kappaM = kappaM, a.sqrteke = sqrteke, a.eke_len = eke_len, a.K_gm = K_gm;
     a.diss_iw = eke_diss_iw, a.diss_tke = eke_diss_tke;
     a.dt = prm->dt_tracer, a.alpha = prm->alpha_eke, a.c_eps = prm->eke_c_eps;
-    const bool vec = turb_vec(a.g, {eke, eke + tau * a.g.ls, eke + taup1 * a.g.ls, kappaM, sqrteke, eke_len,
-                                    K_gm, eke_diss_iw, eke_diss_tke}, a.forc, nullptr);
-    const bool pv = vec || turb_pairs(a.g, {kappaM, sqrteke, eke_len, eke_diss_iw, eke_diss_tke}, a.forc, nullptr);
-    return launch_turb<EkeArgs, EkeK>(a, a.g, vec, pv, (hipStream_t)stream, who);
+    return launch_turb<EkeArgs, EkeK>(a, a.g, (hipStream_t)stream, who);
 }
 
 extern "C" int vx_integrate_idemix_f64(void* stream, const vx_grid* grid, const vx_idemix_params* prm, double* E_iw,
@@ -928,8 +679,5 @@ extern "C" int vx_integrate_idemix_f64(void* stream, const vx_grid* grid, const 
     a.dt = prm->dt_tracer, a.tau_v = prm->tau_v, a.tau_h = prm->tau_h, a.frac = prm->eke_diss_surfbot_frac;
     a.hor = prm->hor_diffusion != 0;
     a.diss_mode = prm->eke_diss_mode;
-    const bool vec = turb_vec(a.g, {E_iw, E_iw + tau * a.g.ls, E_iw + taup1 * a.g.ls, c0, v0, alpha_c, iw_diss},
-                              a.forc, &a.forc_post);
-    const bool pv = vec || turb_pairs(a.g, {c0, alpha_c, iw_diss}, a.forc, &a.forc_post);
-    return launch_turb<IdemixArgs, IdemixK>(a, a.g, vec, pv, (hipStream_t)stream, who);
+    return launch_turb<IdemixArgs, IdemixK>(a, a.g, (hipStream_t)stream, who);
 }
