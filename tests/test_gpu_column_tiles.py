@@ -94,3 +94,48 @@ def test_idemix_depths(nz, levels, shift, monkeypatch):
     lat = TT.ORACLE["idemix"](st).E_iw - off
     got = _run("idemix", st, levels, shift, monkeypatch)["E_iw"] - plain["E_iw"]
     assert np.max(np.abs(got - lat)) <= 1e-12 * np.max(np.abs(off))
+
+
+FORMS = ["contiguous", "offset", "interior", "padded"]
+
+
+def _laid_out(a, form):
+    """A GPU tensor of a's values: contiguous; 8 bytes off 16-byte alignment; the
+    interior of a halo array (rows apart); columns with 3 spare levels."""
+    nx, ny, nz = a.shape
+    t = torch.from_numpy(a).cuda()
+    if form == "offset":
+        buf = torch.zeros(a.size + 1, dtype=t.dtype, device="cuda")
+        w = buf[1:].view(a.shape)
+    elif form == "interior":
+        w = torch.zeros((nx + 4, ny + 4, nz), dtype=t.dtype, device="cuda")[2:-2, 2:-2]
+    elif form == "padded":
+        w = torch.zeros((nx, ny, nz + 3), dtype=t.dtype, device="cuda")[..., :nz]
+    else:
+        return t
+    w.copy_(t)
+    return w
+
+
+@pytest.mark.parametrize("nz", [1, 2, 9, 16, 17, 33, 47, 64, 65, 97, 112, 127])
+@pytest.mark.parametrize("form", FORMS)
+def test_tdma_depths_and_strides(nz, form):
+    """13 x 11 columns: rows of one full and one short tile, and a short last tile when the rows join."""
+    from oracle import tdma as O
+    from veros_amd import workloads as W
+    from veros_amd.batched import TdmaBatch
+    from veros_amd.utilities import solve_implicit_kbot
+    rng = np.random.default_rng(nz)
+    p = W.diffusion_tdma(rng, 13, 11, nz, dz=W.geometric_dz(nz, 10.0, 500.0), land_frac=0.2, independent_ac=True,
+                         with_b_edge=True, with_d_edge=True)
+    p.kbot[0, 0], p.kbot[-1, -1] = 1, nz
+    ref = O.solve_implicit_kbot(p.a, p.b, p.c, p.d, p.kbot, b_edge=p.b_edge, d_edge=p.d_edge)
+    a, b, c, d, be, de = (_laid_out(v, form) for v in (p.a, p.b, p.c, p.d, p.b_edge, p.d_edge))
+    kb = torch.from_numpy(p.kbot).cuda()
+    for mode in ("fp64", "mixed"):
+        out = torch.full_like(a, 7.0) if a.is_contiguous() else _laid_out(np.full(a.shape, 7.0), form)
+        x = solve_implicit_kbot(a, b, c, d, kb, b_edge=be, d_edge=de, precision=mode, out=out)
+        assert rel_err(x.cpu().numpy(), ref) <= 1e-12, mode
+        y = _laid_out(np.full(a.shape, 7.0), form)
+        TdmaBatch([dict(a=a, b=b, c=c, d=d, kbot=kb, x=y, b_edge=be, d_edge=de)], precision=mode).run()
+        assert torch.equal(x, y), mode

@@ -1,6 +1,6 @@
-// Column tiles: a wave owns kTileC consecutive (i, j) columns of an (X, Y, nz)
-// grid, which are one contiguous run of kTileC * nz cells, and sees them in
-// two layouts.
+// Column tiles: a wave owns C = 64 / P consecutive (i, j) columns of an
+// (X, Y, nz) grid (with sy = nz one contiguous run of C * nz cells) and sees
+// them in two layouts.
 //
 //   flat:     element t of lane l is cell 64 t + l of the run. Every global
 //             access is made here: consecutive lanes touch consecutive cells
@@ -10,22 +10,23 @@
 //             lane that must not take part gets an offset past its end, which
 //             the hardware turns into 0 (a dropped store) without traffic and
 //             without a branch, so all loads of a phase are in flight together.
-//   segments: lane s of a column's kTileP lanes holds levels [s S, s S + S),
+//   segments: lane s of a column's P lanes holds levels [s S, s S + S),
 //             the layout of the segmented tridiagonal solve.
 //
 // Values pass between the layouts through an LDS image of the run (odd
 // segment stride, so that the segments' starts spread over the banks).
 // Everything elementwise (forcing sums, right-hand sides, diagnostics, lateral
 // fluxes) is done flat, only the rows' neighbours and the solve need
-// segments. With 16 lanes per column a lane holds nz/16 values per array, half
-// of what 8 lanes need, which leaves registers for twice the waves.
+// segments. P = 16 where many arrays are in flight (a lane holds nz/16 values of
+// each, which leaves registers for more waves), P = 8 where the solve itself is
+// most of the work (half the interface rows per column).
 #pragma once
 #include "tdma_seg.hpp"
 
 namespace vx {
 
-constexpr int kTileP = 16;           // lanes per column: one DPP row
-constexpr int kTileC = 64 / kTileP;  // columns per wave
+constexpr int kTileP = 16;           // lanes per column, unless a kernel says otherwise: one DPP row
+constexpr int kTileC = 64 / kTileP;  // columns per wave then
 
 // levels per lane for a depth nz (>= 2)
 __host__ __device__ constexpr int tile_levels(int nz) {
@@ -51,12 +52,13 @@ __device__ __forceinline__ void buf_store(BufRsrc b, uint32_t off, double v) {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(vx_u2, v), b, off, 0, 0);
 }
 
-template <int S>
+template <int S, int P = kTileP>
 struct Tile {
+    static constexpr int C = 64 / P;              // columns
     static constexpr int SP = S | 1;              // segment stride in an image
-    static constexpr int CS = kTileP * SP;        // column stride
-    static constexpr int DUMMY = kTileC * CS;     // slot of the lanes past the run
-    static constexpr int IMG = kTileC * CS + 2;   // doubles of an image
+    static constexpr int CS = P * SP;             // column stride
+    static constexpr int DUMMY = C * CS;          // slot of the lanes past the run
+    static constexpr int IMG = C * CS + 2;        // doubles of an image
     int lane, s, q;       // lane of the wave; segment and column (segments)
     int lo;               // first level of the segment
     int seg;              // the segment's position in an image
@@ -64,42 +66,43 @@ struct Tile {
     int pos[S];           // their positions in an image
     uint32_t off[S];      // their byte offsets in an (X, Y, nz) array's run
     uint32_t bytes;       // bytes of that run
-    int64_t col0, cell0;  // first column and cell of the run
-    int ncol;             // columns of the run (< kTileC in the last tile)
+    int64_t cell0;        // first cell of the run
+    int ncol;             // columns of the run (< C in a row's or the grid's last tile)
 };
 
-// Tile `w` (wave-uniform) of a grid of `cols` columns.
-template <int S>
-__device__ __forceinline__ Tile<S> make_tile(int64_t w, int64_t cols, int nz) {
-    Tile<S> t;
+// The tile of `ncol` columns of nz levels, `sy` cells apart, from cell0 on
+// (ncol = 0: no columns; the addresses formed are those of cell0). All
+// arguments wave-uniform; C * sy * 8 < kNoAccess.
+template <int S, int P = kTileP>
+__device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz, uint32_t sy) {
+    using T = Tile<S, P>;
+    T t;
     t.lane = (int)(threadIdx.x & 63);
-    t.s = t.lane % kTileP;
-    t.q = t.lane / kTileP;
+    t.s = t.lane % P;
+    t.q = t.lane / P;
     t.lo = t.s * S;
-    t.seg = t.q * Tile<S>::CS + t.s * Tile<S>::SP;
-    const int64_t left = cols - w * kTileC;
-    t.ncol = left < kTileC ? (left < 0 ? 0 : (int)left) : kTileC;
-    t.col0 = t.ncol > 0 ? w * kTileC : 0;  // a tile past the grid: no columns, addresses of the first
-    t.cell0 = t.col0 * nz;
-    t.bytes = (uint32_t)(t.ncol * nz) * 8u;
-    // e / nz for e < 512 + 64, nz <= 128, by a 20-bit reciprocal (exact)
+    t.seg = t.q * T::CS + t.s * T::SP;
+    t.cell0 = cell0;
+    t.ncol = ncol;
+    t.bytes = ncol > 0 ? ((uint32_t)(ncol - 1) * sy + (uint32_t)nz) * 8u : 0u;
+    // e / nz for e <= 1024, nz <= 128, by a 20-bit reciprocal (exact there)
     const uint32_t m = ((1u << 20) + (uint32_t)nz - 1u) / (uint32_t)nz;
 #pragma unroll
     for (int r = 0; r < S; ++r) {
         const uint32_t e = 64u * r + (uint32_t)t.lane;
-        const uint32_t c = (e * m) >> 20;
-        const bool in = (int)e < t.ncol * nz;
-        t.k[r] = (int)(e - c * (uint32_t)nz);
+        const uint32_t c = (e * m) >> 20, k = e - c * (uint32_t)nz;
+        const bool in = (int)c < ncol;
+        t.k[r] = (int)k;
         t.c[r] = in ? (int)c : 0;
-        t.pos[r] = (int)c < kTileC ? (int)c * Tile<S>::CS + t.k[r] + t.k[r] / S * (Tile<S>::SP - S) : Tile<S>::DUMMY;
-        t.off[r] = in ? e * 8u : kNoAccess;
+        t.pos[r] = (int)c < T::C ? (int)(c * T::CS + k + k / S * (T::SP - S)) : T::DUMMY;
+        t.off[r] = in ? (c * sy + k) * 8u : kNoAccess;
     }
     return t;
 }
 
 // The run of a (X, Y, nz) array, `d` cells further on, cs doubles per cell.
-template <int S>
-__device__ __forceinline__ BufRsrc tile_buf(const Tile<S>& t, const double* a, int64_t d = 0, int cs = 1) {
+template <int S, int P>
+__device__ __forceinline__ BufRsrc tile_buf(const Tile<S, P>& t, const double* a, int64_t d = 0, int cs = 1) {
     return make_buf(a + (t.cell0 + d) * cs, t.bytes * (uint32_t)cs);
 }
 
@@ -115,36 +118,36 @@ __device__ __forceinline__ void tile_store(BufRsrc b, const uint32_t (&off)[S], 
     for (int r = 0; r < S; ++r) buf_store(b, off[r] * cs, v[r]);
 }
 // flat <-> image
-template <int S>
-__device__ __forceinline__ void tile_put(const Tile<S>& t, double* img, const double (&v)[S]) {
+template <int S, int P>
+__device__ __forceinline__ void tile_put(const Tile<S, P>& t, double* img, const double (&v)[S]) {
 #pragma unroll
     for (int r = 0; r < S; ++r) img[t.pos[r]] = v[r];
 }
-template <int S>
-__device__ __forceinline__ void tile_get(const Tile<S>& t, const double* img, double (&v)[S]) {
+template <int S, int P>
+__device__ __forceinline__ void tile_get(const Tile<S, P>& t, const double* img, double (&v)[S]) {
 #pragma unroll
     for (int r = 0; r < S; ++r) v[r] = img[t.pos[r]];
 }
 // segments <-> image
-template <int S>
-__device__ __forceinline__ void seg_get(const Tile<S>& t, const double* img, double (&v)[S]) {
+template <int S, int P>
+__device__ __forceinline__ void seg_get(const Tile<S, P>& t, const double* img, double (&v)[S]) {
 #pragma unroll
     for (int r = 0; r < S; ++r) v[r] = img[t.seg + r];
 }
-template <int S>
-__device__ __forceinline__ void seg_put(const Tile<S>& t, double* img, const double (&v)[S]) {
+template <int S, int P>
+__device__ __forceinline__ void seg_put(const Tile<S, P>& t, double* img, const double (&v)[S]) {
 #pragma unroll
     for (int r = 0; r < S; ++r) img[t.seg + r] = v[r];
 }
 // the value of the level below lo (lane s = 0: unspecified) and above lo + S - 1
-// (lane s = kTileP - 1: unspecified) in an image
-template <int S>
-__device__ __forceinline__ double seg_below(const Tile<S>& t, const double* img) {
-    return img[t.s > 0 ? t.seg - 1 - (Tile<S>::SP - S) : t.seg];
+// (lane s = P - 1: unspecified) in an image
+template <int S, int P>
+__device__ __forceinline__ double seg_below(const Tile<S, P>& t, const double* img) {
+    return img[t.s > 0 ? t.seg - 1 - (Tile<S, P>::SP - S) : t.seg];
 }
-template <int S>
-__device__ __forceinline__ double seg_above(const Tile<S>& t, const double* img) {
-    return img[t.s < kTileP - 1 ? t.seg + Tile<S>::SP : t.seg];
+template <int S, int P>
+__device__ __forceinline__ double seg_above(const Tile<S, P>& t, const double* img) {
+    return img[t.s < P - 1 ? t.seg + Tile<S, P>::SP : t.seg];
 }
 
 // ---------------------------------------------------------------------------

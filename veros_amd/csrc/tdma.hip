@@ -6,13 +6,12 @@
 // k = kbot-1 (where b, d may be replaced by b_edge, d_edge) and the
 // super-diagonal is 0 at the top row; x is 0 outside the wet suffix.
 //
-// Layout: (x, y, z) with z contiguous. One lane owns one column and walks it
-// bottom-up; the elimination factors cp/dp live in VGPRs (the level loop is
-// fully unrolled per nz bucket, so the register arrays are statically
-// indexed). Coefficients are read in 16-byte pairs where alignment allows;
-// each lane streams whole cache lines of its own column, so the L1 does the
-// transposition and HBM sees full-line traffic.
-#include "tdma_seg.hpp"
+// Layout: (x, y, z) with z contiguous. Eight lanes own a column (tdma_seg.hpp);
+// a wave brings its eight columns in either flat through registers
+// (tdma_tile.hpp: any alignment, stride and depth) or with 16-byte copies
+// straight into LDS. The lane-per-column kernels at the end of the file walk
+// their column bottom-up with the elimination factors in VGPRs.
+#include "tdma_tile.hpp"
 
 #include <cstdlib>
 
@@ -42,6 +41,17 @@ __global__ __launch_bounds__(kSegLdsBlock) void tdma_segl_mixed_kernel(TdmaArgs 
     extern __shared__ double seg_lds[];
     double* lds = seg_lds + (threadIdx.x / 64) * (seg_lds_wave_bytes(S) / 8);
     seg_mixed_lds<S, REFINE>(p, seg_lane_of(p, S), lds);
+}
+
+// Column tiles, one per wave (two waves per SIMD at least: the mixed form at
+// 16 levels per lane would take the registers of one).
+template <int S, int MODE>
+__global__ __launch_bounds__(kSegLdsBlock) __attribute__((amdgpu_waves_per_eu(2))) void tdma_tile_kernel(TdmaArgs p, TdmaTiling g) {
+    __shared__ double img[kSegLdsBlock / 64][tdma_tile_lds<S>()];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    SegLane L;
+    const Tile<S, kTdmaP> t = tdma_tile_of<S>(p, g, (int64_t)blockIdx.x * (kSegLdsBlock / 64) + wave, L);
+    tdma_tile<S, MODE>(p, t, L, img[wave]);
 }
 
 template <int NZB, bool VEC>
@@ -150,15 +160,10 @@ int validate_tdma(const TdmaArgs& p, int64_t nx, int64_t ny, int32_t nz, const c
     return VX_OK;
 }
 
-bool vec_ok(const TdmaArgs& p) {
-    if ((p.nz & 1) || (p.sx & 1) || (p.sy & 1)) return false;
-    return aligned16(p.a) && aligned16(p.b) && aligned16(p.c) && aligned16(p.d) && aligned16(p.x);
-}
-
 template <template <int, bool> class K>
 int launch_bucket(const TdmaArgs& p, hipStream_t s, const char* who) {
     const int nzb = ((p.nz + 15) / 16) * 16;
-    const bool vec = vec_ok(p);
+    const bool vec = tdma_vec_ok(p);
     const dim3 grid((unsigned)((p.ncol + kTdmaBlock - 1) / kTdmaBlock));
     const dim3 block(kTdmaBlock);
 #define VX_TDMA_CASE(N)                                                                      \
@@ -186,7 +191,7 @@ int launch_bucket(const TdmaArgs& p, hipStream_t s, const char* who) {
 template <template <int, bool> class K>
 int launch_seg(const TdmaArgs& p, hipStream_t s, const char* who) {
     const int S = seg_levels(p.nz);
-    const bool vec = vec_ok(p);
+    const bool vec = tdma_vec_ok(p);
     const int64_t threads = p.ncol * kSegP;
     const dim3 grid((unsigned)((threads + kSegBlock - 1) / kSegBlock));
     const dim3 block(kSegBlock);
@@ -223,19 +228,38 @@ int launch_segl(const TdmaArgs& p, hipStream_t s, const char* who) {
     case N:                                                                 \
         hipLaunchKernelGGL((K<N, true>::fn), grid, block, lds, s, p);       \
         break;
-    switch (S) {
+    switch (S) {  // the depths of tdma_lds_wins
         VX_SEGL_CASE(2)
-        VX_SEGL_CASE(4)
         VX_SEGL_CASE(6)
-        VX_SEGL_CASE(8)
         VX_SEGL_CASE(10)
         VX_SEGL_CASE(12)
-        VX_SEGL_CASE(14)
-        VX_SEGL_CASE(16)
         default:
             return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, p.nz);
     }
 #undef VX_SEGL_CASE
+    return check_launch(who);
+}
+
+template <int MODE>
+int launch_tile(const TdmaArgs& p, hipStream_t s, const char* who) {
+    const TdmaTiling g = tdma_tiling(p);
+    const int waves = kSegLdsBlock / 64;
+    const dim3 grid((unsigned)((g.ntiles + waves - 1) / waves)), block(kSegLdsBlock);
+#define VX_TILE_CASE(N) \
+    case N: hipLaunchKernelGGL((tdma_tile_kernel<N, MODE>), grid, block, 0, s, p, g); break;
+    switch (seg_levels(p.nz)) {
+        VX_TILE_CASE(2)
+        VX_TILE_CASE(4)
+        VX_TILE_CASE(6)
+        VX_TILE_CASE(8)
+        VX_TILE_CASE(10)
+        VX_TILE_CASE(12)
+        VX_TILE_CASE(14)
+        VX_TILE_CASE(16)
+        default:
+            return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, p.nz);
+    }
+#undef VX_TILE_CASE
     return check_launch(who);
 }
 
@@ -274,9 +298,9 @@ struct SegMixK2 {
 };
 
 // Kernel family of the single-grid solves (VX_TDMA_KERNEL, read once):
-// "lds" (default; segmented with LDS-staged coalesced copies when the operands
-// are 16-byte aligned, else "segment"), "segment" (segmented, register loads),
-// "column" (lane per column).
+// default: column tiles, or the LDS-staged kernels where they are faster (see
+// tdma_lds_wins); "segment": segmented, register loads; "column": lane per
+// column.
 int tdma_kernel_family() {
     static const int fam = [] {
         const char* e = std::getenv("VX_TDMA_KERNEL");
@@ -287,7 +311,11 @@ int tdma_kernel_family() {
     return fam;
 }
 bool use_column_kernels() { return tdma_kernel_family() == 0; }
-bool use_lds_kernels(const TdmaArgs& p) { return tdma_kernel_family() == 2 && vec_ok(p); }
+bool use_segment_kernels() { return tdma_kernel_family() == 1; }
+
+bool lds_kernel_wins(const TdmaArgs& p, bool mixed) {
+    return tdma_vec_ok(p) && tdma_lds_wins(seg_levels(p.nz), mixed);
+}
 
 template <int N, bool V>
 struct F64K {
@@ -338,9 +366,10 @@ extern "C" int vx_tdma_f64(void* stream, const double* a, const double* b, const
     TdmaArgs p = make_args(a, b, c, d, b_edge, d_edge, kbot, kbot_sx, kbot_sy, x, nx, ny, nz, sx, sy);
     int rc = validate_tdma(p, nx, ny, nz, "vx_tdma_f64");
     if (rc != VX_OK || p.ncol == 0) return rc;
-    if (use_lds_kernels(p)) return launch_segl<SeglF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
-    if (!use_column_kernels()) return launch_seg<SegF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
-    return launch_bucket<F64K>(p, (hipStream_t)stream, "vx_tdma_f64");
+    if (use_column_kernels()) return launch_bucket<F64K>(p, (hipStream_t)stream, "vx_tdma_f64");
+    if (use_segment_kernels()) return launch_seg<SegF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
+    if (lds_kernel_wins(p, false)) return launch_segl<SeglF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
+    return launch_tile<-1>(p, (hipStream_t)stream, "vx_tdma_f64");
 }
 
 extern "C" int vx_tdma_mixed(void* stream, const double* a, const double* b, const double* c, const double* d,
@@ -353,24 +382,33 @@ extern "C" int vx_tdma_mixed(void* stream, const double* a, const double* b, con
     TdmaArgs p = make_args(a, b, c, d, b_edge, d_edge, kbot, kbot_sx, kbot_sy, x, nx, ny, nz, sx, sy);
     int rc = validate_tdma(p, nx, ny, nz, "vx_tdma_mixed");
     if (rc != VX_OK || p.ncol == 0) return rc;
-    if (use_lds_kernels(p)) {
+    hipStream_t s = (hipStream_t)stream;
+    const char* who = "vx_tdma_mixed";
+    if (use_column_kernels()) {
         switch (refine_steps) {
-            case 0: return launch_segl<SeglMixK0>(p, (hipStream_t)stream, "vx_tdma_mixed");
-            case 1: return launch_segl<SeglMixK1>(p, (hipStream_t)stream, "vx_tdma_mixed");
-            default: return launch_segl<SeglMixK2>(p, (hipStream_t)stream, "vx_tdma_mixed");
+            case 0: return launch_bucket<MixK0>(p, s, who);
+            case 1: return launch_bucket<MixK1>(p, s, who);
+            default: return launch_bucket<MixK2>(p, s, who);
         }
     }
-    if (!use_column_kernels()) {
+    if (use_segment_kernels()) {
         switch (refine_steps) {
-            case 0: return launch_seg<SegMixK0>(p, (hipStream_t)stream, "vx_tdma_mixed");
-            case 1: return launch_seg<SegMixK1>(p, (hipStream_t)stream, "vx_tdma_mixed");
-            default: return launch_seg<SegMixK2>(p, (hipStream_t)stream, "vx_tdma_mixed");
+            case 0: return launch_seg<SegMixK0>(p, s, who);
+            case 1: return launch_seg<SegMixK1>(p, s, who);
+            default: return launch_seg<SegMixK2>(p, s, who);
+        }
+    }
+    if (lds_kernel_wins(p, true)) {
+        switch (refine_steps) {
+            case 0: return launch_segl<SeglMixK0>(p, s, who);
+            case 1: return launch_segl<SeglMixK1>(p, s, who);
+            default: return launch_segl<SeglMixK2>(p, s, who);
         }
     }
     switch (refine_steps) {
-        case 0: return launch_bucket<MixK0>(p, (hipStream_t)stream, "vx_tdma_mixed");
-        case 1: return launch_bucket<MixK1>(p, (hipStream_t)stream, "vx_tdma_mixed");
-        default: return launch_bucket<MixK2>(p, (hipStream_t)stream, "vx_tdma_mixed");
+        case 0: return launch_tile<0>(p, s, who);
+        case 1: return launch_tile<1>(p, s, who);
+        default: return launch_tile<2>(p, s, who);
     }
 }
 

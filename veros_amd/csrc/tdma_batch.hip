@@ -1,18 +1,17 @@
 // Batched TDMA over many independent grids of different shapes and depths.
 //
 // A plan is built once from the list of systems (the arrays of every grid
-// stay where they are): systems are grouped by 16-level nz bucket (8 levels
-// per lane in the segmented solve: S = bucket / 8) and each bucket's columns
-// form one global column space. vx_tdma_plan_run launches one persistent
-// grid-stride kernel per non-empty bucket; a group of kSegP lanes owns one
-// global column at a time, finds its system by binary search over the
-// bucket's column offsets, and runs the segmented solve of the single-grid
-// kernels (tdma_seg.hpp) in float64 (mode 0) or in mixed precision with one
-// refinement step (mode 1). vx_tdma_plan_tune times block-size / grid-size
-// candidates per bucket on the plan's own data and keeps the fastest (a
-// process-wide cache keyed by bucket, mode and size reuses earlier choices);
-// vx_tdma_plan_graph_launch captures run() once into a hipGraph and replays
-// it.
+// stay where they are): systems are grouped by 16-level nz bucket (8 lanes per
+// column in the segmented solve: S = bucket / 8 levels per lane) and cut into
+// tiles of up to 8 columns; each bucket's tiles form one sequence.
+// vx_tdma_plan_run launches one persistent grid-stride kernel per non-empty
+// bucket; a wave takes one tile at a time, finds its system by binary search
+// over the systems' first tiles, and runs the single-grid kernels' solve in
+// float64 (mode 0) or in mixed precision with one refinement step (mode 1).
+// vx_tdma_plan_tune times block-size / grid-size candidates per bucket on the
+// plan's own data and keeps the fastest (a process-wide cache keyed by bucket,
+// mode and size reuses earlier choices); vx_tdma_plan_graph_launch captures
+// run() once into a hipGraph and replays it.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -20,7 +19,7 @@
 #include <tuple>
 #include <vector>
 
-#include "tdma_seg.hpp"
+#include "tdma_tile.hpp"
 
 struct vx_tdma_plan;
 
@@ -28,72 +27,56 @@ namespace vx {
 
 struct SysDesc {
     TdmaArgs args;
-    int64_t col0;  // first column of this system in its bucket's column space
-    int32_t vec;   // 16-byte vector loads allowed
-    int32_t _pad;
+    TdmaTiling tiling;
+    int64_t tile0;  // first tile of this system in its bucket
 };
 
-// One launch per bucket: S levels per lane, MODE 0 = float64, 1 = mixed with
-// one refinement step. Every system's columns start at a multiple of 8 in
-// the bucket's column space (its count padded to a multiple of 8), so the 8
-// columns of a wave's tile always belong to one system: a wave finds it once
-// and, when its arrays allow 16-byte copies, runs the LDS-staged segmented
-// solve of the single-grid kernels; otherwise the register variant.
-template <int S, int MODE>
-__global__ __launch_bounds__(128) void tdma_seg_batch_kernel(const SysDesc* __restrict__ sys, int nsys,
+// LDS doubles of a wave
+template <int S, bool LDSV>
+__host__ __device__ constexpr int batch_lds() {
+    return LDSV ? seg_lds_wave_bytes(S) / 8 : tdma_tile_lds<S>();
+}
+
+// One launch per bucket: S levels per lane, MODE -1 = float64, else mixed with
+// MODE refinement steps. LDSV: every system of the bucket allows 16-byte copies
+// straight into LDS and those are faster at this S (tdma_lds_wins); else the
+// flat loads of tdma_tile.hpp (odd depths, any alignment or strides). Before
+// those, systems of odd depth had each lane load its own levels, 8 bytes at a
+// time, in kernels that held the LDS of the copies.
+template <int S, int MODE, bool LDSV>
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void tdma_seg_batch_kernel(const SysDesc* __restrict__ sys, int nsys,
                                                              int64_t ntiles) {
     extern __shared__ double seg_lds[];
-    double* lds = seg_lds + (threadIdx.x / 64) * (seg_lds_wave_bytes(S) / 8);
+    double* lds = seg_lds + (threadIdx.x / 64) * batch_lds<S, LDSV>();
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / 64);
-    const int lane = threadIdx.x & 63;
-    const int s = lane % kSegP;
-    const int c = lane / kSegP;
     // the tile index is the same in every lane of a wave: keep it (and so
     // the system search and descriptor loads) in scalar registers
     const int64_t w0 = (int64_t)blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     for (int64_t w = w0; w < ntiles; w += wstride) {
-        const int64_t g0 = w * kSegCols;  // the tile's first column
         int lo = 0, hi = nsys - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
-            if (sys[mid].col0 <= g0) lo = mid;
+            if (sys[mid].tile0 <= w) lo = mid;
             else hi = mid - 1;
         }
         lo = __builtin_amdgcn_readfirstlane(lo);
         const SysDesc& sd = sys[lo];
         const TdmaArgs p = sd.args;
-        const int64_t col = g0 + c - sd.col0;
         SegLane L;
-        L.s = s;
-        L.lo = s * S;
-        L.valid = col < p.ncol;
-        L.base = 0;
-        L.k0 = p.nz;
-        if (L.valid) {
-            const int64_t i = col / p.ny;
-            const int64_t j = col - i * p.ny;
-            L.base = i * p.sx + j * p.sy;
-            const int kb = p.kbot[i * p.kx + j * p.ky];
-            L.k0 = (kb >= 1 && kb <= p.nz) ? kb - 1 : p.nz;
-        }
-        double va[S], vb[S], vc[S], vd[S];
-        if (sd.vec) {
+        const Tile<S, kTdmaP> t = tdma_tile_of<S>(p, sd.tiling, w - sd.tile0, L);
+        if constexpr (LDSV) {
+            double va[S], vb[S], vc[S], vd[S];
             seg_rows_lds<S>(p, L, lds, va, vb, vc, vd);
+            if constexpr (MODE < 0) {
+                seg_solve_f64<S>(L, va, vb, vc, vd);
+                seg_store_lds<S>(p, L, lds, vd);
+            } else {
+                double x[S];
+                seg_mixed_core<S, MODE>(L, va, vb, vc, vd, x);
+                seg_store_lds<S>(p, L, lds, x);
+            }
         } else {
-            seg_rows<S, false>(p, L, va, vb, vc, vd);
-        }
-        double x[S];
-        if constexpr (MODE == 0) {
-            seg_solve_f64<S>(L, va, vb, vc, vd);
-#pragma unroll
-            for (int t = 0; t < S; ++t) x[t] = vd[t];
-        } else {
-            seg_mixed_core<S, 1>(L, va, vb, vc, vd, x);
-        }
-        if (sd.vec) {
-            seg_store_lds<S>(p, L, lds, x);
-        } else if (L.valid) {
-            seg_store<S, false>(p.x + L.base, L.lo, p.nz, x);
+            tdma_tile<S, MODE>(p, t, L, lds);
         }
     }
 }
@@ -109,8 +92,9 @@ struct Bucket {
     int nzb = 0;
     int first = 0;       // index of the first system of this bucket in the device table
     int nsys = 0;
-    int64_t total = 0;   // columns, each system's count padded to a multiple of 8
-    int64_t cols = 0;    // columns without the padding
+    int64_t tiles = 0;   // tiles of up to 8 columns
+    int64_t cols = 0;    // columns
+    bool ldsv = true;    // every system's arrays allow 16-byte copies into LDS
     int bs = 128;
     int factor = 0;
 };
@@ -129,22 +113,29 @@ int ilog2(int64_t v) {
 }
 
 template <int S, int MODE>
-void launch_bs(int bs, const SysDesc* d, int nsys, int64_t total, unsigned grid, hipStream_t s) {
-    const size_t lds = (size_t)seg_lds_wave_bytes(S) * (bs / 64);
-    hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE>), dim3(grid), dim3(bs), lds, s, d, nsys, total / kSegCols);
+void launch_bs(int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+    if constexpr (tdma_lds_wins(S, MODE >= 0)) {
+        if (ldsv) {
+            const size_t lds = (size_t)batch_lds<S, true>() * 8 * (bs / 64);
+            hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, true>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
+            return;
+        }
+    }
+    const size_t lds = (size_t)batch_lds<S, false>() * 8 * (bs / 64);
+    hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, false>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
 }
 
 template <int MODE>
-void launch_mode(int nzb, int bs, const SysDesc* d, int nsys, int64_t total, unsigned grid, hipStream_t s) {
+void launch_mode(int nzb, int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
     switch (nzb) {
-        case 16: launch_bs<2, MODE>(bs, d, nsys, total, grid, s); break;
-        case 32: launch_bs<4, MODE>(bs, d, nsys, total, grid, s); break;
-        case 48: launch_bs<6, MODE>(bs, d, nsys, total, grid, s); break;
-        case 64: launch_bs<8, MODE>(bs, d, nsys, total, grid, s); break;
-        case 80: launch_bs<10, MODE>(bs, d, nsys, total, grid, s); break;
-        case 96: launch_bs<12, MODE>(bs, d, nsys, total, grid, s); break;
-        case 112: launch_bs<14, MODE>(bs, d, nsys, total, grid, s); break;
-        default: launch_bs<16, MODE>(bs, d, nsys, total, grid, s); break;
+        case 16: launch_bs<2, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 32: launch_bs<4, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 48: launch_bs<6, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 64: launch_bs<8, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 80: launch_bs<10, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 96: launch_bs<12, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 112: launch_bs<14, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        default: launch_bs<16, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
     }
 }
 
@@ -167,7 +158,7 @@ namespace vx {
 namespace {
 
 unsigned grid_for(const vx_tdma_plan* P, const Bucket& b, int bs, int factor) {
-    const int64_t full = (b.total * kSegP + bs - 1) / bs;  // one 8-column tile per wave
+    const int64_t full = (b.tiles * 64 + bs - 1) / bs;  // one tile per wave
     if (factor == 0) return (unsigned)std::max<int64_t>(1, full);
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(full, (int64_t)factor * P->num_cu));
 }
@@ -175,8 +166,8 @@ unsigned grid_for(const vx_tdma_plan* P, const Bucket& b, int bs, int factor) {
 void launch_bucket(const vx_tdma_plan* P, const Bucket& b, int bs, int factor, hipStream_t s) {
     const SysDesc* d = P->d_sys + b.first;
     const unsigned grid = grid_for(P, b, bs, factor);
-    if (P->mode == 0) launch_mode<0>(b.nzb, bs, d, b.nsys, b.total, grid, s);
-    else launch_mode<1>(b.nzb, bs, d, b.nsys, b.total, grid, s);
+    if (P->mode == 0) launch_mode<-1>(b.nzb, bs, b.ldsv, d, b.nsys, b.tiles, grid, s);
+    else launch_mode<1>(b.nzb, bs, b.ldsv, d, b.nsys, b.tiles, grid, s);
 }
 
 }  // namespace
@@ -209,10 +200,6 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
         p.kbot = y.kbot, p.x = y.x;
         p.ny = y.ny, p.ncol = y.nx * y.ny, p.sx = y.sx, p.sy = y.sy, p.kx = y.kbot_sx, p.ky = y.kbot_sy;
         p.nz = y.nz;
-        sd.vec = (!(y.nz & 1) && !(y.sx & 1) && !(y.sy & 1) && aligned16(y.a) && aligned16(y.b) &&
-                  aligned16(y.c) && aligned16(y.d) && aligned16(y.x))
-                     ? 1
-                     : 0;
         per[(y.nz + 15) / 16 - 1].push_back(sd);
         all.push_back(y);
     }
@@ -233,17 +220,17 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
         b.nzb = kBuckets[bk];
         b.first = (int)table.size();
         b.nsys = (int)per[bk].size();
-        int64_t col = 0;
         for (SysDesc& sd : per[bk]) {
-            sd.col0 = col;
-            col += (sd.args.ncol + kSegCols - 1) / kSegCols * kSegCols;
+            sd.tiling = tdma_tiling(sd.args);
+            sd.tile0 = b.tiles;
+            b.tiles += sd.tiling.ntiles;
             b.cols += sd.args.ncol;
+            b.ldsv = b.ldsv && tdma_vec_ok(sd.args);
             table.push_back(sd);
         }
-        b.total = col;
         {
             std::lock_guard<std::mutex> lk(g_tune_mutex);
-            auto it = g_tune_cache.find(TuneKey{b.nzb, mode, ilog2(b.total), P->num_cu});
+            auto it = g_tune_cache.find(TuneKey{b.nzb, mode, ilog2(b.tiles * kSegCols), P->num_cu});
             if (it != g_tune_cache.end()) {
                 b.bs = it->second.first;
                 b.factor = it->second.second;
@@ -349,7 +336,7 @@ extern "C" int vx_tdma_plan_tune(vx_tdma_plan* plan, void* stream) {
         b.bs = best_bs;
         b.factor = best_f;
         std::lock_guard<std::mutex> lk(g_tune_mutex);
-        g_tune_cache[TuneKey{b.nzb, plan->mode, ilog2(b.total), plan->num_cu}] = {b.bs, b.factor};
+        g_tune_cache[TuneKey{b.nzb, plan->mode, ilog2(b.tiles * kSegCols), plan->num_cu}] = {b.bs, b.factor};
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

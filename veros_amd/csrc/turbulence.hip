@@ -60,6 +60,17 @@ struct TurbLevels {
 
 __device__ __forceinline__ int first_wet_of(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
 
+// The wave's tile: columns [col0, col0 + kTileC) of the X * Y, in order.
+__device__ __forceinline__ int64_t turb_col0(int wave) {
+    return (xcd_contiguous_block() * (kTurbBlock / 64) + wave) * kTileC;
+}
+template <int S>
+__device__ __forceinline__ Tile<S> turb_tile(const TurbGrid& g, int64_t col0) {
+    const int64_t left = (int64_t)g.X * g.Y - col0;
+    const int n = left >= kTileC ? kTileC : (left > 0 ? (int)left : 0);
+    return make_tile<S>(n > 0 ? col0 * g.nz : 0, n, g.nz, (uint32_t)g.nz);
+}
+
 // The lane's group column (segments): what the masks need, known before the
 // first load is issued.
 struct TurbLane {
@@ -68,11 +79,11 @@ struct TurbLane {
     int kw, k0;  // first wet and first solved level (nz: none)
 };
 template <int S>
-__device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S>& t) {
+__device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S>& t, int64_t col0) {
     TurbLane l;
     const bool valid = t.q < t.ncol;
-    const int64_t col = t.col0 + (valid ? t.q : 0);
-    const int kb = t.ncol > 0 ? g.kbot[col] : 0;
+    const int64_t col = valid ? col0 + t.q : 0;
+    const int kb = g.kbot[col];
     l.i = (int)(col / g.Y);
     l.j = (int)(col - (int64_t)l.i * g.Y);
     l.interior = valid && l.i >= 2 && l.i < g.X - 2 && l.j >= 2 && l.j < g.Y - 2;
@@ -267,10 +278,11 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     const TurbGrid& g = a.g;
     __shared__ TurbShared<S> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
+    const int64_t col0 = turb_col0(wave);
+    const Tile<S> t = turb_tile<S>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
-    const TurbLane l = turb_lane(g, t);
+    const TurbLane l = turb_lane(g, t, col0);
     const int nz = g.nz;
     const uint32_t cs = (uint32_t)g.cs;
     const double* E0 = a.tke + a.tau * g.ls;
@@ -282,7 +294,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
         wet[r] = w ? t.off[r] : kNoAccess;
         dry[r] = w ? kNoAccess : t.off[r];
     }
-    const double fsurf = a.forc_surf[t.col0 + (t.q < t.ncol ? t.q : 0)];
+    const double fsurf = a.forc_surf[t.q < t.ncol ? col0 + t.q : 0];
     double e0[S], e1[S], rate[S], f[S];
     {
         double km[S], sq[S], ml[S];
@@ -327,7 +339,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
 #pragma unroll
     for (int r = 0; r < S; ++r) {
         if (t.k[r] == nz - 1 && t.off[r] != kNoAccess) {
-            const int64_t col = t.col0 + t.c[r];
+            const int64_t col = col0 + t.c[r];
             const int i = (int)(col / g.Y), j = (int)(col - (int64_t)i * g.Y);
             if (i >= 2 && i < g.X - 2 && j >= 2 && j < g.Y - 2) {
                 a.surf_corr[col] = v[r] < 0.0 ? -v[r] * 0.5 * sh.lv.zw[nz - 1] / dt : 0.0;
@@ -362,10 +374,11 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     const TurbGrid& g = a.g;
     __shared__ TurbShared<S> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
+    const int64_t col0 = turb_col0(wave);
+    const Tile<S> t = turb_tile<S>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
-    const TurbLane l = turb_lane(g, t);
+    const TurbLane l = turb_lane(g, t, col0);
     const int nz = g.nz;
     const uint32_t cs = (uint32_t)g.cs;
     const double* E0 = a.eke + a.tau * g.ls;
@@ -442,10 +455,11 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     const TurbGrid& g = a.g;
     __shared__ TurbShared<S> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const Tile<S> t = make_tile<S>(xcd_contiguous_block() * (kTurbBlock / 64) + wave, (int64_t)g.X * g.Y, g.nz);
+    const int64_t col0 = turb_col0(wave);
+    const Tile<S> t = turb_tile<S>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
-    const TurbLane l = turb_lane(g, t);
+    const TurbLane l = turb_lane(g, t, col0);
     const int nz = g.nz;
     const uint32_t cs = (uint32_t)g.cs;
     const double* E0 = a.E + a.tau * g.ls;
@@ -457,7 +471,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
         wet[r] = w ? t.off[r] : kNoAccess;
         dry[r] = w ? kNoAccess : t.off[r];
     }
-    const int64_t gcol = t.col0 + (t.q < t.ncol ? t.q : 0);
+    const int64_t gcol = t.q < t.ncol ? col0 + t.q : 0;
     const double fbot = a.forc_bot[gcol], fsurf = a.forc_surf[gcol];
     double e0[S], e1[S], rate[S], f[S];
     {
