@@ -19,7 +19,7 @@
 #include <map>
 #include <mutex>
 
-#include "tdma_seg.hpp"
+#include "col_tile.hpp"
 
 // Tuning knob (compile-time): minimum waves per SIMD requested for the pre
 // kernel (caps its VGPRs).
@@ -1312,10 +1312,12 @@ __global__ __launch_bounds__(kWetThreads) __attribute__((amdgpu_waves_per_eu(VX_
 //   T_new = T[taup1]                                   elsewhere,
 // with D the flux divergence (linear in T[tau], and in K_iso through K1 = K2 =
 // K_iso). Given mu = dL/dT_new:
-//   adj_column : lam = M^-T mu (transposed K33 Thomas, rows re-derived from
-//                K_33), g_taup1 = lam, nu = dt * lam on interior cells
-//   adj_faces  : adjoints of flux_east / flux_north / flux_top from nu
-//   adj_scatter: each face scatters (atomics) into dL/dT[tau] and dL/dK_iso
+//   adj_column : lam = M^-T mu (transposed K33 system, rows re-derived from
+//                K_33), g_taup1 = lam, nu = dt * lam on the interior wet cells and
+//                0 elsewhere, g_tau = g_K = 0
+//   adj_scatter: the adjoints of flux_east / flux_north / flux_top from nu, and
+//                each face's contributions to dL/dT[tau] and dL/dK_iso, summed
+//                over the levels they reach and added to the columns (atomics)
 // ---------------------------------------------------------------------------
 struct AdjArgs {
     const double* tr;       // forward input tracer (X, Y, nz, 3), level tau read
@@ -1324,202 +1326,204 @@ struct AdjArgs {
     const double *Aez, *Anz, *Abx, *Aby, *K11, *K22, *K33;
     const double* mu;       // dL/dT_new (X, Y, nz)
     double *g_tau, *g_taup1, *g_K;
-    double *nu, *mfe, *mfn, *mft;  // workspace (X, Y, nz) each
+    double* nu;             // workspace (X, Y, nz); the caller's holds four such arrays
 };
 
-// g_taup1 = mu, nu = 0 on interior cells below, g_tau = g_K = 0 everywhere
-__global__ __launch_bounds__(256) void iso_adj_init_kernel(int64_t n, AdjArgs a) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    a.g_taup1[t] = a.mu[t];
-    a.g_tau[t] = 0.0;
-    a.g_K[t] = 0.0;
-    a.nu[t] = 0.0;
-    a.mfe[t] = 0.0;
-    a.mfn[t] = 0.0;
-    a.mft[t] = 0.0;
-}
-
-template <int NZB>
-__global__ __launch_bounds__(256) void iso_adj_column_kernel(Grid g, Prm p, AdjArgs a) {
+// A wave per tile of 8 columns of the whole grid (col_tile.hpp): one flat pass
+// over K_33 and mu. A lane per column with the factors in registers, and an
+// initialisation pass before it, took 50 + 8 us on 180x90x40, this @@ us.
+constexpr int kAdjP = 8;
+constexpr int kAdjBlock = 128;
+template <int S>
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2))) void iso_adj_column_kernel(Grid g, Prm p, AdjArgs a) {
+    using T = Tile<S, kAdjP>;
+    __shared__ double lds[kAdjBlock / 64][T::IMG];
+    __shared__ double rdt[kMaxNz], dtw[kMaxNz];  // 1 / dzt, dt / dzw
     const int nz = g.nz;
-    const int ny4 = g.Y - 4;
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= (int64_t)(g.X - 4) * ny4) return;
-    const int i = 2 + (int)(col / ny4);
-    const int j = 2 + (int)(col - (int64_t)(i - 2) * ny4);
-    const int kb = kb_of(g, i, j);
-    const int k0 = (kb >= 1 && kb <= nz) ? kb - 1 : nz;
-    const int64_t o = idx3(g, i, j, 0);
-    const double dt = p.dt_tracer;
-    // transposed rows: sub'[k] = c[k-1] = -delta[k-1]/dzt[k-1], sup'[k] = a[k+1] = -delta[k]/dzt[k+1]
-    double cp[NZB], lm[NZB];
-    double cpp = 0.0, dpp = 0.0, delta_m = 0.0;
+    for (int k = threadIdx.x; k < nz; k += kAdjBlock) {
+        rdt[k] = 1.0 / g.dzt[k];
+        dtw[k] = p.dt_tracer / g.dzw[k];
+    }
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    double* const img = lds[wave];
+    const int64_t col0 = ((int64_t)blockIdx.x * (kAdjBlock / 64) + wave) * T::C;
+    const int64_t left = (int64_t)g.X * g.Y - col0;
+    const int n = left >= T::C ? T::C : (left > 0 ? (int)left : 0);
+    const T t = make_tile<S, kAdjP>(n > 0 ? col0 * nz : 0, n, nz, (uint32_t)nz);
+    SegLane L;
+    L.s = t.s;
+    L.lo = t.lo;
+    L.valid = t.q < n;
+    const int64_t col = L.valid ? col0 + t.q : 0;
+    const int i = (int)(col / g.Y), j = (int)(col - (int64_t)i * g.Y);
+    const bool interior = L.valid && i >= 2 && i <= g.X - 3 && j >= 2 && j <= g.Y - 3;
+    const int kb = g.kbot[col];
+    L.k0 = interior && kb >= 1 && kb <= nz ? kb - 1 : nz;
+    L.base = 0;
+    double mu[S], z[S], va[S], vb[S], vc[S];
+    {
+        double kv[S];
+        uint32_t wet[S];
 #pragma unroll
-    for (int k = 0; k < NZB; ++k) {
-        if (k < nz && k >= k0) {
-            const double delta = (k < nz - 1) ? dt / g.dzw[k] * a.K33[o + k] : 0.0;
-            const bool edge = k == k0;
-            const double dz = g.dzt[k];
-            const double diag = edge ? 1 + delta / dz : 1 + (delta + delta_m) / dz;
-            const double sub = edge ? 0.0 : -delta_m / g.dzt[k - 1];
-            const double sup = (k < nz - 1) ? -delta / g.dzt[k + 1] : 0.0;
-            const double r = 1.0 / (diag - sub * cpp);
-            cpp = sup * r;
-            dpp = (a.mu[o + k] - sub * dpp) * r;
-            delta_m = delta;
-        }
-        cp[k] = cpp;
-        lm[k] = dpp;
+        for (int r = 0; r < S; ++r) wet[r] = t.k[r] >= __shfl(L.k0, t.c[r] * kAdjP) ? t.off[r] : kNoAccess;
+        tile_load(tile_buf(t, a.K33), wet, 1, kv);
+        tile_load(tile_buf(t, a.mu), t.off, 1, mu);
+        tile_put(t, img, kv);
     }
-    double ln = 0.0;
+    double km[S];
+    seg_get(t, img, km);
+    const double below = seg_below(t, img);
+    tile_put(t, img, mu);
+    seg_get(t, img, z);
+    // sub'[k] = c[k-1] = -delta[k-1] / dzt[k-1], sup'[k] = a[k+1] = -delta[k] / dzt[k+1]
+    double dm = L.lo > L.k0 && L.lo < nz ? dtw[L.lo - 1] * below : 0.0;
 #pragma unroll
-    for (int k = NZB - 1; k >= 0; --k) {
-        if (k < nz && k >= k0) {
-            ln = lm[k] - cp[k] * ln;
-            lm[k] = ln;
-        }
+    for (int r = 0; r < S; ++r) {
+        const int k = L.lo + r;
+        const bool w = k >= L.k0 && k < nz;
+        const int kc = k < nz ? k : nz - 1;
+        const double dl = w && k < nz - 1 ? dtw[kc] * km[r] : 0.0;
+        va[r] = w && k > L.k0 ? -dm * rdt[kc > 0 ? kc - 1 : 0] : 0.0;
+        vb[r] = w ? 1 + (dl + dm) * rdt[kc] : 1.0;
+        vc[r] = w && k < nz - 1 ? -dl * rdt[kc < nz - 1 ? kc + 1 : kc] : 0.0;
+        z[r] = w ? z[r] : 0.0;
+        dm = dl;
     }
+    seg_solve_f64<S>(L, va, vb, vc, z);
+    seg_put(t, img, z);
+    double lam[S], nu[S];
+    tile_get(t, img, lam);
 #pragma unroll
-    for (int k = 0; k < NZB; ++k) {
-        if (k < nz) {
-            const double lam = (k >= k0) ? lm[k] : a.mu[o + k];
-            if (k >= k0) a.g_taup1[o + k] = lam;
-            a.nu[o + k] = dt * lam;
-        }
+    for (int r = 0; r < S; ++r) {
+        const bool w = t.k[r] >= __shfl(L.k0, t.c[r] * kAdjP);
+        nu[r] = w ? p.dt_tracer * lam[r] : 0.0;
+        lam[r] = w ? lam[r] : mu[r];
+        z[r] = 0.0;
     }
-}
-
-// adjoints of the face fluxes: dtr = m*((fe - fe_w)/(cost dxt) + (fn - fn_s)/(cost dyt)) + m*(ft - ft_m)/dzt
-__global__ __launch_bounds__(256) void iso_adj_faces_kernel(Grid g, AdjArgs a) {
-    const CellIdx ci = cell_of(1, g.X - 3, 1, g.Y - 3);
-    if (!ci.valid) return;
-    const int i = ci.i, j = ci.j, k = ci.k;
-    const int nz = g.nz;
-    const uint32_t si = (uint32_t)g.Y * (uint32_t)nz, sj = (uint32_t)nz;
-    const uint32_t c = (uint32_t)i * si + (uint32_t)j * sj + (uint32_t)k;
-    auto inner = [&](int ii, int jj) { return ii >= 2 && ii <= g.X - 3 && jj >= 2 && jj <= g.Y - 3; };
-    auto wnu = [&](int ii, int jj, int kk, uint32_t o) {
-        return inner(ii, jj) ? a.nu[o] * m01(kb_of(g, ii, jj), kk) : 0.0;
-    };
-    if (j >= 2) {  // flux_east at (i, j, k): divergence of cells i and i+1
-        a.mfe[c] = wnu(i, j, k, c) / (g.cost[j] * g.dxt[i]) - wnu(i + 1, j, k, c + si) / (g.cost[j] * g.dxt[i + 1]);
-    }
-    if (i >= 2) {  // flux_north at (i, j, k): cells j and j+1
-        a.mfn[c] = wnu(i, j, k, c) / (g.cost[j] * g.dyt[j]) - wnu(i, j + 1, k, c + sj) / (g.cost[j + 1] * g.dyt[j + 1]);
-    }
-    if (i >= 2 && j >= 2 && k < nz - 1) {  // flux_top at (i, j, k): levels k and k+1
-        a.mft[c] = wnu(i, j, k, c) / g.dzt[k] - wnu(i, j, k + 1, c + 1) / g.dzt[k + 1];
-    }
+    tile_store(tile_buf(t, a.g_taup1), t.off, 1, lam);
+    tile_store(tile_buf(t, a.nu), t.off, 1, nu);
+    tile_store(tile_buf(t, a.g_tau), t.off, 1, z);
+    tile_store(tile_buf(t, a.g_K), t.off, 1, z);
 }
 
 __device__ __forceinline__ void adj_add(double* p, double v) {
     if (v != 0.0) unsafeAtomicAdd(p, v);
 }
 
+// Thread per cell (i, j, k), i in [1, X-2), j in [1, Y-2): the three faces whose
+// lower cell it is. A face's contributions go to the levels k-1, k and k+1 of the
+// cell's own, east, north, west and south columns (and of the first three for
+// K_iso); those of the levels next to it pass through LDS to the thread of
+// that level, so each thread adds 8 sums instead of up to 35 single terms
+// (180x90x40: 43 us and 11 us for a kernel that stored the face adjoints first;
+// now @@ us).
 __global__ __launch_bounds__(256) void iso_adj_scatter_kernel(Grid g, AdjArgs a) {
     const CellIdx ci = cell_of(1, g.X - 3, 1, g.Y - 3);
-    if (!ci.valid) return;
-    const int i = ci.i, j = ci.j, k = ci.k;
     const int nz = g.nz;
     const uint32_t si = (uint32_t)g.Y * (uint32_t)nz, sj = (uint32_t)nz;
+    const int i = ci.valid ? ci.i : 1, j = ci.valid ? ci.j : 1, k = ci.k;
     const uint32_t c = (uint32_t)i * si + (uint32_t)j * sj + (uint32_t)k;
+    const uint32_t ce = c + si, cn = c + sj;
     const double* __restrict__ tr = a.tr + (uint32_t)a.tau * g.ls;
-    const bool hm = k >= 1;
-    const uint32_t up = (k + 1 < nz) ? 1u : 0u, dn = hm ? 1u : 0u;
+    const bool hm = k >= 1, hp = k + 1 < nz;
+    const uint32_t up = hp ? 1u : 0u, dn = hm ? 1u : 0u;
     const double* K = a.Kiso;
-
-    if (j >= 2) {  // flux_east (veros/core/isoneutral/diffusion.py:22-47)
-        const double mu = a.mfe[c];
-        if (mu != 0.0) {
-            const uint32_t ce = c + si;
-            const double diffloc = hm ? 0.25 * (K[c] + K[c - 1] + K[ce] + K[ce - 1]) : 0.5 * (K[c] + K[ce]);
-            const double* A = a.Aez + 4u * c;  // (ip, kr) at 2 ip + kr
-            const double q4 = 1.0 / (4.0 * g.dzt[k]);
+    // columns: 0 own, 1 east, 2 north, 3 west, 4 south; at level k, and passed up and down
+    double c0[5] = {}, cu[5] = {}, cd[3] = {}, k0[3] = {}, kd[3] = {};
+    if (ci.valid) {
+        const double nc = a.nu[c], ne = a.nu[ce], nn = a.nu[cn], nt = hp ? a.nu[c + 1] : 0.0;
+        const double cost = g.cost[j];
+        const double mue = j >= 2 ? nc / (cost * g.dxt[i]) - ne / (cost * g.dxt[i + 1]) : 0.0;
+        const double mun =
+            i >= 2 ? (nc / (cost * g.dyt[j]) - nn / (g.cost[j + 1] * g.dyt[j + 1])) * g.cosu[j] : 0.0;
+        const double mut = i >= 2 && j >= 2 && hp ? nc / g.dzt[k] - nt / g.dzt[k + 1] : 0.0;
+        const double q4 = 1.0 / (4.0 * g.dzt[k]);
+        // flux_east and flux_north (veros/core/isoneutral/diffusion.py:22-77)
+        auto lateral = [&](int q, double mu, uint32_t cx, const double* A, double k_over_d) {
+            if (mu == 0.0) return;
+            const double diffloc = hm ? 0.25 * (K[c] + K[c - 1] + K[cx] + K[cx - 1]) : 0.5 * (K[c] + K[cx]);
             const double t0 = tr[g.cs * c], t0u = tr[g.cs * (c + up)], t0d = tr[g.cs * (c - dn)];
-            const double t1 = tr[g.cs * ce], t1u = tr[g.cs * (ce + up)], t1d = tr[g.cs * (ce - dn)];
-            // diffloc terms
-            const double w00 = mu * diffloc * A[0] * q4, w01 = mu * diffloc * A[1] * q4;
-            const double w10 = mu * diffloc * A[2] * q4, w11 = mu * diffloc * A[3] * q4;
-            adj_add(a.g_tau + c, w00 - w01);
-            adj_add(a.g_tau + c - dn, -w00);
-            adj_add(a.g_tau + c + up, w01);
-            adj_add(a.g_tau + ce, w10 - w11);
-            adj_add(a.g_tau + ce - dn, -w10);
-            adj_add(a.g_tau + ce + up, w11);
-            // K_11 term
-            const double wk = mu * a.K11[c] / (g.cost[j] * g.dxu[i]);
-            adj_add(a.g_tau + ce, wk);
-            adj_add(a.g_tau + c, -wk);
-            // K_iso through diffloc
-            const double S = (A[0] * (t0 - t0d) + A[2] * (t1 - t1d) + A[1] * (t0u - t0) + A[3] * (t1u - t1)) * q4;
+            const double t1 = tr[g.cs * cx], t1u = tr[g.cs * (cx + up)], t1d = tr[g.cs * (cx - dn)];
+            const double2 A01 = *reinterpret_cast<const double2*>(A + 4u * c);
+            const double2 A23 = *reinterpret_cast<const double2*>(A + 4u * c + 2);
+            const double m = mu * diffloc * q4, wk = mu * k_over_d;
+            const double w00 = m * A01.x, w01 = m * A01.y, w10 = m * A23.x, w11 = m * A23.y;
+            c0[0] += w00 - w01 - wk;
+            c0[q] += w10 - w11 + wk;
+            // the clamped ends keep their terms
+            c0[0] += (hp ? 0.0 : w01) - (hm ? 0.0 : w00);
+            c0[q] += (hp ? 0.0 : w11) - (hm ? 0.0 : w10);
+            cu[0] += hp ? w01 : 0.0;
+            cu[q] += hp ? w11 : 0.0;
+            cd[0] -= hm ? w00 : 0.0;
+            cd[q] -= hm ? w10 : 0.0;
+            const double S = (A01.x * (t0 - t0d) + A23.x * (t1 - t1d) + A01.y * (t0u - t0) + A23.y * (t1u - t1)) * q4;
             const double wK = mu * S * (hm ? 0.25 : 0.5);
-            adj_add(a.g_K + c, wK);
-            adj_add(a.g_K + ce, wK);
-            if (hm) {
-                adj_add(a.g_K + c - 1, wK);
-                adj_add(a.g_K + ce - 1, wK);
-            }
-        }
-    }
-    if (i >= 2) {  // flux_north (:49-77)
-        const double mu = a.mfn[c] * g.cosu[j];
-        if (mu != 0.0) {
-            const uint32_t cn = c + sj;
-            const double diffloc = hm ? 0.25 * (K[c] + K[c - 1] + K[cn] + K[cn - 1]) : 0.5 * (K[c] + K[cn]);
-            const double* A = a.Anz + 4u * c;
-            const double q4 = 1.0 / (4.0 * g.dzt[k]);
-            const double t0 = tr[g.cs * c], t0u = tr[g.cs * (c + up)], t0d = tr[g.cs * (c - dn)];
-            const double t1 = tr[g.cs * cn], t1u = tr[g.cs * (cn + up)], t1d = tr[g.cs * (cn - dn)];
-            const double w00 = mu * diffloc * A[0] * q4, w01 = mu * diffloc * A[1] * q4;
-            const double w10 = mu * diffloc * A[2] * q4, w11 = mu * diffloc * A[3] * q4;
-            adj_add(a.g_tau + c, w00 - w01);
-            adj_add(a.g_tau + c - dn, -w00);
-            adj_add(a.g_tau + c + up, w01);
-            adj_add(a.g_tau + cn, w10 - w11);
-            adj_add(a.g_tau + cn - dn, -w10);
-            adj_add(a.g_tau + cn + up, w11);
-            const double wk = mu * a.K22[c] / g.dyu[j];
-            adj_add(a.g_tau + cn, wk);
-            adj_add(a.g_tau + c, -wk);
-            const double S = (A[0] * (t0 - t0d) + A[2] * (t1 - t1d) + A[1] * (t0u - t0) + A[3] * (t1u - t1)) * q4;
-            const double wK = mu * S * (hm ? 0.25 : 0.5);
-            adj_add(a.g_K + c, wK);
-            adj_add(a.g_K + cn, wK);
-            if (hm) {
-                adj_add(a.g_K + c - 1, wK);
-                adj_add(a.g_K + cn - 1, wK);
-            }
-        }
-    }
-    if (i >= 2 && j >= 2 && k < nz - 1) {  // flux_top (:79-111)
-        const double mu = a.mft[c];
-        if (mu != 0.0) {
-            const double K2 = K[c];
+            k0[0] += wK;
+            k0[q] += wK;
+            kd[0] += hm ? wK : 0.0;
+            kd[q] += hm ? wK : 0.0;
+        };
+        lateral(1, mue, ce, a.Aez, a.K11[c] / (cost * g.dxu[i]));
+        lateral(2, mun, cn, a.Anz, a.K22[c] / g.dyu[j]);
+        if (mut != 0.0) {  // flux_top (:79-111)
+            const double m = mut * K[c];
             const double* B = a.Abx + 4u * c;
             const double* C = a.Aby + 4u * c;
-            const uint32_t cw = c - si, ce = c + si, cs = c - sj, cn = c + sj;
-            const double fx = 1.0 / (4 * g.dxt[i]) / g.cost[j];
-            const double fy = 1.0 / (4 * g.dyt[j] * g.cost[j]);
+            const uint32_t cw = c - si, cs = c - sj;
+            const double fx = 1.0 / (4 * g.dxt[i]) / cost;
+            const double fy = 1.0 / (4 * g.dyt[j] * cost);
             double S = 0.0;
 #pragma unroll
             for (int kr = 0; kr < 2; ++kr) {
                 // x: (ip=0) tr[i] - tr[i-1], (ip=1) tr[i+1] - tr[i], at level k + kr
                 const double bx0 = B[kr] * fx, bx1 = B[2 + kr] * fx;
                 const double cy0 = C[kr] * g.cosu[j - 1] * fy, cy1 = C[2 + kr] * g.cosu[j] * fy;
-                const uint32_t ck = c + kr;
-                S += bx0 * (tr[g.cs * ck] - tr[g.cs * (cw + kr)]) + bx1 * (tr[g.cs * (ce + kr)] - tr[g.cs * ck]) +
-                     cy0 * (tr[g.cs * ck] - tr[g.cs * (cs + kr)]) + cy1 * (tr[g.cs * (cn + kr)] - tr[g.cs * ck]);
-                const double m = mu * K2;
-                adj_add(a.g_tau + ck, m * (bx0 - bx1 + cy0 - cy1));
-                adj_add(a.g_tau + cw + kr, -m * bx0);
-                adj_add(a.g_tau + ce + kr, m * bx1);
-                adj_add(a.g_tau + cs + kr, -m * cy0);
-                adj_add(a.g_tau + cn + kr, m * cy1);
+                const double t = tr[g.cs * (c + kr)];
+                S += bx0 * (t - tr[g.cs * (cw + kr)]) + bx1 * (tr[g.cs * (ce + kr)] - t) +
+                     cy0 * (t - tr[g.cs * (cs + kr)]) + cy1 * (tr[g.cs * (cn + kr)] - t);
+                double(&o)[5] = kr ? cu : c0;
+                o[0] += m * (bx0 - bx1 + cy0 - cy1);
+                o[1] += m * bx1;
+                o[2] += m * cy1;
+                o[3] -= m * bx0;
+                o[4] -= m * cy0;
             }
-            adj_add(a.g_K + c, mu * S);
+            k0[0] += mut * S;
         }
     }
+    // sums over the levels: from the thread below (its k + 1) and above (its k - 1)
+    __shared__ double lu[5][256], ld[6][256];
+    const int tid = (int)(threadIdx.y * blockDim.x + threadIdx.x);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) lu[q][tid] = cu[q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        ld[q][tid] = cd[q];
+        ld[3 + q][tid] = kd[q];
+    }
+    __syncthreads();
+    if (!ci.valid) return;
+    if (hm) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) c0[q] += lu[q][tid - 1];
+    }
+    if (hp) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            c0[q] += ld[q][tid + 1];
+            k0[q] += ld[3 + q][tid + 1];
+        }
+    }
+    adj_add(a.g_tau + c, c0[0]);
+    adj_add(a.g_tau + ce, c0[1]);
+    adj_add(a.g_tau + cn, c0[2]);
+    adj_add(a.g_tau + (c - si), c0[3]);
+    adj_add(a.g_tau + (c - sj), c0[4]);
+    adj_add(a.g_K + c, k0[0]);
+    adj_add(a.g_K + ce, k0[1]);
+    adj_add(a.g_K + cn, k0[2]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1927,35 +1931,28 @@ extern "C" int vx_iso_diffusion_adjoint_f64(void* stream, const vx_grid* grid, c
         return fail(VX_ERR_INVALID_ARGUMENT, "%s: null array pointer", who);
     if ((int64_t)g.X * g.Y * g.nz * 4 >= ((int64_t)1 << 32))
         return fail(VX_ERR_UNSUPPORTED, "%s: grid too large for 32-bit offsets", who);
-    const int64_t n3 = (int64_t)g.X * g.Y * g.nz;
-    double* w = static_cast<double*>(workspace);
     AdjArgs a{tracer, tau, K_iso, Ai_ez, Ai_nz, Ai_bx, Ai_by, K_11, K_22, K_33, g_new, g_tau, g_taup1, g_K_iso,
-              w, w + n3, w + 2 * n3, w + 3 * n3};
+              static_cast<double*>(workspace)};
     hipStream_t s = (hipStream_t)stream;
     const Prm p = make_prm(prm);
-    hipLaunchKernelGGL(iso_adj_init_kernel, dim3(blocks_for(n3, 256)), dim3(256), 0, s, n3, a);
-    if ((rc = check_launch(who))) return rc;
-    const int64_t ncol = (int64_t)(g.X - 4) * (g.Y - 4);
-    const int nzb = ((g.nz + 15) / 16) * 16;
-    const dim3 cgrid(blocks_for(ncol, 256)), cblk(256);
+    const int64_t ntiles = ((int64_t)g.X * g.Y + 64 / kAdjP - 1) / (64 / kAdjP);
+    const dim3 cgrid(blocks_for(ntiles * 64, kAdjBlock)), cblk(kAdjBlock);
 #define VX_ADJ_CASE(N) \
     case N: hipLaunchKernelGGL(iso_adj_column_kernel<N>, cgrid, cblk, 0, s, g, p, a); break;
-    switch (nzb) {
+    switch (seg_levels(g.nz)) {
+        VX_ADJ_CASE(2)
+        VX_ADJ_CASE(4)
+        VX_ADJ_CASE(6)
+        VX_ADJ_CASE(8)
+        VX_ADJ_CASE(10)
+        VX_ADJ_CASE(12)
+        VX_ADJ_CASE(14)
         VX_ADJ_CASE(16)
-        VX_ADJ_CASE(32)
-        VX_ADJ_CASE(48)
-        VX_ADJ_CASE(64)
-        VX_ADJ_CASE(80)
-        VX_ADJ_CASE(96)
-        VX_ADJ_CASE(112)
-        VX_ADJ_CASE(128)
         default: return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, g.nz);
     }
 #undef VX_ADJ_CASE
     if ((rc = check_launch(who))) return rc;
     const dim3 blk = cell_block(g.nz);
-    hipLaunchKernelGGL(iso_adj_faces_kernel, cell_grid(g.X - 3, g.Y - 3, blk), blk, 0, s, g, a);
-    if ((rc = check_launch(who))) return rc;
     hipLaunchKernelGGL(iso_adj_scatter_kernel, cell_grid(g.X - 3, g.Y - 3, blk), blk, 0, s, g, a);
     return check_launch(who);
 }

@@ -82,64 +82,85 @@ struct TdmaAdjArgs {
     double *gbe, *gde;  // dL/db_edge, dL/dd_edge (nullable; used when b_edge / d_edge were given)
 };
 
-template <int NZB>
-__global__ __launch_bounds__(kTdmaBlock) void tdma_adjoint_kernel(TdmaAdjArgs q) {
+// On column tiles (tdma_tile.hpp): the transposed rows take c from the level
+// below and a from the level above out of the images, lam comes back flat, and
+// every gradient is formed and stored cell by cell. One lane per column with
+// the column's factors in registers (16,200 columns of 180x90x40: 63 blocks)
+// took 72 us there, the tiles @@ us.
+template <int S>
+__global__ __launch_bounds__(kSegLdsBlock) __attribute__((amdgpu_waves_per_eu(2))) void tdma_adjoint_kernel(TdmaAdjArgs q, TdmaTiling g) {
+    __shared__ double lds[kSegLdsBlock / 64][2][tdma_tile_lds<S>()];
     const TdmaArgs& p = q.f;
-    ColumnRef cr;
-    if (!column_of(p, cr)) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    double* const img = lds[wave][0];
+    double* const ximg = lds[wave][1];
+    SegLane L;
+    const Tile<S, kTdmaP> t = tdma_tile_of<S>(p, g, (int64_t)blockIdx.x * (kSegLdsBlock / 64) + wave, L);
     const int nz = p.nz;
-    const int k0 = cr.k0;
-    const int64_t o = cr.base;
-    const bool has_be = p.b_edge != nullptr;
-    const bool has_de = p.d_edge != nullptr;
-    double cp[NZB], lm[NZB];
-    double cpp = 0.0, dpp = 0.0;
+    uint32_t wet[S];
 #pragma unroll
-    for (int k = 0; k < NZB; ++k) {
-        if (k < nz && k >= k0) {
-            const double sub = (k > k0) ? p.c[o + k - 1] : 0.0;
-            const double diag = (k == k0 && has_be) ? p.b_edge[o + k] : p.b[o + k];
-            const double sup = (k < nz - 1) ? p.a[o + k + 1] : 0.0;
-            const double r = 1.0 / (diag - sub * cpp);
-            cpp = sup * r;
-            dpp = (q.g[o + k] - sub * dpp) * r;
-        }
-        cp[k] = cpp;
-        lm[k] = dpp;
-    }
-    double ln = 0.0;
+    for (int r = 0; r < S; ++r) wet[r] = t.k[r] >= __shfl(L.k0, t.c[r] * kTdmaP) ? t.off[r] : kNoAccess;
+    double sub[S], diag[S], sup[S], z[S], x[S], be, de;
+    {
+        double fa[S], fc[S];
+        tile_load(tile_buf(t, p.c), wet, 1, fc);
+        tile_load(tile_buf(t, p.a), wet, 1, fa);
+        tile_load(tile_buf(t, p.b), wet, 1, diag);
+        tile_load(tile_buf(t, q.g), wet, 1, z);
+        tile_load(tile_buf(t, (const double*)p.x), wet, 1, x);
+        seg_edge_values(p, L, S, be, de);
+        double v[S];
+        tile_put(t, img, fc);
+        seg_get(t, img, v);
+        sub[0] = seg_below(t, img);
 #pragma unroll
-    for (int k = NZB - 1; k >= 0; --k) {
-        if (k < nz && k >= k0) {
-            ln = lm[k] - cp[k] * ln;
-            lm[k] = ln;
-        }
-    }
-    double xm = 0.0;  // x[k-1]
+        for (int r = 1; r < S; ++r) sub[r] = v[r - 1];
+        tile_put(t, img, fa);
+        seg_get(t, img, v);
+        sup[S - 1] = seg_above(t, img);
 #pragma unroll
-    for (int k = 0; k < NZB; ++k) {
-        if (k < nz) {
-            double ga = 0.0, gb = 0.0, gc = 0.0, gd = 0.0, gbe = 0.0, gde = 0.0;
-            if (k >= k0) {
-                const double lam = lm[k];
-                const double xk = p.x[o + k];
-                const bool edge = k == k0;
-                if (edge && has_de) gde = lam;
-                else gd = lam;
-                if (edge && has_be) gbe = -lam * xk;
-                else gb = -lam * xk;
-                if (!edge) ga = -lam * xm;
-                if (k < nz - 1) gc = -lam * p.x[o + k + 1];
-                xm = xk;
-            }
-            q.ga[o + k] = ga;
-            q.gb[o + k] = gb;
-            q.gc[o + k] = gc;
-            q.gd[o + k] = gd;
-            if (q.gbe) q.gbe[o + k] = gbe;
-            if (q.gde) q.gde[o + k] = gde;
-        }
+        for (int r = 0; r < S - 1; ++r) sup[r] = v[r + 1];
+        tile_put(t, img, diag);
+        seg_get(t, img, diag);
+        tile_put(t, img, z);
+        seg_get(t, img, z);
+        tile_put(t, ximg, x);
     }
+    seg_mask_rows<S>(p, L, be, 0.0, sub, diag, sup, z, false);
+    seg_solve_f64<S>(L, sub, diag, sup, z);
+    seg_put(t, img, z);
+    double lam[S], ga[S], gb[S], gc[S], gd[S];
+    tile_get(t, img, lam);
+    const bool has_be = p.b_edge != nullptr, has_de = p.d_edge != nullptr;
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        const int k = t.k[r], k0 = __shfl(L.k0, t.c[r] * kTdmaP);
+        const bool w = k >= k0, edge = k == k0;
+        const int seg0 = k % S == 0 ? Tile<S, kTdmaP>::SP - S : 0, seg1 = k % S == S - 1 ? Tile<S, kTdmaP>::SP - S : 0;
+        const double xm = ximg[w && !edge ? t.pos[r] - 1 - seg0 : t.pos[r]];
+        const double xp = ximg[w && k < nz - 1 ? t.pos[r] + 1 + seg1 : t.pos[r]];
+        const double l = w ? lam[r] : 0.0;
+        ga[r] = edge ? 0.0 : -l * xm;
+        gb[r] = -l * x[r];
+        gc[r] = k < nz - 1 ? -l * xp : 0.0;
+        gd[r] = l;
+    }
+    tile_store(tile_buf(t, q.ga), t.off, 1, ga);
+    tile_store(tile_buf(t, q.gc), t.off, 1, gc);
+    // the edge row's derivatives go to the edge arrays when those were given
+    auto split = [&](const double(&v)[S], double* inner, double* at_edge, bool has) {
+        double e[S], i[S];
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const bool edge = has && t.k[r] == __shfl(L.k0, t.c[r] * kTdmaP);
+            e[r] = edge ? v[r] : 0.0;
+            i[r] = edge ? 0.0 : v[r];
+        }
+        tile_store(tile_buf(t, inner), t.off, 1, i);
+        if (at_edge) tile_store(tile_buf(t, at_edge), t.off, 1, e);
+    };
+    split(gb, q.gb, q.gbe, has_be);
+    split(gd, q.gd, q.gde, has_de);
 }
 
 // ---------------------------------------------------------------------------
@@ -428,20 +449,21 @@ extern "C" int vx_tdma_adjoint_f64(void* stream, const double* a, const double* 
         return fail(VX_ERR_INVALID_ARGUMENT, "%s: gb_edge/gd_edge must be given exactly when b_edge/d_edge are",
                     who);
     TdmaAdjArgs q{p, gx, ga, gb, gc, gd, gb_edge, gd_edge};
-    const int nzb = ((nz + 15) / 16) * 16;
-    const dim3 grid((unsigned)((p.ncol + kTdmaBlock - 1) / kTdmaBlock)), block(kTdmaBlock);
+    const TdmaTiling g = tdma_tiling(p);
+    const int waves = kSegLdsBlock / 64;
+    const dim3 grid((unsigned)((g.ntiles + waves - 1) / waves)), block(kSegLdsBlock);
     hipStream_t s = (hipStream_t)stream;
 #define VX_ADJ_CASE(N) \
-    case N: hipLaunchKernelGGL(tdma_adjoint_kernel<N>, grid, block, 0, s, q); break;
-    switch (nzb) {
+    case N: hipLaunchKernelGGL(tdma_adjoint_kernel<N>, grid, block, 0, s, q, g); break;
+    switch (seg_levels(nz)) {
+        VX_ADJ_CASE(2)
+        VX_ADJ_CASE(4)
+        VX_ADJ_CASE(6)
+        VX_ADJ_CASE(8)
+        VX_ADJ_CASE(10)
+        VX_ADJ_CASE(12)
+        VX_ADJ_CASE(14)
         VX_ADJ_CASE(16)
-        VX_ADJ_CASE(32)
-        VX_ADJ_CASE(48)
-        VX_ADJ_CASE(64)
-        VX_ADJ_CASE(80)
-        VX_ADJ_CASE(96)
-        VX_ADJ_CASE(112)
-        VX_ADJ_CASE(128)
         default: return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, nz);
     }
 #undef VX_ADJ_CASE

@@ -226,10 +226,12 @@ __device__ __forceinline__ void iface_solve(int s, double A, double B, double C,
 // The masked system on the lane's levels: identity rows off the wet suffix,
 // a = 0 (and b, d from b_edge, d_edge when given) at the edge row k0, c = 0
 // at the top row nz-1. Values at rows off the wet suffix may be garbage on
-// entry; they are replaced by selects.
+// entry; they are replaced by selects. edge_d off: d_edge is not applied (the
+// adjoint's right-hand side).
 template <int S>
 __device__ __forceinline__ void seg_mask_rows(const TdmaArgs& p, const SegLane& L, double be, double de,
-                                              double (&va)[S], double (&vb)[S], double (&vc)[S], double (&vd)[S]) {
+                                              double (&va)[S], double (&vb)[S], double (&vc)[S], double (&vd)[S],
+                                              bool edge_d = true) {
     const int nz = p.nz;
 #pragma unroll
     for (int t = 0; t < S; ++t) {
@@ -247,7 +249,7 @@ __device__ __forceinline__ void seg_mask_rows(const TdmaArgs& p, const SegLane& 
 #pragma unroll
         for (int t = 0; t < S; ++t) vb[t] = (t == ke) ? be : vb[t];
     }
-    if (p.d_edge != nullptr) {
+    if (edge_d && p.d_edge != nullptr) {
 #pragma unroll
         for (int t = 0; t < S; ++t) vd[t] = (t == ke) ? de : vd[t];
     }
