@@ -38,7 +38,14 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# the current stream's handle without building a Stream object (2.9 us a call),
+# where this torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle() -> int:
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
     return torch.cuda.current_stream().cuda_stream
 
 

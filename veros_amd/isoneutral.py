@@ -31,6 +31,7 @@ present, else from veros's linear EOS module values
 from __future__ import annotations
 
 from collections import namedtuple
+from functools import lru_cache
 
 import torch
 
@@ -44,9 +45,15 @@ LINEAR_EOS_BETA_T = 1.67e-4
 LINEAR_EOS_BETA_S = 0.78e-3
 
 
+@lru_cache(maxsize=64)
+def _output_type(names):
+    # one class per set of names: building it takes longer than most calls
+    return namedtuple("KernelOutput", names)
+
+
 def KernelOutput(**kw):
     """namedtuple built from keyword arguments (veros/state.py:16-20)."""
-    return namedtuple("KernelOutput", list(kw.keys()))(*kw.values())
+    return _output_type(tuple(kw))(*kw.values())
 
 
 def eos_derivatives(settings):

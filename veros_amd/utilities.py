@@ -53,11 +53,50 @@ def _same_layout(ts):
     return all(t.stride() == s for t in ts) and s[-1] == 1
 
 
+def _plain_operands(a, b, c, d, b_edge, d_edge, kbot):
+    """Whether the operands can be handed over as they are: float64 (nx, ny,
+    nz) tensors on the GPU of one layout, z contiguous, and an int32 kbot."""
+    if not (isinstance(a, torch.Tensor) and a.is_cuda and a.dtype == torch.float64 and a.dim() == 3):
+        return False
+    shape, strides = a.shape, a.stride()
+    if strides[2] != 1:
+        return False
+    for t in (b, c, d, b_edge, d_edge):
+        if t is None:
+            continue
+        if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float64 and t.shape == shape
+                and t.stride() == strides):
+            return False
+    if b is None or c is None or d is None:
+        return False
+    return isinstance(kbot, torch.Tensor) and kbot.is_cuda and kbot.dtype == torch.int32 and kbot.shape == shape[:2]
+
+
+def _solve(a, b, c, d, b_edge, d_edge, kb, precision, refine_steps, out):
+    shape, strides = a.shape, a.stride()
+    if out is None:
+        out = torch.empty_strided(shape, strides, dtype=torch.float64, device=a.device)
+    elif out.stride() != strides or out.shape != shape:
+        raise ValueError("out must match the inputs' shape and strides")
+    nx, ny, nz = shape
+    kx, ky = kb.stride()
+    L = _native.lib()
+    args = (stream_handle(), a.data_ptr(), b.data_ptr(), c.data_ptr(), d.data_ptr(), ptr(b_edge), ptr(d_edge),
+            kb.data_ptr(), kx, ky, out.data_ptr(), nx, ny, nz, strides[0], strides[1])
+    if precision == "fp64":
+        _native.check(L.vx_tdma_f64(*args), "vx_tdma_f64")
+    else:
+        _native.check(L.vx_tdma_mixed(*args, int(refine_steps)), "vx_tdma_mixed")
+    return out
+
+
 def solve_implicit_kbot(a, b, c, d, kbot, b_edge=None, d_edge=None, *, precision="fp64",
                         refine_steps=1, out=None):
     """Solve the kbot-masked tridiagonal systems; see include/vxmix.h (vx_tdma_f64)."""
     if precision not in PRECISIONS:
         raise ValueError(f"precision must be one of {PRECISIONS}")
+    if _plain_operands(a, b, c, d, b_edge, d_edge, kbot):
+        return _solve(a, b, c, d, b_edge, d_edge, kbot, precision, refine_steps, out)
     arrs = {"a": a, "b": b, "c": c, "d": d, "b_edge": b_edge, "d_edge": d_edge}
     dev = {}
     from_np = False
@@ -79,7 +118,7 @@ def solve_implicit_kbot(a, b, c, d, kbot, b_edge=None, d_edge=None, *, precision
     (shape,) = shapes
     if len(shape) != 3:
         raise ValueError(f"expected (nx, ny, nz) arrays, got shape {tuple(shape)}")
-    nx, ny, nz = shape
+    nx, ny, _ = shape
     kb, _ = to_device(kbot, torch.int32)
     if tuple(kb.shape) != (nx, ny):
         raise ValueError(f"kbot must have shape {(nx, ny)}, got {tuple(kb.shape)}")
@@ -88,19 +127,7 @@ def solve_implicit_kbot(a, b, c, d, kbot, b_edge=None, d_edge=None, *, precision
         for k in dev:
             if dev[k] is not None:
                 dev[k] = dev[k].contiguous()
-    if out is None:
-        out = torch.empty_strided(shape, dev["a"].stride(), dtype=torch.float64, device=dev["a"].device)
-    elif out.stride() != dev["a"].stride() or out.shape != shape:
-        raise ValueError("out must match the inputs' shape and strides")
-    sx, sy, _ = dev["a"].stride()
-    L = _native.lib()
-    args = [stream_handle(), ptr(dev["a"]), ptr(dev["b"]), ptr(dev["c"]), ptr(dev["d"]),
-            ptr(dev["b_edge"]), ptr(dev["d_edge"]), ptr(kb), kb.stride(0), kb.stride(1), ptr(out),
-            nx, ny, nz, sx, sy]
-    if precision == "fp64":
-        _native.check(L.vx_tdma_f64(*args), "vx_tdma_f64")
-    else:
-        _native.check(L.vx_tdma_mixed(*args, int(refine_steps)), "vx_tdma_mixed")
+    out = _solve(*(dev[k] for k in ("a", "b", "c", "d", "b_edge", "d_edge")), kb, precision, refine_steps, out)
     if from_np:
         return out.cpu().numpy()
     return out
