@@ -627,7 +627,7 @@ def main():
     traffic = PRE_TS_TRAFFIC_BYTES.get((nx, ny, nz, args.levels))
     roof = {"bound": "hbm",
             "kernel": "vx_iso_pre_diffusion_ts_f64 = wet_scan_{count,chunks,columns}_kernel + "
-                      "(iso_pre_dry_kernel || iso_pre_kernel<true> + k33_top_zero_kernel + iso_step_wet_kernel<2>)",
+                      "iso_pre_kernel<true> + iso_step_wet_kernel<2>",
             "achieved": round(gbs[dom], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs[dom] / HBM_PEAK_GBS, 4),
             "traffic": traffic,

@@ -1,7 +1,6 @@
 // Isoneutral triad-tensor stencils for gfx950 (float64).
 //
-//   iso_pre_dry_kernel, iso_pre_kernel
-//                        isoneutral_diffusion_pre  veros/core/isoneutral/isoneutral.py:18-229
+//   iso_pre_kernel       isoneutral_diffusion_pre  veros/core/isoneutral/isoneutral.py:18-229
 //   iso_flux_kernel      _calc_tracer_fluxes       veros/core/isoneutral/diffusion.py:9-113
 //   wet_scan_*_kernel    the wet-cell plan of a step (from kbot)
 //   iso_step_wet_kernel  _calc_explicit_part, _calc_implicit_part, the tracer and
@@ -16,6 +15,7 @@
 // contiguous run. Masks are derived from kbot exactly as calc_topo_kernel
 // builds them (veros/core/numerics.py:195-221): maskT = kbot>0 & k>=kbot-1,
 // maskU/V = min of the two adjacent maskT, maskW = min(maskT[k], maskT[k+1]).
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -24,7 +24,7 @@
 // Tuning knob (compile-time): minimum waves per SIMD requested for the pre
 // kernel (caps its VGPRs).
 #ifndef VX_PRE_MIN_WAVES
-#define VX_PRE_MIN_WAVES 3
+#define VX_PRE_MIN_WAVES 2
 #endif
 
 namespace vx {
@@ -178,13 +178,13 @@ __device__ __forceinline__ double rden(double drodz) { return rcp_nr(fmin(0.0, d
 #define VX_STRIP_BLOCKS 16
 #endif
 constexpr int kStripBlocks = VX_STRIP_BLOCKS;
-// the wet-cell pre kernel's blocks are wider (pre_columns): fewer per strip
-// (4 x 24 columns at nz = 80; measured on 1440x720x80, 16 per strip made the
-// fused pre + temperature/salinity call 1% slower, 8 5% slower)
-#ifndef VX_PRE_STRIP_BLOCKS
-#define VX_PRE_STRIP_BLOCKS 4
+// the pre and flux kernels' strips: columns along j (the fused call on
+// 1440x720x80 and the calls on 360x160x60, levels innermost: 96 columns
+// 6.00 ms and 1176 us, 192 6.05 and 1157, 384 6.09 and 1167)
+#ifndef VX_PRE_STRIP_COLS
+#define VX_PRE_STRIP_COLS 192
 #endif
-constexpr int kPreStripBlocks = VX_PRE_STRIP_BLOCKS;
+constexpr int kPreStripCols = VX_PRE_STRIP_COLS;
 
 struct CellIdx {
     int i, j, k;
@@ -229,48 +229,128 @@ __device__ __forceinline__ double m01(int kb, int k) { return (kb > 0 && kb - 1 
 // gradients are formed from them in registers. Offsets are 32-bit element
 // offsets (the host checks the arrays fit).
 // ---------------------------------------------------------------------------
+// Metric factors of a block's columns and of the levels, in LDS: the cells read
+// them as factors instead of dividing (a float64 division is about 14
+// instructions; pre with its fluxes had 35 divisions and reciprocals per cell).
+// Each is one division, made once per block.
+struct ColMetrics {
+    double rx, rxw;    // 1 / (dxu cost), the same at i-1
+    double ry, rys;    // 1 / dyu, the same at j-1
+    double rcost;      // 1 / cost
+    double cosu, cosus;
+    double fyc, fys;   // cosu dyu, the same at j-1
+    double ryt;        // 1 / (4 dyt cost)
+};
+struct LevelMetrics {
+    double rzw[kMaxNz];   // 1 / dzw
+    double dzw[kMaxNz];
+    double r4zt[kMaxNz];  // 1 / (4 dzt)
+};
+constexpr int kCellBlock = 64;  // threads of a pre or flux block: one wave
+constexpr int kBlockCols = 32;  // most columns of one
+struct BlockMetrics {
+    ColMetrics col[kBlockCols];
+    LevelMetrics lev;
+    int kb[kBlockCols + 2], kbe[kBlockCols], kbw[kBlockCols];  // kbot at j-1 .. j+1 of row i; at rows i+1, i-1
+    int run[kBlockCols + 1];                                   // prefix sums of the columns' run lengths
+};
+// Every thread of the block calls it; visible after the next barrier.
+__device__ __forceinline__ void fill_metrics(const Grid& g, int i, int jb, int ncb, BlockMetrics& m) {
+    const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
+    for (int q = tid; q < ncb; q += nthr) {
+        const int j = jb + q <= g.Y - 3 ? jb + q : g.Y - 3;
+        const double cost = g.cost[j], cosu = g.cosu[j], cosus = g.cosu[j - 1], dyu = g.dyu[j], dyus = g.dyu[j - 1];
+        ColMetrics& c = m.col[q];
+        c.rx = 1.0 / (cost * g.dxu[i]);
+        c.rxw = 1.0 / (cost * g.dxu[i - 1]);
+        c.ry = 1.0 / dyu;
+        c.rys = 1.0 / dyus;
+        c.rcost = 1.0 / cost;
+        c.cosu = cosu;
+        c.cosus = cosus;
+        c.fyc = cosu * dyu;
+        c.fys = cosus * dyus;
+        c.ryt = 1.0 / (4 * g.dyt[j] * cost);
+        m.kbe[q] = g.kbot[(i + 1) * g.Y + j];
+        m.kbw[q] = g.kbot[(i - 1) * g.Y + j];
+    }
+    for (int q = tid; q < ncb + 2; q += nthr) {
+        const int j = jb - 1 + q <= g.Y - 2 ? jb - 1 + q : g.Y - 2;
+        m.kb[q] = g.kbot[i * g.Y + j];
+    }
+    for (int k = tid; k < g.nz; k += nthr) {
+        const double dzw = g.dzw[k];
+        m.lev.dzw[k] = dzw;
+        m.lev.rzw[k] = 1.0 / dzw;
+        m.lev.r4zt[k] = 1.0 / (4.0 * g.dzt[k]);
+    }
+}
+// Turns r[1 .. ncb] (lengths) into prefix sums with r[0] = 0; between barriers.
+__device__ __forceinline__ void scan_runs(int* r, int ncb) {
+    if (threadIdx.x < 64) {
+        const int lane = (int)threadIdx.x;
+        int v = lane < ncb ? r[lane + 1] : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int u = __shfl_up(v, d);
+            v += lane >= d ? u : 0;
+        }
+        if (lane < ncb) r[lane + 1] = v;
+        if (lane == 0) r[0] = 0;
+    }
+}
+// the column q with run[q] <= t < run[q + 1]
+__device__ __forceinline__ int run_column(const BlockMetrics& m, int ncb, int t) {
+    int lo = 0, hi = ncb - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (m.run[mid] <= t) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 // Face-flux arithmetic (veros/core/isoneutral/diffusion.py:22-111), shared by
-// the flux kernel and the fused pre + flux kernel so both produce the same
-// values. A01/A23 are the (ip=0, kr=0..1) / (ip=1, kr=0..1) entries of Ai_ez or
+// the flux kernel and the fused pre + flux kernel; the fused multiply-adds are
+// written out so that both produce the same values, whatever the compiler
+// would contract in either. A01/A23 are the (ip=0, kr=0..1) / (ip=1, kr=0..1) entries of Ai_ez or
 // Ai_nz; t0* the tracer at the cell (u = k+1, d = k-1, clamped at the ends),
 // t1* at the east or north neighbour.
 __device__ __forceinline__ double east_flux_core(double diffloc, double2 A01, double2 A23, double t0, double t0u,
-                                                 double t0d, double t1, double t1u, double t1d, double dzt,
-                                                 double cost, double dxu, double K11) {
-    double sumz = 0.0;
-    sumz = sumz + diffloc * A01.x * (t0 - t0d);  // kr=0, ip=0
-    sumz = sumz + diffloc * A23.x * (t1 - t1d);  // kr=0, ip=1
-    sumz = sumz + diffloc * A01.y * (t0u - t0);  // kr=1, ip=0
-    sumz = sumz + diffloc * A23.y * (t1u - t1);  // kr=1, ip=1
-    return sumz / (4.0 * dzt) + (t1 - t0) / (cost * dxu) * K11;
+                                                 double t0d, double t1, double t1u, double t1d, double r4zt,
+                                                 double rx, double K11) {
+    double sumz = diffloc * A01.x * (t0 - t0d);     // kr=0, ip=0
+    sumz = fma(diffloc * A23.x, t1 - t1d, sumz);  // kr=0, ip=1
+    sumz = fma(diffloc * A01.y, t0u - t0, sumz);  // kr=1, ip=0
+    sumz = fma(diffloc * A23.y, t1u - t1, sumz);  // kr=1, ip=1
+    return fma(sumz, r4zt, (t1 - t0) * rx * K11);
 }
 __device__ __forceinline__ double north_flux_core(double diffloc, double2 A01, double2 A23, double t0, double t0u,
-                                                  double t0d, double t1, double t1u, double t1d, double dzt,
-                                                  double cosu, double dyu, double K22) {
-    double sumz = 0.0;
-    sumz = sumz + diffloc * A01.x * (t0 - t0d);
-    sumz = sumz + diffloc * A23.x * (t1 - t1d);
-    sumz = sumz + diffloc * A01.y * (t0u - t0);
-    sumz = sumz + diffloc * A23.y * (t1u - t1);
-    return cosu * (sumz / (4.0 * dzt) + (t1 - t0) / dyu * K22);
+                                                  double t0d, double t1, double t1u, double t1d, double r4zt,
+                                                  double cosu, double ry, double K22) {
+    double sumz = diffloc * A01.x * (t0 - t0d);
+    sumz = fma(diffloc * A23.x, t1 - t1d, sumz);
+    sumz = fma(diffloc * A01.y, t0u - t0, sumz);
+    sumz = fma(diffloc * A23.y, t1u - t1, sumz);
+    return cosu * fma(sumz, r4zt, (t1 - t0) * ry * K22);
 }
 // tc/tw/te/ts/tn = the tracer at the cell and its west/east/south/north
-// neighbours, levels k (0) and k+1 (1); cosu_s = cosu[j-1]
+// neighbours, levels k (0) and k+1 (1); r4xt = 1 / (4 dxt)
 __device__ __forceinline__ double top_flux_core(double diffloc, double2 B01, double2 B23, double2 C01, double2 C23,
                                                 double tc0, double tc1, double tw0, double tw1, double te0,
                                                 double te1, double ts0, double ts1, double tn0, double tn1,
-                                                double cost, double cosu, double cosu_s, double dxt, double dyt) {
-    double sumx = 0.0;
-    sumx = sumx + diffloc * B01.x / cost * (tc0 - tw0);  // ip=0, kr=0
-    sumx = sumx + diffloc * B01.y / cost * (tc1 - tw1);  // ip=0, kr=1
-    sumx = sumx + diffloc * B23.x / cost * (te0 - tc0);  // ip=1, kr=0
-    sumx = sumx + diffloc * B23.y / cost * (te1 - tc1);  // ip=1, kr=1
-    double sumy = 0.0;
-    sumy = sumy + diffloc * C01.x * cosu_s * (tc0 - ts0);
-    sumy = sumy + diffloc * C01.y * cosu_s * (tc1 - ts1);
-    sumy = sumy + diffloc * C23.x * cosu * (tn0 - tc0);
-    sumy = sumy + diffloc * C23.y * cosu * (tn1 - tc1);
-    return sumx / (4 * dxt) + sumy / (4 * dyt * cost);
+                                                const ColMetrics& m, double r4xt) {
+    const double dx = diffloc * m.rcost;
+    double sumx = dx * B01.x * (tc0 - tw0);    // ip=0, kr=0
+    sumx = fma(dx * B01.y, tc1 - tw1, sumx);  // ip=0, kr=1
+    sumx = fma(dx * B23.x, te0 - tc0, sumx);  // ip=1, kr=0
+    sumx = fma(dx * B23.y, te1 - tc1, sumx);  // ip=1, kr=1
+    const double ds = diffloc * m.cosus, dn = diffloc * m.cosu;
+    double sumy = ds * C01.x * (tc0 - ts0);
+    sumy = fma(ds * C01.y, tc1 - ts1, sumy);
+    sumy = fma(dn * C23.x, tn0 - tc0, sumy);
+    sumy = fma(dn * C23.y, tn1 - tc1, sumy);
+    return fma(sumx, r4xt, sumy * m.ryt);
 }
 
 // Face-flux outputs of the fused pre + flux kernel (temperature, salinity).
@@ -278,18 +358,12 @@ struct PreFlux {
     double *fe[2], *fn[2], *ft[2];
 };
 
-// The dry cells of isoneutral_diffusion_pre. A dry cell has every output
-// exactly zero: its own maskT factor is in maskU (Ai_ez, K_11), maskV (Ai_nz,
-// K_22) and maskW (Ai_bx, Ai_by, K_33), which multiply each entry and each
-// summed term. The dry cells of a column are its levels 0 .. kbot-2, one
-// contiguous run per array, so a wave per column zero-fills those runs with
-// lane-contiguous stores (full cache lines) over the index ranges the
-// reference writes; iso_pre_kernel handles the wet cells.
-// The zeros are stored nontemporal: nothing in the call reads them back, and
-// streaming them past the caches leaves the L2 to the wet-cell kernels beside
-// them (measured on 1440x720x80: pre 4.9 -> 4.6 ms, pre + the
-// temperature/salinity step in one call 8.3 -> 7.5 ms; the same stores for the
-// wet cells' tensor made pre slower).
+// The dry cells of isoneutral_diffusion_pre: every output exactly zero (its own
+// maskT factor is in maskU (Ai_ez, K_11), maskV (Ai_nz, K_22) and maskW (Ai_bx,
+// Ai_by, K_33), which multiply each entry and each summed term), over the index
+// ranges the reference writes: levels 0 .. nd-1 of column (i, j), one run per
+// array, stored by the wave's lanes in order. Nothing in the call reads them, so
+// they are stored nontemporal and leave the L2 to the wet cells.
 typedef double vx_d2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void zero_run(double* __restrict__ p, int n, int lane) {
     for (int m = lane; m < n; m += 64) __builtin_nontemporal_store(0.0, p + m);
@@ -303,101 +377,98 @@ __device__ __forceinline__ void zero_ai_run(double* __restrict__ p, int nd, int 
         else __builtin_nontemporal_store((vx_d2){0.0, 0.0}, reinterpret_cast<vx_d2*>(p + 2 * m));
     }
 }
-
-__global__ __launch_bounds__(256) void iso_pre_dry_kernel(Grid g, double* __restrict__ Aez, double* __restrict__ Anz,
-                                                          double* __restrict__ Abx, double* __restrict__ Aby,
-                                                          double* __restrict__ K11, double* __restrict__ K22,
-                                                          double* __restrict__ K33) {
-    const int lane = (int)(threadIdx.x & 63);
-    const int64_t ni = g.X - 3, nj = g.Y - 3;
-    const int64_t stride = (int64_t)gridDim.x * (blockDim.x >> 6);
-    // grid-stride over the columns (the grid may be smaller than one wave per
-    // column: a background fill beside other kernels)
-    for (int64_t col = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); col < ni * nj; col += stride) {
-        const int i = 1 + (int)(col / nj), j = 1 + (int)(col - (col / nj) * nj);
-        const int nz = g.nz;
-        const int kb = g.kbot[i * g.Y + j];
-        const int nd = (kb >= 1 && kb <= nz) ? kb - 1 : nz;  // dry levels 0 .. nd-1
-        if (nd == 0) continue;
-        const uint32_t c0 = ((uint32_t)i * (uint32_t)g.Y + (uint32_t)j) * (uint32_t)nz;
-        if (j >= 2) {
-            zero_ai_run(Aez + 4u * c0, nd, lane, true);
-            zero_run(K11 + c0, nd, lane);
-        }
-        if (i >= 2) {
-            zero_ai_run(Anz + 4u * c0, nd, lane, true);
-            zero_run(K22 + c0, nd, lane);
-        }
-        if (i >= 2 && j >= 2) {
-            const int nt = nd < nz - 1 ? nd : nz - 1;  // top faces: levels below nz-1
-            zero_ai_run(Abx + 4u * c0, nt, lane, false);
-            zero_ai_run(Aby + 4u * c0, nt, lane, false);
-            zero_run(K33 + c0, nt, lane);
-        }
+__device__ __forceinline__ void zero_column(const Grid& g, int i, int j, int nd, int lane, double* __restrict__ Aez,
+                                            double* __restrict__ Anz, double* __restrict__ Abx,
+                                            double* __restrict__ Aby, double* __restrict__ K11,
+                                            double* __restrict__ K22, double* __restrict__ K33) {
+    const uint32_t c0 = ((uint32_t)i * (uint32_t)g.Y + (uint32_t)j) * (uint32_t)g.nz;
+    if (j >= 2) {
+        zero_ai_run(Aez + 4u * c0, nd, lane, true);
+        zero_run(K11 + c0, nd, lane);
     }
+    if (i >= 2) {
+        zero_ai_run(Anz + 4u * c0, nd, lane, true);
+        zero_run(K22 + c0, nd, lane);
+    }
+    if (i >= 2 && j >= 2) {
+        const int nt = nd < g.nz - 1 ? nd : g.nz - 1;  // top faces: levels below nz-1
+        zero_ai_run(Abx + 4u * c0, nt, lane, false);
+        zero_ai_run(Aby + 4u * c0, nt, lane, false);
+        zero_run(K33 + c0, nd, lane);  // a dry column's top level too
+    }
+}
+
+// The values of one cell's stencil, in flight: the tracers at the cell c, its
+// east (e), west (w), north (n) and south (s) neighbours, levels k, k+1 (p) and
+// k-1 (m), and the diffusivity.
+struct PreIn {
+    double Tc, Tcp, Tcm, Te, Tep, Tem, Tw, Twp, Tn, Tnp, Tnm, Ts, Tsp;
+    double Sc, Scp, Scm, Se, Sep, Sem, Sw, Swp, Sn, Snp, Snm, Ss, Ssp;
+    double Kc, Kcl, Ke, Kel, Kn, Knl;
+};
+// Loaded whether or not they are used (k+1 at the top and k-1 at the bottom
+// are cells of the next and previous columns, in bounds for every cell pre
+// visits, i in [1, X-3], j in [1, Y-3]): a load under a per-lane condition is
+// waited for at once. Offsets are 32-bit element offsets (the host checks the
+// arrays fit).
+__device__ __forceinline__ void pre_load(const Grid& g, const Fields& f, const double* __restrict__ K, int i, int j,
+                                         int k, PreIn& v) {
+    const uint32_t sj = (uint32_t)g.nz, si = (uint32_t)g.Y * (uint32_t)g.nz;
+    const uint32_t c = (uint32_t)i * si + (uint32_t)j * sj + (uint32_t)k;
+    const uint32_t ce = c + si, cw = c - si, cn = c + sj, cs = c - sj;
+    const double* __restrict__ T = f.T + (uint32_t)f.tau * g.ls;
+    const double* __restrict__ S = f.S + (uint32_t)f.tau * g.ls;
+    auto L2 = [&](uint32_t o, double& t, double& sv) {
+        t = T[g.cs * o];
+        sv = S[g.cs * o];
+    };
+    L2(c, v.Tc, v.Sc);
+    L2(c + 1, v.Tcp, v.Scp);
+    L2(c - 1, v.Tcm, v.Scm);
+    L2(ce, v.Te, v.Se);
+    L2(ce + 1, v.Tep, v.Sep);
+    L2(ce - 1, v.Tem, v.Sem);
+    L2(cw, v.Tw, v.Sw);
+    L2(cw + 1, v.Twp, v.Swp);
+    L2(cn, v.Tn, v.Sn);
+    L2(cn + 1, v.Tnp, v.Snp);
+    L2(cn - 1, v.Tnm, v.Snm);
+    L2(cs, v.Ts, v.Ss);
+    L2(cs + 1, v.Tsp, v.Ssp);
+    v.Kc = K[c], v.Kcl = K[c - 1], v.Ke = K[ce], v.Kel = K[ce - 1], v.Kn = K[cn], v.Knl = K[cn - 1];
 }
 
 // One wet cell (i, j, k) of isoneutral_diffusion_pre. FUSED: also the face
 // fluxes of temperature and salinity at level tau from the tensor just formed
 // (the flux kernel's work for the step that follows pre), into `fo`.
 template <bool FUSED>
-__device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const Fields& f,
-                                             const double* __restrict__ K, double* __restrict__ Aez,
+__device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const PreIn& v, double* __restrict__ Aez,
                                              double* __restrict__ Anz, double* __restrict__ Abx,
                                              double* __restrict__ Aby, double* __restrict__ K11,
                                              double* __restrict__ K22, double* __restrict__ K33, const PreFlux& fo,
-                                             const int i, const int j, const int k) {
+                                             const BlockMetrics& bm, const double dxu_i, const double dxu_w,
+                                             const double r4xt, const int i, const int j, const int q, const int k) {
     const int nz = g.nz;
-    const uint32_t sj = (uint32_t)nz, si = (uint32_t)g.Y * (uint32_t)nz;
-    const uint32_t c = (uint32_t)i * si + (uint32_t)j * sj + (uint32_t)k;
-    const uint32_t ce = c + si, cw = c - si, cn = c + sj, cs = c - sj;
+    const ColMetrics& cm = bm.col[q];
+    const uint32_t c = ((uint32_t)i * (uint32_t)g.Y + (uint32_t)j) * (uint32_t)nz + (uint32_t)k;
     const bool hp = k < nz - 1, hm = k >= 1;
-    const double* __restrict__ T = f.T + (uint32_t)f.tau * g.ls;
-    const double* __restrict__ S = f.S + (uint32_t)f.tau * g.ls;
-    const int kb_c = g.kbot[i * g.Y + j], kb_e = g.kbot[(i + 1) * g.Y + j], kb_w = g.kbot[(i - 1) * g.Y + j];
-    const int kb_n = g.kbot[i * g.Y + j + 1], kb_s = g.kbot[i * g.Y + j - 1];
-
-    // tracer values: c(enter), e(ast), w(est), n(orth), s(outh); p = k+1, m = k-1.
-    // Loaded whether or not they are used (k+1 at the top and k-1 at the
-    // bottom are cells of the next and previous columns, in bounds for every
-    // cell pre visits, i in [1, X-3], j in [1, Y-3]): a load under a per-lane
-    // condition is waited for at once.
-    auto L2 = [&](uint32_t o, bool ok, double& t, double& sv) {
-        const double tv = T[g.cs * o], svv = S[g.cs * o];
-        t = ok ? tv : 0.0;
-        sv = ok ? svv : 0.0;
-    };
-    double Tc, Sc, Tcp, Scp, Tcm, Scm, Te, Se, Tep, Sep, Tem, Sem, Tw, Sw, Twp, Swp;
-    double Tn, Sn, Tnp, Snp, Tnm, Snm, Ts, Ss, Tsp, Ssp;
-    L2(c, true, Tc, Sc);
-    L2(c + 1, hp, Tcp, Scp);
-    L2(c - 1, hm, Tcm, Scm);
-    L2(ce, true, Te, Se);
-    L2(ce + 1, hp, Tep, Sep);
-    L2(ce - 1, hm, Tem, Sem);
-    L2(cw, true, Tw, Sw);
-    L2(cw + 1, hp, Twp, Swp);
-    L2(cn, true, Tn, Sn);
-    L2(cn + 1, hp, Tnp, Snp);
-    L2(cn - 1, hm, Tnm, Snm);
-    L2(cs, true, Ts, Ss);
-    L2(cs + 1, hp, Tsp, Ssp);
-
-    // Every other global read up front: reads placed inside the divergent
-    // face branches below would each cost a separate memory round trip.
-    const double dzw_k = g.dzw[k], dzw_l = g.dzw[hm ? k - 1 : k], dzt_k = g.dzt[k];
-    const double dzw_m = hm ? dzw_l : 0.0;
-    const double dxu_i = g.dxu[i], dxu_w = g.dxu[i - 1], dxt_i = g.dxt[i];
-    const double cost_j = g.cost[j], dyu_j = g.dyu[j], dyu_s = g.dyu[j - 1], dyt_j = g.dyt[j];
-    const double cosu_j = g.cosu[j], cosu_s = g.cosu[j - 1];
-    const double Kc = K[c], Kcl = K[c - 1], Ke = K[ce], Kel = K[ce - 1], Kn = K[cn], Knl = K[cn - 1];
-    const double Kcm = hm ? Kcl : 0.0, Kem = hm ? Kel : 0.0, Knm = hm ? Knl : 0.0;
+    const int kb_c = bm.kb[q + 1], kb_e = bm.kbe[q], kb_w = bm.kbw[q];
+    const int kb_n = bm.kb[q + 2], kb_s = bm.kb[q];
+    auto sel = [](bool ok, double x) { return ok ? x : 0.0; };
+    const double Tc = v.Tc, Tcp = sel(hp, v.Tcp), Tcm = sel(hm, v.Tcm), Te = v.Te, Tep = sel(hp, v.Tep);
+    const double Tem = sel(hm, v.Tem), Tw = v.Tw, Twp = sel(hp, v.Twp), Tn = v.Tn, Tnp = sel(hp, v.Tnp);
+    const double Tnm = sel(hm, v.Tnm), Ts = v.Ts, Tsp = sel(hp, v.Tsp);
+    const double Sc = v.Sc, Scp = sel(hp, v.Scp), Scm = sel(hm, v.Scm), Se = v.Se, Sep = sel(hp, v.Sep);
+    const double Sem = sel(hm, v.Sem), Sw = v.Sw, Swp = sel(hp, v.Swp), Sn = v.Sn, Snp = sel(hp, v.Snp);
+    const double Snm = sel(hm, v.Snm), Ss = v.Ss, Ssp = sel(hp, v.Ssp);
+    const double Kc = v.Kc, Kcm = sel(hm, v.Kcl), Ke = v.Ke, Kem = sel(hm, v.Kel), Kn = v.Kn, Knm = sel(hm, v.Knl);
+    const double dzw_k = bm.lev.dzw[k], dzw_m = hm ? bm.lev.dzw[hm ? k - 1 : k] : 0.0;
+    const double r4zt = bm.lev.r4zt[k];
 
     // reciprocal metric factors
-    const double rz_c = hp ? rcp_nr(dzw_k) : 0.0;
-    const double rz_m = hm ? rcp_nr(dzw_m) : 0.0;
-    const double rx_c = rcp_nr(dxu_i * cost_j);
-    const double ry_c = rcp_nr(dyu_j);
+    const double rz_c = hp ? bm.lev.rzw[k] : 0.0;
+    const double rz_m = hm ? bm.lev.rzw[hm ? k - 1 : k] : 0.0;
+    const double rx_c = cm.rx, ry_c = cm.ry;
 
     // masked face gradients (veros/core/isoneutral/isoneutral.py:46-95)
     auto G = [](double m, double a1, double a0, double b1, double b0, double rd) -> Grad {
@@ -464,7 +535,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
         } else {
             Aez[4u * c + 3] = out[3];
         }
-        const double k11v = sumz / (4.0 * dzt_k);
+        const double k11v = sumz * r4zt;
         K11[c] = k11v;
         if constexpr (FUSED) {
             // at level 0 the kr = 0 entries keep their values (their tracer
@@ -472,9 +543,9 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
             const double a0 = hm ? out[0] : Aez[4u * c], a2 = hm ? out[2] : Aez[4u * c + 2];
             const double2 A01 = make_double2(a0, out[1]), A23 = make_double2(a2, out[3]);
             fo.fe[0][c] = east_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Te, hp ? Tep : Te,
-                                         hm ? Tem : Te, dzt_k, cost_j, dxu_i, k11v);
+                                         hm ? Tem : Te, r4zt, rx_c, k11v);
             fo.fe[1][c] = east_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Se, hp ? Sep : Se,
-                                         hm ? Sem : Se, dzt_k, cost_j, dxu_i, k11v);
+                                         hm ? Sem : Se, r4zt, rx_c, k11v);
         }
     }
 
@@ -511,15 +582,15 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
             Anz[4u * c + 1] = out[1];
             Anz[4u * c + 3] = out[3];
         }
-        const double k22v = sumz / (4.0 * dzt_k);
+        const double k22v = sumz * r4zt;
         K22[c] = k22v;
         if constexpr (FUSED) {
             const double a0 = hm ? out[0] : Anz[4u * c], a2 = hm ? out[2] : Anz[4u * c + 2];
             const double2 A01 = make_double2(a0, out[1]), A23 = make_double2(a2, out[3]);
             fo.fn[0][c] = north_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Tn, hp ? Tnp : Tn,
-                                          hm ? Tnm : Tn, dzt_k, cosu_j, dyu_j, k22v);
+                                          hm ? Tnm : Tn, r4zt, cm.cosu, ry_c, k22v);
             fo.fn[1][c] = north_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Sn, hp ? Snp : Sn,
-                                          hm ? Snm : Sn, dzt_k, cosu_j, dyu_j, k22v);
+                                          hm ? Snm : Sn, r4zt, cm.cosu, ry_c, k22v);
         }
     }
 
@@ -527,8 +598,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
     if (i >= 2 && j >= 2 && hp) {
         const int kb_w2 = kb_w, kb_s2 = kb_s;
         const double mW = mc * mcp;
-        const double rx_w = rcp_nr(dxu_w * cost_j);
-        const double ry_s = rcp_nr(dyu_s);
+        const double rx_w = cm.rxw, ry_s = cm.rys;
         const double mw = m01(kb_w2, k), mwp = m01(kb_w2, k + 1);
         const double ms = m01(kb_s2, k), msp = m01(kb_s2, k + 1);
         // horizontal gradients at (i-1+ip, k+kr) and (j-1+jp, k+kr)
@@ -565,7 +635,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
                     sl = -dot(w, gy) * rd;
                     tp = taper(p, ec, tds, sl);
                 }
-                const double facty = jp ? cosu_j * dyu_j : cosu_s * dyu_s;
+                const double facty = jp ? cm.fyc : cm.fys;
                 sumy += facty * Kc * tp * (sl * sl) * mW;
                 oy[jp * 2 + kr] = tp * sl * mW;
             }
@@ -574,70 +644,110 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
         *reinterpret_cast<double2*>(Abx + 4u * c + 2) = make_double2(ox[2], ox[3]);
         *reinterpret_cast<double2*>(Aby + 4u * c) = make_double2(oy[0], oy[1]);
         *reinterpret_cast<double2*>(Aby + 4u * c + 2) = make_double2(oy[2], oy[3]);
-        K33[c] = sumx / (4 * dxt_i) + sumy / (4 * dyt_j * cost_j);
+        K33[c] = sumx * r4xt + sumy * cm.ryt;
         if constexpr (FUSED) {
             const double2 B01 = make_double2(ox[0], ox[1]), B23 = make_double2(ox[2], ox[3]);
             const double2 C01 = make_double2(oy[0], oy[1]), C23 = make_double2(oy[2], oy[3]);
-            fo.ft[0][c] = top_flux_core(Kc, B01, B23, C01, C23, Tc, Tcp, Tw, Twp, Te, Tep, Ts, Tsp, Tn, Tnp, cost_j,
-                                        cosu_j, cosu_s, dxt_i, dyt_j);
-            fo.ft[1][c] = top_flux_core(Kc, B01, B23, C01, C23, Sc, Scp, Sw, Swp, Se, Sep, Ss, Ssp, Sn, Snp, cost_j,
-                                        cosu_j, cosu_s, dxt_i, dyt_j);
+            fo.ft[0][c] = top_flux_core(Kc, B01, B23, C01, C23, Tc, Tcp, Tw, Twp, Te, Tep, Ts, Tsp, Tn, Tnp, cm,
+                                        r4xt);
+            fo.ft[1][c] = top_flux_core(Kc, B01, B23, C01, C23, Sc, Scp, Sw, Swp, Se, Sep, Ss, Ssp, Sn, Snp, cm,
+                                        r4xt);
         }
     }
-    if constexpr (FUSED) {
-        if (i >= 2 && j >= 2 && !hp) {  // no flux through the top level
+    if (i >= 2 && j >= 2 && !hp) {
+        K33[c] = 0.0;  // (:225)
+        if constexpr (FUSED) {  // no flux through the top level
             fo.ft[0][c] = 0.0;
             fo.ft[1][c] = 0.0;
         }
     }
 }
 
-// The wet cells of isoneutral_diffusion_pre (the dry ones are written by
-// iso_pre_dry_kernel). Block-local compaction: a block owns the columns
-// (i, jb .. jb+ncb-1); their wet cells (the wet suffixes) are numbered in
-// column order and dealt round-robin to the block's threads, so the slope work
-// fills whole waves whatever the land fraction.
+// isoneutral_diffusion_pre. Block-local compaction: a block (one wave) owns the
+// columns (i, jb .. jb+ncb-1); their wet cells (the wet suffixes) are numbered
+// in column order and taken 64 at a time, so the slope work fills the wave
+// whatever the land fraction; the dry cells of its columns are zeroed last.
+//
+// A wave waits for its memory operations in order, so a load issued after
+// stores waits until those are acknowledged, which takes several microseconds
+// where writes are the bound: the next round's stencil is therefore loaded
+// before the current round is computed and stored, and the zeros go out when
+// no load is left to wait for. The two stencils in flight take the registers
+// of two waves per SIMD (three spill them and lose more than they hide).
+// Bound by writes: on 1440x720x80 (35% land) the fused call takes 4.58 ms
+// without the 8.7 GB of zeros and 6.04 ms with them; the zeros alone, by a
+// kernel of their own beside this one on a helper stream, and 183 registers of
+// divisions in this one: 6.10 ms. The same on 360x160x60 (levels innermost, all
+// isoneutral calls of a step): 1355 -> 1160 us; 90x40x15, pre + T + S: 77 -> 54 us
+// (no second stream to fork and join).
 template <bool FUSED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FUSED ? 2 : VX_PRE_MIN_WAVES))) void iso_pre_kernel(
+__global__ __launch_bounds__(kCellBlock) __attribute__((amdgpu_waves_per_eu(VX_PRE_MIN_WAVES))) void iso_pre_kernel(
     Grid g, Prm p, Fields f, const double* __restrict__ K, double* __restrict__ Aez, double* __restrict__ Anz,
     double* __restrict__ Abx, double* __restrict__ Aby, double* __restrict__ K11, double* __restrict__ K22,
     double* __restrict__ K33, PreFlux fo, int ncb) {
-    extern __shared__ int pre_counts[];  // prefix sums of the columns' wet counts
-    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripBlocks);
+    __shared__ BlockMetrics bm;
+    const int tid = (int)threadIdx.x, nz = g.nz;
+    // K_33[..., nz-1] = 0 (veros/core/isoneutral/isoneutral.py:225) of the halo
+    // columns: rows 0, 1, X-2, X-1, then columns 0, 1, Y-2, Y-1
+    for (int64_t c = (int64_t)blockIdx.x * kCellBlock + tid; c < 4 * ((int64_t)g.X + g.Y);
+         c += (int64_t)gridDim.x * kCellBlock) {
+        const bool row = c < 4 * (int64_t)g.Y;
+        const int64_t r = row ? c : c - 4 * (int64_t)g.Y;
+        const int64_t n = row ? g.Y : g.X;
+        const int64_t h = r / n, m = r - h * n;  // which of the four, where along it
+        const int64_t e = h < 2 ? h : (row ? g.X : g.Y) - 4 + h;
+        K33[((row ? e * g.Y + m : m * g.Y + e) + 1) * nz - 1] = 0.0;
+    }
+    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripCols / ncb);
     if (!bc.valid) return;  // padding block (uniform)
-    const int nz = g.nz, i = bc.i, jb = bc.j;
-    const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
-    int* sW = pre_counts;
-    for (int q = tid; q < ncb; q += nthr) {
-        const bool col_ok = jb + q <= g.Y - 3;
-        const int kbq = col_ok ? g.kbot[i * g.Y + jb + q] : 0;
-        sW[q + 1] = (kbq >= 1 && kbq <= nz) ? nz - kbq + 1 : 0;
+    const int i = bc.i, jb = bc.j;
+    fill_metrics(g, i, jb, ncb, bm);
+    __syncthreads();
+    if (tid < ncb) {
+        const bool have = jb + tid <= g.Y - 3;
+        const int kbq = bm.kb[tid + 1];
+        const int n = (have && kbq >= 1 && kbq <= nz) ? nz - kbq + 1 : 0;
+        bm.run[tid + 1] = n;
     }
     __syncthreads();
-    if (tid == 0) {
-        sW[0] = 0;
-        for (int q = 0; q < ncb; ++q) sW[q + 1] += sW[q];
-    }
+    scan_runs(bm.run, ncb);
     __syncthreads();
-    const int nwet = sW[ncb];
-    for (int t = tid; t < nwet; t += nthr) {
-        // the column q with sW[q] <= t < sW[q+1]: the last q with sW[q] <= t
-        int lo = 0, hi = ncb - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (sW[mid] <= t) lo = mid;
-            else hi = mid - 1;
+    const int nwet = bm.run[ncb];
+    const double dxu_i = g.dxu[i], dxu_w = g.dxu[i - 1], r4xt = 1.0 / (4 * g.dxt[i]);
+    if (nwet > 0) {
+        // this lane's cell of a round (a lane past the last cell: that cell, not stored)
+        auto locate = [&](int t, int& q, int& k) {
+            const int tt = t < nwet ? t : nwet - 1;
+            q = run_column(bm, ncb, tt);
+            k = nz - (bm.run[q + 1] - bm.run[q]) + (tt - bm.run[q]);  // wet suffix of column q
+        };
+        int q, k;
+        PreIn v;
+        locate(tid, q, k);
+        pre_load(g, f, K, i, jb + q, k, v);
+        for (int t0 = 0;;) {
+            const bool more = t0 + kCellBlock < nwet;
+            int qn = q, kn = k;
+            PreIn vn;
+            if (more) {
+                locate(t0 + kCellBlock + tid, qn, kn);
+                pre_load(g, f, K, i, jb + qn, kn, vn);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (t0 + tid < nwet)
+                pre_wet_cell<FUSED>(g, p, v, Aez, Anz, Abx, Aby, K11, K22, K33, fo, bm, dxu_i, dxu_w, r4xt, i, jb + q,
+                                    q, k);
+            if (!more) break;
+            t0 += kCellBlock;
+            q = qn;
+            k = kn;
+            v = vn;
         }
-        const int k = nz - (sW[lo + 1] - sW[lo]) + (t - sW[lo]);  // wet suffix of column lo
-        pre_wet_cell<FUSED>(g, p, f, K, Aez, Anz, Abx, Aby, K11, K22, K33, fo, i, jb + lo, k);
     }
-}
-
-// K_33[..., nz-1] = 0 over the whole plane (veros/core/isoneutral/isoneutral.py:225)
-__global__ void k33_top_zero_kernel(Grid g, double* __restrict__ K33) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)g.X * g.Y) return;
-    K33[t * g.nz + g.nz - 1] = 0.0;
+    for (int q = 0; q < ncb && jb + q <= g.Y - 3; ++q) {
+        const int nd = nz - (bm.run[q + 1] - bm.run[q]);
+        if (nd > 0) zero_column(g, i, jb + q, nd, tid, Aez, Anz, Abx, Aby, K11, K22, K33);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -674,17 +784,6 @@ struct Strides {
     uint32_t si, sj;
 };
 
-// Inputs of the face fluxes of one cell (i, j, k), read from global memory
-// before any flux is formed. `K` is the one diffusivity of the step (K_iso for
-// the isoneutral step, K_gm for the skew step) at c, c-1, the east column
-// (e, e-1) and the north column (n, n-1).
-struct FaceIn {
-    double K_c, K_cm, K_e, K_em, K_n, K_nm;
-    double2 ez01, ez23, nz01, nz23, bx01, bx23, by01, by23;
-    double K11, K22;
-    double dzt, cost, dxu, cosu, cosu_s, dyu, dxt, dyt;
-};
-
 // K1 = K_iso - K_skew (east/north faces) and K2 = K_iso + K_skew (top faces)
 // (veros/core/isoneutral/diffusion.py:15-16,180-188); one of the two is zero.
 template <bool ISO>
@@ -707,133 +806,120 @@ __device__ __forceinline__ double k2_of(double K) { return ISO ? K : 0.0 + K; }
 // tracer stencil is read straight from global memory (every read issued
 // before the first flux), so no lane of a dry region is launched.
 __device__ __forceinline__ int first_wet(int kb, int nz) { return (kb >= 1 && kb <= nz) ? kb - 1 : nz; }
-__device__ __forceinline__ int flux_run_start(const Grid& g, int i, int j) {
-    const int nz = g.nz;
-    const int fc = first_wet(g.kbot[i * g.Y + j], nz);
+// first level of the run of block column q (row i, column j)
+__device__ __forceinline__ int flux_run_start(const BlockMetrics& m, int nz, int i, int j, int q) {
+    const int fc = first_wet(m.kb[q + 1], nz);
     int s0 = fc < nz ? (fc >= 1 ? fc - 1 : 0) : nz;             // top face of the dry cell below
-    const int fe = j >= 2 ? first_wet(g.kbot[(i + 1) * g.Y + j], nz) : nz;
-    const int fn = i >= 2 ? first_wet(g.kbot[i * g.Y + j + 1], nz) : nz;
+    const int fe = j >= 2 ? first_wet(m.kbe[q], nz) : nz;
+    const int fn = i >= 2 ? first_wet(m.kb[q + 2], nz) : nz;
     s0 = fe < s0 ? fe : s0;
     return fn < s0 ? fn : s0;
 }
 
+typedef unsigned int vx_u4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ double2 buf_load2(BufRsrc b, uint32_t off) {
+    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
+}
+
+// Every read is a buffer load at an offset that is past the buffer's end where
+// the cell does not need it (no traffic, no branch around the load, all of a
+// cell's loads in flight together). A block's cells lie in the columns
+// jb-1 .. jb+ncb of the rows i-1, i, i+1: one buffer per row and array, from
+// column jb-1 on. On 360x160x60, levels innermost, one tracer: 142 us with the
+// loads under the conditions of their faces, 121 now.
 template <int NTR, bool ISO>
-__global__ __launch_bounds__(256) void iso_flux_kernel(Grid g, StepArgs a, int ncb) {
-    extern __shared__ int flux_counts[];  // prefix sums of the columns' run lengths
-    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripBlocks);
+__global__ __launch_bounds__(kCellBlock) void iso_flux_kernel(Grid g, StepArgs a, int ncb) {
+    __shared__ BlockMetrics bm;
+    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripCols / ncb);
     if (!bc.valid) return;  // padding block (uniform)
     const int nz = g.nz, i = bc.i, jb = bc.j;
     const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
-    int* sW = flux_counts;
-    for (int q = tid; q < ncb; q += nthr) sW[q + 1] = jb + q <= g.Y - 3 ? nz - flux_run_start(g, i, jb + q) : 0;
+    fill_metrics(g, i, jb, ncb, bm);
     __syncthreads();
-    if (tid == 0) {
-        sW[0] = 0;
-        for (int q = 0; q < ncb; ++q) sW[q + 1] += sW[q];
-    }
+    for (int q = tid; q < ncb; q += nthr)
+        bm.run[q + 1] = jb + q <= g.Y - 3 ? nz - flux_run_start(bm, nz, i, jb + q, q) : 0;
     __syncthreads();
-    const int ncell = sW[ncb];
-    const uint32_t si = (uint32_t)g.Y * (uint32_t)nz, sj = (uint32_t)nz;
-    const double* __restrict__ Kf = ISO ? a.Kiso : a.Kskew;
+    scan_runs(bm.run, ncb);
+    __syncthreads();
+    const int ncell = bm.run[ncb];
+    const uint32_t sj = (uint32_t)nz;
+    const double r4xt = 1.0 / (4 * g.dxt[i]);
+    // the rows' cells from column jb-1 on, up to column jb+ncb or the row's end
+    const int64_t row = (int64_t)g.Y * nz, o0 = (int64_t)i * row + (int64_t)(jb - 1) * nz;
+    const uint32_t ncells = (uint32_t)(jb + ncb < g.Y ? ncb + 2 : g.Y - jb + 1) * (uint32_t)nz;
+    const double* Kf = ISO ? a.Kiso : a.Kskew;
+    const BufRsrc bK = make_buf(Kf + o0, ncells * 8u), bKe = make_buf(Kf + o0 + row, ncells * 8u);
+    const BufRsrc bez = make_buf(a.Aez + 4 * o0, ncells * 32u), bnz = make_buf(a.Anz + 4 * o0, ncells * 32u);
+    const BufRsrc bbx = make_buf(a.Abx + 4 * o0, ncells * 32u), bby = make_buf(a.Aby + 4 * o0, ncells * 32u);
+    const BufRsrc b11 = make_buf(a.K11 + o0, ncells * 8u), b22 = make_buf(a.K22 + o0, ncells * 8u);
+    const uint32_t cb = 8u * g.cs;  // bytes from a level to the next in the time-level arrays
     for (int t = tid; t < ncell; t += nthr) {
-        int q = 0, hi = ncb - 1;
-        while (q < hi) {
-            const int mid = (q + hi + 1) >> 1;
-            if (sW[mid] <= t) q = mid;
-            else hi = mid - 1;
-        }
+        const int q = run_column(bm, ncb, t);
         const int j = jb + q;
-        const int k = nz - (sW[q + 1] - sW[q]) + (t - sW[q]);
-        const int kb = g.kbot[i * g.Y + j], kb_e = g.kbot[(i + 1) * g.Y + j], kb_n = g.kbot[i * g.Y + j + 1];
+        const int k = nz - (bm.run[q + 1] - bm.run[q]) + (t - bm.run[q]);
+        const int kb = bm.kb[q + 1], kb_e = bm.kbe[q], kb_n = bm.kb[q + 2];
         const bool wc = wet(kb, k);
         const bool need_e = j >= 2 && (wc || wet(kb_e, k));
         const bool need_n = i >= 2 && (wc || wet(kb_n, k));
         const bool need_t = i >= 2 && j >= 2 && (wc || (k + 1 < nz && wet(kb, k + 1)));
-        if (!(need_e || need_n || need_t)) continue;
-        const uint32_t c = (uint32_t)i * si + (uint32_t)j * sj + (uint32_t)k;
         const bool hm = k >= 1, hp = k + 1 < nz;
-        const bool top = need_t && hp;
-        const uint32_t up = hp ? 1u : 0u, dn = hm ? 1u : 0u;  // pad_z_edges clamping
-        // every global read before the first flux
-        FaceIn in{};
-        in.K_c = Kf[c];
-        in.K_cm = hm ? Kf[c - 1] : 0.0;
-        in.dzt = g.dzt[k];
-        in.cost = g.cost[j];
-        in.dxu = g.dxu[i];
-        in.cosu = g.cosu[j];
-        in.cosu_s = g.cosu[j - 1];
-        in.dyu = g.dyu[j];
-        in.dxt = g.dxt[i];
-        in.dyt = g.dyt[j];
-        if (need_e) {
-            in.K_e = Kf[c + si];
-            in.K_em = hm ? Kf[c + si - 1] : 0.0;
-            in.ez01 = *reinterpret_cast<const double2*>(a.Aez + 4u * c);
-            in.ez23 = *reinterpret_cast<const double2*>(a.Aez + 4u * c + 2);
-            in.K11 = a.K11[c];
-        }
-        if (need_n) {
-            in.K_n = Kf[c + sj];
-            in.K_nm = hm ? Kf[c + sj - 1] : 0.0;
-            in.nz01 = *reinterpret_cast<const double2*>(a.Anz + 4u * c);
-            in.nz23 = *reinterpret_cast<const double2*>(a.Anz + 4u * c + 2);
-            in.K22 = a.K22[c];
-        }
-        if (top) {
-            in.bx01 = *reinterpret_cast<const double2*>(a.Abx + 4u * c);
-            in.bx23 = *reinterpret_cast<const double2*>(a.Abx + 4u * c + 2);
-            in.by01 = *reinterpret_cast<const double2*>(a.Aby + 4u * c);
-            in.by23 = *reinterpret_cast<const double2*>(a.Aby + 4u * c + 2);
-        }
+        const bool top = need_t && hp, any = need_e || need_n || need_t;
+        const uint32_t e = (uint32_t)(q + 1) * sj + (uint32_t)k;  // cell in the buffers
+        const uint32_t up = hp ? 1u : 0u, dn = hm ? 1u : 0u;      // pad_z_edges clamping
+        auto at = [](bool on, uint32_t off) { return on ? off : kNoAccess; };
+        const double K_c = buf_load(bK, at(any, 8u * e)), K_cm = buf_load(bK, at(any && hm, 8u * (e - 1u)));
+        const double K_e = buf_load(bKe, at(need_e, 8u * e)), K_em = buf_load(bKe, at(need_e && hm, 8u * (e - 1u)));
+        const double K_n = buf_load(bK, at(need_n, 8u * (e + sj)));
+        const double K_nm = buf_load(bK, at(need_n && hm, 8u * (e + sj - 1u)));
+        const uint32_t oe = at(need_e, 32u * e), on = at(need_n, 32u * e), ot = at(top, 32u * e);
+        const double2 ez01 = buf_load2(bez, oe), ez23 = buf_load2(bez, oe + 16u);
+        const double2 nz01 = buf_load2(bnz, on), nz23 = buf_load2(bnz, on + 16u);
+        const double2 bx01 = buf_load2(bbx, ot), bx23 = buf_load2(bbx, ot + 16u);
+        const double2 by01 = buf_load2(bby, ot), by23 = buf_load2(bby, ot + 16u);
+        const double K11 = buf_load(b11, at(need_e, 8u * e)), K22 = buf_load(b22, at(need_n, 8u * e));
         // tracer at level tau: centre and east/north columns at k, k+up, k-dn;
         // west/south at k, k+1 (top faces only)
         double Tc[NTR], Tcu[NTR], Tcd[NTR], Te[NTR], Teu[NTR], Ted[NTR], Tn[NTR], Tnu[NTR], Tnd[NTR];
         double Tw[NTR], Twu[NTR], Ts[NTR], Tsu[NTR];
+        const bool ue = need_e || top, un = need_n || top;
 #pragma unroll
         for (int r = 0; r < NTR; ++r) {
-            const double* __restrict__ T = a.t[r].tr + (uint32_t)a.tau * g.ls;
-            Tc[r] = T[g.cs * c];
-            Tcu[r] = T[g.cs * (c + up)];
-            Tcd[r] = T[g.cs * (c - dn)];
-            Te[r] = Teu[r] = Ted[r] = Tn[r] = Tnu[r] = Tnd[r] = Tw[r] = Twu[r] = Ts[r] = Tsu[r] = 0.0;
-            if (need_e || top) {
-                Te[r] = T[g.cs * (c + si)];
-                Teu[r] = T[g.cs * (c + si + up)];
-            }
-            if (need_e) Ted[r] = T[g.cs * (c + si - dn)];
-            if (need_n || top) {
-                Tn[r] = T[g.cs * (c + sj)];
-                Tnu[r] = T[g.cs * (c + sj + up)];
-            }
-            if (need_n) Tnd[r] = T[g.cs * (c + sj - dn)];
-            if (top) {
-                Tw[r] = T[g.cs * (c - si)];
-                Twu[r] = T[g.cs * (c - si + 1)];
-                Ts[r] = T[g.cs * (c - sj)];
-                Tsu[r] = T[g.cs * (c - sj + 1)];
-            }
+            const double* T = a.t[r].tr + (int64_t)a.tau * g.ls + o0 * g.cs;
+            const BufRsrc bT = make_buf(T, ncells * cb), bTe = make_buf(T + row * g.cs, ncells * cb);
+            const BufRsrc bTw = make_buf(T - row * g.cs, ncells * cb);
+            Tc[r] = buf_load(bT, at(any, cb * e));
+            Tcu[r] = buf_load(bT, at(any, cb * (e + up)));
+            Tcd[r] = buf_load(bT, at(any, cb * (e - dn)));
+            Te[r] = buf_load(bTe, at(ue, cb * e));
+            Teu[r] = buf_load(bTe, at(ue, cb * (e + up)));
+            Ted[r] = buf_load(bTe, at(need_e, cb * (e - dn)));
+            Tn[r] = buf_load(bT, at(un, cb * (e + sj)));
+            Tnu[r] = buf_load(bT, at(un, cb * (e + sj + up)));
+            Tnd[r] = buf_load(bT, at(need_n, cb * (e + sj - dn)));
+            Tw[r] = buf_load(bTw, at(top, cb * e));
+            Twu[r] = buf_load(bTw, at(top, cb * (e + 1u)));
+            Ts[r] = buf_load(bT, at(top, cb * (e - sj)));
+            Tsu[r] = buf_load(bT, at(top, cb * (e - sj + 1u)));
         }
         // flux_east (:22-47), flux_north (:49-77), flux_top (:79-111)
-        const double dl_e = hm ? 0.25 * (k1_of<ISO>(in.K_c) + k1_of<ISO>(in.K_cm) + k1_of<ISO>(in.K_e) +
-                                         k1_of<ISO>(in.K_em))
-                               : 0.5 * (k1_of<ISO>(in.K_c) + k1_of<ISO>(in.K_e));
-        const double dl_n = hm ? 0.25 * (k1_of<ISO>(in.K_c) + k1_of<ISO>(in.K_cm) + k1_of<ISO>(in.K_n) +
-                                         k1_of<ISO>(in.K_nm))
-                               : 0.5 * (k1_of<ISO>(in.K_c) + k1_of<ISO>(in.K_n));
+        const ColMetrics& cm = bm.col[q];
+        const double r4zt = bm.lev.r4zt[k];
+        const double dl_e = hm ? 0.25 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_cm) + k1_of<ISO>(K_e) + k1_of<ISO>(K_em))
+                               : 0.5 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_e));
+        const double dl_n = hm ? 0.25 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_cm) + k1_of<ISO>(K_n) + k1_of<ISO>(K_nm))
+                               : 0.5 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_n));
 #pragma unroll
         for (int r = 0; r < NTR; ++r) {
-            if (need_e)
-                a.t[r].fe[c] = east_flux_core(dl_e, in.ez01, in.ez23, Tc[r], Tcu[r], Tcd[r], Te[r], Teu[r], Ted[r],
-                                              in.dzt, in.cost, in.dxu, in.K11);
-            if (need_n)
-                a.t[r].fn[c] = north_flux_core(dl_n, in.nz01, in.nz23, Tc[r], Tcu[r], Tcd[r], Tn[r], Tnu[r], Tnd[r],
-                                               in.dzt, in.cosu, in.dyu, in.K22);
-            if (need_t)
-                a.t[r].ft[c] = top ? top_flux_core(k2_of<ISO>(in.K_c), in.bx01, in.bx23, in.by01, in.by23, Tc[r],
-                                                   Tcu[r], Tw[r], Twu[r], Te[r], Teu[r], Ts[r], Tsu[r], Tn[r], Tnu[r],
-                                                   in.cost, in.cosu, in.cosu_s, in.dxt, in.dyt)
-                                   : 0.0;
+            const BufRsrc fe = make_buf(a.t[r].fe + o0, ncells * 8u), fn = make_buf(a.t[r].fn + o0, ncells * 8u);
+            const BufRsrc ft = make_buf(a.t[r].ft + o0, ncells * 8u);
+            buf_store(fe, at(need_e, 8u * e),
+                      east_flux_core(dl_e, ez01, ez23, Tc[r], Tcu[r], Tcd[r], Te[r], Teu[r], Ted[r], r4zt, cm.rx, K11));
+            buf_store(fn, at(need_n, 8u * e),
+                      north_flux_core(dl_n, nz01, nz23, Tc[r], Tcu[r], Tcd[r], Tn[r], Tnu[r], Tnd[r], r4zt, cm.cosu,
+                                      cm.ry, K22));
+            const double ftv = top_flux_core(k2_of<ISO>(K_c), bx01, bx23, by01, by23, Tc[r], Tcu[r], Tw[r], Twu[r],
+                                             Te[r], Teu[r], Ts[r], Tsu[r], Tn[r], Tnu[r], cm, r4xt);
+            buf_store(ft, at(need_t, 8u * e), top ? ftv : 0.0);
         }
     }
 }
@@ -1331,7 +1417,7 @@ struct AdjArgs {
 
 // A wave per tile of 8 columns of the whole grid (col_tile.hpp): one flat pass
 // over K_33 and mu. A lane per column with the factors in registers, and an
-// initialisation pass before it, took 50 + 8 us on 180x90x40, this @@ us.
+// initialisation pass before it, took 50 + 8 us on 180x90x40, this 11 us.
 constexpr int kAdjP = 8;
 constexpr int kAdjBlock = 128;
 template <int S>
@@ -1417,7 +1503,7 @@ __device__ __forceinline__ void adj_add(double* p, double v) {
 // K_iso); those of the levels next to it pass through LDS to the thread of
 // that level, so each thread adds 8 sums instead of up to 35 single terms
 // (180x90x40: 43 us and 11 us for a kernel that stored the face adjoints first;
-// now @@ us).
+// now 26 us).
 __global__ __launch_bounds__(256) void iso_adj_scatter_kernel(Grid g, AdjArgs a) {
     const CellIdx ci = cell_of(1, g.X - 3, 1, g.Y - 3);
     const int nz = g.nz;
@@ -1577,68 +1663,25 @@ Prm make_prm(const vx_iso_params* q) {
     return p;
 }
 
-// A helper stream per device (default priority, non-blocking) with a fork and
-// a join event, created on first use and kept for the process.
-struct AuxStream {
-    hipStream_t s = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
-};
-std::mutex& aux_mutex() {
-    static std::mutex m;
-    return m;
-}
-// Caller holds aux_mutex(). Null when the stream or events cannot be made.
-AuxStream* aux_stream() {
-    static std::map<int, AuxStream> per_device;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-    auto it = per_device.find(dev);
-    if (it != per_device.end()) return &it->second;
-    AuxStream a;
-    if (hipStreamCreateWithFlags(&a.s, hipStreamNonBlocking) != hipSuccess) return nullptr;
-    if (hipEventCreateWithFlags(&a.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&a.join, hipEventDisableTiming) != hipSuccess)
-        return nullptr;
-    return &(per_device[dev] = a);
-}
-
-// Work launched on the returned stream runs after everything enqueued on `s`
-// so far; `s` itself when no helper stream can be had. The fork record and
-// the wait on it form one step under the lock, so calls from other host
-// threads cannot slip their own fork in between.
-hipStream_t fork_aux(hipStream_t s) {
-    std::lock_guard<std::mutex> lk(aux_mutex());
-    AuxStream* ax = aux_stream();
-    if (ax && hipEventRecord(ax->fork, s) == hipSuccess && hipStreamWaitEvent(ax->s, ax->fork, 0) == hipSuccess)
-        return ax->s;
-    return s;
-}
-// Work enqueued on `s` from here on runs after everything enqueued on the
-// helper stream `sd` (a no-op when `sd` is `s`).
-int join_aux(hipStream_t s, hipStream_t sd, const char* who) {
-    if (sd == s) return VX_OK;
-    std::lock_guard<std::mutex> lk(aux_mutex());
-    AuxStream* ax = aux_stream();
-    if (!ax || hipEventRecord(ax->join, sd) != hipSuccess || hipStreamWaitEvent(s, ax->join, 0) != hipSuccess)
-        return fail(VX_ERR_LAUNCH, "%s: joining the helper stream failed", who);
-    return VX_OK;
-}
-
 #ifndef VX_PRE_CELLS
-#define VX_PRE_CELLS 3840
+#define VX_PRE_CELLS 640
 #endif
-// Columns per block of the wet-cell pre kernel: about VX_PRE_CELLS cells
-// (48 columns at nz = 80), so that a block's wet cells fill its 256 threads
-// for several rounds at typical land fractions and the partly filled last
-// round wastes few lanes (on 1440x720x80 with 31% wet cells a block holds
-// about 1180 wet cells: 5 rounds at 92% of the lanes, against 3 at 77% with
-// 24 columns). Measured there, pre + the temperature/salinity step in one
-// call: 240 cells per block 11.7 ms, 640 10.1 ms, 1920 9.8 ms (an earlier
-// build); 1920 against 3840 cells, four runs each alternating on one box:
-// 6.49 / 6.23 / 5.63 / 6.39 against 6.17 / 5.66 / 5.99 / 5.50 ms.
-int pre_columns(int nz) {
-    const int n = (VX_PRE_CELLS + nz - 1) / nz;
-    return n < 1 ? 1 : (n > 64 ? 64 : n);
+// Columns per block (one wave) of the pre and flux kernels: about VX_PRE_CELLS
+// cells (8 columns at nz = 80), so that a wave deals several rounds of cells
+// and the partly filled last one wastes few lanes, but at least four waves per
+// CU on small grids. The fused call on 1440x720x80 and the calls on 360x160x60
+// (levels innermost): 640 cells 6.04 ms and 1162 us, 1280 5.98 and 1204, 2400
+// 6.38 and 1262.
+int cell_columns(const Grid& g) {
+    const int64_t spread = ((int64_t)(g.X - 3) * (g.Y - 3) + 4 * cu_count() - 1) / (4 * cu_count());
+    const int n = (int)std::min<int64_t>((VX_PRE_CELLS + g.nz - 1) / g.nz, spread);
+    return n < 4 ? 4 : (n > kBlockCols ? kBlockCols : n);
+}
+// blocks of ncb columns over the cells' range, for block_cols
+dim3 cell_column_grid(const Grid& g, int ncb) {
+    const int sb = kPreStripCols / ncb;
+    const int64_t nstrips = (g.Y - 3 + (int64_t)sb * ncb - 1) / (sb * ncb);
+    return dim3((unsigned)((nstrips * (g.X - 3) * sb + 7) / 8 * 8));
 }
 
 unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -1647,7 +1690,8 @@ unsigned blocks_xcd(int64_t n, int bs) { return (unsigned)(((n + bs - 1) / bs + 
 // block of nz levels x cpb columns (about 256 threads); 1-D grid of ni row
 // groups, rounded up to a multiple of 8 for the XCD remap
 dim3 cell_block(int nz) { return dim3(nz, nz >= 256 ? 1 : 256 / nz); }
-dim3 cell_grid(int ni, int nj, dim3 blk, int sb = kStripBlocks) {
+dim3 cell_grid(int ni, int nj, dim3 blk) {
+    const int sb = kStripBlocks;
     const int64_t sw = (int64_t)sb * blk.y;
     const int64_t nstrips = (nj + sw - 1) / sw;
     return dim3((unsigned)((nstrips * ni * sb + 7) / 8 * 8));
@@ -1723,9 +1767,9 @@ int launch_step(const Grid& g, const Prm& p, const StepArgs& a, void* workspace,
     const WetPlan wp = wire_wet_plan(g, workspace, NTR);
     int rc = launch_wet_plan(g, wp, s, who);
     if (rc) return rc;
-    const int ncb = pre_columns(g.nz);
-    hipLaunchKernelGGL((iso_flux_kernel<NTR, IMPLICIT>), cell_grid(g.X - 3, g.Y - 3, dim3(1, ncb), kPreStripBlocks),
-                       dim3(256), (size_t)(ncb + 1) * sizeof(int), s, g, a, ncb);
+    const int ncb = cell_columns(g);
+    hipLaunchKernelGGL((iso_flux_kernel<NTR, IMPLICIT>), cell_column_grid(g, ncb), dim3(kCellBlock), 0, s, g, a,
+                       ncb);
     if ((rc = check_launch(who))) return rc;
     return launch_wet_step<NTR, IMPLICIT, false>(g, p, a, wp, s, who);
 }
@@ -1745,58 +1789,15 @@ bool tensor_ok(const double* Ai_ez, const double* Ai_nz, const double* Ai_bx, co
     return Ai_ez && Ai_nz && Ai_bx && Ai_by && K_11 && K_22;
 }
 
-// three flux arrays per tracer
-// isoneutral_diffusion_pre on `s`: the dry-cell zero fill on a helper stream
-// (forked from and joined back into `s`), the wet-cell kernel and the top
-// level of K_33 on `s`; FUSED also writes the step's face fluxes into `fo`.
-// The dry-cell zero fill (store-bound) and the wet-cell slopes (latency-bound)
-// write disjoint cells: the zero fill runs on a helper stream forked from `s`.
-// With `dry_stream` null it is joined back into `s` before returning; else the
-// helper stream goes to *dry_stream and the caller joins it (join_aux) once
-// nothing more it enqueues on `s` reads the dry cells' outputs.
+// isoneutral_diffusion_pre; FUSED also writes the step's face fluxes into `fo`.
 template <bool FUSED>
 int launch_pre(const Grid& g, const Prm& p, const Fields& f, const double* K_iso, double* Ai_ez, double* Ai_nz,
                double* Ai_bx, double* Ai_by, double* K_11, double* K_22, double* K_33, PreFlux fo, hipStream_t s,
-               const char* who, hipStream_t* dry_stream = nullptr, bool use_aux = true) {
-    int rc = VX_OK;
-    const int64_t ncol = (int64_t)(g.X - 3) * (g.Y - 3);  // one wave per column, 4 per block
-    // without the helper stream (use_aux false) the zero fill runs on `s`
-    const hipStream_t sd = use_aux ? fork_aux(s) : s;
-    if (dry_stream) *dry_stream = sd;
-    // Blocks of the zero fill, in eighths of the CU count (0: one wave per
-    // column). Beside the whole one call, fewer blocks than CUs fill in the
-    // background at a modest store rate instead of flooding the memory system
-    // ahead of the wet-cell kernels (measured on 1440x720x80 with the
-    // nontemporal stores, two runs each: 96 blocks 6.34 / 5.61 ms, 128 blocks
-    // 5.95 / 5.79, 160 blocks 5.80 / 5.73, 192 blocks 5.80 / 6.38, one block
-    // per CU 6.90 / 6.61, two per CU 7.05, one wave per column 6.98). Pre
-    // alone is joined at the end of pre, so there the fill must not start
-    // late: one wave per column (4.6 ms; one block per CU gave 4.26 ms on one
-    // box and a 5.1 ms median on another, where the fill's blocks were
-    // dispatched behind the wet cells').
-#ifndef VX_DRY_EIGHTHS_PRE
-#define VX_DRY_EIGHTHS_PRE 0
-#endif
-#ifndef VX_DRY_EIGHTHS_FUSED
-#define VX_DRY_EIGHTHS_FUSED 5
-#endif
-    // (on the caller's stream, without the helper, the fill runs before pre:
-    // the whole grid of it)
-    const unsigned eighths = (dry_stream && use_aux) ? VX_DRY_EIGHTHS_FUSED : VX_DRY_EIGHTHS_PRE;
-    const unsigned dry_full = blocks_for(ncol, 4), ndry = eighths * (unsigned)cu_count() / 8;
-    const unsigned dry_grid = ndry > 0 && ndry < dry_full ? ndry : dry_full;
-    hipLaunchKernelGGL(iso_pre_dry_kernel, dim3(dry_grid), dim3(256), 0, sd, g, Ai_ez, Ai_nz, Ai_bx, Ai_by,
-                       K_11, K_22, K_33);
-    if ((rc = check_launch(who))) return rc;
-    const int ncb = pre_columns(g.nz);
-    const size_t pre_lds = (size_t)(ncb + 1) * sizeof(int);
-    hipLaunchKernelGGL(iso_pre_kernel<FUSED>, cell_grid(g.X - 3, g.Y - 3, dim3(1, ncb), kPreStripBlocks), dim3(256),
-                       pre_lds, s, g, p,
-                       f, K_iso, Ai_ez, Ai_nz, Ai_bx, Ai_by, K_11, K_22, K_33, fo, ncb);
-    if ((rc = check_launch(who))) return rc;
-    hipLaunchKernelGGL(k33_top_zero_kernel, dim3(blocks_for((int64_t)g.X * g.Y, 256)), dim3(256), 0, s, g, K_33);
-    if ((rc = check_launch(who))) return rc;
-    return dry_stream ? VX_OK : join_aux(s, sd, who);
+               const char* who) {
+    const int ncb = cell_columns(g);
+    hipLaunchKernelGGL(iso_pre_kernel<FUSED>, cell_column_grid(g, ncb), dim3(kCellBlock), 0, s, g, p, f, K_iso, Ai_ez,
+                       Ai_nz, Ai_bx, Ai_by, K_11, K_22, K_33, fo, ncb);
+    return check_launch(who);
 }
 
 void wire_workspace(const Grid& g, StepArgs& a, int ntr, void* ws) {
@@ -1961,12 +1962,12 @@ namespace vx {
 namespace {
 
 // The one call (pre, then the temperature and salinity steps) with the given
-// workspace; `use_aux` false keeps every launch on `s` (no helper stream).
+// workspace.
 int pre_diffusion_ts(hipStream_t s, const vx_grid* grid, const vx_iso_params* prm, double* temp, double* salt,
                      int32_t tau, int32_t taup1, const double* K_iso, double* Ai_ez, double* Ai_nz, double* Ai_bx,
                      double* Ai_by, double* K_11, double* K_22, double* K_33, double* dtemp_iso, double* dsalt_iso,
                      const double* int_drhodT, const double* int_drhodS, double* P_diss, void* workspace,
-                     bool use_aux, const char* who) {
+                     const char* who) {
     Grid g;
     int rc = check_common(grid, prm, tau, taup1, g, who);
     if (rc) return rc;
@@ -1997,15 +1998,9 @@ int pre_diffusion_ts(hipStream_t s, const vx_grid* grid, const vx_iso_params* pr
     // the wet-cell plan of the step (reads kbot only)
     const WetPlan wp = wire_wet_plan(g, workspace, 2);
     if ((rc = launch_wet_plan(g, wp, s, who))) return rc;
-    // The step kernel reads no output of a dry cell (its fluxes come from the
-    // wet-cell kernel, and it reads K_33 only on wet cells), so the dry-cell
-    // zero fill overlaps the whole call and is joined at its end.
-    hipStream_t sd = s;
     rc = launch_pre<true>(g, p, Fields{temp, salt, tau}, K_iso, Ai_ez, Ai_nz, Ai_bx, Ai_by, K_11, K_22, K_33, fo, s,
-                          who, &sd, use_aux);
-    if (!rc) rc = launch_wet_step<2, true, true>(g, p, a, wp, s, who);
-    const int rj = join_aux(s, sd, who);
-    return rc ? rc : rj;
+                          who);
+    return rc ? rc : launch_wet_step<2, true, true>(g, p, a, wp, s, who);
 }
 
 }  // namespace
@@ -2019,7 +2014,7 @@ extern "C" int vx_iso_pre_diffusion_ts_f64(void* stream, const vx_grid* grid, co
                                            void* workspace) {
     return vx::pre_diffusion_ts((hipStream_t)stream, grid, prm, temp, salt, tau, taup1, K_iso, Ai_ez, Ai_nz, Ai_bx,
                                 Ai_by, K_11, K_22, K_33, dtemp_iso, dsalt_iso, int_drhodT, int_drhodS, P_diss,
-                                workspace, true, "vx_iso_pre_diffusion_ts_f64");
+                                workspace, "vx_iso_pre_diffusion_ts_f64");
 }
 
 // ---------------------------------------------------------------------------
@@ -2079,8 +2074,7 @@ extern "C" int vx_iso_pre_diffusion_ts_f64_noalloc(void* stream, const vx_grid* 
     void* ws = scratch_on_current_device(who);
     if (!ws) return VX_ERR_LAUNCH;
     return pre_diffusion_ts((hipStream_t)stream, grid, prm, temp, salt, tau, taup1, K_iso, Ai_ez, Ai_nz, Ai_bx,
-                            Ai_by, K_11, K_22, K_33, dtemp_iso, dsalt_iso, int_drhodT, int_drhodS, P_diss, ws, false,
-                            who);
+                            Ai_by, K_11, K_22, K_33, dtemp_iso, dsalt_iso, int_drhodT, int_drhodS, P_diss, ws, who);
 }
 
 extern "C" int vx_iso_pre_f64(void* stream, const vx_grid* grid, const vx_iso_params* prm, const double* temp,

