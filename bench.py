@@ -626,8 +626,7 @@ def main():
     t_dom = parts[dom][0]
     traffic = PRE_TS_TRAFFIC_BYTES.get((nx, ny, nz, args.levels))
     roof = {"bound": "hbm",
-            "kernel": "vx_iso_pre_diffusion_ts_f64 = wet_scan_{count,chunks,columns}_kernel + "
-                      "iso_pre_kernel<true> + iso_step_wet_kernel<2>",
+            "kernel": "vx_iso_pre_diffusion_ts_f64 = iso_pre_kernel<true> + iso_step_wet_kernel<2>",
             "achieved": round(gbs[dom], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs[dom] / HBM_PEAK_GBS, 4),
             "traffic": traffic,

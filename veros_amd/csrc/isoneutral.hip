@@ -2,7 +2,6 @@
 //
 //   iso_pre_kernel       isoneutral_diffusion_pre  veros/core/isoneutral/isoneutral.py:18-229
 //   iso_flux_kernel      _calc_tracer_fluxes       veros/core/isoneutral/diffusion.py:9-113
-//   wet_scan_*_kernel    the wet-cell plan of a step (from kbot)
 //   iso_step_wet_kernel  _calc_explicit_part, _calc_implicit_part, the tracer and
 //                        dtr_iso updates and the energy branch, over the wet cells
 //                                                  veros/core/isoneutral/diffusion.py:116-283,
@@ -300,11 +299,11 @@ __device__ __forceinline__ void scan_runs(int* r, int ncb) {
     }
 }
 // the column q with run[q] <= t < run[q + 1]
-__device__ __forceinline__ int run_column(const BlockMetrics& m, int ncb, int t) {
+__device__ __forceinline__ int run_column(const int* run, int ncb, int t) {
     int lo = 0, hi = ncb - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (m.run[mid] <= t) lo = mid;
+        if (run[mid] <= t) lo = mid;
         else hi = mid - 1;
     }
     return lo;
@@ -355,8 +354,13 @@ __device__ __forceinline__ double top_flux_core(double diffloc, double2 B01, dou
 
 // Face-flux outputs of the fused pre + flux kernel (temperature, salinity).
 struct PreFlux {
-    double *fe[2], *fn[2], *ft[2];
+    double *fe, *fn, *ft;
 };
+// Two tracers' flux at one cell; the caller's workspace may be aligned to 8 bytes only.
+typedef double vx_d2a8 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void store_pair(double* p, double t, double s) {
+    *reinterpret_cast<vx_d2a8*>(p) = (vx_d2a8){t, s};
+}
 
 // The dry cells of isoneutral_diffusion_pre: every output exactly zero (its own
 // maskT factor is in maskU (Ai_ez, K_11), maskV (Ai_nz, K_22) and maskW (Ai_bx,
@@ -542,10 +546,11 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
             // differences vanish there)
             const double a0 = hm ? out[0] : Aez[4u * c], a2 = hm ? out[2] : Aez[4u * c + 2];
             const double2 A01 = make_double2(a0, out[1]), A23 = make_double2(a2, out[3]);
-            fo.fe[0][c] = east_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Te, hp ? Tep : Te,
-                                         hm ? Tem : Te, r4zt, rx_c, k11v);
-            fo.fe[1][c] = east_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Se, hp ? Sep : Se,
-                                         hm ? Sem : Se, r4zt, rx_c, k11v);
+            const double feT = east_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Te, hp ? Tep : Te,
+                hm ? Tem : Te, r4zt, rx_c, k11v);
+            const double feS = east_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Se, hp ? Sep : Se,
+                hm ? Sem : Se, r4zt, rx_c, k11v);
+            store_pair(fo.fe + 2u * c, feT, feS);
         }
     }
 
@@ -587,10 +592,11 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
         if constexpr (FUSED) {
             const double a0 = hm ? out[0] : Anz[4u * c], a2 = hm ? out[2] : Anz[4u * c + 2];
             const double2 A01 = make_double2(a0, out[1]), A23 = make_double2(a2, out[3]);
-            fo.fn[0][c] = north_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Tn, hp ? Tnp : Tn,
-                                          hm ? Tnm : Tn, r4zt, cm.cosu, ry_c, k22v);
-            fo.fn[1][c] = north_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Sn, hp ? Snp : Sn,
-                                          hm ? Snm : Sn, r4zt, cm.cosu, ry_c, k22v);
+            const double fnT = north_flux_core(diffloc, A01, A23, Tc, hp ? Tcp : Tc, hm ? Tcm : Tc, Tn, hp ? Tnp : Tn,
+                hm ? Tnm : Tn, r4zt, cm.cosu, ry_c, k22v);
+            const double fnS = north_flux_core(diffloc, A01, A23, Sc, hp ? Scp : Sc, hm ? Scm : Sc, Sn, hp ? Snp : Sn,
+                hm ? Snm : Sn, r4zt, cm.cosu, ry_c, k22v);
+            store_pair(fo.fn + 2u * c, fnT, fnS);
         }
     }
 
@@ -648,17 +654,17 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
         if constexpr (FUSED) {
             const double2 B01 = make_double2(ox[0], ox[1]), B23 = make_double2(ox[2], ox[3]);
             const double2 C01 = make_double2(oy[0], oy[1]), C23 = make_double2(oy[2], oy[3]);
-            fo.ft[0][c] = top_flux_core(Kc, B01, B23, C01, C23, Tc, Tcp, Tw, Twp, Te, Tep, Ts, Tsp, Tn, Tnp, cm,
-                                        r4xt);
-            fo.ft[1][c] = top_flux_core(Kc, B01, B23, C01, C23, Sc, Scp, Sw, Swp, Se, Sep, Ss, Ssp, Sn, Snp, cm,
-                                        r4xt);
+            const double ftT = top_flux_core(Kc, B01, B23, C01, C23, Tc, Tcp, Tw, Twp, Te, Tep, Ts, Tsp, Tn, Tnp, cm,
+                r4xt);
+            const double ftS = top_flux_core(Kc, B01, B23, C01, C23, Sc, Scp, Sw, Swp, Se, Sep, Ss, Ssp, Sn, Snp, cm,
+                r4xt);
+            store_pair(fo.ft + 2u * c, ftT, ftS);
         }
     }
     if (i >= 2 && j >= 2 && !hp) {
         K33[c] = 0.0;  // (:225)
         if constexpr (FUSED) {  // no flux through the top level
-            fo.ft[0][c] = 0.0;
-            fo.ft[1][c] = 0.0;
+            store_pair(fo.ft + 2u * c, 0.0, 0.0);
         }
     }
 }
@@ -718,7 +724,7 @@ __global__ __launch_bounds__(kCellBlock) __attribute__((amdgpu_waves_per_eu(VX_P
         // this lane's cell of a round (a lane past the last cell: that cell, not stored)
         auto locate = [&](int t, int& q, int& k) {
             const int tt = t < nwet ? t : nwet - 1;
-            q = run_column(bm, ncb, tt);
+            q = run_column(bm.run, ncb, tt);
             k = nz - (bm.run[q + 1] - bm.run[q]) + (tt - bm.run[q]);  // wet suffix of column q
         };
         int q, k;
@@ -759,18 +765,20 @@ __global__ __launch_bounds__(kCellBlock) __attribute__((amdgpu_waves_per_eu(VX_P
 //   iso_step_wet_kernel phase 1 (thread per wet cell): lateral dissipation on
 //     T points, the flux divergence, rhs = tr[taup1] + dt*dtr, and the K33
 //     rows -> LDS
-//   phase 2 (lane per interior column and tracer): Thomas sweep in LDS
+//   phase 2 (8 lanes per interior column and tracer): segmented elimination in LDS
 //   phase 3 (thread per wet cell): tracer, dtr_iso and P_diss updates
 // ---------------------------------------------------------------------------
 struct TracerArgs {
     double* tr;           // (X, Y, nz, 3)
     double* dtr;          // (X, Y, nz)
     const double* I;      // int_drhodX (X, Y, nz, 3), nullable
-    double *fe, *fn, *ft; // workspace: flux_east, flux_north, flux_top (X, Y, nz)
 };
 
 struct StepArgs {
     TracerArgs t[2];
+    // workspace: flux_east, flux_north, flux_top, (X, Y, nz) cells with the
+    // tracers' values side by side
+    double *fe, *fn, *ft;
     int tau, taup1;
     // K1 = K_iso - K_skew (east/north faces), K2 = K_iso + K_skew (top faces);
     // a null pointer is a zero term (veros/core/isoneutral/diffusion.py:15-16,180-188)
@@ -820,6 +828,9 @@ typedef unsigned int vx_u4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ double2 buf_load2(BufRsrc b, uint32_t off) {
     return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(b, off, 0, 0));
 }
+__device__ __forceinline__ void buf_store2(BufRsrc b, uint32_t off, double2 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(vx_u4, v), b, off, 0, 0);
+}
 
 // Every read is a buffer load at an offset that is past the buffer's end where
 // the cell does not need it (no traffic, no branch around the load, all of a
@@ -854,7 +865,7 @@ __global__ __launch_bounds__(kCellBlock) void iso_flux_kernel(Grid g, StepArgs a
     const BufRsrc b11 = make_buf(a.K11 + o0, ncells * 8u), b22 = make_buf(a.K22 + o0, ncells * 8u);
     const uint32_t cb = 8u * g.cs;  // bytes from a level to the next in the time-level arrays
     for (int t = tid; t < ncell; t += nthr) {
-        const int q = run_column(bm, ncb, t);
+        const int q = run_column(bm.run, ncb, t);
         const int j = jb + q;
         const int k = nz - (bm.run[q + 1] - bm.run[q]) + (t - bm.run[q]);
         const int kb = bm.kb[q + 1], kb_e = bm.kbe[q], kb_n = bm.kb[q + 2];
@@ -908,186 +919,30 @@ __global__ __launch_bounds__(kCellBlock) void iso_flux_kernel(Grid g, StepArgs a
                                : 0.5 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_e));
         const double dl_n = hm ? 0.25 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_cm) + k1_of<ISO>(K_n) + k1_of<ISO>(K_nm))
                                : 0.5 * (k1_of<ISO>(K_c) + k1_of<ISO>(K_n));
+        double fe[NTR], fn[NTR], ft[NTR];
 #pragma unroll
         for (int r = 0; r < NTR; ++r) {
-            const BufRsrc fe = make_buf(a.t[r].fe + o0, ncells * 8u), fn = make_buf(a.t[r].fn + o0, ncells * 8u);
-            const BufRsrc ft = make_buf(a.t[r].ft + o0, ncells * 8u);
-            buf_store(fe, at(need_e, 8u * e),
-                      east_flux_core(dl_e, ez01, ez23, Tc[r], Tcu[r], Tcd[r], Te[r], Teu[r], Ted[r], r4zt, cm.rx, K11));
-            buf_store(fn, at(need_n, 8u * e),
-                      north_flux_core(dl_n, nz01, nz23, Tc[r], Tcu[r], Tcd[r], Tn[r], Tnu[r], Tnd[r], r4zt, cm.cosu,
-                                      cm.ry, K22));
+            fe[r] = east_flux_core(dl_e, ez01, ez23, Tc[r], Tcu[r], Tcd[r], Te[r], Teu[r], Ted[r], r4zt, cm.rx, K11);
+            fn[r] = north_flux_core(dl_n, nz01, nz23, Tc[r], Tcu[r], Tcd[r], Tn[r], Tnu[r], Tnd[r], r4zt, cm.cosu,
+                                    cm.ry, K22);
             const double ftv = top_flux_core(k2_of<ISO>(K_c), bx01, bx23, by01, by23, Tc[r], Tcu[r], Tw[r], Twu[r],
                                              Te[r], Teu[r], Ts[r], Tsu[r], Tn[r], Tnu[r], cm, r4xt);
-            buf_store(ft, at(need_t, 8u * e), top ? ftv : 0.0);
+            ft[r] = top ? ftv : 0.0;
         }
+        constexpr uint32_t fb = 8u * NTR;  // bytes of a cell's fluxes
+        auto put = [&](double* f, bool on, const double (&v)[NTR]) {
+            const BufRsrc bf = make_buf(f + o0 * NTR, ncells * fb);
+            if constexpr (NTR == 2) buf_store2(bf, at(on, fb * e), make_double2(v[0], v[1]));
+            else buf_store(bf, at(on, fb * e), v[0]);
+        };
+        put(a.fe, need_e, fe);
+        put(a.fn, need_n, fn);
+        put(a.ft, need_t, ft);
     }
 }
 
-// Workspace fluxes with their valid index ranges (0 elsewhere).
-__device__ __forceinline__ double fe_at(const Grid& g, const TracerArgs& t, int i, int j, uint32_t o) {
-    return (i >= 1 && i <= g.X - 3 && j >= 2 && j <= g.Y - 3) ? t.fe[o] : 0.0;
-}
-__device__ __forceinline__ double fn_at(const Grid& g, const TracerArgs& t, int i, int j, uint32_t o) {
-    return (i >= 2 && i <= g.X - 3 && j >= 1 && j <= g.Y - 3) ? t.fn[o] : 0.0;
-}
-
-
-// ---------------------------------------------------------------------------
-// Wet-cell tracer step. The wet columns of the step's range [1, X-1) x
-// [1, Y-1) are ranked in the strip order of wet_col_ij (rank r, a column's wet
-// cells being its levels kbot-1 .. nz-1), and their cells are numbered in the
-// same order (column r holds cells o_r .. o_r + w_r - 1). The cells are cut
-// into groups: group b takes the wet columns with
-// b*C <= o_r < (b+1)*C, C = kWetThreads - nz + 1, so a group holds at most
-// C + nz - 1 = kWetThreads cells (w_r <= nz). A block steps one group at a
-// time with a thread per cell, so no lane is spent on a dry cell; the plan is
-// built on the device from kbot by three small scan kernels.
-// ---------------------------------------------------------------------------
-constexpr int kWetThreads = 256;
-constexpr int kScanColsPerThread = 8;
-constexpr int kScanChunk = kWetThreads * kScanColsPerThread;  // columns per scan block
-
-struct WetPlan {
-    int* wetcol;  // [ncols]   enumeration index (wet_col_ij) of the wet column of rank r
-    int* wetoff;  // [ncols]   o_r, the number of wet cells before it
-    int* first;   // [ncols+2] first[b] = first rank of group b; first[ngroups] = number of wet columns
-    int* nb;      // [12]      ngroups, wet columns, wet cells, -, then a group counter per XCD
-    int2* chunk;  // [nchunks] (wet columns, wet cells) per scan chunk, then their exclusive sums
-};
-
-// The columns of the step range are enumerated in strips of kWetStrip
-// columns along j, each strip walked row by row along i, so that the rows a
-// group's stencil reaches (i-1, i+1) are stepped close in time and share an
-// L2; the columns past Y-2 in the last strip are padding without wet cells.
-#ifndef VX_WET_STRIP
-#define VX_WET_STRIP 64
-#endif
-constexpr int kWetStrip = VX_WET_STRIP;
-__host__ __device__ inline int64_t wet_enum_cols(int64_t X, int64_t Y) {
-    return (Y - 2 + kWetStrip - 1) / kWetStrip * (X - 2) * kWetStrip;
-}
-__device__ __forceinline__ void wet_col_ij(const Grid& g, int col, int& i, int& j) {
-    const int per = (g.X - 2) * kWetStrip;
-    const int sidx = col / per;
-    const int rem = col - sidx * per;
-    const int ii = rem / kWetStrip;
-    i = 1 + ii;
-    j = 1 + sidx * kWetStrip + (rem - ii * kWetStrip);
-}
-__device__ __forceinline__ int wet_count(const Grid& g, int64_t col, int64_t ncols) {
-    if (col >= ncols) return 0;
-    int i, j;
-    wet_col_ij(g, (int)col, i, j);
-    if (j > g.Y - 2) return 0;
-    const int kb = g.kbot[i * g.Y + j];
-    return (kb >= 1 && kb <= g.nz) ? g.nz - kb + 1 : 0;
-}
-
-// In-place inclusive sum over the block (Hillis-Steele; every thread calls it).
-__device__ __forceinline__ void block_scan2(int* s0, int* s1, int tid) {
-    for (int st = 1; st < kWetThreads; st <<= 1) {
-        const int a0 = tid >= st ? s0[tid - st] : 0, a1 = tid >= st ? s1[tid - st] : 0;
-        __syncthreads();
-        s0[tid] += a0;
-        s1[tid] += a1;
-        __syncthreads();
-    }
-}
-
-// per scan chunk of kScanChunk columns: (wet columns, wet cells)
-__global__ __launch_bounds__(kWetThreads) void wet_scan_count_kernel(Grid g, WetPlan w, int64_t ncols) {
-    __shared__ int s0[kWetThreads], s1[kWetThreads];
-    const int tid = (int)threadIdx.x;
-    const int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)tid * kScanColsPerThread;
-    int nc = 0, ncell = 0;
-    for (int q = 0; q < kScanColsPerThread; ++q) {
-        const int n = wet_count(g, base + q, ncols);
-        nc += n > 0 ? 1 : 0;
-        ncell += n;
-    }
-    s0[tid] = nc;
-    s1[tid] = ncell;
-    __syncthreads();
-    block_scan2(s0, s1, tid);
-    if (tid == kWetThreads - 1) w.chunk[blockIdx.x] = make_int2(s0[tid], s1[tid]);
-}
-
-// one block: exclusive sums of the chunk counts, and the totals
-__global__ __launch_bounds__(kWetThreads) void wet_scan_chunks_kernel(WetPlan w, int nchunks) {
-    __shared__ int s0[kWetThreads], s1[kWetThreads];
-    __shared__ int carry[2];
-    const int tid = (int)threadIdx.x;
-    if (tid == 0) carry[0] = carry[1] = 0;
-    __syncthreads();
-    for (int base = 0; base < nchunks; base += kWetThreads) {
-        const int q = base + tid;
-        const int2 v = q < nchunks ? w.chunk[q] : make_int2(0, 0);
-        s0[tid] = v.x;
-        s1[tid] = v.y;
-        __syncthreads();
-        block_scan2(s0, s1, tid);
-        const int c0 = carry[0], c1 = carry[1];
-        if (q < nchunks) w.chunk[q] = make_int2(c0 + s0[tid] - v.x, c1 + s1[tid] - v.y);
-        __syncthreads();
-        if (tid == kWetThreads - 1) {
-            carry[0] = c0 + s0[tid];
-            carry[1] = c1 + s1[tid];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        w.nb[0] = 0;  // set by wet_scan_columns_kernel when there is a wet column
-        w.nb[1] = carry[0];
-        w.nb[2] = carry[1];
-    }
-    if (tid < 8) w.nb[4 + tid] = 0;  // the step kernel's group counters
-}
-
-// ranks, offsets and the group starts
-__global__ __launch_bounds__(kWetThreads) void wet_scan_columns_kernel(Grid g, WetPlan w, int64_t ncols, int C) {
-    __shared__ int s0[kWetThreads], s1[kWetThreads];
-    const int tid = (int)threadIdx.x;
-    const int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)tid * kScanColsPerThread;
-    int n[kScanColsPerThread];
-    int nc = 0, ncell = 0;
-#pragma unroll
-    for (int q = 0; q < kScanColsPerThread; ++q) {
-        n[q] = wet_count(g, base + q, ncols);
-        nc += n[q] > 0 ? 1 : 0;
-        ncell += n[q];
-    }
-    s0[tid] = nc;
-    s1[tid] = ncell;
-    __syncthreads();
-    block_scan2(s0, s1, tid);
-    const int2 co = w.chunk[blockIdx.x];
-    int r = co.x + s0[tid] - nc, o = co.y + s1[tid] - ncell;
-    const int nwc = w.nb[1];
-#pragma unroll
-    for (int q = 0; q < kScanColsPerThread; ++q) {
-        if (n[q] > 0) {
-            w.wetcol[r] = (int)(base + q);
-            w.wetoff[r] = o;
-            if (r == 0) w.first[0] = 0;
-            // the group boundary m = b*C inside (o, o + n]: the columns before
-            // group b are ranks 0 .. r
-            const int m = (o / C + 1) * C;
-            if (m <= o + n[q]) w.first[m / C] = r + 1;
-            if (r == nwc - 1) {
-                const int ng = o / C + 1;
-                w.first[ng] = nwc;
-                w.nb[0] = ng;
-            }
-            ++r;
-            o += n[q];
-        }
-    }
-}
-
-// Per-tracer LDS arrays of the tracer step: F (flux_top), D (lateral
-// dissipation), R (rhs -> alpha -> new), Q (c' -> gamma), Wk (spike -> beta).
-constexpr int kStepArrays = 5;
+constexpr int kStepThreads = 256;  // threads of a tracer-step block, and the most cells of a group
+constexpr int kStepCols = 64;      // most columns of a block
 
 // One column's K33 system (rows a, b, c of n levels in LDS, right-hand side
 // in r) solved in place into r by the kSegP lanes of a group, lane sg owning
@@ -1159,173 +1014,256 @@ __device__ __forceinline__ void seg_lds_column(const double* a, const double* b,
     if (mL < n) r[mL] = Ls[0];
 }
 
-// Persistent grid (a multiple of 8 blocks): the blocks of XCD x (blockIdx % 8)
-// share the groups [x, x+1) * ngroups / 8, so neighbouring rows share an L2,
-// and take them one at a time from that XCD's counter.
-// IMPLICIT: the K33 part (isoneutral step); else the explicit step only (skew).
-// WETFLUX: the face fluxes exist for wet cells only (the fused pre formed them
-// from the tensor it wrote, in which every face touching a dry cell carries a
-// zero flux), so a face whose other cell is dry reads as zero; else they come
-// from iso_flux_kernel, which writes every face of a wet cell, including the
-// top face of the dry cell below the lowest wet one.
-#ifndef VX_WET_WAVES
-#define VX_WET_WAVES 5  // 96 VGPRs: five blocks per CU
-#endif
-template <int NTR, bool IMPLICIT, bool WETFLUX>
-__global__ __launch_bounds__(kWetThreads) __attribute__((amdgpu_waves_per_eu(VX_WET_WAVES))) void iso_step_wet_kernel(
-    Grid g, Prm p, StepArgs a, WetPlan w) {
-    extern __shared__ double lds[];
-    constexpr int T = kWetThreads;
-    // LDS: rows A, B, C (shared by the tracers), then per tracer F (flux_top),
-    // D (lateral dissipation), R (rhs -> alpha -> new), Q (c' -> gamma), Wk
-    // (spike -> beta), each T cells; then the group's column table
-    double* sA = lds;
-    double* sB = lds + T;
-    double* sC = lds + 2 * T;
-    double* sT = lds + 3 * T;
-    int* sOff = reinterpret_cast<int*>(lds + (3 + kStepArrays * NTR) * T);  // [T+1] first cell of each column
-    int* sCol = sOff + (T + 1);                                   // [T]   its column index
-    const int nz = g.nz;
-    const int tid = (int)threadIdx.x;
-    const int ngroups = w.nb[0];
-    const int xcd = (int)(blockIdx.x & 7);
-    const int gbeg = (int)((int64_t)ngroups * xcd / 8), gend = (int)((int64_t)ngroups * (xcd + 1) / 8);
-    const Strides st{(uint32_t)g.Y * (uint32_t)nz, (uint32_t)nz};
-    const bool energy = a.P != nullptr;
-    const double dt = p.dt_tracer;
-    __shared__ int sGrp;
-    for (;;) {
-        __syncthreads();  // the previous group's LDS (and sGrp) is no longer read
-        if (tid == 0) sGrp = gbeg + atomicAdd(&w.nb[4 + xcd], 1);
-        __syncthreads();
-        const int grp = sGrp;
-        if (grp >= gend) break;  // uniform: every block ends once its XCD's share is taken
-        const int r0 = w.first[grp], r1 = w.first[grp + 1];
-        const int ncolg = r1 - r0;
-        const int o0 = w.wetoff[r0];
-        if (tid < ncolg) {
-            sOff[tid] = w.wetoff[r0 + tid] - o0;
-            sCol[tid] = w.wetcol[r0 + tid];
-        }
-        if (tid == 0) sOff[ncolg] = (grp + 1 < ngroups ? w.wetoff[r1] : w.nb[2]) - o0;
-        __syncthreads();
-        const int ncell = sOff[ncolg];
-        const bool have = tid < ncell;
-        // this thread's cell: the column q with sOff[q] <= tid < sOff[q+1]
-        int q = 0;
-        if (have) {
-            int hi = ncolg - 1;
-            while (q < hi) {
-                const int mid = (q + hi + 1) >> 1;
-                if (sOff[mid] <= tid) q = mid;
-                else hi = mid - 1;
-            }
-        }
-        const int lo = tid;
-        int i, j;
-        wet_col_ij(g, have ? sCol[q] : 0, i, j);
-        const int kb = have ? nz - (sOff[q + 1] - sOff[q]) + 1 : 1;
-        const int k = kb - 1 + (tid - sOff[q]);
-        const bool interior = have && i >= 2 && i <= g.X - 3 && j >= 2 && j <= g.Y - 3;
-        const uint32_t c = (uint32_t)i * st.si + (uint32_t)j * st.sj + (uint32_t)k;
-        bool west_ok = have, south_ok = have;
-        if (WETFLUX && have) {
-            west_ok = wet(g.kbot[(i - 1) * g.Y + j], k);
-            south_ok = wet(g.kbot[i * g.Y + j - 1], k);
-        }
+// Per-block tables of the tracer step, in LDS.
+struct StepTables {
+    double rxc[kStepCols], ryc[kStepCols];             // 1 / (dxt cost), 1 / (dyt cost)
+    double rzt[kMaxNz], rzw[kMaxNz], dzw[kMaxNz];      // 1 / dzt, 1 / dzw, dzw
+    int kb[kStepCols + 1], kbw[kStepCols];             // kbot at j-1 .. of row i; at row i-1
+    int off[kStepCols + 1];                            // prefix sums of the columns' wet cells
+    double rdt, g05, gr;                               // 1 / dt, grav / (2 rho_0), -grav / rho_0
+};
 
-        // ---- every global read first
-        double fe_c[NTR], fe_w[NTR], fn_c[NTR], fn_s[NTR], ft_c[NTR], ft_b[NTR];
-        double Ic[NTR], Ie[NTR], Iw[NTR], In[NTR], Is[NTR], Iu[NTR], trp[NTR], dtr0[NTR];
+// One lane's cell of a group of columns.
+struct StepCell {
+    int q, k, kb;
+    uint32_t e;  // cells from the block's first column's level 0
+    bool have, interior;
+};
+// The global reads of one cell. Every lane loads (a lane past the group's last
+// cell that cell's values), at an offset inside the arrays; what a cell does
+// not have reads a value it has and is set to zero afterwards.
+template <int NTR>
+struct StepIn {
+    double fe_c[NTR], fe_w[NTR], fn_c[NTR], fn_s[NTR], ft_c[NTR], ft_b[NTR];
+    double Ic[NTR], Ie[NTR], Iw[NTR], In[NTR], Is[NTR], Iu[NTR], trp[NTR], dtr0[NTR];
+    double K33k, K33m, P0;
+};
+// Loads at a byte offset from a pointer that is the same for the whole wave:
+// held in scalar registers, they need one vector register of address.
+template <class V>
+__device__ __forceinline__ V load_at(const double* base, uint32_t off) {
+    typedef const __attribute__((address_space(1))) char* gptr;
+    gptr p = (gptr)base;
+    asm("" : "+s"(p));
+    return *(const __attribute__((address_space(1))) V*)(p + off);
+}
+template <int NTR>
+__device__ __forceinline__ void load_fluxes(const double* base, uint32_t e, double (&v)[NTR]) {
+    if constexpr (NTR == 2) {
+        const vx_d2a8 w = load_at<vx_d2a8>(base, 16u * e);
+        v[0] = w.x;
+        v[1] = w.y;
+    } else {
+        v[0] = load_at<double>(base, 8u * e);
+    }
+}
+// o0: the cell of the block's first column's level 0; offsets start one column
+// before it, so that they stay positive for the south column and level k-1
+template <int NTR, bool IMPLICIT, bool WETFLUX>
+__device__ __forceinline__ void step_load(const Grid& g, const StepArgs& a, const StepTables& tb, int64_t o0,
+                                          const StepCell& s, StepIn<NTR>& v) {
+    const uint32_t sj = (uint32_t)g.nz;
+    const int64_t b = o0 - g.nz, row = (int64_t)g.Y * g.nz;
+    const uint32_t e = s.e + sj;
+    const int k = s.k;
+    const bool south = !WETFLUX || wet(tb.kb[s.q], k);
+    load_fluxes<NTR>(a.fe + NTR * b, e, v.fe_c);
+    load_fluxes<NTR>(a.fe + NTR * (b - row), e, v.fe_w);
+    load_fluxes<NTR>(a.fn + NTR * b, e, v.fn_c);
+    load_fluxes<NTR>(a.fn + NTR * b, south ? e - sj : e, v.fn_s);
+    load_fluxes<NTR>(a.ft + NTR * b, e, v.ft_c);
+    // the top face of the dry cell below the lowest wet cell
+    const bool below = !WETFLUX && k == s.kb - 1 && k >= 1;
+    if constexpr (!WETFLUX) load_fluxes<NTR>(a.ft + NTR * b, below ? e - 1u : e, v.ft_b);
+    const uint32_t cb = 8u * g.cs;  // bytes from a level to the next in the time-level arrays
+#pragma unroll
+    for (int t = 0; t < NTR; ++t) {
+        v.trp[t] = load_at<double>(a.t[t].tr + (b * g.cs + (int64_t)a.taup1 * g.ls), cb * e);
+        v.dtr0[t] = load_at<double>(a.t[t].dtr + b, 8u * e);
+    }
+    if constexpr (IMPLICIT) {
+        v.K33k = load_at<double>(a.K33 + b, 8u * e);
+        v.K33m = load_at<double>(a.K33 + b, 8u * (e - 1u));
+    }
+    v.P0 = 0.0;
+    if (a.P) {
+        v.P0 = load_at<double>(a.P + b, 8u * e);
 #pragma unroll
         for (int t = 0; t < NTR; ++t) {
-            const TracerArgs& ta = a.t[t];
-            fe_c[t] = fe_w[t] = fn_c[t] = fn_s[t] = ft_c[t] = ft_b[t] = 0.0;
-            Ic[t] = Ie[t] = Iw[t] = In[t] = Is[t] = Iu[t] = trp[t] = dtr0[t] = 0.0;
-            if (have) {
-                fe_c[t] = fe_at(g, ta, i, j, c);
-                fe_w[t] = west_ok ? fe_at(g, ta, i - 1, j, c - st.si) : 0.0;
-                fn_c[t] = fn_at(g, ta, i, j, c);
-                fn_s[t] = south_ok ? fn_at(g, ta, i, j - 1, c - st.sj) : 0.0;
-                if (interior) {
-                    trp[t] = ta.tr[g.cs * c + (uint32_t)a.taup1 * g.ls];
-                    dtr0[t] = ta.dtr[c];
-                    ft_c[t] = ta.ft[c];
-                    // the top face of the dry cell below the lowest wet cell
-                    if (!WETFLUX && k == kb - 1 && k >= 1) ft_b[t] = ta.ft[c - 1];
-                }
-                if (energy) {
-                    const double* __restrict__ I = ta.I + (uint32_t)a.tau * g.ls;
-                    Ic[t] = I[g.cs * c];
-                    Ie[t] = I[g.cs * (c + st.si)];
-                    Iw[t] = I[g.cs * (c - st.si)];
-                    In[t] = I[g.cs * (c + st.sj)];
-                    Is[t] = I[g.cs * (c - st.sj)];
-                    if (interior && k < nz - 1) Iu[t] = I[g.cs * (c + 1)];
-                }
-            }
+            const double* I = a.t[t].I + (b * g.cs + (int64_t)a.tau * g.ls);
+            v.Ic[t] = load_at<double>(I, cb * e);
+            v.Ie[t] = load_at<double>(I + row * g.cs, cb * e);
+            v.Iw[t] = load_at<double>(I - row * g.cs, cb * e);
+            v.In[t] = load_at<double>(I, cb * (e + sj));
+            v.Is[t] = load_at<double>(I, cb * (e - sj));
+            v.Iu[t] = load_at<double>(I, cb * (e + 1u));
         }
-        double K33k = 0.0, K33m = 0.0;
-        if (IMPLICIT && interior) {
-            K33k = a.K33[c];
-            if (k >= kb) K33m = a.K33[c - 1];  // the edge row k = kbot-1 has no sub-diagonal
-        }
-        const double P0 = (energy && have) ? a.P[c] : 0.0;
-        double dxt_i = 0.0, cost_j = 1.0, dyt_j = 0.0, dzt_k = 1.0, dzw_k = 1.0, dzw_lo = 1.0;
-        if (have) {
-            dxt_i = g.dxt[i];
-            cost_j = g.cost[j];
-            dyt_j = g.dyt[j];
-            dzt_k = g.dzt[k];
-            dzw_k = g.dzw[k];
-            dzw_lo = g.dzw[k >= 1 ? k - 1 : 0];  // pad_z_edges(dzw)[k]
-        }
+    }
+}
+// Fluxes outside the range the flux kernels write (veros/core/isoneutral/
+// diffusion.py:22-111), and those of faces touching a dry cell (WETFLUX), are zero.
+template <int NTR, bool WETFLUX>
+__device__ __forceinline__ void step_mask(const Grid& g, const StepTables& tb, int i, int j, const StepCell& s,
+                                          StepIn<NTR>& v) {
+    const bool jin = j >= 2 && j <= g.Y - 3, iin = i >= 2 && i <= g.X - 3;
+    const bool west = !WETFLUX || wet(tb.kbw[s.q], s.k), south = !WETFLUX || wet(tb.kb[s.q], s.k);
+    const bool ec = jin && i <= g.X - 3, ew = jin && i >= 2 && west;
+    const bool nc = iin && j <= g.Y - 3, ns = iin && j >= 2 && south;
+    const bool below = !WETFLUX && s.k == s.kb - 1 && s.k >= 1;
+#pragma unroll
+    for (int t = 0; t < NTR; ++t) {
+        v.fe_c[t] = ec ? v.fe_c[t] : 0.0;
+        v.fe_w[t] = ew ? v.fe_w[t] : 0.0;
+        v.fn_c[t] = nc ? v.fn_c[t] : 0.0;
+        v.fn_s[t] = ns ? v.fn_s[t] : 0.0;
+        if constexpr (!WETFLUX) v.ft_b[t] = below ? v.ft_b[t] : 0.0;
+    }
+}
+
+// A block owns ncb consecutive columns of row i (strips as in block_cols) and
+// steps their wet cells in groups of whole columns, as many as fit its threads:
+// thread per cell, except in phase 2. IMPLICIT: the K33 part (isoneutral step);
+// else the explicit step only (skew). WETFLUX: the face fluxes exist for wet
+// cells only (the fused pre formed them from the tensor it wrote, in which every
+// face touching a dry cell carries a zero flux), so a face whose other cell is
+// dry counts as zero; else they come from iso_flux_kernel, which writes every
+// face of a wet cell, including the top face of the dry cell below the lowest
+// wet one. The multiply-adds are written out so that all variants round alike.
+//
+// Bound by the wait for its loads: a group's 20 loads are issued together, then
+// the block computes behind barriers while the CU's other blocks load. Blocks
+// over fixed columns replace a plan of all wet cells (three scan kernels a
+// call) with groups taken from a counter (four dependent reads before the first
+// load), the tracers' fluxes side by side halve the flux loads, and the metric
+// factors come from LDS. Four waves per SIMD hold all loads in registers (at
+// five they spill: 1440x720x80 5.90 ms against 5.43). pre + T + S on 1440x720x80
+// 6.05 -> 5.43 ms, on 90x40x15 54 -> 32 us; all isoneutral calls of a step on
+// 360x160x60, levels innermost, 1120 -> 910 us.
+#ifndef VX_STEP_WAVES
+#define VX_STEP_WAVES 4
+#endif
+// columns along j of a strip: 64 and 192 are within 0.2% on 1440x720x80
+#ifndef VX_STEP_STRIP_COLS
+#define VX_STEP_STRIP_COLS 192
+#endif
+constexpr int kStepStripCols = VX_STEP_STRIP_COLS;
+template <int NTR, bool IMPLICIT, bool WETFLUX>
+__global__ __launch_bounds__(kStepThreads) __attribute__((amdgpu_waves_per_eu(VX_STEP_WAVES))) void iso_step_wet_kernel(
+    Grid g, Prm p, StepArgs a, int ncb, int sb) {
+#pragma clang fp contract(off)
+    constexpr int T = kStepThreads;
+    // rows A, B, C, shared by the tracers; per tracer flux_top, then the solve's c' -> gamma; lateral
+    // dissipation; rhs -> alpha -> new; spike -> beta
+    __shared__ double sA[T], sB[T], sC[T], sF[NTR][T], sD[NTR][T], sR[NTR][T], sW[NTR][T];
+    __shared__ StepTables tb;
+    const BlockCols bc = block_cols(1, g.X - 2, 1, g.Y - 2, ncb, sb);
+    if (!bc.valid) return;  // padding block (uniform)
+    const int tid = (int)threadIdx.x, nz = g.nz;
+    const int i = __builtin_amdgcn_readfirstlane(bc.i), jb = __builtin_amdgcn_readfirstlane(bc.j);
+    const int64_t first = ((int64_t)i * g.Y + jb) * nz;
+    const double dt = p.dt_tracer;
+    for (int q = tid; q < ncb; q += T) {
+        const bool real = jb + q <= g.Y - 2;
+        const int j = real ? jb + q : g.Y - 2;
+        const int kb = g.kbot[i * g.Y + j];
+        tb.kb[q + 1] = kb;
+        tb.kbw[q] = g.kbot[(i - 1) * g.Y + j];
+        tb.off[q + 1] = real && kb >= 1 && kb <= nz ? nz - kb + 1 : 0;
+        tb.rxc[q] = 1.0 / (g.dxt[i] * g.cost[j]);
+        tb.ryc[q] = 1.0 / (g.dyt[j] * g.cost[j]);
+    }
+    if (tid == T - 1) {
+        tb.kb[0] = g.kbot[i * g.Y + jb - 1];
+        tb.rdt = 1.0 / dt;
+        tb.g05 = 0.5 * p.grav / p.rho_0;
+        tb.gr = -p.grav / p.rho_0;
+    }
+    for (int k = tid; k < nz; k += T) {
+        const double dzw = g.dzw[k];
+        tb.dzw[k] = dzw;
+        tb.rzw[k] = 1.0 / dzw;
+        tb.rzt[k] = 1.0 / g.dzt[k];
+    }
+    __syncthreads();
+    scan_runs(tb.off, ncb);
+    __syncthreads();
+    const int nwet = tb.off[ncb];
+    const bool iin = i >= 2 && i <= g.X - 3;
+    const bool energy = a.P != nullptr;
+
+    // the group that starts at column q0: its end (as many whole columns as fit) and this thread's cell
+    auto locate = [&](int q0, StepCell& s) {
+        const int p0 = tb.off[q0], lane = tid & 63;
+        const int q = q0 + 1 + lane;
+        const int q1 = q0 + (int)__popcll(__ballot(q <= ncb && tb.off[q <= ncb ? q : ncb] - p0 <= T));
+        const int n = tb.off[q1] - p0;
+        s.have = tid < n;
+        const int t = p0 + (s.have ? tid : n - 1);
+        s.q = run_column(tb.off, ncb, t);
+        s.kb = tb.kb[s.q + 1];
+        s.k = s.kb - 1 + (t - tb.off[s.q]);
+        const int j = jb + s.q;
+        s.interior = s.have && iin && j >= 2 && j <= g.Y - 3;
+        s.e = (uint32_t)(s.q * nz + s.k);
+        return q1;
+    };
+    if (nwet == 0) return;  // uniform
+    for (int q0 = 0;;) {
+        StepCell s;
+        StepIn<NTR> v;
+        const int q1 = locate(q0, s);
+        // what follows from the thread and the block alone (addresses, the
+        // solve's lane numbers) is formed anew for each group: kept over the
+        // loop it takes some 40 registers
+        int64_t o0 = first;
+        int lo = tid;
+        asm volatile("" : "+s"(o0), "+v"(lo));
+        step_load<NTR, IMPLICIT, WETFLUX>(g, a, tb, o0, s, v);
+        __builtin_amdgcn_sched_barrier(0);
+        const int k = s.k;
+        const int j = jb + s.q;
+        step_mask<NTR, WETFLUX>(g, tb, i, j, s, v);
+        const double rzt = tb.rzt[k];
 
         // ---- phase 1a: flux_top and lateral dissipation -> LDS, K33 rows -> LDS
-        if (have) {
+        if (s.have) {
 #pragma unroll
             for (int t = 0; t < NTR; ++t) {
-                double* sTt = sT + t * kStepArrays * T;
-                sTt[lo] = ft_c[t];
+                sF[t][lo] = v.ft_c[t];
                 if (energy) {
                     // compute_dissipation (veros/core/diffusion.py:13-33)
-                    const double de = (Ie[t] - Ic[t]) * fe_c[t] + (Ic[t] - Iw[t]) * fe_w[t];
-                    const double dn = (In[t] - Ic[t]) * fn_c[t] + (Ic[t] - Is[t]) * fn_s[t];
-                    const double g05 = 0.5 * p.grav / p.rho_0;
-                    sTt[T + lo] = g05 * de / (dxt_i * cost_j) + g05 * dn / (dyt_j * cost_j);
+                    const double de = fma(v.Ie[t] - v.Ic[t], v.fe_c[t], (v.Ic[t] - v.Iw[t]) * v.fe_w[t]);
+                    const double dn = fma(v.In[t] - v.Ic[t], v.fn_c[t], (v.Ic[t] - v.Is[t]) * v.fn_s[t]);
+                    sD[t][lo] = tb.g05 * fma(de, tb.rxc[s.q], dn * tb.ryc[s.q]);
                 }
             }
         }
-        if (IMPLICIT && interior) {
+        if (IMPLICIT && s.interior) {
             // rows of the K33 system (veros/core/isoneutral/diffusion.py:154-164); the
             // edge row k = kbot-1 takes b_edge and a = 0 (veros/core/operators.py:72)
-            const double delta = (k < nz - 1) ? dt / dzw_k * K33k : 0.0;
-            const double delta_m = (k >= 1) ? dt / dzw_lo * K33m : 0.0;
-            const double dz = dzt_k;
-            const bool edge = k == kb - 1;
-            sA[lo] = edge ? 0.0 : -delta_m / dz;
-            sB[lo] = edge ? 1 + delta / dz : 1 + (delta + delta_m) / dz;
-            sC[lo] = (k < nz - 1) ? -delta / dz : 0.0;
+            const bool edge = k == s.kb - 1;
+            const double up = (k < nz - 1) ? dt * tb.rzw[k] * v.K33k * rzt : 0.0;
+            const double dn = edge ? 0.0 : dt * tb.rzw[k >= 1 ? k - 1 : 0] * v.K33m * rzt;
+            sA[lo] = -dn;
+            sB[lo] = 1 + (up + dn);
+            sC[lo] = -up;
         }
         __syncthreads();
 
         // ---- phase 1b: divergence and rhs (veros/core/isoneutral/diffusion.py:116-139,196-197)
-        double dtrk[NTR], rhs[NTR];
+        double dtr1[NTR], rhs[NTR], dI[NTR];  // dtr plus the explicit tendency
 #pragma unroll
         for (int t = 0; t < NTR; ++t) {
-            dtrk[t] = rhs[t] = 0.0;
-            if (interior) {
-                double* sTt = sT + t * kStepArrays * T;
-                // below the lowest wet cell: with the fused pre's fluxes the
-                // top face there is zero (its maskW), else it was read above
-                const double ftm = (k >= kb) ? sTt[lo - 1] : ft_b[t];
-                const double hor = (fe_c[t] - fe_w[t]) / (cost_j * dxt_i) +
-                                   (fn_c[t] - fn_s[t]) / (cost_j * dyt_j);
-                const double vert = (k == 0) ? ft_c[t] / dzt_k : (ft_c[t] - ftm) / dzt_k;
-                dtrk[t] = hor + vert;
-                rhs[t] = trp[t] + dt * dtrk[t];
-                sTt[2 * T + lo] = rhs[t];
-            }
+            // below the lowest wet cell: with the fused pre's fluxes the top
+            // face there is zero (its maskW), else it was read above
+            const double ftm = (k >= s.kb) ? sF[t][lo > 0 ? lo - 1 : 0] : (WETFLUX ? 0.0 : v.ft_b[t]);
+            const double hor = fma(v.fe_c[t] - v.fe_w[t], tb.rxc[s.q], (v.fn_c[t] - v.fn_s[t]) * tb.ryc[s.q]);
+            const double vert = (k == 0 ? v.ft_c[t] : v.ft_c[t] - ftm) * rzt;
+            const double dtrk = hor + vert;
+            dtr1[t] = v.dtr0[t] + dtrk;
+            dI[t] = energy ? v.Ic[t] - v.Iu[t] : 0.0;
+            rhs[t] = fma(dt, dtrk, v.trp[t]);
+            sR[t][lo] = rhs[t];
         }
         __syncthreads();
 
@@ -1333,60 +1271,48 @@ __global__ __launch_bounds__(kWetThreads) __attribute__((amdgpu_waves_per_eu(VX_
         // solves the column's run in LDS by the segmented elimination
         // (tdma_seg.hpp), segments of S = max(2, ceil(n / kSegP)) rows, rows
         // past the run identity rows
-        if (IMPLICIT) {
-            const int sg = tid & (kSegP - 1);
-            for (int task = tid / kSegP; task < ncolg * NTR; task += T / kSegP) {
-                const int cq = task % ncolg, t = task / ncolg;
-                int ci, cj;
-                wet_col_ij(g, sCol[cq], ci, cj);
-                if (ci < 2 || ci > g.X - 3 || cj < 2 || cj > g.Y - 3) continue;  // uniform in the group
-                const int b0 = sOff[cq], n = sOff[cq + 1] - b0;
-                double* sTt = sT + t * kStepArrays * T;
-                seg_lds_column(sA + b0, sB + b0, sC + b0, sTt + 2 * T + b0, sTt + 3 * T + b0, sTt + 4 * T + b0, n,
-                               sg);
+        if (IMPLICIT && iin) {
+            const int sg = lo & (kSegP - 1), ncol = q1 - q0, p0 = tb.off[q0];
+            for (int task = lo / kSegP; task < ncol * NTR; task += T / kSegP) {
+                const int t = NTR == 2 && task >= ncol ? 1 : 0, cq = q0 + task - t * ncol;
+                const int cj = jb + cq, b0 = tb.off[cq] - p0, n = tb.off[cq + 1] - tb.off[cq];
+                if (cj < 2 || cj > g.Y - 3 || n == 0) continue;  // uniform in the group
+                seg_lds_column(sA + b0, sB + b0, sC + b0, &sR[t][b0], &sF[t][b0], &sW[t][b0], n, sg);
             }
         }
         __syncthreads();
 
         // ---- phase 3
-        if (have) {
-            double Pk = P0;
+        if (s.have) {
+            double Pk = v.P0;
+            asm volatile("" : "+s"(o0));
+            const double rzw = tb.rzw[k], dzw_lo = tb.dzw[k >= 1 ? k - 1 : 0];  // pad_z_edges(dzw)[k]
 #pragma unroll
             for (int t = 0; t < NTR; ++t) {
-                const double* sTt = sT + t * kStepArrays * T;
-                if (interior) {
-                    const double newk = sTt[2 * T + lo];
-                    a.t[t].tr[g.cs * c + (uint32_t)a.taup1 * g.ls] = newk;
-                    a.t[t].dtr[c] = (dtr0[t] + dtrk[t]) + (newk - rhs[t]) / dt;
+                const double newk = sR[t][lo], newu = sR[t][lo + 1 < T ? lo + 1 : lo];
+                if (s.interior) {
+                    (a.t[t].tr + (o0 * g.cs + (int64_t)a.taup1 * g.ls))[g.cs * s.e] = newk;
+                    (a.t[t].dtr + o0)[s.e] = fma(newk - rhs[t], tb.rdt, dtr1[t]);
                 }
                 if (energy) {
                     // dissipation_on_wgrid (veros/core/diffusion.py:39-62)
-                    const double d0 = sTt[T + lo];
-                    double dw;
-                    if (k == nz - 1) {
-                        dw = d0;
-                    } else {
-                        const double d1 = sTt[T + lo + 1];
-                        const double avg = 0.5 * (d0 + d1);
-                        const bool edge = k == kb - 1;
-                        dw = (avg + 0.5 * (d0 * dzw_lo / dzw_k)) * (edge ? 1.0 : 0.0) + avg * (edge ? 0.0 : 1.0);
-                    }
-                    Pk = Pk + dw;
+                    const double d0 = sD[t][lo];
+                    const double avg = 0.5 * (d0 + sD[t][lo + 1 < T ? lo + 1 : lo]);
+                    const double low = k == s.kb - 1 ? 0.5 * (d0 * dzw_lo * rzw) : 0.0;
+                    Pk = Pk + (k == nz - 1 ? d0 : avg + low);
                     // vertical mixing term (veros/core/isoneutral/diffusion.py:254-279)
-                    if (interior && k < nz - 1) {
-                        const double fxa = (-Iu[t] + Ic[t]) / dzw_k;
-                        const double gr = -p.grav / p.rho_0;
-                        if constexpr (IMPLICIT) {
-                            const double dtrz = sTt[2 * T + lo + 1] - sTt[2 * T + lo];
-                            Pk = Pk + gr * fxa * (ft_c[t] * 1.0 + K33k * dtrz / dzw_k * 1.0);
-                        } else {
-                            Pk = Pk + gr * fxa * ft_c[t] * 1.0;
-                        }
+                    if (s.interior && k < nz - 1) {
+                        const double fxa = dI[t] * rzw;
+                        const double flux = IMPLICIT ? fma(v.K33k * rzw, newu - newk, v.ft_c[t]) : v.ft_c[t];
+                        Pk = fma(tb.gr * fxa, flux, Pk);
                     }
                 }
             }
-            if (energy) a.P[c] = Pk;
+            if (energy) (a.P + o0)[s.e] = Pk;
         }
+        if (tb.off[q1] == nwet) break;  // uniform: only dry columns are left
+        __syncthreads();  // the group's LDS is no longer read
+        q0 = q1;
     }
 }
 
@@ -1706,72 +1632,37 @@ namespace vx {
 namespace {
 
 
-// The wet-cell plan after the tracers' face fluxes in a step's workspace.
-int64_t wet_plan_ncols(int64_t X, int64_t Y) { return wet_enum_cols(X, Y); }
-int64_t wet_plan_nchunks(int64_t X, int64_t Y) { return (wet_plan_ncols(X, Y) + kScanChunk - 1) / kScanChunk; }
-int64_t wet_plan_bytes(int64_t X, int64_t Y) {
-    const int64_t ints = 3 * wet_plan_ncols(X, Y) + 2 + 12;
-    return (ints * (int64_t)sizeof(int) + 7) / 8 * 8 + wet_plan_nchunks(X, Y) * (int64_t)sizeof(int2);
-}
-WetPlan wire_wet_plan(const Grid& g, void* ws, int ntr) {
-    const int64_t ncols = wet_plan_ncols(g.X, g.Y);
-    char* base = static_cast<char*>(ws) + 3 * ntr * (int64_t)g.X * g.Y * g.nz * (int64_t)sizeof(double);
-    WetPlan w;
-    int* ip = reinterpret_cast<int*>(base);
-    w.wetcol = ip;
-    w.wetoff = ip + ncols;
-    w.first = ip + 2 * ncols;
-    w.nb = ip + 3 * ncols + 2;
-    const int64_t ints = 3 * ncols + 2 + 12;
-    w.chunk = reinterpret_cast<int2*>(base + (ints * (int64_t)sizeof(int) + 7) / 8 * 8);
-    return w;
-}
-
-// The wet-cell plan of the step from kbot (three small kernels on `s`).
-int launch_wet_plan(const Grid& g, const WetPlan& wp, hipStream_t s, const char* who) {
-    const int64_t ncols = wet_plan_ncols(g.X, g.Y);
-    const int nchunks = (int)wet_plan_nchunks(g.X, g.Y);
-    const int C = kWetThreads - g.nz + 1;  // >= nz as nz <= kMaxNz
-    hipLaunchKernelGGL(wet_scan_count_kernel, dim3(nchunks), dim3(kWetThreads), 0, s, g, wp, ncols);
-    int rc = check_launch(who);
-    if (rc) return rc;
-    hipLaunchKernelGGL(wet_scan_chunks_kernel, dim3(1), dim3(kWetThreads), 0, s, wp, nchunks);
-    if ((rc = check_launch(who))) return rc;
-    hipLaunchKernelGGL(wet_scan_columns_kernel, dim3(nchunks), dim3(kWetThreads), 0, s, g, wp, ncols, C);
-    return check_launch(who);
-}
-
-#ifndef VX_WET_BPC
-#define VX_WET_BPC 5
+#ifndef VX_STEP_COLS
+#define VX_STEP_COLS 32
 #endif
-// The tracer step over the wet cells: persistent, VX_WET_BPC blocks per CU (as
-// many as fit), a multiple of 8 in all (measured on 1440x720x80: 3 blocks per
-// CU 9.0 ms for the fused pre + temperature/salinity call, 4 8.45 ms, 5 at
-// five waves per SIMD 8.29 ms).
+// Columns per block: a group is about six wet columns at nz = 80, and the last
+// group of a block is partly empty, so the more columns the fewer idle lanes; but
+// at least four blocks per CU on small grids. 1440x720x80 pre + T + S and the
+// calls on 360x160x60: 16 columns 5.00 ms and 958 us, 32 4.89 and 963, 64 4.85
+// and 1006 (one placement of the arrays; 48 0.8% faster and 1.7% slower than 32).
 template <int NTR, bool IMPLICIT, bool WETFLUX>
-int launch_wet_step(const Grid& g, const Prm& p, const StepArgs& a, const WetPlan& wp, hipStream_t s,
-                    const char* who) {
-    const unsigned nblk = (unsigned)((cu_count() * VX_WET_BPC + 7) / 8 * 8);
-    const size_t lds = (size_t)(3 + kStepArrays * NTR) * kWetThreads * sizeof(double) +
-                       (2 * kWetThreads + 1) * sizeof(int);
-    hipLaunchKernelGGL((iso_step_wet_kernel<NTR, IMPLICIT, WETFLUX>), dim3(nblk), dim3(kWetThreads), lds, s, g, p, a,
-                       wp);
+int launch_wet_step(const Grid& g, const Prm& p, const StepArgs& a, hipStream_t s, const char* who) {
+    const int64_t spread = ((int64_t)(g.X - 2) * (g.Y - 2) + 4 * cu_count() - 1) / (4 * cu_count());
+    int ncb = (int)std::min<int64_t>(VX_STEP_COLS, spread);
+    ncb = ncb < 4 ? 4 : ncb;
+    const int sb = (kStepStripCols + ncb - 1) / ncb;
+    const int64_t nstrips = (g.Y - 2 + (int64_t)sb * ncb - 1) / (sb * ncb);
+    const unsigned nblk = (unsigned)((nstrips * (g.X - 2) * sb + 7) / 8 * 8);
+    hipLaunchKernelGGL((iso_step_wet_kernel<NTR, IMPLICIT, WETFLUX>), dim3(nblk), dim3(kStepThreads), 0, s, g, p, a,
+                       ncb, sb);
     return check_launch(who);
 }
 
 template <int NTR, bool IMPLICIT>
-int launch_step(const Grid& g, const Prm& p, const StepArgs& a, void* workspace, hipStream_t s, const char* who) {
+int launch_step(const Grid& g, const Prm& p, const StepArgs& a, hipStream_t s, const char* who) {
     if ((int64_t)g.X * g.Y * g.nz * 4 >= ((int64_t)1 << 32))
         return fail(VX_ERR_UNSUPPORTED, "%s: grid too large for 32-bit offsets", who);
     if (g.nz > kMaxNz) return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d too deep", who, g.nz);
-    const WetPlan wp = wire_wet_plan(g, workspace, NTR);
-    int rc = launch_wet_plan(g, wp, s, who);
-    if (rc) return rc;
     const int ncb = cell_columns(g);
     hipLaunchKernelGGL((iso_flux_kernel<NTR, IMPLICIT>), cell_column_grid(g, ncb), dim3(kCellBlock), 0, s, g, a,
                        ncb);
-    if ((rc = check_launch(who))) return rc;
-    return launch_wet_step<NTR, IMPLICIT, false>(g, p, a, wp, s, who);
+    const int rc = check_launch(who);
+    return rc ? rc : launch_wet_step<NTR, IMPLICIT, false>(g, p, a, s, who);
 }
 
 int check_common(const vx_grid* grid, const vx_iso_params* prm, int32_t tau, int32_t taup1, Grid& g,
@@ -1803,11 +1694,9 @@ int launch_pre(const Grid& g, const Prm& p, const Fields& f, const double* K_iso
 void wire_workspace(const Grid& g, StepArgs& a, int ntr, void* ws) {
     const int64_t n3 = (int64_t)g.X * g.Y * g.nz;
     double* w = static_cast<double*>(ws);
-    for (int t = 0; t < ntr; ++t) {
-        a.t[t].fe = w + (3 * t + 0) * n3;
-        a.t[t].fn = w + (3 * t + 1) * n3;
-        a.t[t].ft = w + (3 * t + 2) * n3;
-    }
+    a.fe = w;
+    a.fn = w + ntr * n3;
+    a.ft = w + 2 * ntr * n3;
 }
 }  // namespace
 }  // namespace vx
@@ -1836,7 +1725,7 @@ extern "C" int vx_iso_diffusion_f64(void* stream, const vx_grid* grid, const vx_
     a.Kskew = nullptr;
     a.Aez = Ai_ez, a.Anz = Ai_nz, a.Abx = Ai_bx, a.Aby = Ai_by, a.K11 = K_11, a.K22 = K_22, a.K33 = K_33;
     a.P = P_diss;
-    return launch_step<1, true>(g, make_prm(prm), a, workspace, (hipStream_t)stream, who);
+    return launch_step<1, true>(g, make_prm(prm), a, (hipStream_t)stream, who);
 }
 
 extern "C" int vx_iso_diffusion_ts_f64(void* stream, const vx_grid* grid, const vx_iso_params* prm, double* temp,
@@ -1870,7 +1759,7 @@ extern "C" int vx_iso_diffusion_ts_f64(void* stream, const vx_grid* grid, const 
     a.Kskew = nullptr;
     a.Aez = Ai_ez, a.Anz = Ai_nz, a.Abx = Ai_bx, a.Aby = Ai_by, a.K11 = K_11, a.K22 = K_22, a.K33 = K_33;
     a.P = P_diss;
-    return launch_step<2, true>(g, make_prm(prm), a, workspace, (hipStream_t)stream, who);
+    return launch_step<2, true>(g, make_prm(prm), a, (hipStream_t)stream, who);
 }
 
 extern "C" int vx_iso_skew_diffusion_f64(void* stream, const vx_grid* grid, const vx_iso_params* prm,
@@ -1898,13 +1787,17 @@ extern "C" int vx_iso_skew_diffusion_f64(void* stream, const vx_grid* grid, cons
     a.Kskew = K_gm;
     a.Aez = Ai_ez, a.Anz = Ai_nz, a.Abx = Ai_bx, a.Aby = Ai_by, a.K11 = K_11, a.K22 = K_22, a.K33 = nullptr;
     a.P = P_diss_skew;
-    return launch_step<1, false>(g, make_prm(prm), a, workspace, (hipStream_t)stream, who);
+    return launch_step<1, false>(g, make_prm(prm), a, (hipStream_t)stream, who);
 }
 
 extern "C" int64_t vx_iso_workspace_bytes(const vx_grid* grid, int32_t ntracers) {
     if (!grid || ntracers < 1 || ntracers > 2 || grid->nx < 1 || grid->ny < 1 || grid->nz < 1) return -1;
-    return 3 * (int64_t)ntracers * (grid->nx + 4) * (grid->ny + 4) * (int64_t)grid->nz * (int64_t)sizeof(double) +
-           vx::wet_plan_bytes(grid->nx + 4, grid->ny + 4);
+    // the face fluxes, and per column and 2048 columns the room of the index
+    // tables that callers' buffers have always held
+    const int64_t X = grid->nx + 4, Y = grid->ny + 4, cols = (Y - 2 + 63) / 64 * (X - 2) * 64;
+    const int64_t ints = 3 * cols + 2 + 12;
+    return 3 * (int64_t)ntracers * X * Y * (int64_t)grid->nz * (int64_t)sizeof(double) +
+           (ints * (int64_t)sizeof(int) + 7) / 8 * 8 + (cols + 2047) / 2048 * 8;
 }
 
 extern "C" int64_t vx_iso_pre_diffusion_ts_workspace_bytes(const vx_grid* grid) {
@@ -1994,13 +1887,10 @@ int pre_diffusion_ts(hipStream_t s, const vx_grid* grid, const vx_iso_params* pr
     a.Aez = Ai_ez, a.Anz = Ai_nz, a.Abx = Ai_bx, a.Aby = Ai_by, a.K11 = K_11, a.K22 = K_22, a.K33 = K_33;
     a.P = P_diss;
     const Prm p = make_prm(prm);
-    const PreFlux fo{{a.t[0].fe, a.t[1].fe}, {a.t[0].fn, a.t[1].fn}, {a.t[0].ft, a.t[1].ft}};
-    // the wet-cell plan of the step (reads kbot only)
-    const WetPlan wp = wire_wet_plan(g, workspace, 2);
-    if ((rc = launch_wet_plan(g, wp, s, who))) return rc;
+    const PreFlux fo{a.fe, a.fn, a.ft};
     rc = launch_pre<true>(g, p, Fields{temp, salt, tau}, K_iso, Ai_ez, Ai_nz, Ai_bx, Ai_by, K_11, K_22, K_33, fo, s,
                           who);
-    return rc ? rc : launch_wet_step<2, true, true>(g, p, a, wp, s, who);
+    return rc ? rc : launch_wet_step<2, true, true>(g, p, a, s, who);
 }
 
 }  // namespace
@@ -2018,9 +1908,8 @@ extern "C" int vx_iso_pre_diffusion_ts_f64(void* stream, const vx_grid* grid, co
 }
 
 // ---------------------------------------------------------------------------
-// The one call without a caller workspace: the face fluxes and the wet-cell
-// plan live in `scratch`, a device array of the library (one per GPU, held
-// until the process ends). Its device address is taken once per device with
+// The one call without a caller workspace: the face fluxes live in `scratch`,
+// a device array of the library (one per GPU, held until the process ends). Its device address is taken once per device with
 // hipGetSymbolAddress; host code never passes the array's own name to a
 // kernel. The entry point allocates nothing: no hipMalloc, no helper stream.
 // ---------------------------------------------------------------------------
