@@ -249,11 +249,15 @@ int launch_segl(const TdmaArgs& p, hipStream_t s, const char* who) {
     case N:                                                                 \
         hipLaunchKernelGGL((K<N, true>::fn), grid, block, lds, s, p);       \
         break;
-    switch (S) {  // the depths of tdma_lds_wins
+    switch (S) {
         VX_SEGL_CASE(2)
+        VX_SEGL_CASE(4)
         VX_SEGL_CASE(6)
+        VX_SEGL_CASE(8)
         VX_SEGL_CASE(10)
         VX_SEGL_CASE(12)
+        VX_SEGL_CASE(14)
+        VX_SEGL_CASE(16)
         default:
             return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, p.nz);
     }
@@ -268,8 +272,7 @@ int launch_tile(const TdmaArgs& p, hipStream_t s, const char* who) {
     const dim3 grid((unsigned)((g.ntiles + waves - 1) / waves)), block(kSegLdsBlock);
 #define VX_TILE_CASE(N) \
     case N: hipLaunchKernelGGL((tdma_tile_kernel<N, MODE>), grid, block, 0, s, p, g); break;
-    switch (seg_levels(p.nz)) {
-        VX_TILE_CASE(2)
+    switch (seg_levels(p.nz)) {  // not 2: tdma_own_levels
         VX_TILE_CASE(4)
         VX_TILE_CASE(6)
         VX_TILE_CASE(8)
@@ -335,7 +338,13 @@ bool use_column_kernels() { return tdma_kernel_family() == 0; }
 bool use_segment_kernels() { return tdma_kernel_family() == 1; }
 
 bool lds_kernel_wins(const TdmaArgs& p, bool mixed) {
-    return tdma_vec_ok(p) && tdma_lds_wins(seg_levels(p.nz), mixed);
+    const int S = seg_levels(p.nz);
+    return tdma_vec_ok(p) && (tdma_lds_wins(S, mixed, false) || tdma_lds_resident(S, tdma_tiling(p).ntiles));
+}
+
+// the segmented kernels with register loads
+bool own_levels(const TdmaArgs& p) {
+    return use_segment_kernels() || (tdma_own_levels(seg_levels(p.nz)) && !tdma_vec_ok(p));
 }
 
 template <int N, bool V>
@@ -388,7 +397,7 @@ extern "C" int vx_tdma_f64(void* stream, const double* a, const double* b, const
     int rc = validate_tdma(p, nx, ny, nz, "vx_tdma_f64");
     if (rc != VX_OK || p.ncol == 0) return rc;
     if (use_column_kernels()) return launch_bucket<F64K>(p, (hipStream_t)stream, "vx_tdma_f64");
-    if (use_segment_kernels()) return launch_seg<SegF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
+    if (own_levels(p)) return launch_seg<SegF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
     if (lds_kernel_wins(p, false)) return launch_segl<SeglF64K>(p, (hipStream_t)stream, "vx_tdma_f64");
     return launch_tile<-1>(p, (hipStream_t)stream, "vx_tdma_f64");
 }
@@ -412,7 +421,7 @@ extern "C" int vx_tdma_mixed(void* stream, const double* a, const double* b, con
             default: return launch_bucket<MixK2>(p, s, who);
         }
     }
-    if (use_segment_kernels()) {
+    if (own_levels(p)) {
         switch (refine_steps) {
             case 0: return launch_seg<SegMixK0>(p, s, who);
             case 1: return launch_seg<SegMixK1>(p, s, who);

@@ -39,10 +39,10 @@ __host__ __device__ constexpr int batch_lds() {
 
 // One launch per bucket: S levels per lane, MODE -1 = float64, else mixed with
 // MODE refinement steps. LDSV: every system of the bucket allows 16-byte copies
-// straight into LDS and those are faster at this S (tdma_lds_wins); else the
-// flat loads of tdma_tile.hpp (odd depths, any alignment or strides). Before
-// those, systems of odd depth had each lane load its own levels, 8 bytes at a
-// time, in kernels that held the LDS of the copies.
+// straight into LDS and those are faster (tdma_lds_wins); else the flat loads of
+// tdma_tile.hpp (odd depths, any alignment or strides), at S = 2 each lane's own
+// levels (tdma_own_levels), as at every S before, in kernels that held the LDS of
+// the copies.
 template <int S, int MODE, bool LDSV>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void tdma_seg_batch_kernel(const SysDesc* __restrict__ sys, int nsys,
                                                              int64_t ntiles) {
@@ -75,6 +75,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void t
                 seg_mixed_core<S, MODE>(L, va, vb, vc, vd, x);
                 seg_store_lds<S>(p, L, lds, x);
             }
+        } else if constexpr (tdma_own_levels(S)) {
+            if constexpr (MODE < 0) seg_f64<S, false>(p, L);
+            else seg_mixed<S, false, MODE>(p, L);
         } else {
             tdma_tile<S, MODE>(p, t, L, lds);
         }
@@ -114,12 +117,10 @@ int ilog2(int64_t v) {
 
 template <int S, int MODE>
 void launch_bs(int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
-    if constexpr (tdma_lds_wins(S, MODE >= 0)) {
-        if (ldsv) {
-            const size_t lds = (size_t)batch_lds<S, true>() * 8 * (bs / 64);
-            hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, true>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
-            return;
-        }
+    if (ldsv && (tdma_lds_wins(S, MODE >= 0, true) || tdma_lds_resident(S, tiles))) {
+        const size_t lds = (size_t)batch_lds<S, true>() * 8 * (bs / 64);
+        hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, true>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
+        return;
     }
     const size_t lds = (size_t)batch_lds<S, false>() * 8 * (bs / 64);
     hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, false>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);

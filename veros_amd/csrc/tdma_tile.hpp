@@ -62,16 +62,37 @@ inline bool tdma_vec_ok(const TdmaArgs& p) {
     return aligned16(p.a) && aligned16(p.b) && aligned16(p.c) && aligned16(p.d) && aligned16(p.x);
 }
 
-// The LDS-staged solve (those copies, tdma_seg.hpp) against the tiles, on 38.4 M
-// cells (us, float64 / mixed with one step): nz 40 189 / 188 against 192 / 196,
-// 60 196 / 195 against 179 / 187, 80 168 / 170 against 173 / 173, 96 188 / 189
-// against 171 / 207, 112 236 / 240 against 194 / 211, 128 246 / 251 against
-// 204 / 233. It wins where the segment stride in its images spreads over the
-// LDS banks (S / 2 odd: 2, 6, 10 levels per lane) and four blocks fit a CU
-// (S <= 10); and for the mixed form at S = 12, where the tiles' flat loads cost
-// a wave per SIMD.
-__host__ __device__ constexpr bool tdma_lds_wins(int S, bool mixed) {
-    return (S <= 10 && (S / 2) % 2 == 1) || (mixed && S == 12);
+// The LDS-staged solve (those copies, tdma_seg.hpp) against the tiles, us,
+// float64 / mixed with one step:
+//   38.4 M cells   nz 40 189 / 188 against 192 / 196, 60 196 / 195 against
+//                  179 / 187, 80 168 / 170 against 173 / 173, 96 188 / 189 against
+//                  171 / 207, 112 236 / 240 against 194 / 211, 128 246 / 251
+//                  against 204 / 233
+//   640x640        nz 24 51 / 50 against 54 / 56, 60 128 / 127 against 119 / 124
+//   128x128        nz 24 4.2 / 4.0 against 4.7 / 4.7, 60 6.5 / 6.3 against 7.3 /
+//                  7.4, 96 10.9 / 11.0 against 10.0 / 11.0
+//   96x96          nz 60 5.4 / 5.2 against 6.1 / 5.9, 96 6.6 / 6.6 against 8.3 /
+//                  6.6, 112 10.1 / 10.3 against 9.3 / 9.2
+// At any size it wins up to S = 6 and at S = 10, and for the mixed form at
+// S = 12, where the tiles' flat loads cost a wave per SIMD. Elsewhere its LDS
+// (one block of two waves holds 8 KB per level of a lane) leaves too few waves on a
+// large grid, and it wins while all of them are resident at once
+// (tdma_lds_resident): nothing waits for a free slot then, and its chain from
+// kbot to the rows is the shorter one. In the batched kernel the tiles' registers
+// cost a wave per SIMD at S = 12, and spill at S = 14 in the mixed form: 640x640x96
+// 198 against 244, x112 mixed 309 against 338 (float64 301 against 281).
+__host__ __device__ constexpr bool tdma_lds_wins(int S, bool mixed, bool batch) {
+    return S <= 6 || S == 10 || (S == 12 && (mixed || batch)) || (S == 14 && mixed && batch);
+}
+// Two levels per lane (nz <= 16) with operands those copies don't fit: each lane
+// loads its own levels; the 8 lanes of a column then read it whole, so the flat
+// loads gain nothing. 320x320x13 10.4 against 10.7 us (tiles), 1200x1200x13 124
+// against 126, 128x128x15 3.5 against 3.8; at four levels (nz 25) 1200x1200 265
+// against 211.
+__host__ __device__ constexpr bool tdma_own_levels(int S) { return S == 2; }
+inline bool tdma_lds_resident(int S, int64_t ntiles) {
+    const int blocks = (160 << 10) / (seg_lds_wave_bytes(S) * (kSegLdsBlock / 64));
+    return ntiles <= (int64_t)blocks * (kSegLdsBlock / 64) * cu_count();
 }
 
 // LDS doubles of a wave
