@@ -139,3 +139,18 @@ def test_tdma_depths_and_strides(nz, form):
         y = _laid_out(np.full(a.shape, 7.0), form)
         TdmaBatch([dict(a=a, b=b, c=c, d=d, kbot=kb, x=y, b_edge=be, d_edge=de)], precision=mode).run()
         assert torch.equal(x, y), mode
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+@pytest.mark.parametrize("levels,shift", [("inner", False), ("outer", True)])
+def test_vertmix_depths(nz, levels, shift):
+    """vertmix_tempsalt on its column tiles: every depth with the time levels
+    innermost, and outermost off 16-byte alignment, against the oracle at the
+    bars of test_gpu_vertmix."""
+    import test_gpu_vertmix as TV
+    from veros_amd import thermodynamics
+    st = TV._state(nz, 9, 6, nz, land=0.3)
+    ds = TV._dev(st, levels)
+    if shift:
+        shift_arrays(ds)
+    TV._check(thermodynamics.vertmix_tempsalt(ds), TV.V.vertmix_tempsalt(st), st)

@@ -72,9 +72,13 @@ struct Tile {
 
 // The tile of `ncol` columns of nz levels, `sy` cells apart, from cell0 on
 // (ncol = 0: no columns; the addresses formed are those of cell0). All
-// arguments wave-uniform; C * sy * 8 < kNoAccess.
+// arguments wave-uniform; C * sy * 8 < kNoAccess. m: depth_reciprocal(nz), with
+// which e / nz is (e * m) >> 20, exactly for e <= 1024, nz <= 128.
+__host__ __device__ __forceinline__ uint32_t depth_reciprocal(int nz) {
+    return ((1u << 20) + (uint32_t)nz - 1u) / (uint32_t)nz;
+}
 template <int S, int P = kTileP>
-__device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz, uint32_t sy) {
+__device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz, uint32_t sy, uint32_t m) {
     using T = Tile<S, P>;
     T t;
     t.lane = (int)(threadIdx.x & 63);
@@ -85,8 +89,6 @@ __device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz,
     t.cell0 = cell0;
     t.ncol = ncol;
     t.bytes = ncol > 0 ? ((uint32_t)(ncol - 1) * sy + (uint32_t)nz) * 8u : 0u;
-    // e / nz for e <= 1024, nz <= 128, by a 20-bit reciprocal (exact there)
-    const uint32_t m = ((1u << 20) + (uint32_t)nz - 1u) / (uint32_t)nz;
 #pragma unroll
     for (int r = 0; r < S; ++r) {
         const uint32_t e = 64u * r + (uint32_t)t.lane;

@@ -1362,7 +1362,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2))) 
     const int64_t col0 = ((int64_t)blockIdx.x * (kAdjBlock / 64) + wave) * T::C;
     const int64_t left = (int64_t)g.X * g.Y - col0;
     const int n = left >= T::C ? T::C : (left > 0 ? (int)left : 0);
-    const T t = make_tile<S, kAdjP>(n > 0 ? col0 * nz : 0, n, nz, (uint32_t)nz);
+    const T t = make_tile<S, kAdjP>(n > 0 ? col0 * nz : 0, n, nz, (uint32_t)nz, depth_reciprocal(nz));
     SegLane L;
     L.s = t.s;
     L.lo = t.lo;

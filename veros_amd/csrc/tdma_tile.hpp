@@ -46,7 +46,7 @@ __device__ __forceinline__ Tile<S, kTdmaP> tdma_tile_of(const TdmaArgs& p, const
     const int64_t left = g.ny - j0;
     const int n = in ? (int)(left < g.cpt ? left : g.cpt) : 0;
     const int64_t base = i * p.sx + j0 * p.sy;
-    const Tile<S, kTdmaP> t = make_tile<S, kTdmaP>(base, n, p.nz, g.cpt > 1 ? (uint32_t)p.sy : 0u);
+    const Tile<S, kTdmaP> t = make_tile<S, kTdmaP>(base, n, p.nz, g.cpt > 1 ? (uint32_t)p.sy : 0u, depth_reciprocal(p.nz));
     L.s = t.s;
     L.lo = t.lo;
     L.valid = t.q < n;

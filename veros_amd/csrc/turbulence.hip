@@ -68,7 +68,7 @@ template <int S>
 __device__ __forceinline__ Tile<S> turb_tile(const TurbGrid& g, int64_t col0) {
     const int64_t left = (int64_t)g.X * g.Y - col0;
     const int n = left >= kTileC ? kTileC : (left > 0 ? (int)left : 0);
-    return make_tile<S>(n > 0 ? col0 * g.nz : 0, n, g.nz, (uint32_t)g.nz);
+    return make_tile<S>(n > 0 ? col0 * g.nz : 0, n, g.nz, (uint32_t)g.nz, depth_reciprocal(g.nz));
 }
 
 // The lane's group column (segments): what the masks need, known before the
