@@ -154,3 +154,18 @@ def test_vertmix_depths(nz, levels, shift):
     if shift:
         shift_arrays(ds)
     TV._check(thermodynamics.vertmix_tempsalt(ds), TV.V.vertmix_tempsalt(st), st)
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+@pytest.mark.parametrize("levels,shift", [("inner", False), ("outer", True)])
+def test_friction_depths(nz, levels, shift):
+    """implicit_vert_friction at every depth, with one column more than a strip
+    holds (8 of 7) and arrays off 16-byte alignment, against the oracle at the
+    bars of test_gpu_friction."""
+    import test_gpu_friction as TF
+    from veros_amd import friction
+    st = TF._state(nz, 9, 7, nz, land=0.3)
+    ds = TF._dev(st, levels)
+    if shift:
+        shift_arrays(ds)
+    TF._check(friction.implicit_vert_friction(ds), TF.F.implicit_vert_friction(st), st)

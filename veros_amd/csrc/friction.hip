@@ -10,17 +10,15 @@
 // tau) / dt_mom over the face range, and adds the dissipation of the solve,
 // interpolated onto the T grid, to K_diss_v.
 //
-// Here a group of kSegP lanes owns a face column (the segmented solve of
-// tdma_seg.hpp, lane s holding levels [s*S, s*S + S)): each lane forms its
-// rows in registers from the face viscosity, the group solves, and each lane
-// writes the new velocity on the wet levels and the tendency on every level,
-// and forms the face's dissipation from the velocities still in registers
-// (the level above from the next lane). A T cell's dissipation needs the u
-// faces i-1 and i and the v faces j-1 and j, so a block owns a strip of T
-// columns and walks a chunk of rows in order: the u faces of the previous row
-// are kept in LDS, and the v faces of the row pass through LDS to the group
-// north of them. No face dissipation goes through memory.
-#include "tdma_seg.hpp"
+// Here a group of 16 lanes owns a face column (col_tile.hpp): it forms its rows
+// in registers from the face viscosity, solves, and the wave writes the new
+// velocity on the wet levels and the tendency on every level; the face's
+// dissipation is formed from the velocities still in registers (the level above
+// from the next lane). A T cell's dissipation needs the u faces i-1 and i and the
+// v faces j-1 and j, so a block owns a strip of T columns and walks a chunk of
+// rows in order: the u faces of the previous row are kept in registers, and the v
+// faces of the row pass through LDS. No face dissipation goes through memory.
+#include "col_tile.hpp"
 
 namespace vx {
 namespace {
@@ -65,216 +63,233 @@ __device__ inline Face face_of(int kb0, int kb1, int nz) {
     return f;
 }
 
-// One face column of component t (face range only when `live`): rows from
-// the face viscosity (veros/core/friction.py:111-126, 161-176), the solve,
-// with `store` the velocity at taup1 on the wet levels and the tendency on
-// every level (:127-130, 178-181), and in ds the face's dissipation on every
-// level (:137-153, 189-201): fxa * (x1[k+1] - x1[k]) / dzw[k] * mask[k+1] *
-// mask[k] times (x0[k+1] - x0[k]) / dzw[k], x0 at tau and x1 at taup1, 0 on
-// the top level. The masks are 0 or 1, so the products are taken as selects.
-// Every lane of the wave calls it (the solve moves data across lanes). zt and
-// zw hold dzt and dzw in LDS: read inside per-level selects, a global load
-// would be waited for at once, level after level.
-template <int S, bool VEC, bool PV>
-__device__ __forceinline__ void fric_face(const FricArgs& p, const double* __restrict__ zt,
-                                          const double* __restrict__ zw, SegLane L, int t, int64_t col, int64_t nb,
-                                          bool live, bool both, bool store, double (&ds)[S]) {
-    const int nz = p.nz;
-    const int lo = L.lo;
-    const int k0 = L.k0;
-    const double dt = p.dt;
-    const int64_t base = col * nz;
-    // face viscosity on the solved levels
-    double ka[S], kn[S], x0[S], x1[S];
-#pragma unroll
-    for (int q = 0; q < S; ++q) ka[q] = kn[q] = x0[q] = x1[q] = 0.0;
-    col_load<S, PV>(p.kappaM + base, 1, lo, nz, [&](int k) { return k >= k0; }, ka);
-    col_load<S, PV>(p.kappaM + nb * nz, 1, lo, nz, [&](int k) { return k >= k0; }, kn);
-    // tau on every level, taup1 below the solve (kept there: du_mix reads it)
-    const double* u0p = p.vel[t] + p.tau * p.ls + p.cs * base;
-    double* u1p = p.vel[t] + p.taup1 * p.ls + p.cs * base;
-    col_load<S, VEC>(u0p, p.cs, lo, nz, [&](int) { return live; }, x0);
-    col_load<S, VEC>(u1p, p.cs, lo, nz, [&](int k) { return live && k < k0; }, x1);
-    double fxa[S];
-#pragma unroll
-    for (int q = 0; q < S; ++q) fxa[q] = 0.5 * (ka[q] + kn[q]);
-    // rows; delta at level lo-1 from the lane below
-    double va[S], vb[S], vc[S], z[S];
-    const double fxm = grp_prev(L.s, fxa[S - 1]);
-    const int kp = lo - 1;
-    double dlm = (both && kp >= k0 && kp < nz - 1) ? dt / zw[kp] * fxm : 0.0;
+// First wet level of a T column (nz: none).
+__device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
+
+// The rows, the solve and the dissipation of a tile's faces of one component.
+// In: flat, the face viscosity fx and tau's velocity x0 (on the solved levels); the
+// lane's column: its first solved level k0, whether both T columns are wet. Out: flat,
+// the solution x1 and the tendency dm; the lane's segment of the face's dissipation
+// (:137-153, 189-201): fxa * (x1[k+1] - x1[k]) / dzw[k] * mask[k+1] * mask[k] times
+// (x0[k+1] - x0[k]) / dzw[k], x0 at tau and x1 at taup1, 0 on the top level. The
+// masks are 0 or 1, so the products are taken as selects. rzt, dtw, rzw: 1 / dzt,
+// dt / dzw and 1 / dzw in LDS.
+template <int S>
+__device__ __forceinline__ void fric_face(const Tile<S>& t, double* img, int nz, const double* __restrict__ rzt,
+                                          const double* __restrict__ dtw, const double* __restrict__ rzw, int k0,
+                                          bool both, double rdt, const double (&fx)[S], const double (&x0)[S],
+                                          double (&x1)[S], double (&dm)[S], double (&ds)[S]) {
+    double f[S], o[S], va[S], vb[S], vc[S], z[1][S];
+    tile_put(t, img, fx);
+    seg_get(t, img, f);
+    const double fm = seg_below(t, img);
+    tile_put(t, img, x0);
+    seg_get(t, img, o);
+    // rows (veros/core/friction.py:111-126, 161-176)
+    double dlm = (both && t.lo > k0 && t.lo < nz) ? dtw[t.lo - 1] * fm : 0.0;
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        const int k = lo + q;
+        const int k = t.lo + q;
         const bool wet = k >= k0 && k < nz;
         const int kc = k < nz ? k : nz - 1;
-        const double dz = zt[kc];
-        const double dl = (both && wet && k < nz - 1) ? dt / zw[kc] * fxa[q] : 0.0;
-        const bool edge = k == k0;
-        va[q] = (wet && !edge) ? -dlm / dz : 0.0;
-        vb[q] = wet ? (edge ? 1 + dl / dz : (1 + dlm / dz) + dl / dz) : 1.0;
-        vc[q] = wet ? -dl / dz : 0.0;
-        z[q] = wet ? x0[q] : 0.0;
+        const double rz = rzt[kc];
+        const double dl = (both && wet && k < nz - 1) ? dtw[kc] * f[q] : 0.0;
+        va[q] = (wet && k != k0) ? -dlm * rz : 0.0;
+        vb[q] = wet ? (k == k0 ? 1 + dl * rz : (1 + dlm * rz) + dl * rz) : 1.0;
+        vc[q] = wet ? -dl * rz : 0.0;
+        z[0][q] = wet ? o[q] : 0.0;
         dlm = dl;
     }
-    seg_solve_f64<S>(L, va, vb, vc, z);
-#pragma unroll
-    for (int q = 0; q < S; ++q) {
-        const int k = lo + q;
-        x1[q] = (k >= k0 && k < nz) ? z[q] : x1[q];
-    }
+    tile_solve<S, 1>(t, va, vb, vc, z);
+    seg_put(t, img, z[0]);
     // level lo+S from the lane above (every lane takes part in the moves)
-    const double x1n = grp_next(L.s, x1[0]);
-    const double x0n = grp_next(L.s, x0[0]);
+    const double zn = dpp_move<kDppShl + 1>(z[0][0]), on = dpp_move<kDppShl + 1>(o[0]);
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        const int k = lo + q;
-        const double a1 = q < S - 1 ? x1[q < S - 1 ? q + 1 : 0] : x1n;
-        const double a0 = q < S - 1 ? x0[q < S - 1 ? q + 1 : 0] : x0n;
-        const int kc = k < nz - 1 ? k : 0;
-        const double dzw = zw[kc];
-        ds[q] = (both && k >= k0 && k < nz - 1) ? ((a0 - x0[q]) * ((fxa[q] * (a1 - x1[q])) / dzw)) / dzw : 0.0;
+        const int k = t.lo + q;
+        const double z1 = q < S - 1 ? z[0][q < S - 1 ? q + 1 : 0] : zn;
+        const double o1 = q < S - 1 ? o[q < S - 1 ? q + 1 : 0] : on;
+        const bool d = both && k >= k0 && k < nz - 1;
+        const double rw = rzw[d ? k : 0];
+        ds[q] = d ? ((o1 - o[q]) * (f[q] * (z1 - z[0][q])) * rw) * rw : 0.0;
     }
-    if (!(live && store)) return;
-    bool st[S];
-    double dm[S];
+    tile_get(t, img, x1);
 #pragma unroll
-    for (int q = 0; q < S; ++q) {
-        const int k = lo + q;
-        st[q] = k >= k0;
-        dm[q] = (x1[q] - x0[q]) / dt;
-    }
-    // the levels below the solve hold taup1's own values, so a pair store
-    // that covers one of them writes back what is there
-    col_store_if<S, VEC>(u1p, p.cs, lo, nz, x1, st);
-    col_store<S, PV>(p.dmix[t] + base, 1, lo, nz, dm);
+    for (int q = 0; q < S; ++q) z[0][q] = (z[0][q] - o[q]) * rdt;
+    seg_put(t, img, z[0]);
+    tile_get(t, img, dm);
 }
 
-// A block of 32 face-column groups owns a strip of 31 T columns j (group g at
-// column jb - 1 + g; group 0 solves the v face south of the strip for group
-// 1) and walks the rows of a chunk [ib, ie) in order, starting one row early
-// for the u faces west of the chunk. Per row: the v face, then the u face of
-// each column. The u-face dissipation of the previous row stays in LDS, each
-// lane reading back only what it wrote; the v-face dissipation of the row
-// goes through LDS to the group north of it (two buffers, one barrier per
-// row). Each face is stored by exactly one block. K_diss_v +=
-// ugrid_to_tgrid(diss_u), then += vgrid_to_tgrid(diss_v)
-// (veros/core/friction.py:154-155, 203-204; veros/core/numerics.py:313-336):
-// at T cell (i, j) the u faces i and i-1 weighted dxu / (2 dxt) for 2 <= i <
-// X-2 (face i alone for i = 1), the v faces j and j-1 weighted area_v / (2
-// area_t) for 2 <= j < Y-2 (face j alone for j = 1), formed as (K + u part)
-// + v part on the levels
-// below the top one (which dissipates nothing). Blocks are XCD-contiguous,
-// strips fastest. Two waves per SIMD: 218 VGPRs at nz = 80.
-// VEC: levels outermost, nz even and every array 16-byte aligned. PV (implied
-// by VEC): nz even and the arrays without time levels (kappaM, du_mix, dv_mix,
-// K_diss_v) 16-byte aligned, which then move in level pairs whatever the
-// layout of u and v.
-template <int S, bool VEC, bool PV>
-__global__ __launch_bounds__(kSegBlock) __attribute__((amdgpu_waves_per_eu(2))) void friction_walk_kernel(FricArgs p, int rows, int64_t nstrips,
-                                                                  int64_t nblocks) {
-    __shared__ double dsu[S * kSegBlock];
-    __shared__ double dsv[2][S * kSegBlock];
+// A block owns a strip of T columns j and walks the rows of a chunk [ib, ie) in
+// order, starting one row early for the u faces west of the chunk. Half of its
+// waves solve the row's v faces, the other half its u faces, four columns each, on
+// column tiles (col_tile.hpp); the strip's first column is solved for its v face
+// only. The v faces' dissipation goes through LDS to the u waves (two images per
+// wave, one barrier per row), which keep that of the previous row's u faces and
+// update K_diss_v. Each face is stored by exactly one block.
+// K_diss_v += ugrid_to_tgrid(diss_u), then += vgrid_to_tgrid(diss_v)
+// (veros/core/friction.py:154-155, 203-204; veros/core/numerics.py:313-336): at T cell
+// (i, j) the u faces i and i-1 weighted dxu / (2 dxt) for 2 <= i < X-2 (face i alone
+// for i = 1), the v faces j and j-1 weighted area_v / (2 area_t) for 2 <= j < Y-2
+// (face j alone for j = 1), on the wet levels below the top one (no face of a dry
+// cell dissipates). Blocks are XCD-contiguous, strips fastest.
+//
+// A row's chain (kbot, the loads, the solve through LDS) is what bounds it, with
+// 5.1 GB on 1440x720x80 at 3.2 TB/s. What lies below the solve is loaded and stored
+// before it, so that no flat value but the operands lives across it. Blocks of
+// four waves: with eight, one block fills a CU's registers and nothing runs
+// while it waits at its barrier (2.22 -> 2.68 ms for the vertical step there).
+// Loading the next row ahead took the registers that hold a second block's waves
+// (2.55 ms). Eight lanes per column, each loading and storing its own levels,
+// and every row's divisions in the lane: friction 1.94 ms there, now 1.60; 163
+// us on 360x160x60, levels innermost, now 103.
+constexpr int kFricGroups = 2;                                // column groups of a block
+constexpr int kFricBlock = 2 * 64 * kFricGroups;              // a u and a v wave for each
+constexpr int kFricCols = kFricGroups * (64 / kTileP) - 1;    // T columns of a strip
+// waves per SIMD (and blocks per CU) that the registers allow
+template <int S>
+constexpr int kFricWaves = S <= 3 ? 4 : S == 4 ? 3 : 2;
+template <int S>
+__global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFricWaves<S>))) void friction_walk_kernel(
+    FricArgs p, int rows, int64_t nstrips, int64_t nblocks, uint32_t rnz) {
+    using T = Tile<S>;
+    constexpr int G = kFricGroups;
+    __shared__ double work[2 * G][T::IMG];
+    __shared__ double dsv[2][G][T::IMG];
+    __shared__ double sdz[3][kMaxNz];
     const int64_t b = xcd_contiguous_block();
     if (b >= nblocks) return;
-    const int tid = threadIdx.x;
-    __shared__ double sdz[2 * kMaxNz];  // dzt, then dzw
-    for (int k = tid; k < p.nz; k += kSegBlock) {
-        sdz[k] = p.dzt[k];
-        sdz[kMaxNz + k] = p.dzw[k];
+    const int nz = p.nz;
+    for (int k = threadIdx.x; k < nz; k += kFricBlock) {
+        const double zw = p.dzw[k];
+        sdz[0][k] = 1.0 / p.dzt[k];
+        sdz[1][k] = p.dt / zw;
+        sdz[2][k] = 1.0 / zw;
     }
     __syncthreads();
-    const double* zt = sdz;
-    const double* zw = sdz + kMaxNz;
-    const int g = tid / kSegP;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const bool vface = wave < G;
+    const int grp = vface ? wave : wave - G, comp = vface ? 1 : 0;
+    double* const img = work[wave];
     const int64_t strip = b % nstrips, chunk = b / nstrips;
-    const int64_t j = 31 * strip + g;  // the strip's T columns are [31 strip + 1, 31 strip + 32)
     const int64_t ib = 1 + (int64_t)rows * chunk;
     const int64_t ie = ib + rows < p.X - 2 ? ib + rows : p.X - 2;
-    const bool jlive = j >= 1 && j <= p.Y - 3;
-    const bool jown = g >= 1 && jlive;
-    const int nz = p.nz;
-    SegLane L;
-    L.s = tid % kSegP;
-    L.lo = L.s * S;
-    L.valid = true;
+    const int64_t j0 = kFricCols * strip + T::C * grp;  // the wave's columns
+    const int64_t left = p.Y - 2 - j0;
+    const int n = left >= T::C ? T::C : (left > 0 ? (int)left : 0);
+    const int64_t next = vface ? 1 : p.Y;  // the face's other column
+    const uint32_t cs = (uint32_t)p.cs;
+    const double rdt = 1.0 / p.dt;
+    double* const vel = p.vel[comp];
+    T t = make_tile<S>(0, n, nz, (uint32_t)nz, rnz);
+    const int64_t j = t.q < n ? j0 + t.q : (n > 0 ? j0 : 0);  // the lane's column
+    const bool jlive = t.q < n && j >= 1, jown = jlive && (grp > 0 || t.q > 0);
+    // the block's own elements: not the strip's first column, nor j = 0
+    auto own = [&](int r) { return t.off[r] != kNoAccess && (grp > 0 || t.c[r] > 0); };
+    double du[S];  // the previous row's u faces' dissipation
+#pragma unroll
+    for (int r = 0; r < S; ++r) du[r] = 0.0;
 #pragma unroll 1
     for (int64_t i = ib >= 2 ? ib - 1 : ib; i < ie; ++i) {
-        // the grid spacings are loaded again in each face (kept across the
-        // row loop they would double the registers of the solve)
-        asm volatile("" ::: "memory");
         const bool pre = i < ib;
-        const int64_t col = jlive ? i * p.Y + j : 0;
-        L.base = col * nz;
-        const int kb = jlive ? p.kbot[col] : 0;
-        const int buf = (int)(i & 1);
-        if (!pre) {
-            const int64_t nb = jlive ? col + 1 : col;
-            const Face f = face_of(kb, jlive ? p.kbot[nb] : 0, nz);
-            L.k0 = f.k0;
-            double ds[S];
-            fric_face<S, VEC, PV>(p, zt, zw, L, 1, col, nb, jlive, f.both, jown, ds);
+        const int64_t col = i * p.Y + j;
+        t.cell0 = (i * p.Y + j0) * nz;
+        double ds[S];
+        int kb = 0;
+        if (n > 0 && !(pre && vface)) {
+            kb = p.kbot[col];
+            const bool live = vface ? jlive : jown;
+            const Face f = face_of(live ? kb : 0, live ? p.kbot[col + next] : 0, nz);
+            const BufRsrc b0 = tile_buf(t, vel + p.tau * p.ls, 0, (int)cs);
+            const BufRsrc b1 = tile_buf(t, vel + p.taup1 * p.ls, 0, (int)cs);
+            const BufRsrc bd = tile_buf(t, p.dmix[comp]);
+            double fx[S], kn[S], x0[S], x1[S];
+            uint32_t on[S];  // the solved levels
 #pragma unroll
-            for (int q = 0; q < S; ++q) dsv[buf][q * kSegBlock + tid] = ds[q];
+            for (int r = 0; r < S; ++r) on[r] = t.k[r] >= __shfl(f.k0, t.c[r] * kTileP) ? t.off[r] : kNoAccess;
+            tile_load(tile_buf(t, p.kappaM), on, 1, fx);
+            tile_load(tile_buf(t, p.kappaM, next * nz), on, 1, kn);
+            tile_load(b0, on, cs, x0);
+#pragma unroll
+            for (int r = 0; r < S; ++r) on[r] = own(r) && !pre ? on[r] : kNoAccess;
+            if (!pre) {  // below the solve taup1 keeps its value
+                double y0[S], dm[S];
+                uint32_t below[S];
+#pragma unroll
+                for (int r = 0; r < S; ++r) below[r] = own(r) && on[r] == kNoAccess ? t.off[r] : kNoAccess;
+                tile_load(b0, below, cs, y0);
+                tile_load(b1, below, cs, dm);
+#pragma unroll
+                for (int r = 0; r < S; ++r) dm[r] = (dm[r] - y0[r]) * rdt;
+                tile_store(bd, below, 1, dm);
+            }
+#pragma unroll
+            for (int r = 0; r < S; ++r) fx[r] = 0.5 * (fx[r] + kn[r]);
+            fric_face<S>(t, img, nz, sdz[0], sdz[1], sdz[2], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
+            if (vface) seg_put(t, dsv[i & 1][grp], ds);
+            tile_store(b1, on, cs, x1);
+            tile_store(bd, on, 1, kn);
+        }
+        if (vface || n == 0) {
+            if (!pre) __syncthreads();
+            continue;
         }
         double bu[S];
-        asm volatile("" ::: "memory");
         {
-            const bool ulive = jown;
-            const int64_t nb = ulive ? col + p.Y : col;
-            const Face f = face_of(ulive ? kb : 0, ulive ? p.kbot[nb] : 0, nz);
-            L.k0 = f.k0;
-            double ds[S];
-            fric_face<S, VEC, PV>(p, zt, zw, L, 0, col, nb, ulive, f.both, !pre, ds);
-            const double wi = p.dxu[i], wm = p.dxu[i - 1], den = 2 * p.dxt[i];
+            const double wi = p.dxu[i], wm = p.dxu[i - 1], rden = 1.0 / (2 * p.dxt[i]);
 #pragma unroll
-            for (int q = 0; q < S; ++q) {
-                bu[q] = i >= 2 ? (wi * ds[q] + wm * dsu[q * kSegBlock + tid]) / den : ds[q];
-                dsu[q * kSegBlock + tid] = ds[q];
+            for (int r = 0; r < S; ++r) {
+                bu[r] = i >= 2 ? (wi * ds[r] + wm * du[r]) * rden : ds[r];
+                du[r] = ds[r];
             }
         }
-        if (pre) continue;
+        if (pre) continue;  // uniform in the block
         // K_diss_v and the weights are loaded before the barrier, which their
         // latency then overlaps
-        double K[S];
+        const BufRsrc bK = tile_buf(t, p.K_diss_v);
+        double K[S], wj = 1.0, wjm = 0.0;
+        uint32_t ow[S];
+        const int wc = jown ? first_wet_level(kb, nz) : nz;
 #pragma unroll
-        for (int q = 0; q < S; ++q) K[q] = 0.0;
-        double* Kp = p.K_diss_v + L.base;
-        double wj = 0.0, wjm = 0.0, dnj = 1.0;
-        if (jown) {
-            col_load<S, PV>(Kp, 1, L.lo, nz, [&](int k) { return k < nz - 1; }, K);
-            wj = p.area_v[col], wjm = p.area_v[col - 1], dnj = 2 * p.area_t[col];
+        for (int r = 0; r < S; ++r)
+            ow[r] = t.k[r] >= __shfl(wc, t.c[r] * kTileP) && t.k[r] < nz - 1 ? t.off[r] : kNoAccess;
+        tile_load(bK, ow, 1, K);
+        const bool south = jown && j >= 2;
+        if (south) {
+            const double rd = 1.0 / (2 * p.area_t[col]);
+            wj = p.area_v[col] * rd;
+            wjm = p.area_v[col - 1] * rd;
         }
         __syncthreads();
-        if (jown) {
-            bool st[S];
+        // the v faces of the lane's column and of the column south, which may be
+        // the last of the wave before
+        const double* vn = dsv[i & 1][grp];
+        const double* vs = t.q > 0 ? vn - T::CS : dsv[i & 1][grp > 0 ? grp - 1 : 0] + (T::C - 1) * T::CS;
 #pragma unroll
-            for (int q = 0; q < S; ++q) {
-                const double dv = dsv[buf][q * kSegBlock + tid];
-                const double bv = j >= 2 ? (wj * dv + wjm * dsv[buf][q * kSegBlock + tid - kSegP]) / dnj : dv;
-                st[q] = L.lo + q < nz - 1;
-                K[q] = st[q] ? (K[q] + bu[q]) + bv : K[q];
-            }
-            col_store_if<S, PV>(Kp, 1, L.lo, nz, K, st);
+        for (int r = 0; r < S; ++r) {
+            const double dn = vn[t.seg + r], dd = vs[t.seg + r];
+            bu[r] = bu[r] + (south ? wj * dn + wjm * dd : dn);
         }
+        seg_put(t, img, bu);
+        tile_get(t, img, bu);
+#pragma unroll
+        for (int r = 0; r < S; ++r) buf_store(bK, ow[r], K[r] + bu[r]);
     }
 }
 
-// Rows per block of the walk kernel. A block walks `rows` rows of two face
-// solves each and one extra row of u faces, and two blocks fit a CU (one from
-// 14 levels per lane on, by their LDS), so a launch of n blocks takes about ceil(n / slots) passes of 2 * rows + 1 solves;
-// the row count with the cheapest product is taken (at most 24: longer chunks
-// leave the last pass emptier than the row they save). With 24 rows whatever
-// the grid, 360x160x60 (levels innermost) launched 96 blocks for 256 CUs: 459 us,
-// 163 us with the 5 rows (438 blocks) chosen here; 1440x720x80: 2.01 -> 1.94 ms
-// with 23.
+// Rows per block of the walk kernel. A block walks `rows` rows and one extra row of
+// u faces, and a launch of n blocks takes about ceil(n / slots) passes of rows + 1
+// rows; the row count with the cheapest product is taken (at most 24: longer
+// chunks leave the last pass emptier than the row they save). With 24 rows
+// whatever the grid, an earlier form of the kernel launched 96 blocks for 256 CUs
+// on 360x160x60: 459 us, 163 us with the rows chosen here.
 int fric_rows(int64_t nrows, int64_t nstrips, int blocks_per_cu) {
     const int64_t slots = (int64_t)blocks_per_cu * cu_count();
     int best = 1;
     int64_t best_cost = INT64_MAX;
     for (int rows = 1; rows <= 24; ++rows) {
         const int64_t nblocks = nstrips * ((nrows + rows - 1) / rows);
-        const int64_t cost = (nblocks + slots - 1) / slots * (2 * rows + 1);
+        const int64_t cost = (nblocks + slots - 1) / slots * (rows + 1);
         if (cost <= best_cost) {
             best_cost = cost;
             best = rows;
@@ -284,21 +299,12 @@ int fric_rows(int64_t nrows, int64_t nstrips, int blocks_per_cu) {
 }
 
 template <int S>
-void launch_fric_walk(const FricArgs& p, bool vec, bool pv, hipStream_t s) {
-    const int64_t nstrips = (p.Y - 3 + 30) / 31;
-    const int rows = fric_rows(p.X - 3, nstrips, S >= 14 ? 1 : 2);
-    const int64_t nchunks = (p.X - 3 + rows - 1) / rows;
-    const int64_t nblocks = nstrips * nchunks;
-    const dim3 grid((unsigned)((nblocks + 7) / 8 * 8));
-    if (vec)
-        hipLaunchKernelGGL((friction_walk_kernel<S, true, true>), grid, dim3(kSegBlock), 0, s, p, rows, nstrips,
-                           nblocks);
-    else if (pv)
-        hipLaunchKernelGGL((friction_walk_kernel<S, false, true>), grid, dim3(kSegBlock), 0, s, p, rows, nstrips,
-                           nblocks);
-    else
-        hipLaunchKernelGGL((friction_walk_kernel<S, false, false>), grid, dim3(kSegBlock), 0, s, p, rows, nstrips,
-                           nblocks);
+void launch_fric_walk(const FricArgs& p, hipStream_t s) {
+    const int64_t nstrips = (p.Y - 3 + kFricCols - 1) / kFricCols;
+    const int rows = fric_rows(p.X - 3, nstrips, kFricWaves<S>);
+    const int64_t nblocks = nstrips * ((p.X - 3 + rows - 1) / rows);
+    hipLaunchKernelGGL(friction_walk_kernel<S>, dim3((unsigned)((nblocks + 7) / 8 * 8)), dim3(kFricBlock), 0, s, p,
+                       rows, nstrips, nblocks, depth_reciprocal(p.nz));
 }
 
 }  // namespace
@@ -349,18 +355,15 @@ extern "C" int vx_implicit_vert_friction_f64(void* stream, const vx_grid* grid, 
     const bool outer = grid->time_layout == VX_LEVELS_OUTER;
     p.cs = outer ? 1 : 3;
     p.ls = outer ? p.X * p.Y * p.nz : 1;
-    const bool pv = !(p.nz & 1) && aligned16(kappaM) && aligned16(du_mix) && aligned16(dv_mix) && aligned16(K_diss_v);
-    const bool vec = pv && outer && aligned16(u) && aligned16(v);
     hipStream_t s = (hipStream_t)stream;
-    switch (seg_levels(p.nz)) {
-        case 2: launch_fric_walk<2>(p, vec, pv, s); break;
-        case 4: launch_fric_walk<4>(p, vec, pv, s); break;
-        case 6: launch_fric_walk<6>(p, vec, pv, s); break;
-        case 8: launch_fric_walk<8>(p, vec, pv, s); break;
-        case 10: launch_fric_walk<10>(p, vec, pv, s); break;
-        case 12: launch_fric_walk<12>(p, vec, pv, s); break;
-        case 14: launch_fric_walk<14>(p, vec, pv, s); break;
-        default: launch_fric_walk<16>(p, vec, pv, s); break;
+    switch (tile_levels(p.nz)) {
+        case 2: launch_fric_walk<2>(p, s); break;
+        case 3: launch_fric_walk<3>(p, s); break;
+        case 4: launch_fric_walk<4>(p, s); break;
+        case 5: launch_fric_walk<5>(p, s); break;
+        case 6: launch_fric_walk<6>(p, s); break;
+        case 7: launch_fric_walk<7>(p, s); break;
+        default: launch_fric_walk<8>(p, s); break;
     }
     return check_launch(who);
 }

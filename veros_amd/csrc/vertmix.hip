@@ -80,12 +80,11 @@ __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __res
     }
 }
 
-// Column tiles (any layout, depth and alignment): a wave's four
-// columns are loaded flat, the two tracers' old values stay with the lanes that
-// loaded them, and everything goes back flat. Bound by HBM: on 1440x720x80, levels
-// outermost, 2.4 GB in 0.60 ms, as long as 8 lanes per column with 16-byte copies
-// into LDS took there; 360x160x60, levels innermost, 71 -> 46 us against each
-// lane loading its own levels.
+// Column tiles (any layout, depth and alignment): a wave's four columns are loaded
+// flat, the two tracers' old values stay with the lanes that loaded them, and
+// everything goes back flat. Bound by HBM: on 1440x720x80, levels outermost, 2.6 GB
+// in 0.59 ms (8 lanes per column with 16-byte copies into LDS: 0.60); 360x160x60,
+// levels innermost, 71 -> 46 us against each lane loading its own levels.
 constexpr int kVmixBlock = 128;
 template <int S>
 __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, uint32_t rnz) {
