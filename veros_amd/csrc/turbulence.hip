@@ -132,7 +132,9 @@ __device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S>& t, 
 // F and the coefficient come from the arrays A and B (one or two of them):
 // COMB(face values of the neighbour's A and B, the cell's a and b) returns
 // coefficient * difference. Two directions at a time, so that the loads of a
-// pair are in flight together and hold few registers.
+// pair are in flight together and hold few registers. The kernels store their
+// diagnostics after it: a load waits for the stores issued before it (the three
+// models on 1440x720x80: 4.13 -> 4.10 ms).
 template <int S, bool TWO, class COMB>
 __device__ __forceinline__ void add_lateral(const TurbGrid& g, const Tile<S>& t, const TurbCols& tc, const double* A,
                                             uint32_t csA, const double* B, const double (&a)[S],
@@ -334,24 +336,26 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
         dg[r] = rate[r] * v[r];  // tke_diss over the whole array (:230)
         st[r] = wet[r];
     }
-    tile_store(tile_buf(t, a.diss), t.off, 1, dg);
     // surface correction and clamp of every interior column (:235-244)
+    double corr[S];
+    bool top[S];
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        if (t.k[r] == nz - 1 && t.off[r] != kNoAccess) {
-            const int64_t col = col0 + t.c[r];
-            const int i = (int)(col / g.Y), j = (int)(col - (int64_t)i * g.Y);
-            if (i >= 2 && i < g.X - 2 && j >= 2 && j < g.Y - 2) {
-                a.surf_corr[col] = v[r] < 0.0 ? -v[r] * 0.5 * sh.lv.zw[nz - 1] / dt : 0.0;
-                v[r] = fmax(0.0, v[r]);
-                st[r] = t.off[r];
-            }
-        }
+        const int in = __shfl((int)l.interior, t.c[r] * kTileP);
+        top[r] = in != 0 && t.k[r] == nz - 1 && t.off[r] != kNoAccess;
+        corr[r] = v[r];
+        v[r] = top[r] ? fmax(0.0, v[r]) : v[r];
+        st[r] = top[r] ? t.off[r] : st[r];
     }
     if (a.hor) {
         const double none[1] = {0.0};
         add_lateral<S, false>(g, t, tc, E0, cs, nullptr, e0, none,
                               [](double nA, double, double ea, double) { return nA - ea; }, v);
+    }
+    tile_store(tile_buf(t, a.diss), t.off, 1, dg);
+#pragma unroll
+    for (int r = 0; r < S; ++r) {
+        if (top[r]) a.surf_corr[col0 + t.c[r]] = corr[r] < 0.0 ? -corr[r] * 0.5 * sh.lv.zw[nz - 1] / dt : 0.0;
     }
     tile_store(tile_buf(t, E1, 0, (int)cs), st, cs, v);
 }
@@ -424,13 +428,13 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
         v[r] = wet[r] != kNoAccess ? v[r] : e1[r];
         dg[r] = cint[r] * v[r];  // (:151)
     }
+    add_lateral<S, true>(g, t, tc, E0, cs, a.K_gm, e0, kg, [](double nE, double nK, double ea, double ka) {
+        return 0.5 * fmax(500.0, nK + ka) * (nE - ea);
+    }, v);
     tile_store(tile_buf(t, a.diss_iw), t.off, 1, dg);
 #pragma unroll
     for (int r = 0; r < S; ++r) dg[r] = 0.0;  // (:152)
     tile_store(tile_buf(t, a.diss_tke), t.off, 1, dg);
-    add_lateral<S, true>(g, t, tc, E0, cs, a.K_gm, e0, kg, [](double nE, double nK, double ea, double ka) {
-        return 0.5 * fmax(500.0, nK + ka) * (nE - ea);
-    }, v);
     tile_store(tile_buf(t, E1, 0, (int)cs), wet, cs, v);
 }
 
@@ -537,7 +541,6 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
         v[r] = wet[r] != kNoAccess ? v[r] : e1[r];
         dg[r] = rate[r] * v[r];  // (:174)
     }
-    tile_store(tile_buf(t, a.iw_diss), t.off, 1, dg);
     if (a.hor) {  // (:186-218): the fluxes of v0 E with the coefficient 0.5 tau_h (v0 + v0')
         double v0[S];
         tile_load(tile_buf(t, a.v0), wet, 1, v0);
@@ -545,6 +548,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
             return (nV + va) * (nV * nE - va * ea);
         }, v);
     }
+    tile_store(tile_buf(t, a.iw_diss), t.off, 1, dg);
     tile_store(tile_buf(t, E1, 0, (int)cs), wet, cs, v);
 }
 
