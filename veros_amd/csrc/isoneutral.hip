@@ -1594,12 +1594,13 @@ Prm make_prm(const vx_iso_params* q) {
 #endif
 // Columns per block (one wave) of the pre and flux kernels: about VX_PRE_CELLS
 // cells (8 columns at nz = 80), so that a wave deals several rounds of cells
-// and the partly filled last one wastes few lanes, but at least four waves per
-// CU on small grids. The fused call on 1440x720x80 and the calls on 360x160x60
-// (levels innermost): 640 cells 6.04 ms and 1162 us, 1280 5.98 and 1204, 2400
-// 6.38 and 1262.
+// and the partly filled last one wastes few lanes, but at least eight waves per CU
+// on small grids, as many as pre's registers allow at once (pre + T + S on
+// 180x90x40, levels innermost: 90 us with four, 77 with eight, 80 with 16). The
+// fused call on 1440x720x80 and the calls on 360x160x60 (levels innermost): 640
+// cells 6.04 ms and 1162 us, 1280 5.98 and 1204, 2400 6.38 and 1262.
 int cell_columns(const Grid& g) {
-    const int64_t spread = ((int64_t)(g.X - 3) * (g.Y - 3) + 4 * cu_count() - 1) / (4 * cu_count());
+    const int64_t spread = ((int64_t)(g.X - 3) * (g.Y - 3) + 8 * cu_count() - 1) / (8 * cu_count());
     const int n = (int)std::min<int64_t>((VX_PRE_CELLS + g.nz - 1) / g.nz, spread);
     return n < 4 ? 4 : (n > kBlockCols ? kBlockCols : n);
 }
@@ -1637,12 +1638,14 @@ namespace {
 #endif
 // Columns per block: a group is about six wet columns at nz = 80, and the last
 // group of a block is partly empty, so the more columns the fewer idle lanes; but
-// at least four blocks per CU on small grids. 1440x720x80 pre + T + S and the
+// at least eight blocks per CU on small grids, the four that run at once and
+// four to follow (pre + T + S on 180x90x40, levels innermost: 77 us with four, 73 with
+// eight, 75 with 12). 1440x720x80 pre + T + S and the
 // calls on 360x160x60: 16 columns 5.00 ms and 958 us, 32 4.89 and 963, 64 4.85
 // and 1006 (one placement of the arrays; 48 0.8% faster and 1.7% slower than 32).
 template <int NTR, bool IMPLICIT, bool WETFLUX>
 int launch_wet_step(const Grid& g, const Prm& p, const StepArgs& a, hipStream_t s, const char* who) {
-    const int64_t spread = ((int64_t)(g.X - 2) * (g.Y - 2) + 4 * cu_count() - 1) / (4 * cu_count());
+    const int64_t spread = ((int64_t)(g.X - 2) * (g.Y - 2) + 8 * cu_count() - 1) / (8 * cu_count());
     int ncb = (int)std::min<int64_t>(VX_STEP_COLS, spread);
     ncb = ncb < 4 ? 4 : ncb;
     const int sb = (kStepStripCols + ncb - 1) / ncb;
