@@ -261,4 +261,42 @@ __device__ __forceinline__ void tile_solve(const Tile<S>& t, double (&va)[S], co
     }
 }
 
+// The same with P lanes per column: kTileP as above, or kSegP by the
+// elimination of tdma_seg.hpp.
+template <int S, int NR, int P>
+__device__ __forceinline__ void col_solve(const Tile<S, P>& t, double (&va)[S], const double (&vb)[S], double (&vc)[S],
+                                          double (&z)[NR][S]) {
+    if constexpr (P == kTileP) {
+        tile_solve<S, NR>(t, va, vb, vc, z);
+    } else {
+        SegLane L;
+        L.s = t.s;
+        L.lo = t.lo;
+        L.valid = true;
+        L.base = 0;
+        L.k0 = 0;
+        if constexpr (NR == 1) seg_solve_f64<S>(L, va, vb, vc, z[0]);
+        else seg_solve2_f64<S>(L, va, vb, vc, z[0], z[1]);
+    }
+}
+// the next lane's value of the column (last lane: unspecified)
+template <int P>
+__device__ __forceinline__ double col_next(int s, double x) {
+    if constexpr (P == kTileP) return dpp_move<kDppShl + 1>(x);
+    else return grp_next(s, x);
+}
+
+// Lanes per column and levels per lane of the kernels that choose between the two:
+// 8 lanes up to 32 levels, so that a wave takes 8 columns, else 16, which halve a
+// lane's registers. us on 1435x896 (friction, vertical mixing) and 1000x600 (TKE +
+// EKE + IDEMIX), 16 lanes / 8 lanes: nz 9 853 / 416, 287 / 177, 885 / 535; 17 936 /
+// 606, 322 / 261, 977 / 774; 24 983 / 637, 341 / 322, 1043 / 845; 32 1031 / 853, 405 /
+// 391, 1080 / 1017. Eight lanes from 33 levels on need five or more levels a lane,
+// whose registers cost a wave per SIMD.
+constexpr int col_lanes(int nz) { return nz <= 32 ? kSegP : kTileP; }
+constexpr int col_levels(int nz) {
+    const int s = (nz + col_lanes(nz) - 1) / col_lanes(nz);
+    return s < 2 ? 2 : s;
+}
+
 }  // namespace vx

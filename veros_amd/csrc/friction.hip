@@ -10,8 +10,8 @@
 // tau) / dt_mom over the face range, and adds the dissipation of the solve,
 // interpolated onto the T grid, to K_diss_v.
 //
-// Here a group of 16 lanes owns a face column (col_tile.hpp): it forms its rows
-// in registers from the face viscosity, solves, and the wave writes the new
+// Here a group of 8 or 16 lanes owns a face column (col_tile.hpp): it forms its
+// rows in registers from the face viscosity, solves, and the wave writes the new
 // velocity on the wet levels and the tendency on every level; the face's
 // dissipation is formed from the velocities still in registers (the level above
 // from the next lane). A T cell's dissipation needs the u faces i-1 and i and the
@@ -74,8 +74,8 @@ __device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 
 // (x0[k+1] - x0[k]) / dzw[k], x0 at tau and x1 at taup1, 0 on the top level. The
 // masks are 0 or 1, so the products are taken as selects. rzt, dtw, rzw: 1 / dzt,
 // dt / dzw and 1 / dzw in LDS.
-template <int S>
-__device__ __forceinline__ void fric_face(const Tile<S>& t, double* img, int nz, const double* __restrict__ rzt,
+template <int S, int P>
+__device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int nz, const double* __restrict__ rzt,
                                           const double* __restrict__ dtw, const double* __restrict__ rzw, int k0,
                                           bool both, double rdt, const double (&fx)[S], const double (&x0)[S],
                                           double (&x1)[S], double (&dm)[S], double (&ds)[S]) {
@@ -100,10 +100,10 @@ __device__ __forceinline__ void fric_face(const Tile<S>& t, double* img, int nz,
         z[0][q] = wet ? o[q] : 0.0;
         dlm = dl;
     }
-    tile_solve<S, 1>(t, va, vb, vc, z);
+    col_solve<S, 1>(t, va, vb, vc, z);
     seg_put(t, img, z[0]);
     // level lo+S from the lane above (every lane takes part in the moves)
-    const double zn = dpp_move<kDppShl + 1>(z[0][0]), on = dpp_move<kDppShl + 1>(o[0]);
+    const double zn = col_next<P>(t.s, z[0][0]), on = col_next<P>(t.s, o[0]);
 #pragma unroll
     for (int q = 0; q < S; ++q) {
         const int k = t.lo + q;
@@ -122,7 +122,7 @@ __device__ __forceinline__ void fric_face(const Tile<S>& t, double* img, int nz,
 
 // A block owns a strip of T columns j and walks the rows of a chunk [ib, ie) in
 // order, starting one row early for the u faces west of the chunk. Half of its
-// waves solve the row's v faces, the other half its u faces, four columns each, on
+// waves solve the row's v faces, the other half its u faces, four or eight columns each, on
 // column tiles (col_tile.hpp); the strip's first column is solved for its v face
 // only. The v faces' dissipation goes through LDS to the u waves (two images per
 // wave, one barrier per row), which keep that of the previous row's u faces and
@@ -142,17 +142,20 @@ __device__ __forceinline__ void fric_face(const Tile<S>& t, double* img, int nz,
 // Loading the next row ahead took the registers that hold a second block's waves
 // (2.55 ms). Eight lanes per column, each loading and storing its own levels,
 // and every row's divisions in the lane: friction 1.94 ms there, now 1.60; 163
-// us on 360x160x60, levels innermost, now 103.
+// us on 360x160x60, levels innermost, now 92.
 constexpr int kFricGroups = 2;                                // column groups of a block
 constexpr int kFricBlock = 2 * 64 * kFricGroups;              // a u and a v wave for each
-constexpr int kFricCols = kFricGroups * (64 / kTileP) - 1;    // T columns of a strip
-// waves per SIMD (and blocks per CU) that the registers allow
-template <int S>
-constexpr int kFricWaves = S <= 3 ? 4 : S == 4 ? 3 : 2;
-template <int S>
-__global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFricWaves<S>))) void friction_walk_kernel(
+template <int P>
+constexpr int kFricCols = kFricGroups * (64 / P) - 1;         // T columns of a strip
+// waves per SIMD (and blocks per CU): what the registers allow, but two for four
+// levels on 8 lanes (1435x896x32 849 us with three, 813 with two; 360x160x60, 16
+// lanes, 92 with three, 104 with two)
+template <int S, int P>
+constexpr int kFricWaves = S <= 3 ? 4 : S == 4 && P == kTileP ? 3 : 2;
+template <int S, int P>
+__global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFricWaves<S, P>))) void friction_walk_kernel(
     FricArgs p, int rows, int64_t nstrips, int64_t nblocks, uint32_t rnz) {
-    using T = Tile<S>;
+    using T = Tile<S, P>;
     constexpr int G = kFricGroups;
     __shared__ double work[2 * G][T::IMG];
     __shared__ double dsv[2][G][T::IMG];
@@ -174,14 +177,14 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
     const int64_t strip = b % nstrips, chunk = b / nstrips;
     const int64_t ib = 1 + (int64_t)rows * chunk;
     const int64_t ie = ib + rows < p.X - 2 ? ib + rows : p.X - 2;
-    const int64_t j0 = kFricCols * strip + T::C * grp;  // the wave's columns
+    const int64_t j0 = kFricCols<P> * strip + T::C * grp;  // the wave's columns
     const int64_t left = p.Y - 2 - j0;
     const int n = left >= T::C ? T::C : (left > 0 ? (int)left : 0);
     const int64_t next = vface ? 1 : p.Y;  // the face's other column
     const uint32_t cs = (uint32_t)p.cs;
     const double rdt = 1.0 / p.dt;
     double* const vel = p.vel[comp];
-    T t = make_tile<S>(0, n, nz, (uint32_t)nz, rnz);
+    T t = make_tile<S, P>(0, n, nz, (uint32_t)nz, rnz);
     const int64_t j = t.q < n ? j0 + t.q : (n > 0 ? j0 : 0);  // the lane's column
     const bool jlive = t.q < n && j >= 1, jown = jlive && (grp > 0 || t.q > 0);
     // the block's own elements: not the strip's first column, nor j = 0
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
             double fx[S], kn[S], x0[S], x1[S];
             uint32_t on[S];  // the solved levels
 #pragma unroll
-            for (int r = 0; r < S; ++r) on[r] = t.k[r] >= __shfl(f.k0, t.c[r] * kTileP) ? t.off[r] : kNoAccess;
+            for (int r = 0; r < S; ++r) on[r] = t.k[r] >= __shfl(f.k0, t.c[r] * P) ? t.off[r] : kNoAccess;
             tile_load(tile_buf(t, p.kappaM), on, 1, fx);
             tile_load(tile_buf(t, p.kappaM, next * nz), on, 1, kn);
             tile_load(b0, on, cs, x0);
@@ -225,7 +228,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
             }
 #pragma unroll
             for (int r = 0; r < S; ++r) fx[r] = 0.5 * (fx[r] + kn[r]);
-            fric_face<S>(t, img, nz, sdz[0], sdz[1], sdz[2], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
+            fric_face<S, P>(t, img, nz, sdz[0], sdz[1], sdz[2], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
             if (vface) seg_put(t, dsv[i & 1][grp], ds);
             tile_store(b1, on, cs, x1);
             tile_store(bd, on, 1, kn);
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         const int wc = jown ? first_wet_level(kb, nz) : nz;
 #pragma unroll
         for (int r = 0; r < S; ++r)
-            ow[r] = t.k[r] >= __shfl(wc, t.c[r] * kTileP) && t.k[r] < nz - 1 ? t.off[r] : kNoAccess;
+            ow[r] = t.k[r] >= __shfl(wc, t.c[r] * P) && t.k[r] < nz - 1 ? t.off[r] : kNoAccess;
         tile_load(bK, ow, 1, K);
         const bool south = jown && j >= 2;
         if (south) {
@@ -298,12 +301,12 @@ int fric_rows(int64_t nrows, int64_t nstrips, int blocks_per_cu) {
     return best;
 }
 
-template <int S>
+template <int S, int P>
 void launch_fric_walk(const FricArgs& p, hipStream_t s) {
-    const int64_t nstrips = (p.Y - 3 + kFricCols - 1) / kFricCols;
-    const int rows = fric_rows(p.X - 3, nstrips, kFricWaves<S>);
+    const int64_t nstrips = (p.Y - 3 + kFricCols<P> - 1) / kFricCols<P>;
+    const int rows = fric_rows(p.X - 3, nstrips, kFricWaves<S, P>);
     const int64_t nblocks = nstrips * ((p.X - 3 + rows - 1) / rows);
-    hipLaunchKernelGGL(friction_walk_kernel<S>, dim3((unsigned)((nblocks + 7) / 8 * 8)), dim3(kFricBlock), 0, s, p,
+    hipLaunchKernelGGL((friction_walk_kernel<S, P>), dim3((unsigned)((nblocks + 7) / 8 * 8)), dim3(kFricBlock), 0, s, p,
                        rows, nstrips, nblocks, depth_reciprocal(p.nz));
 }
 
@@ -356,14 +359,21 @@ extern "C" int vx_implicit_vert_friction_f64(void* stream, const vx_grid* grid, 
     p.cs = outer ? 1 : 3;
     p.ls = outer ? p.X * p.Y * p.nz : 1;
     hipStream_t s = (hipStream_t)stream;
-    switch (tile_levels(p.nz)) {
-        case 2: launch_fric_walk<2>(p, s); break;
-        case 3: launch_fric_walk<3>(p, s); break;
-        case 4: launch_fric_walk<4>(p, s); break;
-        case 5: launch_fric_walk<5>(p, s); break;
-        case 6: launch_fric_walk<6>(p, s); break;
-        case 7: launch_fric_walk<7>(p, s); break;
-        default: launch_fric_walk<8>(p, s); break;
+    if (col_lanes(p.nz) == kSegP) {
+        switch (col_levels(p.nz)) {
+            case 2: launch_fric_walk<2, kSegP>(p, s); break;
+            case 3: launch_fric_walk<3, kSegP>(p, s); break;
+            default: launch_fric_walk<4, kSegP>(p, s); break;
+        }
+    } else {
+        switch (col_levels(p.nz)) {
+            case 3: launch_fric_walk<3, kTileP>(p, s); break;
+            case 4: launch_fric_walk<4, kTileP>(p, s); break;
+            case 5: launch_fric_walk<5, kTileP>(p, s); break;
+            case 6: launch_fric_walk<6, kTileP>(p, s); break;
+            case 7: launch_fric_walk<7, kTileP>(p, s); break;
+            default: launch_fric_walk<8, kTileP>(p, s); break;
+        }
     }
     return check_launch(who);
 }

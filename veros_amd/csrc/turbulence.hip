@@ -3,7 +3,7 @@
 // integrate_eke_kernel (veros/core/eke.py:93-255) and integrate_idemix_kernel
 // (veros/core/idemix.py:47-265), without their advection branches.
 //
-// One kernel per model. A wave owns a tile of four columns of the whole (X, Y)
+// One kernel per model. A wave owns a tile of four or eight columns of the whole (X, Y)
 // grid (col_tile.hpp): it loads its cells flat and coalesced, sums the forcing
 // terms and forms the right-hand side and the dissipation coefficient cell by
 // cell, passes those and the diffusivity through LDS to the segment layout,
@@ -48,8 +48,8 @@ struct Terms {
 
 // The lateral faces of a tile's columns: east, west, north, south.
 struct TurbCols {
-    double w[kTileC][4];  // weights
-    int face[kTileC][4];  // first level at which the face is wet (nz: none)
+    double w[64 / kSegP][4];  // weights
+    int face[64 / kSegP][4];  // first level at which the face is wet (nz: none)
 };
 
 // Level tables of a block: dd[k] = the diffusivity's factor in delta at level k
@@ -60,15 +60,16 @@ struct TurbLevels {
 
 __device__ __forceinline__ int first_wet_of(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
 
-// The wave's tile: columns [col0, col0 + kTileC) of the X * Y, in order.
+// The wave's tile: columns [col0, col0 + 64 / P) of the X * Y, in order.
+template <int P>
 __device__ __forceinline__ int64_t turb_col0(int wave) {
-    return (xcd_contiguous_block() * (kTurbBlock / 64) + wave) * kTileC;
+    return (xcd_contiguous_block() * (kTurbBlock / 64) + wave) * (64 / P);
 }
-template <int S>
-__device__ __forceinline__ Tile<S> turb_tile(const TurbGrid& g, int64_t col0) {
+template <int S, int P>
+__device__ __forceinline__ Tile<S, P> turb_tile(const TurbGrid& g, int64_t col0) {
     const int64_t left = (int64_t)g.X * g.Y - col0;
-    const int n = left >= kTileC ? kTileC : (left > 0 ? (int)left : 0);
-    return make_tile<S>(n > 0 ? col0 * g.nz : 0, n, g.nz, (uint32_t)g.nz, depth_reciprocal(g.nz));
+    const int n = left >= 64 / P ? 64 / P : (left > 0 ? (int)left : 0);
+    return make_tile<S, P>(n > 0 ? col0 * g.nz : 0, n, g.nz, (uint32_t)g.nz, depth_reciprocal(g.nz));
 }
 
 // The lane's group column (segments): what the masks need, known before the
@@ -78,8 +79,8 @@ struct TurbLane {
     bool interior;
     int kw, k0;  // first wet and first solved level (nz: none)
 };
-template <int S>
-__device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S>& t, int64_t col0) {
+template <int S, int P>
+__device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S, P>& t, int64_t col0) {
     TurbLane l;
     const bool valid = t.q < t.ncol;
     const int64_t col = valid ? col0 + t.q : 0;
@@ -96,8 +97,8 @@ __device__ __forceinline__ TurbLane turb_lane(const TurbGrid& g, const Tile<S>& 
 // columns; every thread of the block calls it, after it has issued its first
 // loads (whose latency the divisions here hide). `lateral`: the weights times
 // `lw` and the faces are wanted.
-template <int S>
-__device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S>& t, const TurbLane& l, double scale,
+template <int S, int P>
+__device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S, P>& t, const TurbLane& l, double scale,
                                            double lw, bool lateral, TurbLevels& lv, TurbCols& tc) {
     const int nz = g.nz;
     for (int k = threadIdx.x; k < nz; k += kTurbBlock) {
@@ -135,8 +136,8 @@ __device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S>& t, 
 // pair are in flight together and hold few registers. The kernels store their
 // diagnostics after it: a load waits for the stores issued before it (the three
 // models on 1440x720x80: 4.13 -> 4.10 ms).
-template <int S, bool TWO, class COMB>
-__device__ __forceinline__ void add_lateral(const TurbGrid& g, const Tile<S>& t, const TurbCols& tc, const double* A,
+template <int S, bool TWO, int P, class COMB>
+__device__ __forceinline__ void add_lateral(const TurbGrid& g, const Tile<S, P>& t, const TurbCols& tc, const double* A,
                                             uint32_t csA, const double* B, const double (&a)[S],
                                             const double (&b)[TWO ? S : 1], COMB comb, double (&v)[S]) {
     const int64_t nz = g.nz, row = (int64_t)g.Y * nz;
@@ -172,8 +173,8 @@ __device__ __forceinline__ void add_lateral(const TurbGrid& g, const Tile<S>& t,
 // f plus the signed forcing terms on the cells of `off`, summed left to right;
 // with `first` the sum replaces f. VX_TERMS_GROUP terms are loaded at a time,
 // before the group's first use.
-template <int S>
-__device__ __forceinline__ void add_terms(const Terms& T, const Tile<S>& t, const uint32_t (&off)[S], bool first,
+template <int S, int P>
+__device__ __forceinline__ void add_terms(const Terms& T, const Tile<S, P>& t, const uint32_t (&off)[S], bool first,
                                           double (&f)[S]) {
     constexpr int G = VX_TERMS_GROUP;
     for (int q0 = 0; q0 < T.n; q0 += G) {
@@ -198,8 +199,8 @@ __device__ __forceinline__ void add_terms(const Terms& T, const Tile<S>& t, cons
 // dissipation) and rhs images in, the solution into the rhs image. MUL (IDEMIX):
 // the rows are scaled by kap at their own column's level,
 // a = -delta[k-1] kap[k-1], b = 1 + (delta[k] + delta[k-1]) kap[k], c = -delta[k] kap[k+1].
-template <int S, bool MUL>
-__device__ __forceinline__ void turb_solve(const Tile<S>& t, const TurbLevels& lv, int nz, int k0, const double* kap,
+template <int S, bool MUL, int P>
+__device__ __forceinline__ void turb_solve(const Tile<S, P>& t, const TurbLevels& lv, int nz, int k0, const double* kap,
                                            const double* diss, double* rhs) {
     double km[S], va[S], vb[S], vc[S], z[1][S];
     seg_get(t, kap, km);
@@ -244,14 +245,14 @@ __device__ __forceinline__ void turb_solve(const Tile<S>& t, const TurbLevels& l
         z[0][r] = wet ? z[0][r] : 0.0;
         dm = dk;
     }
-    tile_solve<S, 1>(t, va, vb, vc, z);
+    col_solve<S, 1>(t, va, vb, vc, z);
     seg_put(t, rhs, z[0]);
 }
 
 // LDS of a block: three images per wave, the columns, the level tables.
-template <int S>
+template <int S, int P>
 struct TurbShared {
-    double img[kTurbBlock / 64][3][Tile<S>::IMG];
+    double img[kTurbBlock / 64][3][Tile<S, P>::IMG];
     TurbCols cols[kTurbBlock / 64];
     TurbLevels lv;
 };
@@ -275,13 +276,13 @@ struct TkeArgs {
     int hor;
 };
 
-template <int S>
+template <int S, int P>
 __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void tke_kernel(TkeArgs a) {
     const TurbGrid& g = a.g;
-    __shared__ TurbShared<S> sh;
+    __shared__ TurbShared<S, P> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int64_t col0 = turb_col0(wave);
-    const Tile<S> t = turb_tile<S>(g, col0);
+    const int64_t col0 = turb_col0<P>(wave);
+    const Tile<S, P> t = turb_tile<S, P>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
     const TurbLane l = turb_lane(g, t, col0);
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     uint32_t wet[S], dry[S];  // solved cells; the others of the run
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP);
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * P);
         wet[r] = w ? t.off[r] : kNoAccess;
         dry[r] = w ? kNoAccess : t.off[r];
     }
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             x[r] = e0[r] + dt * f[r];
-            const double fs = __shfl(fsurf, t.c[r] * kTileP);
+            const double fs = __shfl(fsurf, t.c[r] * P);
             if (t.k[r] == nz - 1) x[r] += rtop * fs;
         }
         tile_put(t, sh.img[wave][2], x);
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     bool top[S];
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        const int in = __shfl((int)l.interior, t.c[r] * kTileP);
+        const int in = __shfl((int)l.interior, t.c[r] * P);
         top[r] = in != 0 && t.k[r] == nz - 1 && t.off[r] != kNoAccess;
         corr[r] = v[r];
         v[r] = top[r] ? fmax(0.0, v[r]) : v[r];
@@ -373,13 +374,13 @@ struct EkeArgs {
     double dt, alpha, c_eps;
 };
 
-template <int S>
+template <int S, int P>
 __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void eke_kernel(EkeArgs a) {
     const TurbGrid& g = a.g;
-    __shared__ TurbShared<S> sh;
+    __shared__ TurbShared<S, P> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int64_t col0 = turb_col0(wave);
-    const Tile<S> t = turb_tile<S>(g, col0);
+    const int64_t col0 = turb_col0<P>(wave);
+    const Tile<S, P> t = turb_tile<S, P>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
     const TurbLane l = turb_lane(g, t, col0);
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     uint32_t wet[S], sea[S], halo[S];
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP), m = t.k[r] >= __shfl(l.kw, t.c[r] * kTileP);
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * P), m = t.k[r] >= __shfl(l.kw, t.c[r] * P);
         wet[r] = w ? t.off[r] : kNoAccess;
         sea[r] = m ? t.off[r] : kNoAccess;
         halo[r] = m && !w ? t.off[r] : kNoAccess;
@@ -454,13 +455,13 @@ struct IdemixArgs {
     int diss_mode;  // 0: as is; 1: column integral at the bottom cell; 2: split bottom / surface
 };
 
-template <int S>
+template <int S, int P>
 __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_TURB_WAVES(S)))) void idemix_kernel(IdemixArgs a) {
     const TurbGrid& g = a.g;
-    __shared__ TurbShared<S> sh;
+    __shared__ TurbShared<S, P> sh;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const int64_t col0 = turb_col0(wave);
-    const Tile<S> t = turb_tile<S>(g, col0);
+    const int64_t col0 = turb_col0<P>(wave);
+    const Tile<S, P> t = turb_tile<S, P>(g, col0);
     const double dt = a.dt;
     TurbCols& tc = sh.cols[wave];
     const TurbLane l = turb_lane(g, t, col0);
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     uint32_t wet[S], dry[S];
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * kTileP);
+        const bool w = t.k[r] >= __shfl(l.k0, t.c[r] * P);
         wet[r] = w ? t.off[r] : kNoAccess;
         dry[r] = w ? kNoAccess : t.off[r];
     }
@@ -502,16 +503,16 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
             const double fk = img[t.seg + r];
             if (k >= k0 && k < nz) part += (k < nz - 1 ? sh.lv.zw[k] : 0.5 * sh.lv.zw[k]) * fk;
         }
-        part += __shfl_xor(part, 1, kTileP);
-        part += __shfl_xor(part, 2, kTileP);
-        part += __shfl_xor(part, 4, kTileP);
-        part += __shfl_xor(part, 8, kTileP);
+        part += __shfl_xor(part, 1, P);
+        part += __shfl_xor(part, 2, P);
+        part += __shfl_xor(part, 4, P);
+        if constexpr (P == 16) part += __shfl_xor(part, 8, P);
 #pragma unroll
         for (int r = 0; r < S; ++r) {
-            const double a_loc = __shfl(part, t.c[r] * kTileP);
+            const double a_loc = __shfl(part, t.c[r] * P);
             const int k = t.k[r];
             double x = 0.0;
-            if (k == __shfl(l.k0, t.c[r] * kTileP)) x = (a.diss_mode == 1 ? 1.0 : a.frac) * a_loc / sh.lv.zw[k];
+            if (k == __shfl(l.k0, t.c[r] * P)) x = (a.diss_mode == 1 ? 1.0 : a.frac) * a_loc / sh.lv.zw[k];
             if (a.diss_mode == 2 && k == nz - 1) x = (1.0 - a.frac) * a_loc / (0.5 * sh.lv.zw[k]);
             f[r] = x;
         }
@@ -526,8 +527,8 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             x[r] = e0[r] + dt * f[r];
-            const bool edge = t.k[r] == __shfl(l.k0, t.c[r] * kTileP);
-            const double fb = __shfl(fbot, t.c[r] * kTileP), fs = __shfl(fsurf, t.c[r] * kTileP);
+            const bool edge = t.k[r] == __shfl(l.k0, t.c[r] * P);
+            const double fb = __shfl(fbot, t.c[r] * P), fs = __shfl(fsurf, t.c[r] * P);
             if (edge) x[r] += dt * fb / sh.lv.zw[t.k[r]];  // d_edge (:157-159)
             else if (t.k[r] == nz - 1) x[r] += rtop * fs;
         }
@@ -592,34 +593,41 @@ int make_terms(const vx_terms* in, Terms& t, bool allow_empty, const char* who) 
     return VX_OK;
 }
 
-template <class Args, template <int> class K>
+template <class Args, template <int, int> class K>
 int launch_turb(const Args& a, const TurbGrid& g, hipStream_t s, const char* who) {
-    const int64_t threads = ((int64_t)g.X * g.Y + kTileC - 1) / kTileC * 64;
+    const int lanes = col_lanes(g.nz), cols = 64 / lanes;
+    const int64_t threads = ((int64_t)g.X * g.Y + cols - 1) / cols * 64;
     const dim3 grid(blocks_mult8(threads, kTurbBlock)), block(kTurbBlock);
-    switch (tile_levels(g.nz)) {
-        case 2: hipLaunchKernelGGL(K<2>::fn, grid, block, 0, s, a); break;
-        case 3: hipLaunchKernelGGL(K<3>::fn, grid, block, 0, s, a); break;
-        case 4: hipLaunchKernelGGL(K<4>::fn, grid, block, 0, s, a); break;
-        case 5: hipLaunchKernelGGL(K<5>::fn, grid, block, 0, s, a); break;
-        case 6: hipLaunchKernelGGL(K<6>::fn, grid, block, 0, s, a); break;
-        case 7: hipLaunchKernelGGL(K<7>::fn, grid, block, 0, s, a); break;
-        case 8: hipLaunchKernelGGL(K<8>::fn, grid, block, 0, s, a); break;
+    switch (col_levels(g.nz)) {
+        case 2: hipLaunchKernelGGL((K<2, kSegP>::fn), grid, block, 0, s, a); break;
+        case 3:
+            if (lanes == kSegP) hipLaunchKernelGGL((K<3, kSegP>::fn), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((K<3, kTileP>::fn), grid, block, 0, s, a);
+            break;
+        case 4:
+            if (lanes == kSegP) hipLaunchKernelGGL((K<4, kSegP>::fn), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((K<4, kTileP>::fn), grid, block, 0, s, a);
+            break;
+        case 5: hipLaunchKernelGGL((K<5, kTileP>::fn), grid, block, 0, s, a); break;
+        case 6: hipLaunchKernelGGL((K<6, kTileP>::fn), grid, block, 0, s, a); break;
+        case 7: hipLaunchKernelGGL((K<7, kTileP>::fn), grid, block, 0, s, a); break;
+        case 8: hipLaunchKernelGGL((K<8, kTileP>::fn), grid, block, 0, s, a); break;
         default: return fail(VX_ERR_UNSUPPORTED, "%s: nz=%d", who, g.nz);
     }
     return check_launch(who);
 }
 
-template <int N>
+template <int N, int P>
 struct TkeK {
-    static constexpr auto fn = tke_kernel<N>;
+    static constexpr auto fn = tke_kernel<N, P>;
 };
-template <int N>
+template <int N, int P>
 struct EkeK {
-    static constexpr auto fn = eke_kernel<N>;
+    static constexpr auto fn = eke_kernel<N, P>;
 };
-template <int N>
+template <int N, int P>
 struct IdemixK {
-    static constexpr auto fn = idemix_kernel<N>;
+    static constexpr auto fn = idemix_kernel<N, P>;
 };
 
 bool levels_ok(int tau, int taup1) { return tau >= 0 && tau <= 2 && taup1 >= 0 && taup1 <= 2 && tau != taup1; }

@@ -9,7 +9,7 @@
 // then forms the tendencies (new - old) / dt over the whole array and copies
 // the cyclic x halos.
 //
-// Here a group of 16 lanes owns a column (col_tile.hpp): it forms the rows in
+// Here a group of 8 or 16 lanes owns a column (col_tile.hpp): it forms the rows in
 // registers, solves temperature and salinity with one factorisation, and the
 // wave writes the new tracers on the wet levels and both tendencies on every
 // level. The coefficients never touch memory: the kernel reads kappaH and the
@@ -80,15 +80,15 @@ __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __res
     }
 }
 
-// Column tiles (any layout, depth and alignment): a wave's four columns are loaded
+// Column tiles (any layout, depth and alignment): a wave's columns are loaded
 // flat, the two tracers' old values stay with the lanes that loaded them, and
 // everything goes back flat. Bound by HBM: on 1440x720x80, levels outermost, 2.6 GB
 // in 0.59 ms (8 lanes per column with 16-byte copies into LDS: 0.60); 360x160x60,
 // levels innermost, 71 -> 46 us against each lane loading its own levels.
 constexpr int kVmixBlock = 128;
-template <int S>
+template <int S, int P>
 __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, uint32_t rnz) {
-    using T = Tile<S>;
+    using T = Tile<S, P>;
     __shared__ double sdz[2 * kMaxNz];
     __shared__ double lds[kVmixBlock / 64][T::IMG];
     vmix_stage_dz(p, sdz);
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
     const int64_t left = p.X * p.Y - col0;
     if (left <= 0) return;  // uniform in the wave; no barrier follows
     const int n = left >= T::C ? T::C : (int)left;
-    const T t = make_tile<S>(col0 * nz, n, nz, (uint32_t)nz, rnz);
+    const T t = make_tile<S, P>(col0 * nz, n, nz, (uint32_t)nz, rnz);
     SegLane L;
     L.s = t.s;
     L.lo = t.lo;
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
     double oT[S], oS[S], nT[S], nS[S];
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        wet[r] = t.k[r] >= __shfl(L.k0, t.c[r] * kTileP) ? t.off[r] : kNoAccess;
+        wet[r] = t.k[r] >= __shfl(L.k0, t.c[r] * P) ? t.off[r] : kNoAccess;
         nT[r] = nS[r] = 0.0;
     }
     if (__any(L.k0 < nz)) {
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
         tile_put(t, img, oS);
         seg_get(t, img, z[1]);
         vmix_rows<S>(p, sdz, sdz + kMaxNz, L, [&](int k) { return km[k - L.lo + 1]; }, fT, fS, va, vb, vc, z[0], z[1]);
-        tile_solve<S, 2>(t, va, vb, vc, z);
+        col_solve<S, 2>(t, va, vb, vc, z);
         seg_put(t, img, z[0]);
         tile_get(t, img, nT);
         seg_put(t, img, z[1]);
@@ -173,10 +173,10 @@ __global__ __launch_bounds__(256) void vertmix_cyclic_kernel(VmixArgs p) {
     tr[p.cs * (dst * plane + off)] = tr[p.cs * (src * plane + off)];
 }
 
-template <int S>
+template <int S, int P>
 void launch_vmix(const VmixArgs& p, hipStream_t s) {
-    const int64_t threads = p.X * p.Y * kTileP;
-    hipLaunchKernelGGL(vertmix_tile_kernel<S>, dim3((unsigned)((threads + kVmixBlock - 1) / kVmixBlock)),
+    const int64_t threads = (p.X * p.Y + 64 / P - 1) / (64 / P) * 64;
+    hipLaunchKernelGGL((vertmix_tile_kernel<S, P>), dim3((unsigned)((threads + kVmixBlock - 1) / kVmixBlock)),
                        dim3(kVmixBlock), 0, s, p, depth_reciprocal(p.nz));
 }
 
@@ -227,14 +227,21 @@ extern "C" int vx_vertmix_tempsalt_f64(void* stream, const vx_grid* grid, double
     p.cs = outer ? 1 : 3;
     p.ls = outer ? p.X * p.Y * p.nz : 1;
     hipStream_t s = (hipStream_t)stream;
-    switch (tile_levels(p.nz)) {
-        case 2: launch_vmix<2>(p, s); break;
-        case 3: launch_vmix<3>(p, s); break;
-        case 4: launch_vmix<4>(p, s); break;
-        case 5: launch_vmix<5>(p, s); break;
-        case 6: launch_vmix<6>(p, s); break;
-        case 7: launch_vmix<7>(p, s); break;
-        default: launch_vmix<8>(p, s); break;
+    if (col_lanes(p.nz) == kSegP) {
+        switch (col_levels(p.nz)) {
+            case 2: launch_vmix<2, kSegP>(p, s); break;
+            case 3: launch_vmix<3, kSegP>(p, s); break;
+            default: launch_vmix<4, kSegP>(p, s); break;
+        }
+    } else {
+        switch (col_levels(p.nz)) {
+            case 3: launch_vmix<3, kTileP>(p, s); break;
+            case 4: launch_vmix<4, kTileP>(p, s); break;
+            case 5: launch_vmix<5, kTileP>(p, s); break;
+            case 6: launch_vmix<6, kTileP>(p, s); break;
+            case 7: launch_vmix<7, kTileP>(p, s); break;
+            default: launch_vmix<8, kTileP>(p, s); break;
+        }
     }
     int rc = check_launch(who);
     if (rc) return rc;
