@@ -25,14 +25,12 @@ REPO = Path(__file__).resolve().parent
 sys.path.insert(0, str(REPO))
 
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per call of vx_iso_pre_diffusion_ts_f64 (its seven kernels) on
-# 1440x720x80, from the FETCH_SIZE and WRITE_SIZE rocprofv3 passes recorded in
-# profiles/mixing_step_1440x720x80.md (read bytes = 2.0 x FETCH_SIZE, write
-# bytes = 1.0 x WRITE_SIZE, calibrated on a 1 GiB device copy), per layout of
-# the time-level variables
-# (the levels-innermost figure predates the segmented K33 solve of the step
-# kernel and pre's unconditional neighbour loads)
-PRE_TS_TRAFFIC_BYTES = {(1440, 720, 80, "outer"): 21_844_174_848, (1440, 720, 80, "inner"): 27_204_216_832}
+# HBM bytes per call of vx_iso_pre_diffusion_ts_f64 (its two kernels) on
+# 1440x720x80, time levels outermost, from the FETCH_SIZE and WRITE_SIZE
+# rocprofv3 passes recorded in profiles/mixing_step_1440x720x80.md (read bytes =
+# 2.0 x FETCH_SIZE, write bytes = 1.0 x WRITE_SIZE, calibrated on a 1 GiB device
+# copy); not measured with the levels innermost
+PRE_TS_TRAFFIC_BYTES = {(1440, 720, 80, "outer"): 21_926_504_320}
 # the minimum bytes per interior cell of pre + the temperature + salinity step
 # in one call: K_iso read (8), Ai_* and K_11/22/33 written once and not read
 # back (128 + 24), P_diss read and written (16), and per tracer tr[tau] (8),
