@@ -25,8 +25,7 @@
 
 namespace vx {
 
-constexpr int kTileP = 16;           // lanes per column, unless a kernel says otherwise: one DPP row
-constexpr int kTileC = 64 / kTileP;  // columns per wave then
+constexpr int kTileP = 16;  // lanes per column, unless a kernel says otherwise: one DPP row
 
 // levels per lane for a depth nz (>= 2)
 __host__ __device__ constexpr int tile_levels(int nz) {

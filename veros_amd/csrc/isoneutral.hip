@@ -1612,7 +1612,6 @@ dim3 cell_column_grid(const Grid& g, int ncb) {
 }
 
 unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-unsigned blocks_xcd(int64_t n, int bs) { return (unsigned)(((n + bs - 1) / bs + 7) / 8 * 8); }
 
 // block of nz levels x cpb columns (about 256 threads); 1-D grid of ni row
 // groups, rounded up to a multiple of 8 for the XCD remap
