@@ -76,6 +76,23 @@ struct Tile {
 __host__ __device__ __forceinline__ uint32_t depth_reciprocal(int nz) {
     return ((1u << 20) + (uint32_t)nz - 1u) / (uint32_t)nz;
 }
+// Flat element e of such a tile.
+struct FlatCell {
+    int k, c, pos;
+    uint32_t off;  // kNoAccess past the run; c is 0 there
+};
+template <int S, int P>
+__host__ __device__ __forceinline__ FlatCell flat_cell(uint32_t e, int ncol, int nz, uint32_t sy, uint32_t m) {
+    using T = Tile<S, P>;
+    const uint32_t c = (e * m) >> 20, k = e - c * (uint32_t)nz;
+    const bool in = (int)c < ncol;
+    FlatCell f;
+    f.k = (int)k;
+    f.c = in ? (int)c : 0;
+    f.pos = (int)c < T::C ? (int)(c * T::CS + k + k / S * (T::SP - S)) : T::DUMMY;
+    f.off = in ? (c * sy + k) * 8u : kNoAccess;
+    return f;
+}
 template <int S, int P = kTileP>
 __device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz, uint32_t sy, uint32_t m) {
     using T = Tile<S, P>;
@@ -90,15 +107,23 @@ __device__ __forceinline__ Tile<S, P> make_tile(int64_t cell0, int ncol, int nz,
     t.bytes = ncol > 0 ? ((uint32_t)(ncol - 1) * sy + (uint32_t)nz) * 8u : 0u;
 #pragma unroll
     for (int r = 0; r < S; ++r) {
-        const uint32_t e = 64u * r + (uint32_t)t.lane;
-        const uint32_t c = (e * m) >> 20, k = e - c * (uint32_t)nz;
-        const bool in = (int)c < ncol;
-        t.k[r] = (int)k;
-        t.c[r] = in ? (int)c : 0;
-        t.pos[r] = (int)c < T::C ? (int)(c * T::CS + k + k / S * (T::SP - S)) : T::DUMMY;
-        t.off[r] = in ? (c * sy + k) * 8u : kNoAccess;
+        const FlatCell f = flat_cell<S, P>(64u * r + (uint32_t)t.lane, ncol, nz, sy, m);
+        t.k[r] = f.k;
+        t.c[r] = f.c;
+        t.pos[r] = f.pos;
+        t.off[r] = f.off;
     }
     return t;
+}
+// Image positions of the levels below and above a flat element in its column;
+// the element's own where the column has no level from k0 on there, and for an
+// element past the run, whose slot may be the image's last.
+template <int S, int P>
+__host__ __device__ __forceinline__ void flat_neighbours(const FlatCell& f, int k0, int nz, int& below, int& above) {
+    constexpr int step = Tile<S, P>::SP - S;  // more between two segments
+    const bool on = f.off != kNoAccess && f.k >= k0;
+    below = on && f.k > k0 ? f.pos - 1 - (f.k % S == 0 ? step : 0) : f.pos;
+    above = on && f.k < nz - 1 ? f.pos + 1 + (f.k % S == S - 1 ? step : 0) : f.pos;
 }
 
 // The run of a (X, Y, nz) array, `d` cells further on, cs doubles per cell.

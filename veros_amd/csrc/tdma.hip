@@ -136,9 +136,9 @@ __global__ __launch_bounds__(kSegLdsBlock) __attribute__((amdgpu_waves_per_eu(2)
     for (int r = 0; r < S; ++r) {
         const int k = t.k[r], k0 = __shfl(L.k0, t.c[r] * kTdmaP);
         const bool w = k >= k0, edge = k == k0;
-        const int seg0 = k % S == 0 ? Tile<S, kTdmaP>::SP - S : 0, seg1 = k % S == S - 1 ? Tile<S, kTdmaP>::SP - S : 0;
-        const double xm = ximg[w && !edge ? t.pos[r] - 1 - seg0 : t.pos[r]];
-        const double xp = ximg[w && k < nz - 1 ? t.pos[r] + 1 + seg1 : t.pos[r]];
+        int below, above;
+        flat_neighbours<S, kTdmaP>({k, t.c[r], t.pos[r], t.off[r]}, k0, nz, below, above);
+        const double xm = ximg[below], xp = ximg[above];
         const double l = w ? lam[r] : 0.0;
         ga[r] = edge ? 0.0 : -l * xm;
         gb[r] = -l * x[r];
