@@ -16,6 +16,7 @@ import numpy as np
 import pytest
 import torch
 
+import test_gpu_friction as TF
 import test_gpu_vertmix as TV
 
 pytestmark = [pytest.mark.gpu,
@@ -88,3 +89,13 @@ def test_vertmix(nz):
     plain = _as_dict(TV.V.vertmix_tempsalt(st, solver="thomas"))
     exact = _as_dict(_extended("vertmix").vertmix_tempsalt(_wide(st), solver="thomas"))
     _check(out, plain, exact, TV.KEYS)
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+def test_friction(nz):
+    from veros_amd import friction
+    st = TF._state(nz, 60, 50, nz)
+    out = _as_dict(friction.implicit_vert_friction(TF._dev(st, "inner")))
+    plain = _as_dict(TF.F.implicit_vert_friction(st, solver="thomas"))
+    exact = _as_dict(_extended("friction").implicit_vert_friction(_wide(st), solver="thomas"))
+    _check(out, plain, exact, TF.KEYS)

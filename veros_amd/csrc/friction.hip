@@ -63,6 +63,9 @@ __device__ inline Face face_of(int kb0, int kb1, int nz) {
     return f;
 }
 
+// x (h + l): x / y rounded once, for h = 1 / y and l = h (1 - h y), its rounding's rest.
+__device__ __forceinline__ double scaled(double x, double h, double l) { return fma(x, h, x * l); }
+
 // First wet level of a T column (nz: none).
 __device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
 
@@ -72,11 +75,13 @@ __device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 
 // the solution x1 and the tendency dm; the lane's segment of the face's dissipation
 // (:137-153, 189-201): fxa * (x1[k+1] - x1[k]) / dzw[k] * mask[k+1] * mask[k] times
 // (x0[k+1] - x0[k]) / dzw[k], x0 at tau and x1 at taup1, 0 on the top level. The
-// masks are 0 or 1, so the products are taken as selects. rzt, dtw, rzw: 1 / dzt,
-// dt / dzw and 1 / dzw in LDS.
+// masks are 0 or 1, so the products are taken as selects. rzt, dtw, rzw2, rzw2l:
+// 1 / dzt, dt / dzw and 1 / dzw^2 with what its rounding cuts off, in LDS: the
+// dissipation is then rounded no more often than by the reference's divisions.
 template <int S, int P>
 __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int nz, const double* __restrict__ rzt,
-                                          const double* __restrict__ dtw, const double* __restrict__ rzw, int k0,
+                                          const double* __restrict__ dtw, const double* __restrict__ rzw2,
+                                          const double* __restrict__ rzw2l, int k0,
                                           bool both, double rdt, const double (&fx)[S], const double (&x0)[S],
                                           double (&x1)[S], double (&dm)[S], double (&ds)[S]) {
     double f[S], o[S], va[S], vb[S], vc[S], z[1][S];
@@ -110,8 +115,7 @@ __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int 
         const double z1 = q < S - 1 ? z[0][q < S - 1 ? q + 1 : 0] : zn;
         const double o1 = q < S - 1 ? o[q < S - 1 ? q + 1 : 0] : on;
         const bool d = both && k >= k0 && k < nz - 1;
-        const double rw = rzw[d ? k : 0];
-        ds[q] = d ? ((o1 - o[q]) * (f[q] * (z1 - z[0][q])) * rw) * rw : 0.0;
+        ds[q] = d ? scaled((o1 - o[q]) * (f[q] * (z1 - z[0][q])), rzw2[d ? k : 0], rzw2l[d ? k : 0]) : 0.0;
     }
     tile_get(t, img, x1);
 #pragma unroll
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
     constexpr int G = kFricGroups;
     __shared__ double work[2 * G][T::IMG];
     __shared__ double dsv[2][G][T::IMG];
-    __shared__ double sdz[3][kMaxNz];
+    __shared__ double sdz[4][kMaxNz];
     const int64_t b = xcd_contiguous_block();
     if (b >= nblocks) return;
     const int nz = p.nz;
@@ -167,7 +171,9 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         const double zw = p.dzw[k];
         sdz[0][k] = 1.0 / p.dzt[k];
         sdz[1][k] = p.dt / zw;
-        sdz[2][k] = 1.0 / zw;
+        const double sq = zw * zw, r = 1.0 / sq;
+        sdz[2][k] = r;
+        sdz[3][k] = r * fma(-r, fma(zw, zw, -sq), fma(-r, sq, 1.0));
     }
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -228,7 +234,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
             }
 #pragma unroll
             for (int r = 0; r < S; ++r) fx[r] = 0.5 * (fx[r] + kn[r]);
-            fric_face<S, P>(t, img, nz, sdz[0], sdz[1], sdz[2], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
+            fric_face<S, P>(t, img, nz, sdz[0], sdz[1], sdz[2], sdz[3], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
             if (vface) seg_put(t, dsv[i & 1][grp], ds);
             tile_store(b1, on, cs, x1);
             tile_store(bd, on, 1, kn);
@@ -239,10 +245,11 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         }
         double bu[S];
         {
-            const double wi = p.dxu[i], wm = p.dxu[i - 1], rden = 1.0 / (2 * p.dxt[i]);
+            const double wi = p.dxu[i], wm = p.dxu[i - 1], den = 2 * p.dxt[i], rden = 1.0 / den;
+            const double rdenl = rden * fma(-rden, den, 1.0);
 #pragma unroll
             for (int r = 0; r < S; ++r) {
-                bu[r] = i >= 2 ? (wi * ds[r] + wm * du[r]) * rden : ds[r];
+                bu[r] = i >= 2 ? scaled(wi * ds[r] + wm * du[r], rden, rdenl) : ds[r];
                 du[r] = ds[r];
             }
         }
@@ -250,7 +257,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         // K_diss_v and the weights are loaded before the barrier, which their
         // latency then overlaps
         const BufRsrc bK = tile_buf(t, p.K_diss_v);
-        double K[S], wj = 1.0, wjm = 0.0;
+        double K[S], wj = 1.0, wjm = 0.0, rden = 1.0, rdenl = 0.0;
         uint32_t ow[S];
         const int wc = jown ? first_wet_level(kb, nz) : nz;
 #pragma unroll
@@ -259,9 +266,11 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         tile_load(bK, ow, 1, K);
         const bool south = jown && j >= 2;
         if (south) {
-            const double rd = 1.0 / (2 * p.area_t[col]);
-            wj = p.area_v[col] * rd;
-            wjm = p.area_v[col - 1] * rd;
+            const double den = 2 * p.area_t[col];
+            rden = 1.0 / den;
+            rdenl = rden * fma(-rden, den, 1.0);
+            wj = p.area_v[col];
+            wjm = p.area_v[col - 1];
         }
         __syncthreads();
         // the v faces of the lane's column and of the column south, which may be
@@ -271,7 +280,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             const double dn = vn[t.seg + r], dd = vs[t.seg + r];
-            bu[r] = bu[r] + (south ? wj * dn + wjm * dd : dn);
+            bu[r] = bu[r] + (south ? scaled(wj * dn + wjm * dd, rden, rdenl) : dn);
         }
         seg_put(t, img, bu);
         tile_get(t, img, bu);
