@@ -17,6 +17,7 @@ import pytest
 import torch
 
 import test_gpu_friction as TF
+import test_gpu_turbulence as TT
 import test_gpu_vertmix as TV
 
 pytestmark = [pytest.mark.gpu,
@@ -99,3 +100,13 @@ def test_friction(nz):
     plain = _as_dict(TF.F.implicit_vert_friction(st, solver="thomas"))
     exact = _as_dict(_extended("friction").implicit_vert_friction(_wide(st), solver="thomas"))
     _check(out, plain, exact, TF.KEYS)
+
+
+@pytest.mark.parametrize("nz", DEPTHS)
+@pytest.mark.parametrize("model,keys", [("tke", ("tke", "tke_diss")), ("eke", ("eke", "eke_diss_iw"))])
+def test_energies(model, keys, nz):
+    st = TT._state(nz, 60, 50, nz, enable_eke=True, enable_tke_hor_diffusion=True)
+    out = TT._gpu(model, st, "outer")
+    fn = TT.ORACLE[model]
+    exact = getattr(_extended("turbulence"), fn.__name__)(_wide(st), solver="thomas")
+    _check(out, _as_dict(fn(st, solver="thomas")), _as_dict(exact), keys)
