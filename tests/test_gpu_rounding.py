@@ -110,3 +110,42 @@ def test_energies(model, keys, nz):
     fn = TT.ORACLE[model]
     exact = getattr(_extended("turbulence"), fn.__name__)(_wide(st), solver="thomas")
     _check(out, _as_dict(fn(st, solver="thomas")), _as_dict(exact), keys)
+
+
+def _solve_and_gradients(p, g, dtype):
+    """x, lam = A^-T g and the gradients of sum(g x), by sweeps over the masked rows."""
+    tdma = _extended("tdma") if dtype is LD else importlib.import_module("oracle.tdma")
+    a, b, c, d, be, g = (v.astype(dtype) for v in (p.a, p.b, p.c, p.d, p.b_edge, g))
+    _, water, edge = tdma.create_water_masks(p.kbot, a.shape[2])
+    zero = np.zeros((), dtype)
+    b = np.where(edge, be, b)
+    a, c = np.where(water & ~edge, a, zero), np.where(water, c, zero)
+    c[..., -1] = 0
+    x = tdma.solve_tridiagonal_thomas(a, b, c, d, water, edge)
+
+    def down(t):  # the level below
+        return np.concatenate([np.zeros_like(t[..., :1]), t[..., :-1]], -1)
+
+    def up(t):
+        return np.concatenate([t[..., 1:], np.zeros_like(t[..., :1])], -1)
+
+    # the row below the edge is not part of the system: its c does not enter
+    lam = tdma.solve_tridiagonal_thomas(down(c), b, up(a), g, water, edge)
+    gb = -lam * x
+    return dict(a=np.where(water & ~edge, -lam * down(x), zero), b=gb, c=up(x) * -lam, d=lam)
+
+
+@pytest.mark.parametrize("nz", [3, 9, 20, 33, 47, 60, 77, 100, 128])
+def test_solve_gradients(nz):
+    from veros_amd import workloads as W
+    from veros_amd.autodiff import solve_implicit_ad
+    rng = np.random.default_rng(nz)
+    p = W.diffusion_tdma(rng, 50, 40, nz, dz=W.geometric_dz(nz, 10.0, 500.0), land_frac=0.2, independent_ac=True,
+                         with_b_edge=True)
+    g = rng.standard_normal(p.a.shape)
+    leaf = {n: torch.from_numpy(getattr(p, n)).cuda().requires_grad_(True) for n in ("a", "b", "c", "d", "b_edge")}
+    x = solve_implicit_ad(leaf["a"], leaf["b"], leaf["c"], leaf["d"], torch.from_numpy(p.kbot).cuda(), leaf["b_edge"])
+    x.backward(torch.from_numpy(g).cuda())
+    out = {n: t.grad.cpu().numpy() for n, t in leaf.items()}
+    out["b"] += out.pop("b_edge")  # the diagonal in use: b, at the edge b_edge
+    _check(out, _solve_and_gradients(p, g, np.float64), _solve_and_gradients(p, g, LD), tuple(out))

@@ -1402,7 +1402,7 @@ __global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(2))) 
         z[r] = w ? z[r] : 0.0;
         dm = dl;
     }
-    seg_solve_f64<S>(L, va, vb, vc, z);
+    seg_solve_f64<S, 2>(L, va, vb, vc, z);
     seg_put(t, img, z);
     double lam[S], nu[S];
     tile_get(t, img, lam);

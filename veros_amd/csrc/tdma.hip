@@ -127,7 +127,25 @@ __global__ __launch_bounds__(kSegLdsBlock) __attribute__((amdgpu_waves_per_eu(2)
         tile_put(t, ximg, x);
     }
     seg_mask_rows<S>(p, L, be, 0.0, sub, diag, sup, z, false);
-    seg_solve_f64<S>(L, sub, diag, sup, z);
+    if constexpr (S <= 8) {
+        // lam shares x's pivots, so that in gb = -lam x their roundings add up (nz 9 to 60:
+        // 1.09 to 1.02 times the error of a sequential lam): one step of refinement
+        double a[S], c[S], d[S];
+#pragma unroll
+        for (int r = 0; r < S; ++r) a[r] = sub[r], c[r] = sup[r], d[r] = z[r];
+        seg_solve_f64<S, 2>(L, sub, diag, sup, z);
+        const double zm = grp_prev(L.s, z[S - 1]), zp = grp_next(L.s, z[0]);
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const double m = r > 0 ? z[r > 0 ? r - 1 : 0] : zm, p = r < S - 1 ? z[r < S - 1 ? r + 1 : 0] : zp;
+            d[r] = fma(-a[r], m, fma(-c[r], p, fma(-diag[r], z[r], d[r])));
+        }
+        seg_solve_f64<S>(L, a, diag, c, d);
+#pragma unroll
+        for (int r = 0; r < S; ++r) z[r] += fabs(d[r]) < HUGE_VAL ? d[r] : 0.0;
+    } else {
+        seg_solve_f64<S, 2>(L, sub, diag, sup, z);
+    }
     seg_put(t, img, z);
     double lam[S], ga[S], gb[S], gc[S], gd[S];
     tile_get(t, img, lam);
