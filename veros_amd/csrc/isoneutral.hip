@@ -185,6 +185,16 @@ constexpr int kStripBlocks = VX_STRIP_BLOCKS;
 #endif
 constexpr int kPreStripCols = VX_PRE_STRIP_COLS;
 
+// Blocks of ncb columns in a strip of about `cols` columns; as many as a row of nj
+// columns needs where more than a quarter of the strip would be padding. The fused
+// call with whole strips / with shortened ones, us: 4000x2x40 241 / 59, 20000x3x80
+// 1328 / 542, 1200x7x60 107 / 65, 2000x20x50 213 / 206; where an eighth is padding the
+// shortened strip is no faster (calls on 360x160x60 914 / 921).
+__host__ __device__ __forceinline__ int strip_blocks(int cols, int ncb, int nj) {
+    const int most = (nj + ncb - 1) / ncb, sb = cols / ncb;
+    return 4 * most < 3 * sb ? most : sb;
+}
+
 struct CellIdx {
     int i, j, k;
     bool valid;
@@ -704,7 +714,7 @@ __global__ __launch_bounds__(kCellBlock) __attribute__((amdgpu_waves_per_eu(VX_P
         const int64_t e = h < 2 ? h : (row ? g.X : g.Y) - 4 + h;
         K33[((row ? e * g.Y + m : m * g.Y + e) + 1) * nz - 1] = 0.0;
     }
-    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripCols / ncb);
+    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, strip_blocks(kPreStripCols, ncb, g.Y - 3));
     if (!bc.valid) return;  // padding block (uniform)
     const int i = bc.i, jb = bc.j;
     fill_metrics(g, i, jb, ncb, bm);
@@ -841,7 +851,7 @@ __device__ __forceinline__ void buf_store2(BufRsrc b, uint32_t off, double2 v) {
 template <int NTR, bool ISO>
 __global__ __launch_bounds__(kCellBlock) void iso_flux_kernel(Grid g, StepArgs a, int ncb) {
     __shared__ BlockMetrics bm;
-    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, kPreStripCols / ncb);
+    const BlockCols bc = block_cols(1, g.X - 3, 1, g.Y - 3, ncb, strip_blocks(kPreStripCols, ncb, g.Y - 3));
     if (!bc.valid) return;  // padding block (uniform)
     const int nz = g.nz, i = bc.i, jb = bc.j;
     const int tid = (int)threadIdx.x, nthr = (int)blockDim.x;
@@ -1606,7 +1616,7 @@ int cell_columns(const Grid& g) {
 }
 // blocks of ncb columns over the cells' range, for block_cols
 dim3 cell_column_grid(const Grid& g, int ncb) {
-    const int sb = kPreStripCols / ncb;
+    const int sb = strip_blocks(kPreStripCols, ncb, g.Y - 3);
     const int64_t nstrips = (g.Y - 3 + (int64_t)sb * ncb - 1) / (sb * ncb);
     return dim3((unsigned)((nstrips * (g.X - 3) * sb + 7) / 8 * 8));
 }
@@ -1647,7 +1657,7 @@ int launch_wet_step(const Grid& g, const Prm& p, const StepArgs& a, hipStream_t 
     const int64_t spread = ((int64_t)(g.X - 2) * (g.Y - 2) + 8 * cu_count() - 1) / (8 * cu_count());
     int ncb = (int)std::min<int64_t>(VX_STEP_COLS, spread);
     ncb = ncb < 4 ? 4 : ncb;
-    const int sb = (kStepStripCols + ncb - 1) / ncb;
+    const int sb = strip_blocks(kStepStripCols + ncb - 1, ncb, g.Y - 2);
     const int64_t nstrips = (g.Y - 2 + (int64_t)sb * ncb - 1) / (sb * ncb);
     const unsigned nblk = (unsigned)((nstrips * (g.X - 2) * sb + 7) / 8 * 8);
     hipLaunchKernelGGL((iso_step_wet_kernel<NTR, IMPLICIT, WETFLUX>), dim3(nblk), dim3(kStepThreads), 0, s, g, p, a,
