@@ -208,5 +208,6 @@ def mixing_step(state, a, b, c, d, T_tau, K_iso, b_edge=None, d_edge=None, *, pr
     if tuple(a.shape) != (X - 4, Y - 4, nz):
         raise ValueError(f"the systems must have the interior's shape {(X - 4, Y - 4, nz)}, got {tuple(a.shape)}")
     kb, _ = to_device(vs.kbot, torch.int32)
-    return _MixingStep.apply(a, b, c, d, b_edge, d_edge, T_tau, K_iso.contiguous(), base, kb[2:-2, 2:-2], state,
-                             precision, refine_steps)
+    # the solve's own copy: kbot may change in place before backward
+    return _MixingStep.apply(a, b, c, d, b_edge, d_edge, T_tau, K_iso.contiguous(), base, kb[2:-2, 2:-2].clone(),
+                             state, precision, refine_steps)
