@@ -332,7 +332,8 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
             const double q = a.c_eps / ml[r];
             rate[r] = q * sq[r];
             const double x = dt * rate[r];
-            sq[r] = fma(fma(-x, ml[r], dtc * sq[r]), q * rc, x);
+            const double y = fma(fma(-x, ml[r], dtc * sq[r]), q * rc, x);
+            sq[r] = y == y ? y : x;  // an infinite mxl dissipates nothing, but leaves 0 * inf in the remainder
         }
         tile_put(t, sh.img[wave][1], sq);
     }
