@@ -10,7 +10,7 @@
 // float64 (mode 0) or in mixed precision with one refinement step (mode 1).
 // vx_tdma_plan_tune times block-size / grid-size candidates per bucket on the
 // plan's own data and keeps the fastest (a process-wide cache keyed by bucket,
-// mode and size reuses earlier choices); vx_tdma_plan_graph_launch captures
+// mode, kernel and size reuses earlier choices); vx_tdma_plan_graph_launch captures
 // run() once into a hipGraph and replays it.
 #include <algorithm>
 #include <cstring>
@@ -89,7 +89,7 @@ namespace {
 constexpr int kBuckets[] = {16, 32, 48, 64, 80, 96, 112, 128};
 constexpr int kNumBuckets = 8;
 constexpr int kBlockSizes[] = {64, 128};  // one or two waves (LDS: seg_lds_wave_bytes(S) per wave)
-constexpr int kGridFactors[] = {1, 2, 4, 8, 0};  // blocks per CU; 0 = one block per 256 columns
+constexpr int kGridFactors[] = {1, 2, 4, 8, 0};  // blocks per CU; 0 = one tile per wave
 
 struct Bucket {
     int nzb = 0;
@@ -97,12 +97,13 @@ struct Bucket {
     int nsys = 0;
     int64_t tiles = 0;   // tiles of up to 8 columns
     int64_t cols = 0;    // columns
-    bool ldsv = true;    // every system's arrays allow 16-byte copies into LDS
+    bool lds = true;     // solved by the kernel with 16-byte copies into LDS (else on flat loads)
     int bs = 128;
     int factor = 0;
 };
 
-using TuneKey = std::tuple<int, int, int64_t, int>;  // nzb, mode, log2(columns), CUs
+// nzb, mode, kernel (Bucket::lds: its LDS and registers differ from the other's), log2(columns), CUs
+using TuneKey = std::tuple<int, int, bool, int, int>;
 std::mutex g_tune_mutex;
 std::map<TuneKey, std::pair<int, int>> g_tune_cache;
 
@@ -115,9 +116,13 @@ int ilog2(int64_t v) {
     return r;
 }
 
+TuneKey tune_key(const Bucket& b, int mode, int num_cu) {
+    return {b.nzb, mode, b.lds, ilog2(b.tiles * kSegCols), num_cu};
+}
+
 template <int S, int MODE>
-void launch_bs(int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
-    if (ldsv && (tdma_lds_wins(S, MODE >= 0, true) || tdma_lds_resident(S, tiles))) {
+void launch_bs(int bs, bool use_lds, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+    if (use_lds) {
         const size_t lds = (size_t)batch_lds<S, true>() * 8 * (bs / 64);
         hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, true>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
         return;
@@ -127,16 +132,16 @@ void launch_bs(int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, uns
 }
 
 template <int MODE>
-void launch_mode(int nzb, int bs, bool ldsv, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+void launch_mode(int nzb, int bs, bool lds, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
     switch (nzb) {
-        case 16: launch_bs<2, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 32: launch_bs<4, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 48: launch_bs<6, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 64: launch_bs<8, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 80: launch_bs<10, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 96: launch_bs<12, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        case 112: launch_bs<14, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
-        default: launch_bs<16, MODE>(bs, ldsv, d, nsys, tiles, grid, s); break;
+        case 16: launch_bs<2, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 32: launch_bs<4, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 48: launch_bs<6, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 64: launch_bs<8, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 80: launch_bs<10, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 96: launch_bs<12, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 112: launch_bs<14, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        default: launch_bs<16, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
     }
 }
 
@@ -167,8 +172,8 @@ unsigned grid_for(const vx_tdma_plan* P, const Bucket& b, int bs, int factor) {
 void launch_bucket(const vx_tdma_plan* P, const Bucket& b, int bs, int factor, hipStream_t s) {
     const SysDesc* d = P->d_sys + b.first;
     const unsigned grid = grid_for(P, b, bs, factor);
-    if (P->mode == 0) launch_mode<-1>(b.nzb, bs, b.ldsv, d, b.nsys, b.tiles, grid, s);
-    else launch_mode<1>(b.nzb, bs, b.ldsv, d, b.nsys, b.tiles, grid, s);
+    if (P->mode == 0) launch_mode<-1>(b.nzb, bs, b.lds, d, b.nsys, b.tiles, grid, s);
+    else launch_mode<1>(b.nzb, bs, b.lds, d, b.nsys, b.tiles, grid, s);
 }
 
 }  // namespace
@@ -226,12 +231,14 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
             sd.tile0 = b.tiles;
             b.tiles += sd.tiling.ntiles;
             b.cols += sd.args.ncol;
-            b.ldsv = b.ldsv && tdma_vec_ok(sd.args);
+            b.lds = b.lds && tdma_vec_ok(sd.args);
             table.push_back(sd);
         }
+        const int S = b.nzb / kTdmaP;
+        b.lds = b.lds && (tdma_lds_wins(S, mode != 0, true) || tdma_lds_resident(S, b.tiles));
         {
             std::lock_guard<std::mutex> lk(g_tune_mutex);
-            auto it = g_tune_cache.find(TuneKey{b.nzb, mode, ilog2(b.tiles * kSegCols), P->num_cu});
+            auto it = g_tune_cache.find(tune_key(b, mode, P->num_cu));
             if (it != g_tune_cache.end()) {
                 b.bs = it->second.first;
                 b.factor = it->second.second;
@@ -337,7 +344,7 @@ extern "C" int vx_tdma_plan_tune(vx_tdma_plan* plan, void* stream) {
         b.bs = best_bs;
         b.factor = best_f;
         std::lock_guard<std::mutex> lk(g_tune_mutex);
-        g_tune_cache[TuneKey{b.nzb, plan->mode, ilog2(b.tiles * kSegCols), plan->num_cu}] = {b.bs, b.factor};
+        g_tune_cache[tune_key(b, plan->mode, plan->num_cu)] = {b.bs, b.factor};
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
