@@ -44,19 +44,10 @@ struct Prm {
     double drhodT, drhodS, K_iso_steep, iso_slopec, iso_dslope, dt_tracer, grav, rho_0;
 };
 
-__device__ __forceinline__ int64_t cidx(const Grid& g, int i, int j) { return (int64_t)i * g.Y + j; }
-__device__ __forceinline__ int64_t idx3(const Grid& g, int i, int j, int k) { return cidx(g, i, j) * g.nz + k; }
-__device__ __forceinline__ int kb_of(const Grid& g, int i, int j) { return g.kbot[cidx(g, i, j)]; }
-__device__ __forceinline__ double mT(int kb, int k) { return (kb > 0 && kb - 1 <= k) ? 1.0 : 0.0; }
 // Level k of a column with bottom index kb is a wet T cell (maskT = 1).
 __device__ __forceinline__ bool wet(int kb, int k) { return kb > 0 && kb - 1 <= k; }
 
-// Tracer value at time level `lev` of a time-level array.
-__device__ __forceinline__ double tr3(const double* __restrict__ f, const Grid& g, int i, int j, int k, int lev) {
-    return f[(uint32_t)idx3(g, i, j, k) * g.cs + (uint32_t)lev * g.ls];
-}
-
-// Masked face gradients (veros/core/isoneutral/isoneutral.py:46-95).
+// temp and salt and the time level that the stencil reads.
 struct Fields {
     const double* __restrict__ T;
     const double* __restrict__ S;
@@ -81,32 +72,10 @@ __device__ __forceinline__ double rcp_nr(double x) {
     return fma(r, e, r);
 }
 
-// Masked face gradients (veros/core/isoneutral/isoneutral.py:46-95); `rd` is
-// the reciprocal of the metric factor (dxu*cost, dyu or dzw).
+// Masked face gradients of the two tracers (veros/core/isoneutral/isoneutral.py:46-95).
 struct Grad {
     double T, S;
 };
-
-__device__ __forceinline__ Grad grad_x(const Grid& g, const Fields& f, int i, int j, int k, double rd) {
-    const double m = mT(kb_of(g, i, j), k) * mT(kb_of(g, i + 1, j), k);
-    return {m * (tr3(f.T, g, i + 1, j, k, f.tau) - tr3(f.T, g, i, j, k, f.tau)) * rd,
-            m * (tr3(f.S, g, i + 1, j, k, f.tau) - tr3(f.S, g, i, j, k, f.tau)) * rd};
-}
-
-__device__ __forceinline__ Grad grad_y(const Grid& g, const Fields& f, int i, int j, int k, double rd) {
-    const double m = mT(kb_of(g, i, j), k) * mT(kb_of(g, i, j + 1), k);
-    return {m * (tr3(f.T, g, i, j + 1, k, f.tau) - tr3(f.T, g, i, j, k, f.tau)) * rd,
-            m * (tr3(f.S, g, i, j + 1, k, f.tau) - tr3(f.S, g, i, j, k, f.tau)) * rd};
-}
-
-// dT/dz at the top face of (i, j, k); 0 at the top level and below k = 0.
-__device__ __forceinline__ Grad grad_z(const Grid& g, const Fields& f, int i, int j, int k, double rd) {
-    if (k < 0 || k >= g.nz - 1) return {0.0, 0.0};
-    const int kb = kb_of(g, i, j);
-    const double m = mT(kb, k) * mT(kb, k + 1);
-    return {m * (tr3(f.T, g, i, j, k + 1, f.tau) - tr3(f.T, g, i, j, k, f.tau)) * rd,
-            m * (tr3(f.S, g, i, j, k + 1, f.tau) - tr3(f.S, g, i, j, k, f.tau)) * rd};
-}
 
 // exp(x) for |x| <= 64 by Cody-Waite reduction: x = n ln2 + r with ln2 split
 // into a 32-bit-exact high part and a low part, |r| <= ln2/2, e^r from its
@@ -796,10 +765,6 @@ struct StepArgs {
     const double* Kskew;
     const double *Aez, *Anz, *Abx, *Aby, *K11, *K22, *K33;
     double* P;            // P_diss_iso / P_diss_skew, nullable (energy branch off)
-};
-
-struct Strides {
-    uint32_t si, sj;
 };
 
 // K1 = K_iso - K_skew (east/north faces) and K2 = K_iso + K_skew (top faces)
@@ -1632,15 +1597,6 @@ dim3 cell_grid(int ni, int nj, dim3 blk) {
     const int64_t nstrips = (nj + sw - 1) / sw;
     return dim3((unsigned)((nstrips * ni * sb + 7) / 8 * 8));
 }
-
-}  // namespace
-}  // namespace vx
-
-
-
-namespace vx {
-namespace {
-
 
 #ifndef VX_STEP_COLS
 #define VX_STEP_COLS 32
