@@ -31,10 +31,13 @@ def create_water_masks(ks, nz):
     return land, water, edge
 
 
+_KBOT_KERNEL_LEVELS = 1 << 20  # the most levels vx_kbot_from_edge_mask takes
+
+
 def kbot_from_masks(water_mask, edge_mask):
     """kbot = (index of the edge cell) + 1, 0 where a column has no edge."""
     edge, _ = to_device(edge_mask)
-    if (edge.dtype == torch.bool and edge.dim() == 3 and edge.numel() > 0
+    if (edge.dtype == torch.bool and edge.dim() == 3 and edge.numel() > 0 and edge.shape[2] <= _KBOT_KERNEL_LEVELS
             and edge.device.index == torch.cuda.current_device()):
         edge = edge.contiguous()
         nx, ny, nz = edge.shape
