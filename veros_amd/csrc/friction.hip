@@ -63,9 +63,6 @@ __device__ inline Face face_of(int kb0, int kb1, int nz) {
     return f;
 }
 
-// x (h + l): x / y rounded once, for h = 1 / y and l = h (1 - h y), its rounding's rest.
-__device__ __forceinline__ double scaled(double x, double h, double l) { return fma(x, h, x * l); }
-
 // First wet level of a T column (nz: none).
 __device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
 
@@ -75,14 +72,15 @@ __device__ __forceinline__ int first_wet_level(int kb, int nz) { return kb >= 1 
 // the solution x1 and the tendency dm; the lane's segment of the face's dissipation
 // (:137-153, 189-201): fxa * (x1[k+1] - x1[k]) / dzw[k] * mask[k+1] * mask[k] times
 // (x0[k+1] - x0[k]) / dzw[k], x0 at tau and x1 at taup1, 0 on the top level. The
-// masks are 0 or 1, so the products are taken as selects. rzt, dtw, rzw2, rzw2l:
-// 1 / dzt, dt / dzw and 1 / dzw^2 with what its rounding cuts off, in LDS: the
-// dissipation is then rounded no more often than by the reference's divisions.
+// masks are 0 or 1, so the products are taken as selects. rzt, rztl, dtw, rzw2, rzw2l:
+// 1 / dzt, dt / dzw and 1 / dzw^2, the reciprocals with what their rounding cuts off,
+// in LDS: rows, tendency and dissipation are then rounded no more often than by the
+// reference's divisions.
 template <int S, int P>
 __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int nz, const double* __restrict__ rzt,
-                                          const double* __restrict__ dtw, const double* __restrict__ rzw2,
-                                          const double* __restrict__ rzw2l, int k0,
-                                          bool both, double rdt, const double (&fx)[S], const double (&x0)[S],
+                                          const double* __restrict__ rztl, const double* __restrict__ dtw,
+                                          const double* __restrict__ rzw2, const double* __restrict__ rzw2l, int k0,
+                                          bool both, const Recip& rdt, const double (&fx)[S], const double (&x0)[S],
                                           double (&x1)[S], double (&dm)[S], double (&ds)[S]) {
     double f[S], o[S], va[S], vb[S], vc[S], z[1][S];
     tile_put(t, img, fx);
@@ -97,11 +95,12 @@ __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int 
         const int k = t.lo + q;
         const bool wet = k >= k0 && k < nz;
         const int kc = k < nz ? k : nz - 1;
-        const double rz = rzt[kc];
+        const double rz = rzt[kc], rl = rztl[kc];
         const double dl = (both && wet && k < nz - 1) ? dtw[kc] * f[q] : 0.0;
-        va[q] = (wet && k != k0) ? -dlm * rz : 0.0;
-        vb[q] = wet ? (k == k0 ? 1 + dl * rz : (1 + dlm * rz) + dl * rz) : 1.0;
-        vc[q] = wet ? -dl * rz : 0.0;
+        const double below = scaled(dlm, rz, rl), above = scaled(dl, rz, rl);
+        va[q] = (wet && k != k0) ? -below : 0.0;
+        vb[q] = wet ? (k == k0 ? 1 + above : (1 + below) + above) : 1.0;
+        vc[q] = wet ? -above : 0.0;
         z[0][q] = wet ? o[q] : 0.0;
         dlm = dl;
     }
@@ -119,7 +118,7 @@ __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int 
     }
     tile_get(t, img, x1);
 #pragma unroll
-    for (int q = 0; q < S; ++q) z[0][q] = (z[0][q] - o[q]) * rdt;
+    for (int q = 0; q < S; ++q) z[0][q] = scaled(z[0][q] - o[q], rdt.h, rdt.l);
     seg_put(t, img, z[0]);
     tile_get(t, img, dm);
 }
@@ -163,13 +162,15 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
     constexpr int G = kFricGroups;
     __shared__ double work[2 * G][T::IMG];
     __shared__ double dsv[2][G][T::IMG];
-    __shared__ double sdz[4][kMaxNz];
+    __shared__ double sdz[5][kMaxNz];
     const int64_t b = xcd_contiguous_block();
     if (b >= nblocks) return;
     const int nz = p.nz;
     for (int k = threadIdx.x; k < nz; k += kFricBlock) {
         const double zw = p.dzw[k];
-        sdz[0][k] = 1.0 / p.dzt[k];
+        const Recip rzt = recip(p.dzt[k]);
+        sdz[0][k] = rzt.h;
+        sdz[4][k] = rzt.l;
         sdz[1][k] = p.dt / zw;
         const double sq = zw * zw, r = 1.0 / sq;
         sdz[2][k] = r;
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
     const int n = left >= T::C ? T::C : (left > 0 ? (int)left : 0);
     const int64_t next = vface ? 1 : p.Y;  // the face's other column
     const uint32_t cs = (uint32_t)p.cs;
-    const double rdt = 1.0 / p.dt;
+    const Recip rdt = recip(p.dt);
     double* const vel = p.vel[comp];
     T t = make_tile<S, P>(0, n, nz, (uint32_t)nz, rnz);
     const int64_t j = t.q < n ? j0 + t.q : (n > 0 ? j0 : 0);  // the lane's column
@@ -229,12 +230,12 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
                 tile_load(b0, below, cs, y0);
                 tile_load(b1, below, cs, dm);
 #pragma unroll
-                for (int r = 0; r < S; ++r) dm[r] = (dm[r] - y0[r]) * rdt;
+                for (int r = 0; r < S; ++r) dm[r] = scaled(dm[r] - y0[r], rdt.h, rdt.l);
                 tile_store(bd, below, 1, dm);
             }
 #pragma unroll
             for (int r = 0; r < S; ++r) fx[r] = 0.5 * (fx[r] + kn[r]);
-            fric_face<S, P>(t, img, nz, sdz[0], sdz[1], sdz[2], sdz[3], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
+            fric_face<S, P>(t, img, nz, sdz[0], sdz[4], sdz[1], sdz[2], sdz[3], f.k0, f.both, rdt, fx, x0, x1, kn, ds);
             if (vface) seg_put(t, dsv[i & 1][grp], ds);
             tile_store(b1, on, cs, x1);
             tile_store(bd, on, 1, kn);
@@ -245,11 +246,11 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         }
         double bu[S];
         {
-            const double wi = p.dxu[i], wm = p.dxu[i - 1], den = 2 * p.dxt[i], rden = 1.0 / den;
-            const double rdenl = rden * fma(-rden, den, 1.0);
+            const double wi = p.dxu[i], wm = p.dxu[i - 1];
+            const Recip rden = recip(2 * p.dxt[i]);
 #pragma unroll
             for (int r = 0; r < S; ++r) {
-                bu[r] = i >= 2 ? scaled(wi * ds[r] + wm * du[r], rden, rdenl) : ds[r];
+                bu[r] = i >= 2 ? scaled(wi * ds[r] + wm * du[r], rden.h, rden.l) : ds[r];
                 du[r] = ds[r];
             }
         }
@@ -257,7 +258,8 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         // K_diss_v and the weights are loaded before the barrier, which their
         // latency then overlaps
         const BufRsrc bK = tile_buf(t, p.K_diss_v);
-        double K[S], wj = 1.0, wjm = 0.0, rden = 1.0, rdenl = 0.0;
+        double K[S], wj = 1.0, wjm = 0.0;
+        Recip rden{1.0, 0.0};
         uint32_t ow[S];
         const int wc = jown ? first_wet_level(kb, nz) : nz;
 #pragma unroll
@@ -266,9 +268,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
         tile_load(bK, ow, 1, K);
         const bool south = jown && j >= 2;
         if (south) {
-            const double den = 2 * p.area_t[col];
-            rden = 1.0 / den;
-            rdenl = rden * fma(-rden, den, 1.0);
+            rden = recip(2 * p.area_t[col]);
             wj = p.area_v[col];
             wjm = p.area_v[col - 1];
         }
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kFricBlock) __attribute__((amdgpu_waves_per_eu(kFri
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             const double dn = vn[t.seg + r], dd = vs[t.seg + r];
-            bu[r] = bu[r] + (south ? scaled(wj * dn + wjm * dd, rden, rdenl) : dn);
+            bu[r] = bu[r] + (south ? scaled(wj * dn + wjm * dd, rden.h, rden.l) : dn);
         }
         seg_put(t, img, bu);
         tile_get(t, img, bu);

@@ -53,9 +53,10 @@ struct TurbCols {
 };
 
 // Level tables of a block: dd[k] = the diffusivity's factor in delta at level k
-// (0 on the top level), rz[k] = 1 / dzw (1 / (0.5 dzw) on the top level).
+// (0 on the top level), rz[k], rl[k] = 1 / dzw (1 / (0.5 dzw) on the top level) and its
+// rounding's rest, with which the rows round as with the reference's divisions.
 struct TurbLevels {
-    double dd[kMaxNz], rz[kMaxNz], zw[kMaxNz];
+    double dd[kMaxNz], rz[kMaxNz], rl[kMaxNz], zw[kMaxNz];
 };
 
 __device__ __forceinline__ int first_wet_of(int kb, int nz) { return kb >= 1 && kb <= nz ? kb - 1 : nz; }
@@ -104,7 +105,9 @@ __device__ __forceinline__ void turb_setup(const TurbGrid& g, const Tile<S, P>& 
     for (int k = threadIdx.x; k < nz; k += kTurbBlock) {
         const double dzw = g.dzw[k];
         lv.zw[k] = dzw;
-        lv.rz[k] = 1.0 / (k == nz - 1 ? 0.5 * dzw : dzw);
+        const Recip r = recip(k == nz - 1 ? 0.5 * dzw : dzw);
+        lv.rz[k] = r.h;
+        lv.rl[k] = r.l;
         lv.dd[k] = k < nz - 1 ? scale / g.dzt[k + 1] * 0.5 : 0.0;
     }
     if (lateral) {
@@ -248,10 +251,10 @@ __device__ __forceinline__ void turb_solve(const Tile<S, P>& t, const TurbLevels
             }
             C = -dk / zw * kn;
         } else {
-            const double rz = lv.rz[kc];
-            A = -dm * rz;
-            B = 1 + (dk + (edge ? 0.0 : dm)) * rz + vb[r];
-            C = -dk * rz;
+            const double rz = lv.rz[kc], rl = lv.rl[kc];
+            A = -scaled(dm, rz, rl);
+            B = 1 + scaled(dk + (edge ? 0.0 : dm), rz, rl) + vb[r];
+            C = -scaled(dk, rz, rl);
         }
         va[r] = wet && !edge ? A : 0.0;
         vb[r] = wet ? B : 1.0;
@@ -339,12 +342,12 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
     }
     {
         double x[S];
-        const double rtop = dt * sh.lv.rz[nz - 1];
+        const double ftop = scaled(dt * fsurf, sh.lv.rz[nz - 1], sh.lv.rl[nz - 1]);
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             x[r] = e0[r] + dt * f[r];
-            const double fs = __shfl(fsurf, t.c[r] * P);
-            if (t.k[r] == nz - 1) x[r] += rtop * fs;
+            const double fs = __shfl(ftop, t.c[r] * P);
+            if (t.k[r] == nz - 1) x[r] += fs;
         }
         tile_put(t, sh.img[wave][2], x);
     }
@@ -544,14 +547,14 @@ __global__ __launch_bounds__(kTurbBlock) __attribute__((amdgpu_waves_per_eu(VX_T
 #pragma unroll
         for (int r = 0; r < S; ++r) x[r] = dt * rate[r];
         tile_put(t, sh.img[wave][1], x);
-        const double rtop = dt * sh.lv.rz[nz - 1];
+        const double ftop = scaled(dt * fsurf, sh.lv.rz[nz - 1], sh.lv.rl[nz - 1]);
 #pragma unroll
         for (int r = 0; r < S; ++r) {
             x[r] = e0[r] + dt * f[r];
             const bool edge = t.k[r] == __shfl(l.k0, t.c[r] * P);
-            const double fb = __shfl(fbot, t.c[r] * P), fs = __shfl(fsurf, t.c[r] * P);
+            const double fb = __shfl(fbot, t.c[r] * P), fs = __shfl(ftop, t.c[r] * P);
             if (edge) x[r] += dt * fb / sh.lv.zw[t.k[r]];  // d_edge (:157-159)
-            else if (t.k[r] == nz - 1) x[r] += rtop * fs;
+            else if (t.k[r] == nz - 1) x[r] += fs;
         }
         tile_put(t, sh.img[wave][2], x);
     }

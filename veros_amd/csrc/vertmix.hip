@@ -35,13 +35,15 @@ struct VmixArgs {
     int64_t cs, ls;
 };
 
-// 1 / dzt (s[0, nz)) and dt / dzw (s[kMaxNz, kMaxNz + nz)) in LDS; every thread
-// of the block calls it. The rows read them inside per-level selects, where a
-// global load is waited for at once, level after level.
+// 1 / dzt (s[0, nz)), the rest of its rounding (from kMaxNz on) and dt / dzw (from
+// 2 kMaxNz on) in LDS; every thread of the block calls it. The rows read them
+// inside per-level selects, where a global load is waited for at once, level after level.
 __device__ __forceinline__ void vmix_stage_dz(const VmixArgs& p, double* s) {
     for (int k = threadIdx.x; k < p.nz; k += blockDim.x) {
-        s[k] = 1.0 / p.dzt[k];
-        s[kMaxNz + k] = p.dt / p.dzw[k];
+        const Recip r = recip(p.dzt[k]);
+        s[k] = r.h;
+        s[kMaxNz + k] = r.l;
+        s[2 * kMaxNz + k] = p.dt / p.dzw[k];
     }
     __syncthreads();
 }
@@ -49,12 +51,13 @@ __device__ __forceinline__ void vmix_stage_dz(const VmixArgs& p, double* s) {
 // The rows of the lane's levels (veros/core/thermodynamics.py:267-277),
 // identity rows off the wet suffix; z1, z2 get the surface forcing on the top
 // level. KM(k) is kappaH at level k of the column, for k in [lo-1, lo+S); its
-// value matters for k0 <= k < nz-1 only. rzt, dtw: 1 / dzt and dt / dzw (in LDS).
+// value matters for k0 <= k < nz-1 only. rzt, rztl, dtw: 1 / dzt with its rest and
+// dt / dzw (in LDS): every entry rounds as with the reference's divisions.
 template <int S, class KMF>
 __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __restrict__ rzt,
-                                          const double* __restrict__ dtw, const SegLane& L, KMF KM, double fT, double fS,
-                                          double (&va)[S], double (&vb)[S], double (&vc)[S], double (&z1)[S],
-                                          double (&z2)[S]) {
+                                          const double* __restrict__ rztl, const double* __restrict__ dtw,
+                                          const SegLane& L, KMF KM, double fT, double fS, double (&va)[S],
+                                          double (&vb)[S], double (&vc)[S], double (&z1)[S], double (&z2)[S]) {
     const int nz = p.nz;
     const double dt = p.dt;
     const int kp = L.lo - 1;  // delta at the level below the segment
@@ -64,15 +67,15 @@ __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __res
         const int k = L.lo + t;
         const bool wet = k >= L.k0 && k < nz;
         const int kc = k < nz ? k : nz - 1;
-        const double rz = rzt[kc];
+        const double rz = rzt[kc], rl = rztl[kc];
         const double dl = (wet && k < nz - 1) ? dtw[kc] * KM(k) : 0.0;
         const bool edge = k == L.k0;
-        va[t] = (wet && !edge) ? -dlm * rz : 0.0;
-        vb[t] = wet ? (edge ? 1 + dl * rz : 1 + (dl + dlm) * rz) : 1.0;
-        vc[t] = (wet && k < nz - 1) ? -dl * rz : 0.0;
+        va[t] = (wet && !edge) ? -scaled(dlm, rz, rl) : 0.0;
+        vb[t] = wet ? 1 + scaled(edge ? dl : dl + dlm, rz, rl) : 1.0;
+        vc[t] = (wet && k < nz - 1) ? -scaled(dl, rz, rl) : 0.0;
         if (k == nz - 1) {  // surface forcing (:277, :284)
-            z1[t] = z1[t] + dt * fT * rz;
-            z2[t] = z2[t] + dt * fS * rz;
+            z1[t] = z1[t] + scaled(dt * fT, rz, rl);
+            z2[t] = z2[t] + scaled(dt * fS, rz, rl);
         }
         z1[t] = wet ? z1[t] : 0.0;
         z2[t] = wet ? z2[t] : 0.0;
@@ -89,7 +92,7 @@ constexpr int kVmixBlock = 128;
 template <int S, int P>
 __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, uint32_t rnz) {
     using T = Tile<S, P>;
-    __shared__ double sdz[2 * kMaxNz];
+    __shared__ double sdz[3 * kMaxNz];
     __shared__ double lds[kVmixBlock / 64][T::IMG];
     vmix_stage_dz(p, sdz);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), nz = p.nz;
@@ -137,7 +140,8 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
         seg_get(t, img, z[0]);
         tile_put(t, img, oS);
         seg_get(t, img, z[1]);
-        vmix_rows<S>(p, sdz, sdz + kMaxNz, L, [&](int k) { return km[k - L.lo + 1]; }, fT, fS, va, vb, vc, z[0], z[1]);
+        vmix_rows<S>(p, sdz, sdz + kMaxNz, sdz + 2 * kMaxNz, L, [&](int k) { return km[k - L.lo + 1]; }, fT, fS, va, vb, vc,
+                     z[0], z[1]);
         col_solve<S, 2>(t, va, vb, vc, z);
         seg_put(t, img, z[0]);
         tile_get(t, img, nT);
@@ -145,11 +149,11 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
         tile_get(t, img, nS);
         tile_store(bT, wet, cs, nT);
         tile_store(bS, wet, cs, nS);
-        const double rdt = 1.0 / p.dt;
+        const Recip rdt = recip(p.dt);
 #pragma unroll
         for (int r = 0; r < S; ++r) {  // (new - old) / dt; 0 where unchanged
-            nT[r] = wet[r] != kNoAccess ? (nT[r] - oT[r]) * rdt : 0.0;
-            nS[r] = wet[r] != kNoAccess ? (nS[r] - oS[r]) * rdt : 0.0;
+            nT[r] = wet[r] != kNoAccess ? scaled(nT[r] - oT[r], rdt.h, rdt.l) : 0.0;
+            nS[r] = wet[r] != kNoAccess ? scaled(nS[r] - oS[r], rdt.h, rdt.l) : 0.0;
         }
     }
     tile_store(tile_buf(t, p.dvmix[0]), t.off, 1, nT);
