@@ -209,13 +209,17 @@ __device__ __forceinline__ double tile_rhs_step(double R, double al, double ga) 
 // of iterative refinement (the rows' float64 residual, solved with the same
 // factors). With eight lanes (iface_solve) only columns with a weakly dominant row
 // need the step; the fourth stride's roundings make up for it on every column.
-// Root mean square error of friction and energy columns of 34 to 128 levels
-// against extended precision, in units of that of a sequential sweep: eight lanes
-// 1.11 to 1.21, sixteen lanes 1.16 to 1.32 with the step on weak columns only,
-// 1.10 to 1.14 with it on all of them and the sum of tile_solve.
-template <int NR>
-__device__ __forceinline__ void tile_iface(int s, double A, double B, double C, const double (&R)[NR],
-                                           double (&Ls)[NR], double (&Lm)[NR]) {
+// The residual starts with R - B x, whose terms cancel, and REST: takes in what the
+// forming of B and R cut off (Bl, Rl), so that a strongly dominant row's level is
+// rounded about once; it is one level in nz / 16. Mean error of columns of 34 to 113
+// levels against extended precision, in units of that of a sequential sweep, with the
+// residual summed first and without Bl, Rl / now: temperature 1.02 to 1.07 / 0.86 to
+// 1.00, velocity 1.05 to 1.12 / 0.93 to 1.07, energies 1.04 to 1.07 / 0.91 to 1.04. The
+// same from the interface level's own row after the solve keeps ten registers more:
+// vertical mixing and friction on 1440x720x80 2.26 -> 2.72 ms, now 2.27.
+template <int NR, bool REST>
+__device__ __forceinline__ void tile_iface(int s, double A, double B, double Bl, double C, const double (&R)[NR],
+                                           const double (&Rl)[NR], double (&Ls)[NR], double (&Lm)[NR]) {
     double a = A, b = B, c = C, al[4], ga[4];
 #pragma unroll
     for (int q = 0; q < NR; ++q) Ls[q] = R[q];
@@ -227,7 +231,10 @@ __device__ __forceinline__ void tile_iface(int s, double A, double B, double C, 
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
         Ls[q] *= rb;
-        double r = R[q] - (A * dpp_move<kDppShr + 1>(Ls[q]) + B * Ls[q] + C * dpp_move<kDppShl + 1>(Ls[q]));
+        double r = fma(-B, Ls[q], R[q]);
+        if constexpr (REST) r += fma(-Bl, Ls[q], Rl[q]);
+        r = fma(-A, dpp_move<kDppShr + 1>(Ls[q]), r);
+        r = fma(-C, dpp_move<kDppShl + 1>(Ls[q]), r);
         r = tile_rhs_step<1>(r, al[0], ga[0]);
         r = tile_rhs_step<2>(r, al[1], ga[1]);
         r = tile_rhs_step<4>(r, al[2], ga[2]);
@@ -238,8 +245,10 @@ __device__ __forceinline__ void tile_iface(int s, double A, double B, double C, 
 }
 
 // NR right-hand sides of one matrix; z in, their solutions out. va and vc are
-// overwritten by the sweep's factors (see seg_solve_f64).
-template <int S, int NR>
+// overwritten by the sweep's factors (see seg_solve_f64). REST: see tile_iface (off for
+// IDEMIX, whose rows' conditioning sets the error: 0.2% of it, and its four registers
+// cost a wave at three levels per lane, 600x400x40 597 -> 610 us for the three models).
+template <int S, int NR, bool REST>
 __device__ __forceinline__ void tile_solve(const Tile<S>& t, double (&va)[S], const double (&vb)[S], double (&vc)[S],
                                            double (&z)[NR][S]) {
     const double aL = va[S - 1], bL = vb[S - 1], cL = vc[S - 1];
@@ -269,13 +278,18 @@ __device__ __forceinline__ void tile_solve(const Tile<S>& t, double (&va)[S], co
         va[i] = -va[i] - cp * va[i + 1];
         vc[i] = -cp * vc[i + 1];
     }
-    const double RA = aL * va[S - 2];
-    const double RB = bL + aL * vc[S - 2] + cL * dpp_move<kDppShl + 1>(va[0]);
+    const double RA = aL * va[S - 2], nb = dpp_move<kDppShl + 1>(va[0]);
+    const double RB = fma(cL, nb, fma(aL, vc[S - 2], bL));
+    const double RBl = fma(cL, nb, fma(aL, vc[S - 2], bL - RB));
     const double RC = cL * dpp_move<kDppShl + 1>(vc[0]);
-    double RD[NR], Ls[NR], Lm[NR];
+    double RD[NR], RDl[NR], Ls[NR], Lm[NR];
 #pragma unroll
-    for (int q = 0; q < NR; ++q) RD[q] = z[q][S - 1] - aL * z[q][S - 2] - cL * dpp_move<kDppShl + 1>(z[q][0]);
-    tile_iface<NR>(t.s, RA, RB, RC, RD, Ls, Lm);
+    for (int q = 0; q < NR; ++q) {
+        const double na = dpp_move<kDppShl + 1>(z[q][0]);
+        RD[q] = fma(-cL, na, fma(-aL, z[q][S - 2], z[q][S - 1]));
+        RDl[q] = fma(-cL, na, fma(-aL, z[q][S - 2], z[q][S - 1] - RD[q]));
+    }
+    tile_iface<NR, REST>(t.s, RA, RB, RBl, RC, RD, RDl, Ls, Lm);
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
 #pragma unroll
@@ -286,11 +300,11 @@ __device__ __forceinline__ void tile_solve(const Tile<S>& t, double (&va)[S], co
 
 // The same with P lanes per column: kTileP as above, or kSegP by the
 // elimination of tdma_seg.hpp.
-template <int S, int NR, int P>
+template <int S, int NR, bool REST = true, int P>
 __device__ __forceinline__ void col_solve(const Tile<S, P>& t, double (&va)[S], const double (&vb)[S], double (&vc)[S],
                                           double (&z)[NR][S]) {
     if constexpr (P == kTileP) {
-        tile_solve<S, NR>(t, va, vb, vc, z);
+        tile_solve<S, NR, REST>(t, va, vb, vc, z);
     } else {
         SegLane L;
         L.s = t.s;

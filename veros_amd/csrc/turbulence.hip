@@ -262,7 +262,7 @@ __device__ __forceinline__ void turb_solve(const Tile<S, P>& t, const TurbLevels
         z[0][r] = wet ? z[0][r] : 0.0;
         dm = dk;
     }
-    col_solve<S, 1>(t, va, vb, vc, z);
+    col_solve<S, 1, !MUL>(t, va, vb, vc, z);
     seg_put(t, rhs, z[0]);
 }
 

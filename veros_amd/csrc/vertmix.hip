@@ -49,17 +49,15 @@ __device__ __forceinline__ void vmix_stage_dz(const VmixArgs& p, double* s) {
 }
 
 // The rows of the lane's levels (veros/core/thermodynamics.py:267-277),
-// identity rows off the wet suffix; z1, z2 get the surface forcing on the top
-// level. KM(k) is kappaH at level k of the column, for k in [lo-1, lo+S); its
-// value matters for k0 <= k < nz-1 only. rzt, rztl, dtw: 1 / dzt with its rest and
-// dt / dzw (in LDS): every entry rounds as with the reference's divisions.
+// identity rows off the wet suffix. KM(k) is kappaH at level k of the column, for
+// k in [lo-1, lo+S); its value matters for k0 <= k < nz-1 only. rzt, rztl, dtw:
+// 1 / dzt with its rest and dt / dzw (in LDS): every entry rounds as with the
+// reference's divisions.
 template <int S, class KMF>
 __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __restrict__ rzt,
                                           const double* __restrict__ rztl, const double* __restrict__ dtw,
-                                          const SegLane& L, KMF KM, double fT, double fS, double (&va)[S],
-                                          double (&vb)[S], double (&vc)[S], double (&z1)[S], double (&z2)[S]) {
+                                          const SegLane& L, KMF KM, double (&va)[S], double (&vb)[S], double (&vc)[S]) {
     const int nz = p.nz;
-    const double dt = p.dt;
     const int kp = L.lo - 1;  // delta at the level below the segment
     double dlm = (kp >= L.k0 && kp < nz - 1) ? dtw[kp > 0 ? kp : 0] * KM(kp) : 0.0;
 #pragma unroll
@@ -73,12 +71,6 @@ __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __res
         va[t] = (wet && !edge) ? -scaled(dlm, rz, rl) : 0.0;
         vb[t] = wet ? 1 + scaled(edge ? dl : dl + dlm, rz, rl) : 1.0;
         vc[t] = (wet && k < nz - 1) ? -scaled(dl, rz, rl) : 0.0;
-        if (k == nz - 1) {  // surface forcing (:277, :284)
-            z1[t] = z1[t] + scaled(dt * fT, rz, rl);
-            z2[t] = z2[t] + scaled(dt * fS, rz, rl);
-        }
-        z1[t] = wet ? z1[t] : 0.0;
-        z2[t] = wet ? z2[t] : 0.0;
         dlm = dl;
     }
 }
@@ -123,6 +115,20 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
         wet[r] = t.k[r] >= __shfl(L.k0, t.c[r] * P) ? t.off[r] : kNoAccess;
         nT[r] = nS[r] = 0.0;
     }
+    // a tracer's right-hand sides: its old values and the surface forcing (:277, :284)
+    auto rhs = [&](const double(&old)[S], double forc, double(&z)[S]) {
+        const double ftop = scaled(p.dt * forc, sdz[nz - 1], sdz[kMaxNz + nz - 1]);
+        double x[S];
+#pragma unroll
+        for (int r = 0; r < S; ++r) {
+            const double f = __shfl(ftop, t.c[r] * P);
+            x[r] = t.k[r] == nz - 1 ? old[r] + f : old[r];
+        }
+        tile_put(t, img, x);
+        seg_get(t, img, z);
+#pragma unroll
+        for (int r = 0; r < S; ++r) z[r] = L.lo + r >= L.k0 && L.lo + r < nz ? z[r] : 0.0;
+    };
     if (__any(L.k0 < nz)) {
         double km[S + 1], va[S], vb[S], vc[S], z[2][S];
         {
@@ -136,12 +142,9 @@ __global__ __launch_bounds__(kVmixBlock) void vertmix_tile_kernel(VmixArgs p, ui
 #pragma unroll
             for (int r = 0; r < S; ++r) km[r + 1] = kv[r];
         }
-        tile_put(t, img, oT);
-        seg_get(t, img, z[0]);
-        tile_put(t, img, oS);
-        seg_get(t, img, z[1]);
-        vmix_rows<S>(p, sdz, sdz + kMaxNz, sdz + 2 * kMaxNz, L, [&](int k) { return km[k - L.lo + 1]; }, fT, fS, va, vb, vc,
-                     z[0], z[1]);
+        vmix_rows<S>(p, sdz, sdz + kMaxNz, sdz + 2 * kMaxNz, L, [&](int k) { return km[k - L.lo + 1]; }, va, vb, vc);
+        rhs(oT, fT, z[0]);
+        rhs(oS, fS, z[1]);
         col_solve<S, 2>(t, va, vb, vc, z);
         seg_put(t, img, z[0]);
         tile_get(t, img, nT);
