@@ -146,23 +146,14 @@ __device__ __forceinline__ double rden(double drodz) { return rcp_nr(fmin(0.0, d
 #define VX_STRIP_BLOCKS 16
 #endif
 constexpr int kStripBlocks = VX_STRIP_BLOCKS;
-// the pre and flux kernels' strips: columns along j (the fused call on
-// 1440x720x80 and the calls on 360x160x60, levels innermost: 96 columns
-// 6.00 ms and 1176 us, 192 6.05 and 1157, 384 6.09 and 1167)
+// the pre and flux kernels' strips: at most so many columns along j (strip_blocks; the
+// fused call on 1440x720x80, on 300x200x128 and the calls on 360x160x60, the last two
+// with the levels innermost: 64 columns 6.04 ms, 773 and 958 us, 96 5.97, 752 and 966,
+// 192 5.87, 737 and 956, 256 5.98, 735 and 955)
 #ifndef VX_PRE_STRIP_COLS
 #define VX_PRE_STRIP_COLS 192
 #endif
 constexpr int kPreStripCols = VX_PRE_STRIP_COLS;
-
-// Blocks of ncb columns in a strip of about `cols` columns; as many as a row of nj
-// columns needs where more than a quarter of the strip would be padding. The fused
-// call with whole strips / with shortened ones, us: 4000x2x40 241 / 59, 20000x3x80
-// 1328 / 542, 1200x7x60 107 / 65, 2000x20x50 213 / 206; where an eighth is padding the
-// shortened strip is no faster (calls on 360x160x60 914 / 921).
-__host__ __device__ __forceinline__ int strip_blocks(int cols, int ncb, int nj) {
-    const int most = (nj + ncb - 1) / ncb, sb = cols / ncb;
-    return 4 * most < 3 * sb ? most : sb;
-}
 
 struct CellIdx {
     int i, j, k;

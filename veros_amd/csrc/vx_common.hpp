@@ -42,6 +42,19 @@ constexpr int kMaxNz = 128;
 // per device.
 int cu_count();
 
+// Blocks of ncb columns in a strip, where a row of nj columns is cut into equal strips of
+// at most `cols` columns (one block at least). Equal, since every block of the last strip
+// that lies past the row is padding, and the blocks of a strip go to neighbouring XCDs: with
+// full strips of 192 and the rest in a narrow one, half of the XCDs had next to nothing
+// to do on 200 columns. The isoneutral call there, nz 128, levels innermost, 946 -> 737 us;
+// 700x400x9 407 -> 369, 400x400x60 1045 -> 956; rows shorter than a strip take one of their
+// own width (4000x2x40 241 -> 64).
+__host__ __device__ __forceinline__ int strip_blocks(int cols, int ncb, int nj) {
+    const int row = (nj + ncb - 1) / ncb, most = cols > ncb ? cols / ncb : 1;
+    const int nstrips = (row + most - 1) / most;
+    return (row + nstrips - 1) / nstrips;
+}
+
 // Blocks are dispatched round-robin over the 8 XCDs, each with its own L2.
 // With gridDim.x a multiple of 8 this gives block b the index of the
 // (b / 8)-th block of the x-th eighth of the grid (x = b % 8), so that each
