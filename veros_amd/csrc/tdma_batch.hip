@@ -29,25 +29,36 @@ struct SysDesc {
     TdmaArgs args;
     TdmaTiling tiling;
     int64_t tile0;  // first tile of this system in its bucket
+    int32_t vec;    // its arrays allow 16-byte copies into LDS
 };
 
+// How a bucket's systems are solved: on flat loads (tdma_tile.hpp; any depth, alignment and
+// strides), with 16-byte copies straight into LDS, or each as its arrays allow.
+enum BatchKind { kFlat = 0, kCopies = 1, kEither = 2 };
+
+// Whether a bucket whose systems allow the copies in part takes them system by system, the
+// others with each lane's own loads: where the copies win at any size (tdma_lds_wins) by more than
+// those loads lose, if at least half of the columns allow them. Six systems of 300x200, one off
+// alignment, all on flat loads / by system, us, float64 and mixed: nz 80 165 and 182 / 163 and 164,
+// 96 224 and 224 / 209 and 212; four of 60x50: 8.5 and 8.3 / 8.1, 9.7 and 9.5 / 9.1 and 9.0. On flat
+// loads throughout, where by system took (300x200): nz 48 98 / 101, 64 125 / 140, 112 257 and 313 / 306
+// and 308, 128 278 and 300 / 367 and 380.
+__host__ __device__ constexpr bool batch_either(int S) { return S == 10 || S == 12; }
+
 // LDS doubles of a wave
-template <int S, bool LDSV>
+template <int S, int KIND>
 __host__ __device__ constexpr int batch_lds() {
-    return LDSV ? seg_lds_wave_bytes(S) / 8 : tdma_tile_lds<S>();
+    return KIND == kFlat ? tdma_tile_lds<S>() : seg_lds_wave_bytes(S) / 8;
 }
 
 // One launch per bucket: S levels per lane, MODE -1 = float64, else mixed with
-// MODE refinement steps. LDSV: every system of the bucket allows 16-byte copies
-// straight into LDS and those are faster (tdma_lds_wins); else the flat loads of
-// tdma_tile.hpp (odd depths, any alignment or strides), at S = 2 each lane's own
-// levels (tdma_own_levels), as at every S before, in kernels that held the LDS of
-// the copies.
-template <int S, int MODE, bool LDSV>
+// MODE refinement steps. On flat loads at S = 2 each lane loads its own levels
+// (tdma_own_levels).
+template <int S, int MODE, int KIND>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void tdma_seg_batch_kernel(const SysDesc* __restrict__ sys, int nsys,
                                                              int64_t ntiles) {
     extern __shared__ double seg_lds[];
-    double* lds = seg_lds + (threadIdx.x / 64) * batch_lds<S, LDSV>();
+    double* lds = seg_lds + (threadIdx.x / 64) * batch_lds<S, KIND>();
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x / 64);
     // the tile index is the same in every lane of a wave: keep it (and so
     // the system search and descriptor loads) in scalar registers
@@ -64,22 +75,25 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void t
         const TdmaArgs p = sd.args;
         SegLane L;
         const Tile<S, kTdmaP> t = tdma_tile_of<S>(p, sd.tiling, w - sd.tile0, L);
-        if constexpr (LDSV) {
-            double va[S], vb[S], vc[S], vd[S];
-            seg_rows_lds<S>(p, L, lds, va, vb, vc, vd);
-            if constexpr (MODE < 0) {
-                seg_solve_f64<S>(L, va, vb, vc, vd);
-                seg_store_lds<S>(p, L, lds, vd);
-            } else {
-                double x[S];
-                seg_mixed_core<S, MODE>(L, va, vb, vc, vd, x);
-                seg_store_lds<S>(p, L, lds, x);
-            }
-        } else if constexpr (tdma_own_levels(S)) {
+        if constexpr (KIND == kFlat && tdma_own_levels(S)) {
             if constexpr (MODE < 0) seg_f64<S, false>(p, L);
             else seg_mixed<S, false, MODE>(p, L);
-        } else {
+        } else if constexpr (KIND == kFlat) {
             tdma_tile<S, MODE>(p, t, L, lds);
+        } else {
+            const bool copies = KIND == kCopies || sd.vec;
+            double va[S], vb[S], vc[S], vd[S], x[S];
+            if (copies) seg_rows_lds<S>(p, L, lds, va, vb, vc, vd);
+            else seg_rows<S, false>(p, L, va, vb, vc, vd);
+            if constexpr (MODE < 0) {
+                seg_solve_f64<S>(L, va, vb, vc, vd);
+#pragma unroll
+                for (int q = 0; q < S; ++q) x[q] = vd[q];
+            } else {
+                seg_mixed_core<S, MODE>(L, va, vb, vc, vd, x);
+            }
+            if (copies) seg_store_lds<S>(p, L, lds, x);
+            else if (L.valid) seg_store<S, false>(p.x + L.base, L.lo, p.nz, x);
         }
     }
 }
@@ -97,13 +111,13 @@ struct Bucket {
     int nsys = 0;
     int64_t tiles = 0;   // tiles of up to 8 columns
     int64_t cols = 0;    // columns
-    bool lds = true;     // solved by the kernel with 16-byte copies into LDS (else on flat loads)
+    int kind = kFlat;    // BatchKind
     int bs = 128;
     int factor = 0;
 };
 
-// nzb, mode, kernel (Bucket::lds: its LDS and registers differ from the other's), log2(columns), CUs
-using TuneKey = std::tuple<int, int, bool, int, int>;
+// nzb, mode, kind (each has other LDS and registers), log2(columns), CUs
+using TuneKey = std::tuple<int, int, int, int, int>;
 std::mutex g_tune_mutex;
 std::map<TuneKey, std::pair<int, int>> g_tune_cache;
 
@@ -117,31 +131,34 @@ int ilog2(int64_t v) {
 }
 
 TuneKey tune_key(const Bucket& b, int mode, int num_cu) {
-    return {b.nzb, mode, b.lds, ilog2(b.tiles * kSegCols), num_cu};
+    return {b.nzb, mode, b.kind, ilog2(b.tiles * kSegCols), num_cu};
 }
 
+template <int S, int MODE, int KIND>
+void launch_kind(int bs, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+    const size_t lds = (size_t)batch_lds<S, KIND>() * 8 * (bs / 64);
+    hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, KIND>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
+}
 template <int S, int MODE>
-void launch_bs(int bs, bool use_lds, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
-    if (use_lds) {
-        const size_t lds = (size_t)batch_lds<S, true>() * 8 * (bs / 64);
-        hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, true>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
-        return;
+void launch_bs(int bs, int kind, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+    if constexpr (batch_either(S)) {
+        if (kind == kEither) return launch_kind<S, MODE, kEither>(bs, d, nsys, tiles, grid, s);
     }
-    const size_t lds = (size_t)batch_lds<S, false>() * 8 * (bs / 64);
-    hipLaunchKernelGGL((tdma_seg_batch_kernel<S, MODE, false>), dim3(grid), dim3(bs), lds, s, d, nsys, tiles);
+    if (kind == kCopies) launch_kind<S, MODE, kCopies>(bs, d, nsys, tiles, grid, s);
+    else launch_kind<S, MODE, kFlat>(bs, d, nsys, tiles, grid, s);
 }
 
 template <int MODE>
-void launch_mode(int nzb, int bs, bool lds, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
+void launch_mode(int nzb, int bs, int kind, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
     switch (nzb) {
-        case 16: launch_bs<2, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 32: launch_bs<4, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 48: launch_bs<6, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 64: launch_bs<8, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 80: launch_bs<10, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 96: launch_bs<12, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        case 112: launch_bs<14, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
-        default: launch_bs<16, MODE>(bs, lds, d, nsys, tiles, grid, s); break;
+        case 16: launch_bs<2, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 32: launch_bs<4, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 48: launch_bs<6, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 64: launch_bs<8, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 80: launch_bs<10, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 96: launch_bs<12, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        case 112: launch_bs<14, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
+        default: launch_bs<16, MODE>(bs, kind, d, nsys, tiles, grid, s); break;
     }
 }
 
@@ -172,8 +189,8 @@ unsigned grid_for(const vx_tdma_plan* P, const Bucket& b, int bs, int factor) {
 void launch_bucket(const vx_tdma_plan* P, const Bucket& b, int bs, int factor, hipStream_t s) {
     const SysDesc* d = P->d_sys + b.first;
     const unsigned grid = grid_for(P, b, bs, factor);
-    if (P->mode == 0) launch_mode<-1>(b.nzb, bs, b.lds, d, b.nsys, b.tiles, grid, s);
-    else launch_mode<1>(b.nzb, bs, b.lds, d, b.nsys, b.tiles, grid, s);
+    if (P->mode == 0) launch_mode<-1>(b.nzb, bs, b.kind, d, b.nsys, b.tiles, grid, s);
+    else launch_mode<1>(b.nzb, bs, b.kind, d, b.nsys, b.tiles, grid, s);
 }
 
 }  // namespace
@@ -226,16 +243,21 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
         b.nzb = kBuckets[bk];
         b.first = (int)table.size();
         b.nsys = (int)per[bk].size();
+        int64_t vec_tiles = 0;
         for (SysDesc& sd : per[bk]) {
             sd.tiling = tdma_tiling(sd.args);
             sd.tile0 = b.tiles;
             b.tiles += sd.tiling.ntiles;
             b.cols += sd.args.ncol;
-            b.lds = b.lds && tdma_vec_ok(sd.args);
+            sd.vec = tdma_vec_ok(sd.args) ? 1 : 0;
+            vec_tiles += sd.vec ? sd.tiling.ntiles : 0;
             table.push_back(sd);
         }
         const int S = b.nzb / kTdmaP;
-        b.lds = b.lds && (tdma_lds_wins(S, mode != 0, true) || tdma_lds_resident(S, b.tiles));
+        if (vec_tiles == b.tiles && (tdma_lds_wins(S, mode != 0, true) || tdma_lds_resident(S, b.tiles)))
+            b.kind = kCopies;
+        else if (vec_tiles < b.tiles && 2 * vec_tiles >= b.tiles && batch_either(S))
+            b.kind = kEither;
         {
             std::lock_guard<std::mutex> lk(g_tune_mutex);
             auto it = g_tune_cache.find(tune_key(b, mode, P->num_cu));
