@@ -37,13 +37,14 @@ struct SysDesc {
 enum BatchKind { kFlat = 0, kCopies = 1, kEither = 2 };
 
 // Whether a bucket whose systems allow the copies in part takes them system by system, the
-// others with each lane's own loads: where the copies win at any size (tdma_lds_wins) by more than
-// those loads lose, if at least half of the columns allow them. Six systems of 300x200, one off
-// alignment, all on flat loads / by system, us, float64 and mixed: nz 80 165 and 182 / 163 and 164,
-// 96 224 and 224 / 209 and 212; four of 60x50: 8.5 and 8.3 / 8.1, 9.7 and 9.5 / 9.1 and 9.0. On flat
-// loads throughout, where by system took (300x200): nz 48 98 / 101, 64 125 / 140, 112 257 and 313 / 306
-// and 308, 128 278 and 300 / 367 and 380.
-__host__ __device__ constexpr bool batch_either(int S) { return S == 10 || S == 12; }
+// others with each lane's own loads, if at least half of the columns allow them: at 10 and
+// 12 levels per lane, where the copies win at any size (tdma_lds_wins) by more than those loads lose,
+// and up to 8 while all tiles are resident. Six systems of 300x200, one off alignment, all on
+// flat loads / by system, us, float64 and mixed: nz 80 165 and 182 / 163 and 164, 96 224 and 224 / 209
+// and 212, but 48 98 / 101, 64 125 / 140, 112 257 and 313 / 306 and 308, 128 278 and 300 / 367 and
+// 380. 22 systems of up to 66x66 and 18 to 85 levels: 30.4 / 30.0 and 29.7 / 29.3, with no
+// division before the loads (tdma_tile_of) 29.4 and 29.4.
+inline bool batch_either(int S, int64_t tiles) { return S == 10 || S == 12 || (S <= 8 && tdma_lds_resident(S, tiles)); }
 
 // LDS doubles of a wave
 template <int S, int KIND>
@@ -141,7 +142,7 @@ void launch_kind(int bs, const SysDesc* d, int nsys, int64_t tiles, unsigned gri
 }
 template <int S, int MODE>
 void launch_bs(int bs, int kind, const SysDesc* d, int nsys, int64_t tiles, unsigned grid, hipStream_t s) {
-    if constexpr (batch_either(S)) {
+    if constexpr (S <= 12) {
         if (kind == kEither) return launch_kind<S, MODE, kEither>(bs, d, nsys, tiles, grid, s);
     }
     if (kind == kCopies) launch_kind<S, MODE, kCopies>(bs, d, nsys, tiles, grid, s);
@@ -256,7 +257,7 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
         const int S = b.nzb / kTdmaP;
         if (vec_tiles == b.tiles && (tdma_lds_wins(S, mode != 0, true) || tdma_lds_resident(S, b.tiles)))
             b.kind = kCopies;
-        else if (vec_tiles < b.tiles && 2 * vec_tiles >= b.tiles && batch_either(S))
+        else if (vec_tiles < b.tiles && 2 * vec_tiles >= b.tiles && batch_either(S, b.tiles))
             b.kind = kEither;
         {
             std::lock_guard<std::mutex> lk(g_tune_mutex);

@@ -41,7 +41,7 @@ inline TdmaTiling tdma_tiling(const TdmaArgs& p) {
 template <int S>
 __device__ __forceinline__ Tile<S, kTdmaP> tdma_tile_of(const TdmaArgs& p, const TdmaTiling& g, int64_t w, SegLane& L) {
     const bool in = w < g.ntiles;
-    const int64_t i = in ? w / g.tpr : 0;
+    const int64_t i = in && w >= g.tpr ? w / g.tpr : 0;  // columns in one row: no division in the chain to the loads
     const int64_t j0 = in ? (w - i * g.tpr) * g.cpt : 0;
     const int64_t left = g.ny - j0;
     const int n = in ? (int)(left < g.cpt ? left : g.cpt) : 0;
