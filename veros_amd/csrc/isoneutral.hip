@@ -213,7 +213,8 @@ struct ColMetrics {
 struct LevelMetrics {
     double rzw[kMaxNz];   // 1 / dzw
     double dzw[kMaxNz];
-    double r4zt[kMaxNz];  // 1 / (4 dzt)
+    double r4zt[kMaxNz];   // 1 / (4 dzt)
+    double r4ztl[kMaxNz];  // what its rounding cuts off: K_11 and K_22 round as when divided
 };
 constexpr int kCellBlock = 64;  // threads of a pre or flux block: one wave
 constexpr int kBlockCols = 32;  // most columns of one
@@ -251,7 +252,9 @@ __device__ __forceinline__ void fill_metrics(const Grid& g, int i, int jb, int n
         const double dzw = g.dzw[k];
         m.lev.dzw[k] = dzw;
         m.lev.rzw[k] = 1.0 / dzw;
-        m.lev.r4zt[k] = 1.0 / (4.0 * g.dzt[k]);
+        const Recip r4zt = recip(4.0 * g.dzt[k]);
+        m.lev.r4zt[k] = r4zt.h;
+        m.lev.r4ztl[k] = r4zt.l;
     }
 }
 // Turns r[1 .. ncb] (lengths) into prefix sums with r[0] = 0; between barriers.
@@ -437,7 +440,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
     const double Snm = sel(hm, v.Snm), Ss = v.Ss, Ssp = sel(hp, v.Ssp);
     const double Kc = v.Kc, Kcm = sel(hm, v.Kcl), Ke = v.Ke, Kem = sel(hm, v.Kel), Kn = v.Kn, Knm = sel(hm, v.Knl);
     const double dzw_k = bm.lev.dzw[k], dzw_m = hm ? bm.lev.dzw[hm ? k - 1 : k] : 0.0;
-    const double r4zt = bm.lev.r4zt[k];
+    const double r4zt = bm.lev.r4zt[k], r4ztl = bm.lev.r4ztl[k];
 
     // reciprocal metric factors
     const double rz_c = hp ? bm.lev.rzw[k] : 0.0;
@@ -509,7 +512,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
         } else {
             Aez[4u * c + 3] = out[3];
         }
-        const double k11v = sumz * r4zt;
+        const double k11v = scaled(sumz, r4zt, r4ztl);
         K11[c] = k11v;
         if constexpr (FUSED) {
             // at level 0 the kr = 0 entries keep their values (their tracer
@@ -557,7 +560,7 @@ __device__ __forceinline__ void pre_wet_cell(const Grid& g, const Prm& p, const 
             Anz[4u * c + 1] = out[1];
             Anz[4u * c + 3] = out[3];
         }
-        const double k22v = sumz * r4zt;
+        const double k22v = scaled(sumz, r4zt, r4ztl);
         K22[c] = k22v;
         if constexpr (FUSED) {
             const double a0 = hm ? out[0] : Anz[4u * c], a2 = hm ? out[2] : Anz[4u * c + 2];
