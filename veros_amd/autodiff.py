@@ -203,6 +203,8 @@ def mixing_step(state, a, b, c, d, T_tau, K_iso, b_edge=None, d_edge=None, *, pr
     vs = state.variables
     a, b, c, d, b_edge, d_edge = _solve_operands(a, b, c, d, b_edge, d_edge)
     base = vs.temp[..., vs.taup1]
+    if isinstance(base, torch.Tensor) and not base.is_complex():
+        base = base.to(torch.float64)
     _check_step_inputs(state, T_tau=T_tau, T_taup1=base, K_iso=K_iso)
     X, Y, nz = K_iso.shape
     if tuple(a.shape) != (X - 4, Y - 4, nz):
