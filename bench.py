@@ -628,7 +628,8 @@ def main():
             "achieved": round(gbs[dom], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs[dom] / HBM_PEAK_GBS, 4),
             "traffic": traffic,
-            "traffic_source": "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes over this call on this workload "
+            "traffic_source": None if traffic is None else
+                              "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes over this call on this workload "
                               f"with the time levels {args.levels}most (read = 2.0 x FETCH_SIZE, write = 1.0 x "
                               "WRITE_SIZE, factors from a 1 GiB copy); profiles/mixing_step_1440x720x80.md",
             "algorithmic_bytes_per_launch": B8_step,
