@@ -36,15 +36,20 @@ struct SysDesc {
 // strides), with 16-byte copies straight into LDS, or each as its arrays allow.
 enum BatchKind { kFlat = 0, kCopies = 1, kEither = 2 };
 
-// Whether a bucket whose systems allow the copies in part takes them system by system, the
-// others with each lane's own loads, if at least half of the columns allow them: at 10 and
-// 12 levels per lane, where the copies win at any size (tdma_lds_wins) by more than those loads lose,
-// and up to 8 while all tiles are resident. Six systems of 300x200, one off alignment, all on
-// flat loads / by system, us, float64 and mixed: nz 80 165 and 182 / 163 and 164, 96 224 and 224 / 209
-// and 212, but 48 98 / 101, 64 125 / 140, 112 257 and 313 / 306 and 308, 128 278 and 300 / 367 and
-// 380. 22 systems of up to 66x66 and 18 to 85 levels: 30.4 / 30.0 and 29.7 / 29.3, with no
-// division before the loads (tdma_tile_of) 29.4 and 29.4.
-inline bool batch_either(int S, int64_t tiles) { return S == 10 || S == 12 || (S <= 8 && tdma_lds_resident(S, tiles)); }
+// Whether a bucket of which only the systems with vec_tiles of its tiles allow the copies
+// takes those system by system, the others with each lane's own loads, which lose against
+// the flat loads by more than the copies win. Six systems of one size, us, all on flat loads /
+// by system, float64 and mixed:
+//   resident tiles, 4 of 6 allowing: nz 32 1878 tiles 5.1 and 5.0 / 4.8 and 4.7; 48, 2700 8.3 and
+//   8.3 / 7.9 and 7.6; 64, 2274 9.1 and 9.1 / 8.8 and 8.7; 80, 1806 9.9 and 9.9 / 9.1 and 9.2; 96, 1392
+//   9.2 and 9.1 / 9.0 and 8.9. With 3 of 6: nz 64 9.2 / 11.6, 80 9.3 / 9.6. Fewer than two tiles per CU:
+//   nz 80, 432 5.6 / 5.9; more than 16: nz 32, 4686 8.5 / 8.9. 14 and 16 levels per lane: no difference.
+//   any size: nz 80, 67500 tiles, mixed, 5 of 6 257 / 241, 4 of 6 259 / 268; float64 235 / 240; nz 96 304 / 307.
+inline bool batch_either(int S, bool mixed, int64_t vec_tiles, int64_t tiles) {
+    const int64_t cus = cu_count();
+    if (S == 10 && mixed && 6 * vec_tiles >= 5 * tiles) return true;
+    return S <= 12 && 3 * vec_tiles >= 2 * tiles && tiles > 2 * cus && tiles <= 16 * cus && tdma_lds_resident(S, tiles);
+}
 
 // LDS doubles of a wave
 template <int S, int KIND>
@@ -257,7 +262,7 @@ extern "C" int vx_tdma_plan_create(const vx_tdma_system* systems, int32_t nsys, 
         const int S = b.nzb / kTdmaP;
         if (vec_tiles == b.tiles && (tdma_lds_wins(S, mode != 0, true) || tdma_lds_resident(S, b.tiles)))
             b.kind = kCopies;
-        else if (vec_tiles < b.tiles && 2 * vec_tiles >= b.tiles && batch_either(S, b.tiles))
+        else if (vec_tiles < b.tiles && batch_either(S, mode != 0, vec_tiles, b.tiles))
             b.kind = kEither;
         {
             std::lock_guard<std::mutex> lk(g_tune_mutex);
