@@ -30,7 +30,7 @@ HBM_PEAK_GBS = 8000.0
 # rocprofv3 passes recorded in profiles/mixing_step_1440x720x80.md (read bytes =
 # 2.0 x FETCH_SIZE, write bytes = 1.0 x WRITE_SIZE, calibrated on a 1 GiB device
 # copy); not measured with the levels innermost
-PRE_TS_TRAFFIC_BYTES = {(1440, 720, 80, "outer"): 21_926_504_320}
+PRE_TS_TRAFFIC_BYTES = {(1440, 720, 80, "outer"): 21_985_082_368}
 # the minimum bytes per interior cell of pre + the temperature + salinity step
 # in one call: K_iso read (8), Ai_* and K_11/22/33 written once and not read
 # back (128 + 24), P_diss read and written (16), and per tracer tr[tau] (8),

@@ -138,7 +138,7 @@ __device__ __forceinline__ void fric_face(const Tile<S, P>& t, double* img, int 
 // cell dissipates). Blocks are XCD-contiguous, strips fastest.
 //
 // A row's chain (kbot, the loads, the solve through LDS) is what bounds it, with
-// 5.1 GB on 1440x720x80 at 3.2 TB/s. What lies below the solve is loaded and stored
+// 5.1 GB on 1440x720x80 at 3.1 TB/s. What lies below the solve is loaded and stored
 // before it, so that no flat value but the operands lives across it. Blocks of
 // four waves: with eight, one block fills a CU's registers and nothing runs
 // while it waits at its barrier (2.22 -> 2.68 ms for the vertical step there).

@@ -78,7 +78,7 @@ __device__ __forceinline__ void vmix_rows(const VmixArgs& p, const double* __res
 // Column tiles (any layout, depth and alignment): a wave's columns are loaded
 // flat, the two tracers' old values stay with the lanes that loaded them, and
 // everything goes back flat. Bound by HBM: on 1440x720x80, levels outermost, 2.6 GB
-// in 0.59 ms (8 lanes per column with 16-byte copies into LDS: 0.60); 360x160x60,
+// in 0.60 ms (8 lanes per column with 16-byte copies into LDS: 0.60); 360x160x60,
 // levels innermost, 71 -> 46 us against each lane loading its own levels.
 constexpr int kVmixBlock = 128;
 template <int S, int P>
